@@ -3,10 +3,12 @@
 The local kernel comes in three tile families with identical results: voxel
 tiles (32x8x8, one union-find node per voxel, 256 threads; csrc/local.hpp),
 tall voxel tiles (32x16x8, 512 threads: fewer tile borders and a smaller halo
-per voxel for a larger LDS footprint) and row tiles (64x8x8, x-runs as nodes;
-csrc/rows.hpp).  Which is fastest depends on the connectivity, the voxel
-type, the volume's size and how much of it is foreground.  `tile_table.json`
-(next to this file) holds, per key
+per voxel for a larger LDS footprint) and row tiles (64x8x8, link bit masks
+of 16-voxel row segments; csrc/rows.hpp).  Which is fastest can depend on the
+connectivity, the voxel type, the volume's size and how much of it is
+foreground.  `tile_table.json`
+(next to this file; row tiles are the fastest family for every key it holds)
+has, per key
 
     connectivity / mode / voxel bytes / size class / density class
 
@@ -19,7 +21,7 @@ device volume (4096 evenly spaced voxels, one small reduction and a host
 synchronisation) only when the table's choice for that key depends on it and
 the best single family for the key would lose more than one sample costs on
 some density class; otherwise that family is used unsampled.  Keys missing
-from the table keep the default family (rows for 6, voxels otherwise).
+from the table take the library's default (rows).
 """
 from __future__ import annotations
 

@@ -29,6 +29,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/cc3d_amd.h"
@@ -155,12 +156,12 @@ __global__ __launch_bounds__(WG) void k_tile_counters(const TileCnt* tc, int64_t
 struct GlobalParams {
   int64_t sx, sy, sz, osx;
   int64_t ntx, nty, ntz, ntiles;
-  uint32_t* GP;
-  uint32_t* RL;
+  uint2* GP;
   const uint32_t* TR;
   const uint8_t* J8;
   const uint16_t* J16;
   const uint32_t* REQ;
+  int64_t reqcap;  // row tiles: requests per tile (16-bit entries)
   const uint32_t* TQ;
   uint32_t* bits;
   uint32_t* prefix;
@@ -252,8 +253,72 @@ __global__ __launch_bounds__(WG) void k_requests(GlobalParams p) {
       G::halo_coords(rq & 0xFFFF, bx, by, bz);
       const int64_t gx = x0 + bx - 1, gy = y0 + by - 1, gz = G::IS3D ? z0 + bz - 1 : 0;
       const uint32_t b = lroot_index<G>(p, v, gx, gy, gz);
-      if (b != 0xFFFFFFFFu) kunion(p.GP, p.RL, p.bits, a, b);
+      if (b != 0xFFFFFFFFu) kunion(p.GP, p.bits, a, b);
     }
+  }
+}
+
+// The same for row tiles, whose requests are (voxel position in the tile |
+// relation << 12): the forest entries of the two voxels, both foreground.
+// One wave per tile.  The links of a border join the same few pairs of local
+// roots again and again, so a wave drops the pairs that one of its lanes has
+// taken before: a table of the tile's pairs in LDS, and within the 64
+// requests of a round the lane that wrote a slot last stands for the others
+// with its pair.  A table slot that another pair took only costs a repeated
+// union.
+constexpr int RRQ_SLOTS = 256;
+__global__ __launch_bounds__(WG) void k_rrequests(GlobalParams p) {
+  using G = GeoR;
+  __shared__ uint2 tab[WG / 64][RRQ_SLOTS];
+  __shared__ uint32_t own[WG / 64][RRQ_SLOTS];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t w0 = (int64_t)blockIdx.x * (WG / 64) + wv;
+  const int64_t nw = (int64_t)gridDim.x * (WG / 64);
+  const uint16_t* REQ = reinterpret_cast<const uint16_t*>(p.REQ);
+  for (int64_t slot = w0; slot < p.ntiles; slot += nw) {
+    const uint32_t nq = p.TQ[slot];
+    if (nq == 0) continue;
+    const VolGeo v = vol_geo(p, slot);
+    const int64_t tile = slot - v.tile0;
+    const int64_t tz = tile / (v.ntx * v.nty);
+    const int64_t tr = tile - tz * v.ntx * v.nty;
+    const int64_t ty = tr / v.ntx, tx = tr - ty * v.ntx;
+    const uint32_t root0 = tile_root0<G>(v.sx, v.sy, v.sz, tx, ty, tz, v.key0);
+    const bool j8 = p.TR[slot] <= 255;
+#pragma unroll
+    for (int k = 0; k < RRQ_SLOTS / 64; k++) tab[wv][lane + 64 * k] = make_uint2(0xFFFFFFFFu, 0xFFFFFFFFu);
+    wave_order();
+    for (uint32_t i0 = 0; i0 < nq; i0 += 64) {
+      const uint32_t i = i0 + (uint32_t)lane;
+      uint32_t a = 0xFFFFFFFFu, b = 0xFFFFFFFFu;
+      if (i < nq) {
+        const uint32_t rq = REQ[slot * p.reqcap + i];
+        const int ps = (int)(rq & 0xFFFu);
+        const uint32_t j = j8 ? p.J8[slot * G::TV + ps] : p.J16[slot * G::TV + ps];
+        int dx, dy, dz;
+        rel_decode(rq >> 12, dx, dy, dz);
+        const int64_t gx = tx * G::TX + (ps & 63) + dx;
+        const int64_t gy = ty * G::TY + ((ps >> 6) & (G::TY - 1)) + dy;
+        const int64_t gz = tz * G::TZ + (ps >> 9) + dz;
+        b = lroot_index<G>(p, v, gx, gy, gz);
+        a = root0 + j - 1;
+      }
+      bool live = b != 0xFFFFFFFFu;
+      const uint32_t h = (((a * 0x9E3779B1u) ^ (b * 0x85EBCA77u)) >> 24) & (RRQ_SLOTS - 1);
+      if (live) {
+        const uint2 q = tab[wv][h];
+        live = q.x != a || q.y != b;
+      }
+      if (live) own[wv][h] = (uint32_t)lane;
+      wave_order();
+      const int o = live ? (int)own[wv][h] : lane;
+      const uint32_t oa = __shfl(a, o), ob = __shfl(b, o);
+      if (live && o != lane && oa == a && ob == b) live = false;
+      if (live) tab[wv][h] = make_uint2(a, b);
+      wave_order();
+      if (live) kunion(p.GP, p.bits, a, b);
+    }
+    wave_order();
   }
 }
 
@@ -360,7 +425,7 @@ __global__ __launch_bounds__(WG) void k_periodic(GlobalParams p, const T* in, in
     if (!link) continue;
     const VolGeo v = vol_geo(p, 0);
     const uint32_t ka = lroot_index<G>(p, v, ax, ay, az), kb = lroot_index<G>(p, v, bx, by, bz);
-    if (ka != 0xFFFFFFFFu && kb != 0xFFFFFFFFu) kunion(p.GP, p.RL, p.bits, ka, kb);
+    if (ka != 0xFFFFFFFFu && kb != 0xFFFFFFFFu) kunion(p.GP, p.bits, ka, kb);
   }
 }
 
@@ -577,7 +642,7 @@ __device__ inline void fin_load(const GlobalParams& p, int64_t slot, uint32_t ro
     }
   }
   lab[0] = 0u;
-  for (uint32_t i = t; i < R; i += WG) lab[i + 1] = root_label(p, kroot_key(p.GP, p.RL, root0 + i), base);
+  for (uint32_t i = t; i < R; i += WG) lab[i + 1] = root_label(p, kroot_key(p.GP, root0 + i), base);
 }
 
 // Thread t's EPT output voxels of tile `tile` of volume v (after a barrier
@@ -662,57 +727,65 @@ hipError_t scan_root_bits(const uint32_t* bits, int64_t nwords, uint32_t* bsum, 
   return hipGetLastError();
 }
 
-// Row tiles (GeoR): one workgroup per tile; thread t owns J entries
-// 16t .. 16t + 15, i.e. 16 consecutive voxels of one row, loaded with one
-// (J8) or two (J16) 16-byte loads and written as one contiguous run.
-constexpr int RFIN_PT = GeoR::TV / WG;
-static_assert(RFIN_PT == 16, "16 voxels per thread");
-
+// Row tiles (GeoR): one workgroup per tile.  In pass i thread t takes the 4
+// voxels at x = 4 (t & 15) of row 16 i + (t >> 4): 16 lanes read and write
+// one row, so a wave's stores cover whole 256-byte rows (uint32 labels) at
+// any row alignment.  All loads of the passes come before the label table's
+// barrier.  Rows that start on a 128-byte line are written past the caches
+// (512^3 uint32: 179 -> 166 us, with one component 148 -> 110 us); other rows
+// share lines with their neighbours and are merged in L2 instead (383 x 401 x
+// 367: 62 us, 105 us past the caches).
 template <class OUT>
 __device__ inline void rfin_tile(const GlobalParams& p, const VolGeo& v, int64_t tile, int64_t slot, uint32_t base,
                                  OUT* __restrict__ out, uint32_t* lab) {
+  constexpr int PASSES = GeoR::TV / (4 * WG);
   const int t = threadIdx.x;
   const uint32_t R = p.TR[slot];
-  uint32_t j[RFIN_PT];
+  uint32_t j[PASSES][2];  // two 16-bit entries per word
   if (R <= 255) {
-    const uint4 w = reinterpret_cast<const uint4*>(p.J8 + slot * GeoR::TV)[t];
-    const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
-    for (int k = 0; k < RFIN_PT; k++) j[k] = (ws[k >> 2] >> (8 * (k & 3))) & 0xFFu;
-  } else {
-    const uint4 w0 = reinterpret_cast<const uint4*>(p.J16 + slot * GeoR::TV)[2 * t];
-    const uint4 w1 = reinterpret_cast<const uint4*>(p.J16 + slot * GeoR::TV)[2 * t + 1];
-    const uint32_t ws[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-#pragma unroll
-    for (int k = 0; k < RFIN_PT; k++) j[k] = (ws[k >> 1] >> (16 * (k & 1))) & 0xFFFFu;
-  }
-  const uint32_t root0 = slot_root0<GeoR>(v, slot);
-  if (t == 0) lab[0] = 0u;
-  for (uint32_t i = t; i < R; i += WG) lab[i + 1] = root_label(p, kroot_key(p.GP, p.RL, root0 + i), base);
-  __syncthreads();
-  const int e0 = RFIN_PT * t;
-  const int lx = e0 & 63, ly = (e0 >> 6) & (GeoR::TY - 1), lz = e0 >> 9;
-  const int64_t tz = tile / (v.ntx * v.nty);
-  const int64_t tr = tile - tz * v.ntx * v.nty;
-  const int64_t ty = tr / v.ntx, tx = tr - ty * v.ntx;
-  const int64_t gx = tx * GeoR::TX + lx, gy = ty * GeoR::TY + ly, gz = tz * GeoR::TZ + lz;
-  if (gy >= v.sy || gz >= v.sz || gx >= v.sx) return;
-  OUT* o = out + gx + v.sx * (gy + v.sy * gz);
-  OUT vals[RFIN_PT];
-#pragma unroll
-  for (int k = 0; k < RFIN_PT; k++) vals[k] = (OUT)lab[j[k]];
-  if (gx + RFIN_PT <= v.sx && (reinterpret_cast<uintptr_t>(o) & 15) == 0) {
-    constexpr int NV = RFIN_PT * (int)sizeof(OUT) / 16;
-#pragma unroll
-    for (int i = 0; i < NV; i++) {
-      uint4 w;
-      __builtin_memcpy(&w, reinterpret_cast<const char*>(vals) + 16 * i, 16);
-      reinterpret_cast<uint4*>(o)[i] = w;
+    for (int i = 0; i < PASSES; i++) {
+      const uint32_t w = reinterpret_cast<const uint32_t*>(p.J8 + slot * GeoR::TV)[t + WG * i];
+      j[i][0] = (w & 0xFFu) | ((w & 0xFF00u) << 8);
+      j[i][1] = ((w >> 16) & 0xFFu) | ((w >> 8) & 0xFF0000u);
     }
   } else {
 #pragma unroll
-    for (int k = 0; k < RFIN_PT; k++)
-      if (gx + k < v.sx) o[k] = vals[k];
+    for (int i = 0; i < PASSES; i++) {
+      const uint2 w = reinterpret_cast<const uint2*>(p.J16 + slot * GeoR::TV)[t + WG * i];
+      j[i][0] = w.x;
+      j[i][1] = w.y;
+    }
+  }
+  const uint32_t root0 = slot_root0<GeoR>(v, slot);
+  if (t == 0) lab[0] = 0u;
+  for (uint32_t i = t; i < R; i += WG) lab[i + 1] = root_label(p, kroot_key(p.GP, root0 + i), base);
+  __syncthreads();
+  const int64_t tz = tile / (v.ntx * v.nty);
+  const int64_t tr = tile - tz * v.ntx * v.nty;
+  const int64_t ty = tr / v.ntx, tx = tr - ty * v.ntx;
+  const int64_t gx = tx * GeoR::TX + 4 * (t & 15);
+  typedef OUT Pack __attribute__((ext_vector_type(4), aligned(sizeof(OUT))));
+  const bool whole = ((uint64_t)v.sx * sizeof(OUT) % 128 | reinterpret_cast<uintptr_t>(out) % 128) == 0;
+#pragma unroll
+  for (int i = 0; i < PASSES; i++) {
+    const int row = 16 * i + (t >> 4);
+    const int64_t gy = ty * GeoR::TY + (row & (GeoR::TY - 1)), gz = tz * GeoR::TZ + row / GeoR::TY;
+    Pack k;
+    k[0] = (OUT)lab[j[i][0] & 0xFFFFu];
+    k[1] = (OUT)lab[j[i][0] >> 16];
+    k[2] = (OUT)lab[j[i][1] & 0xFFFFu];
+    k[3] = (OUT)lab[j[i][1] >> 16];
+    if (gx >= v.sx || gy >= v.sy || gz >= v.sz) continue;
+    OUT* o = out + gx + v.sx * (gy + v.sy * gz);
+    if (gx + 4 <= v.sx) {
+      if (whole) __builtin_nontemporal_store(k, reinterpret_cast<Pack*>(o));
+      else *reinterpret_cast<Pack*>(o) = k;
+    } else {
+#pragma unroll
+      for (int q = 0; q < 3; q++)
+        if (gx + q < v.sx) o[q] = k[q];
+    }
   }
 }
 
@@ -1186,10 +1259,12 @@ struct Geometry {
   bool rows = false;  // row tiles (GeoR): 3D multilabel and binary
   bool tall = false;  // tall voxel tiles (Geo3T) instead of Geo3
   int64_t ntx = 0, nty = 0, ntz = 0, ntiles = 0;
-  int TV = 0, HALO = 0;
+  int TV = 0;
+  size_t req_bytes = 0;  // request storage of one tile
+  int64_t reqcap = 0;    // row tiles: requests in it
   int64_t nwords = 0, nblk = 0;
   int64_t qblocks = 0, qwords = 0, qnblk = 0;  // binary 2D-8 block bitmask
-  size_t oGP, oRL, oTR, oTQ, oTC, oJ8, oJ16, oREQ, oBITS, oPRE, oBSUM, oCTR, oMM, oQB, oQP, oQS, total;
+  size_t oGP, oTR, oTQ, oTC, oJ8, oJ16, oREQ, oBITS, oPRE, oBSUM, oCTR, oMM, oQB, oQP, oQS, total;
 };
 
 // tiles: CC3D_AMD_TILES_ROWS / _VOXELS / _TALL bits (else the default family)
@@ -1221,21 +1296,23 @@ static int plan(Geometry& g, int64_t sx, int64_t sy, int64_t sz, int64_t connect
   if (g.K >= 0xFFFFFFFFll || g.V >= 0xFFFFFFFFll)
     return fail(CC3D_AMD_ERR_INVALID, "volumes of 2^32-1 voxels or more are not supported");
   int TX, TY, TZ;
-  // Row tiles for 6-connected 3D volumes (multilabel or binary): measured
-  // faster there than the voxel tiles; the voxel tiles stay faster at 26/18.
+  // Row tiles for 3D multilabel and binary volumes.
   g.rows = g.is3d && g.mode != M_CONT &&
-           ((tiles & CC3D_AMD_TILES_ROWS)                            ? true
-            : (tiles & (CC3D_AMD_TILES_VOXELS | CC3D_AMD_TILES_TALL)) ? false
-                                                                      : connectivity == 6);
+           ((tiles & CC3D_AMD_TILES_ROWS) || !(tiles & (CC3D_AMD_TILES_VOXELS | CC3D_AMD_TILES_TALL)));
   g.tall = g.is3d && !g.rows && (tiles & CC3D_AMD_TILES_TALL) && !(tiles & CC3D_AMD_TILES_VOXELS);
   if (g.rows) {
-    TX = GeoR::TX; TY = GeoR::TY; TZ = GeoR::TZ; g.TV = GeoR::TV; g.HALO = GeoR::HALO;
+    TX = GeoR::TX; TY = GeoR::TY; TZ = GeoR::TZ; g.TV = GeoR::TV;
+    g.reqcap = row_req_cap(g.mode == M_CONT, g.nb);
+    g.req_bytes = (size_t)g.reqcap * sizeof(uint16_t);
   } else if (g.tall) {
-    TX = Geo3T::TX; TY = Geo3T::TY; TZ = Geo3T::TZ; g.TV = Geo3T::TV; g.HALO = Geo3T::HALO;
+    TX = Geo3T::TX; TY = Geo3T::TY; TZ = Geo3T::TZ; g.TV = Geo3T::TV;
+    g.req_bytes = (size_t)Geo3T::HALO * 4;
   } else if (g.is3d) {
-    TX = Geo3::TX; TY = Geo3::TY; TZ = Geo3::TZ; g.TV = Geo3::TV; g.HALO = Geo3::HALO;
+    TX = Geo3::TX; TY = Geo3::TY; TZ = Geo3::TZ; g.TV = Geo3::TV;
+    g.req_bytes = (size_t)Geo3::HALO * 4;
   } else {
-    TX = Geo2::TX; TY = Geo2::TY; TZ = 1; g.TV = Geo2::TV; g.HALO = Geo2::HALO;
+    TX = Geo2::TX; TY = Geo2::TY; TZ = 1; g.TV = Geo2::TV;
+    g.req_bytes = (size_t)Geo2::HALO * 4;
   }
   g.ntx = (sx + TX - 1) / TX;
   g.nty = (sy + TY - 1) / TY;
@@ -1255,14 +1332,13 @@ static int plan(Geometry& g, int64_t sx, int64_t sy, int64_t sz, int64_t connect
     return r;
   };
   const size_t slots = (size_t)g.ntiles * g.TV;
-  g.oGP = take((size_t)g.K * 4);
-  g.oRL = take((size_t)g.K * 4);
+  g.oGP = take((size_t)g.K * sizeof(uint2));
   g.oTR = take((size_t)g.ntiles * 4);
   g.oTQ = take((size_t)g.ntiles * 4);
   g.oTC = take((size_t)g.ntiles * sizeof(TileCnt));
   g.oJ8 = take(slots);
   g.oJ16 = take(slots * 2);
-  g.oREQ = take((size_t)g.ntiles * g.HALO * 4);
+  g.oREQ = take((size_t)g.ntiles * g.req_bytes);
   g.oBITS = take((size_t)g.nwords * 4);
   g.oPRE = take((size_t)g.nwords * 4);
   g.oBSUM = take((size_t)(g.nblk + 1) * 4);
@@ -1308,7 +1384,7 @@ struct cc3d_amd_batch {
   bool own_ws = false;
   size_t total = 0;
   int64_t ntiles = 0, nkeys = 0, nwords = 0, nblk = 0;
-  size_t oVOL = 0, oGP = 0, oRL = 0, oBITS = 0, oPRE = 0, oBSUM = 0, oCTR = 0;
+  size_t oVOL = 0, oGP = 0, oBITS = 0, oPRE = 0, oBSUM = 0, oCTR = 0;
   BatchVol* h_tab = nullptr;  // pinned host copy of the volume table
   int64_t* h_t0 = nullptr;    // pinned: first tile of each volume, per tile group (n + tile groups)
   Counters* h_ctr = nullptr;  // pinned: entry 0 whole batch, 1 + k table entry k
@@ -1329,6 +1405,7 @@ struct cc3d_amd_batch {
     bool rows() const { return fam == FAM_ROWS; }
     int v0 = 0, v1 = 0;  // table entries
     int64_t tiles = 0;
+    int64_t reqcap = 0;  // row tiles: requests per tile, for the group's largest neighbourhood
     size_t oT0 = 0, oVIX = 0, oTR = 0, oTQ = 0, oTC = 0, oJ8 = 0, oJ16 = 0, oREQ = 0;
     GlobalParams gp{};
     LocalParams lp{};
@@ -1379,13 +1456,18 @@ void launch_requests(const GlobalParams& p, int64_t ntiles, int mode, hipStream_
   else hipLaunchKernelGGL((k_requests<G, QK, 8>), dim3(grid_for(ntiles, WG / 8, 65536)), dim3(WG), 0, s, p);
 }
 
+void launch_rrequests(const GlobalParams& p, int64_t ntiles, hipStream_t s) {
+  hipLaunchKernelGGL(k_rrequests, dim3(grid_for(ntiles, WG / 64, 65536)), dim3(WG), 0, s, p);
+}
+
 template <class G>
 int run_global(cc3d_amd_job* j) {
   const GlobalParams& p = j->gp;
   hipStream_t s = j->stream;
   {
   ProfScope ps_("k_requests", s);
-  if (j->g.qk == Q_BLOCK8) launch_requests<G, Q_BLOCK8>(p, j->g.ntiles, j->g.mode, s);
+  if constexpr (std::is_same<G, GeoR>::value) launch_rrequests(p, j->g.ntiles, s);
+  else if (j->g.qk == Q_BLOCK8) launch_requests<G, Q_BLOCK8>(p, j->g.ntiles, j->g.mode, s);
   else launch_requests<G, Q_NONE>(p, j->g.ntiles, j->g.mode, s);
   }
   HIPCHECK(hipGetLastError());
@@ -1653,12 +1735,12 @@ static int job_begin(cc3d_amd_job* j, const void* in, int in_dtype, int64_t sx, 
   GlobalParams& gp = j->gp;
   gp.sx = g.sx; gp.sy = g.sy; gp.sz = g.sz; gp.osx = g.osx;
   gp.ntx = g.ntx; gp.nty = g.nty; gp.ntz = g.ntz; gp.ntiles = g.ntiles;
-  gp.GP = reinterpret_cast<uint32_t*>(ws + g.oGP);
-  gp.RL = reinterpret_cast<uint32_t*>(ws + g.oRL);
+  gp.GP = reinterpret_cast<uint2*>(ws + g.oGP);
   gp.TR = reinterpret_cast<uint32_t*>(ws + g.oTR);
   gp.J8 = reinterpret_cast<uint8_t*>(ws + g.oJ8);
   gp.J16 = reinterpret_cast<uint16_t*>(ws + g.oJ16);
   gp.REQ = reinterpret_cast<uint32_t*>(ws + g.oREQ);
+  gp.reqcap = g.reqcap;
   gp.TQ = reinterpret_cast<uint32_t*>(ws + g.oTQ);
   gp.bits = reinterpret_cast<uint32_t*>(ws + g.oBITS);
   gp.prefix = reinterpret_cast<uint32_t*>(ws + g.oPRE);
@@ -1713,12 +1795,12 @@ static int job_begin(cc3d_amd_job* j, const void* in, int in_dtype, int64_t sx, 
   lp.delta_bits = j->delta_bits;
   lp.minmax = reinterpret_cast<const uint64_t*>(mm);
   lp.GP = gp.GP;
-  lp.RL = gp.RL;
   lp.bits = gp.bits;
   lp.TR = reinterpret_cast<uint32_t*>(ws + g.oTR);
   lp.J8 = reinterpret_cast<uint8_t*>(ws + g.oJ8);
   lp.J16 = reinterpret_cast<uint16_t*>(ws + g.oJ16);
   lp.REQ = reinterpret_cast<uint32_t*>(ws + g.oREQ);
+  lp.reqcap = g.reqcap;
   lp.TQ = reinterpret_cast<uint32_t*>(ws + g.oTQ);
   lp.tcnt = reinterpret_cast<TileCnt*>(ws + g.oTC);
   hipError_t e;
@@ -1891,7 +1973,8 @@ uint64_t cc3d_amd_union_find_length(int64_t max_labels, int64_t voxels, int64_t 
 // (the job lives on the stack and its workspace is `scratch`).
 static int cc_core(const void* in, int in_dtype, int64_t sx, int64_t sy, int64_t sz, int64_t max_labels,
                    int64_t connectivity, const void* delta, void* out, int out_dtype, uint64_t* N,
-                   int periodic_boundary, int binary_image, void* stream, char* scratch, size_t scratch_bytes) {
+                   int periodic_boundary, int binary_image, void* stream, char* scratch, size_t scratch_bytes,
+                   int tiles) {
   if (!out || !N) return fail(CC3D_AMD_ERR_INVALID, "NULL output");
   if (out_dtype != DT_U16 && out_dtype != DT_U32 && out_dtype != DT_U64)
     return fail(CC3D_AMD_ERR_INVALID, "output dtype must be uint16, uint32 or uint64");
@@ -1922,7 +2005,7 @@ static int cc_core(const void* in, int in_dtype, int64_t sx, int64_t sy, int64_t
     return CC3D_AMD_OK;
   }
   const bool b8 = binary_image && connectivity == 8 && sz == 1;
-  int flags = (continuous ? CC3D_AMD_CONTINUOUS : 0) | CC3D_AMD_NO_SINGLE_ROW_RULE;
+  int flags = (continuous ? CC3D_AMD_CONTINUOUS : 0) | CC3D_AMD_NO_SINGLE_ROW_RULE | tiles;
   if (b8 && (uint64_t)(((sx + 1) >> 1) * ((sy + 1) >> 1)) >= L) flags |= CC3D_AMD_COUNT_PROVISIONAL;
   cc3d_amd_job local_job;
   cc3d_amd_job* j = scratch ? &local_job : new cc3d_amd_job();
@@ -1952,7 +2035,7 @@ int cc3d_amd_connected_components3d(const void* in, int in_dtype, int64_t sx, in
                                     int out_dtype, uint64_t* N, int periodic_boundary, int binary_image,
                                     void* stream) {
   return cc_core(in, in_dtype, sx, sy, sz, max_labels, connectivity, delta, out, out_dtype, N, periodic_boundary,
-                 binary_image, stream, nullptr, 0);
+                 binary_image, stream, nullptr, 0, 0);
 }
 
 int cc3d_amd_connected_components3d_noalloc(const void* in, int in_dtype, int64_t sx, int64_t sy, int64_t sz,
@@ -1963,8 +2046,14 @@ int cc3d_amd_connected_components3d_noalloc(const void* in, int in_dtype, int64_
   uint64_t db = 0;
   delta_bits_of(in_dtype, delta, db);
   const bool continuous = !binary_image && !delta_is_zero(in_dtype, db);
-  if (sx > 0 && sy > 0 && sz > 0 && plan(g, sx, sy, sz, connectivity, binary_image, continuous) == CC3D_AMD_OK &&
-      g.total > CC3D_AMD_NOALLOC_SCRATCH_BYTES)
+  auto too_large = [&](int tiles) {
+    return sx > 0 && sy > 0 && sz > 0 &&
+           plan(g, sx, sy, sz, connectivity, binary_image, continuous, tiles) == CC3D_AMD_OK &&
+           g.total > CC3D_AMD_NOALLOC_SCRATCH_BYTES;
+  };
+  // volumes of ragged sides near the limit fit on the smaller voxel tiles only
+  const int tiles = too_large(0) ? CC3D_AMD_TILES_VOXELS : 0;
+  if (tiles && too_large(tiles))
     return fail(CC3D_AMD_ERR_INVALID, "cc3d_amd_connected_components3d_noalloc: the volume needs " +
                                           std::to_string(g.total) + " bytes of scratch; the limit is " +
                                           std::to_string((unsigned long long)CC3D_AMD_NOALLOC_SCRATCH_BYTES));
@@ -1975,7 +2064,7 @@ int cc3d_amd_connected_components3d_noalloc(const void* in, int in_dtype, int64_
   const bool was_suspended = g_prof_suspended;
   g_prof_suspended = true;
   rc = cc_core(in, in_dtype, sx, sy, sz, max_labels, connectivity, delta, out, out_dtype, N, periodic_boundary,
-               binary_image, stream, ptr, CC3D_AMD_NOALLOC_SCRATCH_BYTES);
+               binary_image, stream, ptr, CC3D_AMD_NOALLOC_SCRATCH_BYTES, tiles);
   g_prof_suspended = was_suspended;
   return rc;
 }
@@ -2073,14 +2162,14 @@ static int batch_layout(const cc3d_amd_volume* vols, int n, int mode, std::vecto
     }
     nbs[i] = nb;
     // the single-volume path's choice (plan): rows unless continuous, then
-    // voxels, then tall; by default rows at 6-connectivity, else voxels
+    // voxels, then tall; by default rows, voxels if continuous
     const int pref = (int)((v.connectivity >> 8) & 0xFF);
     const bool cont = mode == CC3D_AMD_BATCH_CONTINUOUS;
     famv[i] = qks[i] != Q_NONE                           ? cc3d_amd_batch::FAM_PLANE
               : (!cont && (pref & CC3D_AMD_TILES_ROWS))  ? cc3d_amd_batch::FAM_ROWS
               : (pref & CC3D_AMD_TILES_VOXELS)          ? cc3d_amd_batch::FAM_VOXELS
               : (pref & CC3D_AMD_TILES_TALL)            ? cc3d_amd_batch::FAM_TALL
-              : (!cont && nb == 6)                      ? cc3d_amd_batch::FAM_ROWS
+              : !cont                                   ? cc3d_amd_batch::FAM_ROWS
                                                         : cc3d_amd_batch::FAM_VOXELS;
     b.perm[i] = i;
   }
@@ -2165,8 +2254,7 @@ static int batch_layout(const cc3d_amd_volume* vols, int n, int mode, std::vecto
     return r;
   };
   b.oVOL = take((size_t)n * sizeof(BatchVol));
-  b.oGP = take((size_t)b.nkeys * 4);
-  b.oRL = take((size_t)b.nkeys * 4);
+  b.oGP = take((size_t)b.nkeys * sizeof(uint2));
   b.oBITS = take((size_t)b.nwords * 4);
   b.oPRE = take((size_t)b.nwords * 4);
   b.oBSUM = take((size_t)(b.nblk + 1) * 4);
@@ -2175,10 +2263,13 @@ static int batch_layout(const cc3d_amd_volume* vols, int n, int mode, std::vecto
     int TXg, TYg, TZg;
     batch_tile_dims(tg.fam, TXg, TYg, TZg);
     const size_t TVg = (size_t)TXg * TYg * TZg;
-    const size_t HALOg = tg.rows()                              ? GeoR::HALO
-                         : tg.fam == cc3d_amd_batch::FAM_TALL  ? Geo3T::HALO
-                         : tg.fam == cc3d_amd_batch::FAM_PLANE ? Geo2::HALO
-                                                               : Geo3::HALO;
+    tg.reqcap = 0;
+    for (int k = tg.v0; tg.rows() && k < tg.v1; k++)
+      tg.reqcap = std::max<int64_t>(tg.reqcap, row_req_cap(mode == CC3D_AMD_BATCH_CONTINUOUS, tab[k].nb));
+    const size_t req_bytes = tg.rows() ? (size_t)tg.reqcap * sizeof(uint16_t)
+                             : tg.fam == cc3d_amd_batch::FAM_TALL  ? (size_t)Geo3T::HALO * 4
+                             : tg.fam == cc3d_amd_batch::FAM_PLANE ? (size_t)Geo2::HALO * 4
+                                                                   : (size_t)Geo3::HALO * 4;
     const size_t slots = (size_t)tg.tiles * TVg;
     tg.oT0 = take((size_t)(tg.v1 - tg.v0 + 1) * sizeof(int64_t));
     tg.oVIX = take((size_t)tg.tiles * 4);
@@ -2187,7 +2278,7 @@ static int batch_layout(const cc3d_amd_volume* vols, int n, int mode, std::vecto
     tg.oTC = take((size_t)tg.tiles * sizeof(TileCnt));
     tg.oJ8 = take(slots);
     tg.oJ16 = take(slots * 2);
-    tg.oREQ = take((size_t)tg.tiles * HALOg * 4);
+    tg.oREQ = take((size_t)tg.tiles * req_bytes);
   }
   for (auto& m : b.minmax) m.oMM = take(64);  // {min, max} and the last NaN index
   for (auto& st : b.stale) {
@@ -2259,7 +2350,7 @@ int cc3d_amd_batch_create(cc3d_amd_batch** out_batch, const cc3d_amd_volume* vol
     return fail(CC3D_AMD_ERR_HIP, "could not upload the batch table");
   }
   GlobalParams& gp = b->gp;
-  gp.GP = reinterpret_cast<uint32_t*>(ws + b->oGP);
+  gp.GP = reinterpret_cast<uint2*>(ws + b->oGP);
   gp.bits = reinterpret_cast<uint32_t*>(ws + b->oBITS);
   gp.prefix = reinterpret_cast<uint32_t*>(ws + b->oPRE);
   gp.bsum = reinterpret_cast<uint32_t*>(ws + b->oBSUM);
@@ -2280,11 +2371,11 @@ int cc3d_amd_batch_create(cc3d_amd_batch** out_batch, const cc3d_amd_volume* vol
     GlobalParams& q = tg.gp;
     q = gp;
     q.ntiles = tg.tiles;
-    q.RL = reinterpret_cast<uint32_t*>(ws + b->oRL);
     q.TR = reinterpret_cast<uint32_t*>(ws + tg.oTR);
     q.J8 = reinterpret_cast<uint8_t*>(ws + tg.oJ8);
     q.J16 = reinterpret_cast<uint16_t*>(ws + tg.oJ16);
     q.REQ = reinterpret_cast<uint32_t*>(ws + tg.oREQ);
+    q.reqcap = tg.reqcap;
     q.TQ = reinterpret_cast<uint32_t*>(ws + tg.oTQ);
     q.vols = gp.vols + tg.v0;
     q.vtile0 = reinterpret_cast<const int64_t*>(ws + tg.oT0);
@@ -2302,12 +2393,12 @@ int cc3d_amd_batch_create(cc3d_amd_batch** out_batch, const cc3d_amd_volume* vol
     lp.delta_bits = 0;
     lp.minmax = nullptr;
     lp.GP = gp.GP;
-    lp.RL = q.RL;
     lp.bits = gp.bits;
     lp.TR = reinterpret_cast<uint32_t*>(ws + tg.oTR);
     lp.J8 = reinterpret_cast<uint8_t*>(ws + tg.oJ8);
     lp.J16 = reinterpret_cast<uint16_t*>(ws + tg.oJ16);
     lp.REQ = reinterpret_cast<uint32_t*>(ws + tg.oREQ);
+    lp.reqcap = tg.reqcap;
     lp.TQ = reinterpret_cast<uint32_t*>(ws + tg.oTQ);
     lp.tcnt = reinterpret_cast<TileCnt*>(ws + tg.oTC);
     need_utab = need_utab || !tg.rows();
@@ -2414,7 +2505,7 @@ int cc3d_amd_batch_begin(cc3d_amd_batch* b) {
   {
     ProfScope ps_("k_requests", s);
     for (const auto& tg : b->tgroups) {
-      if (tg.rows()) launch_requests<GeoR, Q_NONE>(tg.gp, tg.tiles, b->mode, s);
+      if (tg.rows()) launch_rrequests(tg.gp, tg.tiles, s);
       else if (tg.fam == cc3d_amd_batch::FAM_TALL) launch_requests<Geo3T, Q_NONE>(tg.gp, tg.tiles, b->mode, s);
       else if (tg.fam == cc3d_amd_batch::FAM_PLANE) launch_requests<Geo2, Q_NONE>(tg.gp, tg.tiles, b->mode, s);
       else launch_requests<Geo3, Q_NONE>(tg.gp, tg.tiles, b->mode, s);

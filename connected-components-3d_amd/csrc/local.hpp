@@ -38,12 +38,11 @@
 // common.hpp), so tiles never lean on each other's cross-tile links.
 //
 // Outputs per tile:
-//   RL[root0 + r]    global key of local root r (root0 = tile_root0)
 //   TR[tile]         number of local roots R
 //   J8/J16           per voxel (thread-major: thread t's column is entries
 //                    8t..8t+7): 0 (background) or 1 + index of its local root;
 //                    8-bit when R <= 255, else 16-bit
-//   GP[root0 + r]    initialised to itself for every local root
+//   GP[root0 + r]    {itself, its global key} for every local root r (root0 = tile_root0)
 //   bits             bit (key) set for every local root's key (kunion clears
 //                    those of the roots it buries)
 //   REQ/TQ           cross-tile union requests: (root index r, halo index)
@@ -66,13 +65,13 @@ struct LocalParams {
   int64_t ntx, nty, ntz, ntiles;
   uint64_t delta_bits;
   const uint64_t* minmax;  // Q_CONT8: global {min, max} bit patterns
-  uint32_t* GP;
-  uint32_t* RL;
+  uint2* GP;       // {parent, key} per local root
   uint32_t* bits;  // root bitmask over keys, cleared beforehand
   uint32_t* TR;
   uint8_t* J8;
   uint16_t* J16;
   uint32_t* REQ;
+  int64_t reqcap;        // row tiles: requests per tile (16-bit entries)
   uint32_t* TQ;
   TileCnt* tcnt;
   const uint16_t* utab;  // union tables (UTab), UTAB_TOTAL entries
@@ -437,7 +436,7 @@ struct LocalLds {
 };
 
 // Labels tile `tile` of the volume described by p.  Per-tile outputs go to
-// index `slot` of RL/J/REQ/TR/TQ/tcnt; keys are offset by `keybase` (both
+// index `slot` of J/REQ/TR/TQ/tcnt; keys are offset by `keybase` (both
 // are `tile` and 0 for a single volume; a batch concatenates volumes).
 //
 // Union-find nodes are box positions numbered in global key order (tile and
@@ -1084,7 +1083,6 @@ __device__ inline void local_tile(const LocalParams& p, int64_t tile, int64_t sl
     return L.late.rprefix[r >> 5] + (uint32_t)__popc(L.w.rbits[r >> 5] & ((1u << (r & 31)) - 1u));
   };
   const uint32_t root0 = tile_root0<G>(sx, sy, sz, tx, ty, tz, keybase);
-  uint32_t* RLt = p.RL + root0;
   // Keys are below 2^32, so they can be formed in 32-bit arithmetic: the
   // wrap-around of the intermediate terms cancels.  Box position (bx, by, bz)
   // is voxel (x0 + bx - 1, y0 + by - 1, z0 + bz - 1).
@@ -1104,8 +1102,8 @@ __device__ inline void local_tile(const LocalParams& p, int64_t tile, int64_t sl
         key = kbox0 + (uint32_t)bx + (uint32_t)sx * ((uint32_t)by + (uint32_t)sy * (uint32_t)bz) + keybase;
       else
         key = kbox0 + (uint32_t)sx * (uint32_t)sy + (uint32_t)bx + (uint32_t)sx * (uint32_t)by + keybase;
-      p.GP[root0 + rk] = root0 + rk;
-      RLt[rk++] = key;
+      p.GP[root0 + rk] = make_uint2(root0 + rk, key);
+      rk++;
       atomicOr(p.bits + (key >> 5), 1u << (key & 31));
     }
   }

@@ -1,36 +1,46 @@
-// Row kernel: local labelling of 3D multilabel and binary volumes
-// (connectivity 26, 18, 6) with one voxel per lane.
+// Row kernel: local labelling of multilabel, binary and continuous volumes on
+// link bit masks, one 16-voxel row segment per lane.
 //
 // Replaces the first raster pass of the reference for these paths
-// (cc3d/cc3d.hpp:344-1076, cc3d/cc3d_binary.hpp:31-761).  The tile is
-// 64 x 8 x 8 voxels; a 512-thread workgroup gives one wave to each z-plane,
-// and a lane to each x.  A row (64 voxels along x) is handled with 64-bit
-// lane masks:
+// (cc3d/cc3d.hpp:344-1076, cc3d/cc3d_binary.hpp:31-761,
+// cc3d/cc3d_continuous.hpp:90-296).  The tile is 64 x 8 x 8 voxels, 64 rows
+// of 64; a 256-thread workgroup gives every lane one row and every wave one
+// 16-voxel segment of all rows.  A lane reads its own row and the four
+// backward rows its connectivity reaches (B: y-1; C, D, E: z-1 at y, y-1,
+// y+1) from the tile staged in LDS and holds, per relation p -> q, one bit
+// for each voxel of the segment:
 //
-//   F      foreground                       (v != 0)
-//   S      run starts: foreground voxels not equal (multilabel) / not linked
-//          (binary) to the voxel before them in the row; lane 0 always starts
-//          a run, so runs never leave the tile
-//   E_d    links of the row to a backward row r' at x + d, d in {-1, 0, +1}
-//          (equal values / both foreground), from DPP-shifted copies of r'
-//          whose shifted-in lane is the x-halo voxel of r'
+//   F            foreground
+//   a            linked to the voxel before it in the row
+//   b0 bm bp     linked to (x, y-1, z), (x-1, y-1, z), (x+1, y-1, z); the
+//   c* d* e*     same for the rows C, D, E
 //
-// Union-find nodes are the runs (identified by their first voxel) and the
-// halo nodes: runs of the halo rows and the x-halo voxels.  Node ids are box
-// positions (bx, by, bz) = (x + 1, y + 1, z + 1) in raster order, which is
-// global key order, so every tree is rooted at its member with the smallest
-// key.  A run makes one union with each run of r' it touches: at the first
-// voxel of each maximal E_0 interval inside it (U0), and through the
-// diagonals only where nothing else joins the two runs -- at its first voxel
-// for d = -1 (Um) and at its last voxel for d = +1 (Up).  Unions are appended
-// to a per-wave queue in LDS and made 64 at a time, one per lane.
+// multilabel: a bit is one compare and one add-with-carry (push_*), which
+// shifts the condition into the mask: 2 VALU operations per voxel and
+// relation.  binary: the segments are staged as foreground bits and every
+// relation is a shift and an AND.
 //
-// Halo pieces (halo nodes connected through links inside one neighbouring
-// tile) are unioned first, and their roots recorded; after the tile's own
-// unions each piece whose tree holds tile voxels makes one cross-tile request
-// (root index, piece node), resolved by the global kernels.  Outputs (RL, TR,
-// J8/J16, GP, REQ/TQ, tcnt) have the same meaning as those of the voxel
-// kernel in local.hpp; J is row-major: entry x + 64 * (y + 8 * z).
+// A link is dropped when another one covers it: p's link to q is implied by
+// a linked backward neighbour r of p that is taken before q in the order a,
+// c0, b0, bm, bp, cm, cp, e0, d0, em, ep, dm, dp, is adjacent to q and is
+// linked to q (equal values are, so adjacency is enough for multilabel and
+// binary; continuous links need the bit of the pair r - q, which is another
+// bit of the same masks).  The pair r - q belongs to a voxel before p, so by
+// induction over (voxel, order) every dropped link follows from kept ones,
+// whatever tiles its voxels lie in.  At a tile's first column the link a
+// crosses into the next tile: there it comes last in the order and covers
+// nothing.  On the 512^3 uint32 Voronoi workload at 26-connectivity this
+// leaves 0.10 unions and 0.017 cross-tile requests per voxel.
+//
+// Union-find nodes are the tile's voxels (LDS position row * 68 + x, raster
+// order, so every tree is rooted at its member with the smallest key); a
+// voxel points at its run's first voxel in the segment, and the first voxel of a
+// segment that continues a run at the voxel before it, from the start.  Kept
+// links go to a per-wave queue and are made 64 at a time, one per lane: links
+// inside the tile as LDS unions, links out of it as cross-tile requests
+// (voxel position | relation << 12) for the global kernels.  Outputs (GP, TR,
+// J8/J16, REQ/TQ, tcnt) are those of the voxel kernel in local.hpp except
+// for the request format; J is row-major: entry x + 64 * (y + 8 * z).
 #pragma once
 
 #include "common.hpp"
@@ -38,118 +48,198 @@
 
 namespace cc3d_amd {
 
-// Tile geometry of the row kernels.  Box positions: bx in [0, 65]
-// (x = -1 .. 64), by in [0, TY + 1], bz in [0, TZ].  Halo index = box index.
+// Tile geometry of the row kernels: 64 rows of 64 voxels.  Box rows (by, bz):
+// by = y + 1, bz = z + 1, one halo row or plane on each side that backward
+// neighbours reach.
 template <int TY_, int TZ_>
 struct RowGeo {
   static constexpr int TX = 64, TY = TY_, TZ = TZ_;
   static constexpr bool IS3D = true;
-  static constexpr int NT = 64 * TZ;  // one wave per plane
-  static constexpr int NW = TZ;
+  static constexpr int NT = 256;
   static constexpr int TV = TX * TY * TZ;
-  static constexpr int BX = TX + 2, BY = TY + 2, BZ = TZ + 1;
-  static constexpr int BOXN = BX * BY * BZ;
+  static constexpr int BY = TY + 2, BZ = TZ + 1;
   static constexpr int NROWS = BY * BZ;
-  // box positions that can be halo nodes: plane bz = 0; rows by = 0 of
-  // planes 1..TZ; rows by = TY + 1 of planes 1..TZ-1; the x-halo of the tile
-  // rows.  Bounds the requests of a tile.
-  static constexpr int HALO = BX * BY + BX * TZ + BX * (TZ - 1) + 2 * TY * TZ;
-  static_assert(BOXN < 65536, "16-bit nodes");
-
-  __host__ __device__ static constexpr int box(int bx, int by, int bz) { return bx + BX * (by + BY * bz); }
-  __host__ __device__ static constexpr int rid(int by, int bz) { return by + BY * bz; }
-  __device__ static inline void halo_coords(int h, int& bx, int& by, int& bz) {
-    bz = h / (BX * BY);
-    const int r = h - bz * (BX * BY);
-    by = r / BX;
-    bx = r - by * BX;
-  }
-  template <int QK>
-  __device__ static inline void nid_box(int n, int& bx, int& by, int& bz) {
-    halo_coords(n, bx, by, bz);
-  }
+  static_assert(TY * TZ == 64, "one row per lane of a wave");
   __device__ static inline int jidx(int lx, int ly, int lz) { return lx + TX * (ly + TY * lz); }
 };
 using GeoR = RowGeo<8, 8>;
 
+// Relations in covering order; index 12 is a.  Offsets as (d + 1) in 2-bit
+// fields per axis.
+enum : int { R_C0, R_B0, R_BM, R_BP, R_CM, R_CP, R_E0, R_D0, R_EM, R_EP, R_DM, R_DP, R_A, R_N };
+__host__ __device__ constexpr Off rel_off(int r) {
+  switch (r) {
+    case R_C0: return {0, 0, -1};
+    case R_B0: return {0, -1, 0};
+    case R_BM: return {-1, -1, 0};
+    case R_BP: return {1, -1, 0};
+    case R_CM: return {-1, 0, -1};
+    case R_CP: return {1, 0, -1};
+    case R_E0: return {0, 1, -1};
+    case R_D0: return {0, -1, -1};
+    case R_EM: return {-1, 1, -1};
+    case R_EP: return {1, 1, -1};
+    case R_DM: return {-1, -1, -1};
+    case R_DP: return {1, -1, -1};
+    default: return {-1, 0, 0};
+  }
+}
+__host__ __device__ constexpr uint32_t rel_packed(int axis) {
+  uint32_t m = 0;
+  for (int r = 0; r < R_N; r++) {
+    const Off o = rel_off(r);
+    m |= (uint32_t)((axis == 0 ? o.dx : axis == 1 ? o.dy : o.dz) + 1) << (2 * r);
+  }
+  return m;
+}
+// Does an offset belong to connectivity nb?  (Also: are two voxels that far
+// apart adjacent.)
+__host__ __device__ constexpr bool off_in(int dx, int dy, int dz, int nb) {
+  const int ax = dx < 0 ? -dx : dx, ay = dy < 0 ? -dy : dy, az = dz < 0 ? -dz : dz;
+  const int l1 = ax + ay + az;
+  if (ax > 1 || ay > 1 || az > 1) return false;
+  return nb == 26 || (nb == 18 && l1 <= 2) || (nb == 6 && l1 <= 1);
+}
+__host__ __device__ constexpr bool rel_in(int r, int nb) {
+  return off_in(rel_off(r).dx, rel_off(r).dy, rel_off(r).dz, nb);
+}
+__host__ __device__ constexpr bool rel_adj(int i, int j, int nb) {
+  const Off a = rel_off(i), b = rel_off(j);
+  return off_in(a.dx - b.dx, a.dy - b.dy, a.dz - b.dz, nb);
+}
+// Offset of relation r (run time).
+__device__ inline void rel_decode(uint32_t r, int& dx, int& dy, int& dz) {
+  constexpr uint32_t PX = rel_packed(0), PY = rel_packed(1), PZ = rel_packed(2);
+  dx = (int)((PX >> (2 * r)) & 3u) - 1;
+  dy = (int)((PY >> (2 * r)) & 3u) - 1;
+  dz = (int)((PZ >> (2 * r)) & 3u) - 1;
+}
+
+// Bound on the requests of a tile.  Multilabel and binary: the largest number
+// of kept relations that leave the tile, over every set of links a voxel can
+// have, summed over the tile's voxels (4,036 at 26-connectivity, 2,537 at
+// 18, 1,088 at 6).  Continuous: all relations that leave the tile.
+__host__ __device__ constexpr int row_req_cap(bool cont, int nb) {
+  return nb == 6 ? 1088 : nb == 18 ? (cont ? 5280 : 2540) : (cont ? 9316 : 4036);
+}
+
+// Staged voxel type: 4 bytes for every type up to 4 bytes, else the type.
 template <class T>
-struct RowLds {
-  using G = GeoR;
-  static constexpr int QCAP = 128;  // per-wave union queue: 64 pending + one append
-  static constexpr int RW = (G::BOXN + 31) / 32;
-  T v[G::BOXN];                                 // box values
-  alignas(4) uint16_t par[(G::BOXN + 1) & ~1];  // parents (pmin works on aligned words)
-  uint32_t rbits[RW];                           // roots of trees that hold tile voxels
-  union {
-    uint32_t q[G::NW][QCAP];  // union queues (phases 2 and 4)
-    uint32_t rprefix[RW];     // exclusive popcount prefix of rbits (phases 6-7)
-  } u;
-  uint16_t plist[G::HALO];  // piece roots
-  uint32_t npiece, nreq, nroots;
-  uint32_t red_epl[G::NW], red_prov[G::NW];
-  int32_t red_first[G::NW], red_last[G::NW];
+struct RowVal {
+  using type = uint32_t;
+};
+template <>
+struct RowVal<float> {
+  using type = float;
+};
+template <>
+struct RowVal<uint64_t> {
+  using type = uint64_t;
+};
+template <>
+struct RowVal<double> {
+  using type = double;
 };
 
-// DPP lane shifts across the whole wave (wave_shr:1 / wave_shl:1): lane x
-// receives src from lane x - 1 (x + 1); the lane with no source keeps `old`.
-__device__ inline uint32_t shr1_u32(uint32_t old, uint32_t src) {
-  return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)src, 0x138, 0xf, 0xf, false);
+constexpr int RSTR = 68;     // row stride of staged values and nodes: 16-byte accesses of 64 rows spread over all banks
+constexpr int RQCAP = 1024;  // queued links per wave; one relation of a wave's segments always fits
+
+template <class T, int MODE>
+struct RowLds {
+  using G = GeoR;
+  using VT = typename RowVal<T>::type;
+  struct Work {
+    uint32_t par[64 * RSTR];
+    uint16_t queue[4][RQCAP];  // per wave; later, per wave: segment bits [row] and root bits [row]
+  };
+  union alignas(16) {
+    // staged box: x = -1 at 3, x = 0..63 at 4..67, x = 64 at 68 (the next row's unused first element)
+    VT v[MODE == M_BINARY ? 1 : G::NROWS * RSTR + 4];
+    // staged foreground bits, 16 per half-word: x = -1 in bit 15 of 0, segments in 1..4, x = 64 in bit 0 of 5
+    uint16_t fb[G::NROWS][6];
+    Work w;
+  } u;
+  uint32_t nreq;
+  uint32_t wtot[4], red_epl[4], red_prov[4];
+  uint64_t rows[4];
+};
+
+// m = 2 m + condition
+__device__ inline void push_bit(uint32_t& m, bool c) { m = m + m + (c ? 1u : 0u); }
+__device__ inline void push_eq(uint32_t& m, uint32_t a, uint32_t b) {
+  asm("v_cmp_eq_u32_e32 vcc, %1, %2\n\tv_addc_co_u32_e32 %0, vcc, %0, %0, vcc" : "+v"(m) : "v"(a), "v"(b) : "vcc");
 }
-__device__ inline uint32_t shl1_u32(uint32_t old, uint32_t src) {
-  return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)src, 0x130, 0xf, 0xf, false);
+__device__ inline void push_eq(uint32_t& m, float a, float b) {
+  asm("v_cmp_eq_f32_e32 vcc, %1, %2\n\tv_addc_co_u32_e32 %0, vcc, %0, %0, vcc" : "+v"(m) : "v"(a), "v"(b) : "vcc");
 }
-template <class T>
-__device__ inline T lane_shift(T old, T src, bool right) {
-  if constexpr (sizeof(T) <= 4) {
-    uint32_t o = 0, s = 0;
-    __builtin_memcpy(&o, &old, sizeof(T));
-    __builtin_memcpy(&s, &src, sizeof(T));
-    const uint32_t r = right ? shr1_u32(o, s) : shl1_u32(o, s);
-    T out;
-    __builtin_memcpy(&out, &r, sizeof(T));
-    return out;
-  } else {
-    uint64_t o, s;
-    __builtin_memcpy(&o, &old, 8);
-    __builtin_memcpy(&s, &src, 8);
-    const uint32_t lo = right ? shr1_u32((uint32_t)o, (uint32_t)s) : shl1_u32((uint32_t)o, (uint32_t)s);
-    const uint32_t hi =
-      right ? shr1_u32((uint32_t)(o >> 32), (uint32_t)(s >> 32)) : shl1_u32((uint32_t)(o >> 32), (uint32_t)(s >> 32));
-    const uint64_t r = (uint64_t)lo | ((uint64_t)hi << 32);
-    T out;
-    __builtin_memcpy(&out, &r, 8);
-    return out;
-  }
+__device__ inline void push_eq(uint32_t& m, uint64_t a, uint64_t b) {
+  asm("v_cmp_eq_u64_e32 vcc, %1, %2\n\tv_addc_co_u32_e32 %0, vcc, %0, %0, vcc" : "+v"(m) : "v"(a), "v"(b) : "vcc");
+}
+__device__ inline void push_eq(uint32_t& m, double a, double b) {
+  asm("v_cmp_eq_f64_e32 vcc, %1, %2\n\tv_addc_co_u32_e32 %0, vcc, %0, %0, vcc" : "+v"(m) : "v"(a), "v"(b) : "vcc");
+}
+__device__ inline void push_fg(uint32_t& m, uint32_t a) {
+  asm("v_cmp_ne_u32_e32 vcc, 0, %1\n\tv_addc_co_u32_e32 %0, vcc, %0, %0, vcc" : "+v"(m) : "v"(a) : "vcc");
+}
+__device__ inline void push_fg(uint32_t& m, float a) {
+  asm("v_cmp_neq_f32_e32 vcc, 0, %1\n\tv_addc_co_u32_e32 %0, vcc, %0, %0, vcc" : "+v"(m) : "v"(a) : "vcc");
+}
+template <class V>
+__device__ inline void push_fg(uint32_t& m, V a) {
+  push_bit(m, a != V(0));
+}
+
+// Continuous link between two values of one volume type T, background
+// excluded (cc3d/cc3d_continuous.hpp:79-88).
+template <class T, class V>
+__device__ inline bool cont_link(V a, V b, V delta) {
+  return a != V(0) && b != V(0) && match<V>(a, b, delta);
+}
+
+// Orders the wave's memory accesses before and after (its LDS accesses are
+// performed in order, so this is a matter for the compiler only).
+__device__ inline void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 __device__ inline uint64_t wave_ballot(bool p) { return (uint64_t)__ballot(p); }
 
-// lfind_h / lunion (common.hpp) with every loop bounded by the node count of
-// a box: parents only decrease, so a correct forest never needs more hops;
-// the bound only guarantees that the kernel ends.
-constexpr int RHOPS = 6000;
-__device__ inline uint32_t rfind(uint16_t* par, uint32_t a) {
-  uint32_t p = pload(par, a);
-  for (int i = 0; p != a && i < RHOPS; i++) {
-    const uint32_t gp = pload(par, p);
+// Lanes below this one in m.
+__device__ inline uint32_t mbcnt64(uint64_t m) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+// LDS union-find over 32-bit parents.  A parent is never larger than its
+// node, so walks end; a union lowers the larger root's parent with an atomic
+// minimum and goes on from the parent it displaced, so a link is never lost
+// to a racing one.  Path halving stores an ancestor of a node that is no
+// root any more.
+__device__ inline void lstore(uint32_t* p, uint32_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ inline uint32_t rfind(uint32_t* par, uint32_t a) {
+  uint32_t p = lload(par + a);
+  while (p != a) {
+    const uint32_t gp = lload(par + p);
     if (gp == p) return p;
-    pstore(par, a, gp);
+    lstore(par + a, gp);
     a = gp;
-    p = pload(par, a);
+    p = lload(par + a);
   }
   return a;
 }
-// Root of a, reading only (bounded like rfind).
-__device__ inline uint32_t rfind_ro(const uint16_t* par, uint32_t a) {
-  for (int i = 0; i < RHOPS; i++) {
-    const uint32_t p = pload(par, a);
-    if (p == a) break;
+__device__ inline uint32_t rfind_ro(const uint32_t* par, uint32_t a) {
+  uint32_t p = lload(par + a);
+  while (p != a) {
     a = p;
+    p = lload(par + a);
   }
   return a;
 }
-__device__ inline void runion(uint16_t* par, uint32_t a, uint32_t b) {
-  for (int i = 0; i < RHOPS; i++) {
+__device__ inline void runion(uint32_t* par, uint32_t a, uint32_t b) {
+  while (true) {
     a = rfind(par, a);
     b = rfind(par, b);
     if (a == b) return;
@@ -158,499 +248,478 @@ __device__ inline void runion(uint16_t* par, uint32_t a, uint32_t b) {
       a = b;
       b = t;
     }
-    const uint32_t old = pmin(par, a, b);
+    const uint32_t old = atomicMin(par + a, b);
     if (old == a) return;
     a = old;
   }
 }
 
-// The n queued unions (a << 16 | b) of a wave, one per lane.  Called from a
-// few places only, out of line: one copy of the union loops keeps the
-// kernel's code small.
-__device__ __noinline__ void run_queue(uint16_t* par, const uint32_t* q, uint32_t n, int lane) {
-  for (uint32_t i = lane; i < n; i += 64) {
-    const uint32_t e = q[i];
-    runion(par, e >> 16, e & 0xFFFFu);
-  }
+// N consecutive voxels from p (aligned to a voxel), as the widest loads that
+// alignment allows.
+template <class T, int N>
+__device__ inline void load_run(const T* p, T (&v)[N]) {
+  struct __attribute__((packed, aligned(sizeof(T)))) Pack {
+    T e[N];
+  };
+  const Pack k = *reinterpret_cast<const Pack*>(p);
+#pragma unroll
+  for (int i = 0; i < N; i++) v[i] = k.e[i];
 }
 
-
-// Lanes below x (1-based rank of x among the set bits of m, minus one).
-__device__ inline uint32_t mbcnt64(uint64_t m) {
-  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-}
-
-// Position of the highest set bit of m at or below lane x (m & lemask != 0).
-__device__ inline uint32_t run_start(uint64_t m, uint64_t lemask) {
-  const uint64_t b = m & lemask;
-  const uint32_t hi = (uint32_t)(b >> 32);
-  return hi ? 63u - (uint32_t)__builtin_clz(hi) : 31u - (uint32_t)__builtin_clz((uint32_t)b | 1u);
-}
-
-// Buffer loads of box positions (raw buffer loads at 32-bit byte offsets
-// from box position (0, 0, 0); an offset at or above the record count reads
-// 0), or 64-bit addresses when the box spans 2 GiB or more.
-template <class T>
-struct BoxLoader {
-  __amdgpu_buffer_rsrc_t rs;
-  const T* in;
-  int64_t x0, y0, z0, sx, sy, sz;
-  bool buf;
-  uint32_t RB, PB;
-
-  __device__ inline void init(const T* in_, int64_t x0_, int64_t y0_, int64_t z0_, int64_t sx_, int64_t sy_,
-                              int64_t sz_, int BXn, int BYn, int BZn) {
-    in = in_;
-    x0 = x0_;
-    y0 = y0_;
-    z0 = z0_;
-    sx = sx_;
-    sy = sy_;
-    sz = sz_;
-    buf = (uint64_t)(BXn + sx * BYn + sx * sy * BZn) * sizeof(T) < (uint64_t)0x80000000u;
-    RB = (uint32_t)(sx * (int64_t)sizeof(T));
-    PB = (uint32_t)(sx * sy * (int64_t)sizeof(T));
-    if (buf) {
-      const int64_t base_el = (x0 - 1) + sx * ((y0 - 1) + sy * (z0 - 1));
-      const uint64_t rem = (uint64_t)(sx * sy * sz - base_el) * sizeof(T);
-      const int nrec = (int)(rem < 0x80000000ull ? rem : 0x7FFFFFFFull);
-      const char* bp = reinterpret_cast<const char*>(in) + base_el * (int64_t)sizeof(T);
-      rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(bp), 0, nrec, 0x00020000);
+// Bit k of the result: byte k of w is not zero, for the 16 bytes of four
+// words; t has 0x80 in each such byte and a dot product gathers them.
+__device__ inline uint32_t nonzero_bytes(const uint32_t (&w)[4]) {
+  uint32_t acc = 0, out[2];
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    acc = 0;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const uint32_t x = w[2 * h + i];
+      const uint32_t t = (((x & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | x) & 0x80808080u;
+      acc = __builtin_amdgcn_udot4(t, i ? 0x80402010u : 0x08040201u, acc, false);
     }
+    out[h] = acc >> 7;
   }
-  // value of box position (bx, by, bz); 0 outside the volume
-  __device__ inline T load(int bx, int by, int bz) const {
-    const int64_t gx = x0 + bx - 1, gy = y0 + by - 1, gz = z0 + bz - 1;
-    const bool ok = gx >= 0 && gx < sx && gy >= 0 && gy < sy && gz >= 0 && gz < sz;
-    if (buf) {
-      const uint32_t off = ok ? (uint32_t)bx * (uint32_t)sizeof(T) + (uint32_t)by * RB + (uint32_t)bz * PB : 0x80000000u;
-      if constexpr (sizeof(T) == 1) {
-        return __builtin_bit_cast(T, (uint8_t)__builtin_amdgcn_raw_buffer_load_b8(rs, off, 0, 0));
-      } else if constexpr (sizeof(T) == 2) {
-        return __builtin_bit_cast(T, (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rs, off, 0, 0));
-      } else if constexpr (sizeof(T) == 4) {
-        return __builtin_bit_cast(T, (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0));
-      } else {
-        return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, 0));
-      }
-    }
-    const T v = in[ok ? gx + sx * (gy + sy * gz) : 0];
-    return ok ? v : T(0);
-  }
-};
-
-// Link masks of row `cur` (foreground F) to a backward row r' (values w,
-// x-halo values hl / hr, foreground Fw): bit x of E0 / Em / Ep when cur[x]
-// links to r'[x] / r'[x - 1] / r'[x + 1].
-template <class T, int MODE>
-__device__ inline void row_links(T cur, uint64_t F, T w, T hl, T hr, uint64_t Fw, bool diag, uint64_t& E0,
-                                 uint64_t& Em, uint64_t& Ep) {
-  if constexpr (MODE == M_MULTI) {
-    E0 = wave_ballot(cur == w) & F;
-    if (diag) {
-      Em = wave_ballot(cur == lane_shift<T>(hl, w, true)) & F;
-      Ep = wave_ballot(cur == lane_shift<T>(hr, w, false)) & F;
-    } else {
-      Em = Ep = 0;
-    }
-  } else {
-    E0 = F & Fw;
-    if (diag) {
-      Em = F & ((Fw << 1) | (fg(hl) ? 1ull : 0ull));
-      Ep = F & ((Fw >> 1) | (fg(hr) ? (1ull << 63) : 0ull));
-    } else {
-      Em = Ep = 0;
-    }
-  }
+  return out[0] | (out[1] << 8);
 }
 
 template <class T, int MODE, int NB>
 __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, int64_t sy, int64_t sz, int64_t ntx,
-                                 int64_t nty, int64_t tile, int64_t slot, uint32_t keybase, RowLds<T>& L) {
+                                 int64_t nty, int64_t tile, int64_t slot, uint32_t keybase, RowLds<T, MODE>& L) {
   using G = GeoR;
-  constexpr int BX = G::BX;
-  constexpr int QCAP = RowLds<T>::QCAP;
-  constexpr int RW = RowLds<T>::RW;
-  constexpr bool DIAG = NB != 6;  // x +- 1 neighbours in the rows the connectivity reaches
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  using VT = typename RowVal<T>::type;
+  const int t = threadIdx.x, lane = t & 63;
+  const int seg = __builtin_amdgcn_readfirstlane(t >> 6);  // one segment per wave
   const int64_t tz = tile / (ntx * nty);
   const int64_t trem = tile - tz * ntx * nty;
   const int64_t ty = trem / ntx, tx = trem - ty * ntx;
   const int64_t x0 = tx * G::TX, y0 = ty * G::TY, z0 = tz * G::TZ;
-  uint16_t* par = L.par;
-  uint32_t* q = L.u.q[wv];
-  const uint64_t lemask = lane == 63 ? ~0ull : ((2ull << lane) - 1ull);  // lanes <= x
+  uint32_t my_epl = 0, my_prov = 0;
+  if (t == 0) L.nreq = 0;
 
-  for (int i = t; i < RW; i += G::NT) L.rbits[i] = 0u;
-  if (t == 0) {
-    L.npiece = 0;
-    L.nreq = 0;
-  }
-
-  BoxLoader<T> ld;
-  ld.init(in, x0, y0, z0, sx, sy, sz, G::BX, G::BY, G::BZ);
-
-  // 1. staging.  Wave wv loads the rows by = 0..8 of its plane bz = wv + 1
-  //    (kept in registers), row by = 9 of that plane (wv < 7) and rows wv
-  //    and wv + 8 of the halo plane bz = 0: every box row but (9, 8), which
-  //    no voxel of the tile reaches.  Each row: values to LDS, run starts,
-  //    parents of run starts, the run start of every lane.
-  const int bzo = wv + 1;
-  auto stage_row = [&](T v, int by, int bz) {
-    const int r = G::rid(by, bz);
-    L.v[r * BX + 1 + lane] = v;
-    const uint64_t F = wave_ballot(fg(v));
-    uint64_t S;
-    if constexpr (MODE == M_MULTI) {
-      const uint64_t eq = wave_ballot(v == lane_shift<T>(v, v, true));
-      S = F & ~(eq & ~1ull);
-    } else {
-      S = F & ~(F << 1);
-    }
-    if ((S >> lane) & 1ull) par[r * BX + 1 + lane] = (uint16_t)(r * BX + 1 + lane);
+  // 1. stage the box: rows r = by + BY * bz.  Row BY - 1 of the last plane is
+  //    reached by no voxel.  Voxels outside the volume are background.
+  const T* box = in + ((x0 - 1) + sx * ((y0 - 1) + sy * (z0 - 1)));  // box position (-1, -1, -1); dereferenced inside the volume only
+  const int64_t xleft = sx - x0;                                     // voxels of a row from x0 on
+  auto row_ok = [&](int by, int bz) -> bool {
+    const int64_t gy = y0 + by - 1, gz = z0 + bz - 1;
+    return gy >= 0 && gy < sy && gz >= 0 && gz < sz;
   };
-  {
-    T own[G::TY + 1];  // rows by = 0..8 of plane bzo
-    T extra[3];
-    const int eby0 = wv, eby1 = wv + 8;
+  auto row_ptr = [&](int by, int bz) -> const T* { return box + (1 + sx * (by + sy * (int64_t)bz)); };  // its x0
+  if constexpr (MODE == M_BINARY) {
+    // 16 voxels (one segment) per thread and pass
+    constexpr int ITEMS = 4 * G::NROWS;
+    constexpr int PASSES = (ITEMS + G::NT - 1) / G::NT;
 #pragma unroll
-    for (int k = 0; k <= G::TY; k++) own[k] = ld.load(1 + lane, k, bzo);
-    extra[0] = wv < G::TZ - 1 ? ld.load(1 + lane, G::TY + 1, bzo) : T(0);
-    extra[1] = ld.load(1 + lane, eby0, 0);
-    extra[2] = eby1 <= G::TY + 1 ? ld.load(1 + lane, eby1, 0) : T(0);
-    // x-halo of these rows: lane 2k + side, k over the rows above in order
-    const int nrow = (G::TY + 1) + (wv < G::TZ - 1 ? 1 : 0) + 1 + (eby1 <= G::TY + 1 ? 1 : 0);
-    int hrow = lane >> 1;
-    int hby, hbz;
-    if (hrow <= G::TY) {
-      hby = hrow;
-      hbz = bzo;
-    } else if (hrow == G::TY + 1 && wv < G::TZ - 1) {
-      hby = G::TY + 1;
-      hbz = bzo;
-    } else {
-      const int e = hrow - (G::TY + 1) - (wv < G::TZ - 1 ? 1 : 0);
-      hby = e == 0 ? eby0 : eby1;
-      hbz = 0;
-    }
-    const bool hlive = hrow < nrow;
-    const int hbx = (lane & 1) ? BX - 1 : 0;
-    const T hv = hlive ? ld.load(hbx, hby, hbz) : T(0);
+    for (int q = 0; q < PASSES; q++) {
+      const int i = t + G::NT * q;
+      if (i >= ITEMS) break;
+      const int r = i >> 2, s = i & 3;
+      const int bz = r / G::BY, by = r - bz * G::BY;
+      uint32_t F = 0, NE = 0;  // NE: differs from the voxel before it (tile rows)
+      if (row_ok(by, bz) && 16 * s < xleft) {
+        const T* e = row_ptr(by, bz) + 16 * s;
+        const bool own = by >= 1 && by <= G::TY && bz >= 1;
+        T prev = T(0);
+        if (own && x0 + 16 * s > 0) prev = e[-1];
+        if (16 * s + 16 <= xleft) {
+          T v[16];
+          load_run<T, 16>(e, v);
+          if constexpr (sizeof(T) == 1) {
+            uint32_t w[4], d[4];
+            __builtin_memcpy(w, v, 16);
+            F = nonzero_bytes(w);
+            d[0] = w[0] ^ ((w[0] << 8) | (uint32_t)(uint8_t)prev);
 #pragma unroll
-    for (int k = 0; k <= G::TY; k++) stage_row(own[k], k, bzo);
-    if (wv < G::TZ - 1) stage_row(extra[0], G::TY + 1, bzo);
-    stage_row(extra[1], eby0, 0);
-    if (eby1 <= G::TY + 1) stage_row(extra[2], eby1, 0);
-    if (hlive) {
-      const int n = G::box(hbx, hby, hbz);
-      L.v[n] = hv;
-      if (fg(hv)) par[n] = (uint16_t)n;
+            for (int k = 1; k < 4; k++) d[k] = w[k] ^ __builtin_amdgcn_alignbyte(w[k], w[k - 1], 3);
+            NE = nonzero_bytes(d);
+          } else {
+#pragma unroll
+            for (int k = 15; k >= 0; k--) {
+              push_bit(F, v[k] != T(0));
+              push_bit(NE, v[k] != (k > 0 ? v[k - 1] : prev));
+            }
+          }
+        } else {
+          const int n = (int)(xleft - 16 * s);
+          for (int k = 0; k < n; k++) {
+            const T c = e[k];
+            F |= (uint32_t)(c != T(0)) << k;
+            NE |= (uint32_t)(c != prev) << k;
+            prev = c;
+          }
+        }
+        if (own) my_epl += (uint32_t)__popc(F & NE);
+      }
+      L.u.fb[r][s + 1] = (uint16_t)F;
     }
-  }
-  __syncthreads();
-
-  // union queue of this wave
-  uint32_t qn = 0;
-  auto flush = [&]() {
-    run_queue(par, q, qn, lane);
-    qn = 0;
-  };
-  auto append = [&](uint64_t U, uint32_t a, uint32_t b) {
-    if (U == 0) return;
-    if ((U >> lane) & 1ull) q[qn + mbcnt64(U)] = (a << 16) | b;
-    qn += (uint32_t)__builtin_popcountll(U);
-    if (qn >= 64) flush();
-  };
-  const uint64_t ltmask = lemask >> 1;            // lanes below x
-  const uint64_t le1mask = (lemask << 1) | 1ull;  // lanes up to x + 1
-  auto row_vals = [&](int r) -> T { return L.v[r * BX + 1 + lane]; };
-  auto row_F = [&](T v) -> uint64_t { return wave_ballot(fg(v)); };
-  auto row_S = [&](T v, uint64_t F) -> uint64_t {
-    if constexpr (MODE == M_MULTI) {
-      const uint64_t eq = wave_ballot(v == lane_shift<T>(v, v, true));
-      return F & ~(eq & ~1ull);
-    } else {
-      return F & ~(F << 1);
+    if (t < 2 * G::NROWS) {
+      const int r = t >> 1, right = t & 1;
+      const int bz = r / G::BY, by = r - bz * G::BY;
+      const bool ok = row_ok(by, bz) && (right ? xleft > 64 : x0 > 0);
+      const bool f = ok && row_ptr(by, bz)[right ? 64 : -1] != T(0);
+      L.u.fb[r][right ? 5 : 0] = (uint16_t)(f ? (right ? 1u : 0x8000u) : 0u);
     }
-  };
-  // Unions of row r (values cur, F, S) with backward row rp.  Links in
-  // sk0 / skm / skp (offsets 0, -1, +1) are implied by others and make no
-  // union; E0 / Em / Ep return the row's links to rp.
-  // a: node of the run of each lane of row r.  Partner nodes come from the
-  // run starts of rp, recomputed from its values.
-  auto contact = [&](uint32_t a, T cur, uint64_t F, uint64_t S, uint64_t Send, int rp, bool diag, bool halo_only,
-                     uint64_t& any, uint64_t sk0, uint64_t skm, uint64_t skp, uint64_t& E0, uint64_t& Em,
-                     uint64_t& Ep) {
-    const T w = row_vals(rp);
-    const T hl = L.v[rp * BX], hr = L.v[rp * BX + BX - 1];
-    const uint64_t Fw = row_F(w);
-    row_links<T, MODE>(cur, F, w, hl, hr, Fw, diag, E0, Em, Ep);
-    if (halo_only) {  // the x-halo voxels of r' lie in other tiles
-      Em &= ~1ull;
-      Ep &= ~(1ull << 63);
-    }
-    any |= E0 | Em | Ep;
-    const uint64_t E0u = E0 & ~sk0;
-    const uint64_t U0 = E0u & ~((E0u << 1) & ~S);
-    const uint64_t Um = Em & ~skm & ~E0 & S;
-    const uint64_t Up = Ep & ~skp & ~E0 & Send;
-    if ((U0 | Um | Up) == 0) return;
-    const uint64_t Sw = row_S(w, Fw);
-    const uint32_t base = (uint32_t)(rp * BX + 1);
-    if (U0) append(U0, a, base + run_start(Sw, lemask));
-    if (Um) append(Um, a, lane == 0 ? base - 1u : base + run_start(Sw, ltmask));
-    if (Up) append(Up, a, lane == 63 ? base + 64u : base + run_start(Sw, le1mask));
-  };
-
-  // 2. halo pieces: links between halo nodes of one neighbouring tile.
-  //    Row pairs: plane 0 rows 2..8 with the row before (the tile below);
-  //    rows by = 0 of planes 2..8 and rows by = 9 of planes 2..7 with the
-  //    same row of the plane before (the tiles beside in y).
-  for (int pi = wv; pi < 20; pi += G::NW) {
-    int r, rp;
-    if (pi < 7) {
-      r = G::rid(pi + 2, 0);
-      rp = G::rid(pi + 1, 0);
-    } else if (pi < 14) {
-      r = G::rid(0, pi - 5);
-      rp = G::rid(0, pi - 6);
-    } else {
-      r = G::rid(G::TY + 1, pi - 12);
-      rp = G::rid(G::TY + 1, pi - 13);
-    }
-    const T cur = row_vals(r);
-    const uint64_t F = row_F(cur);
-    const uint64_t S = row_S(cur, F);
-    const uint64_t Send = F & ~((F & ~S) >> 1);
-    uint64_t any = 0, e0, em, ep;
-    const uint32_t a = (uint32_t)(r * BX + 1) + run_start(S, lemask);
-    contact(a, cur, F, S, Send, rp, DIAG, true, any, 0, 0, 0, e0, em, ep);
-  }
-  flush();
-  // x-halo columns of the tile rows (the tiles beside in x): each voxel with
-  // the voxels of its column before it, as the connectivity reaches them
-  if (t < 128) {
-    const int bxh = t < 64 ? 0 : BX - 1;
-    const int k = t & 63, by = 1 + (k & 7), bz = 1 + (k >> 3);
-    const uint32_t n = (uint32_t)G::box(bxh, by, bz);
-    const T cur = L.v[n];
-    if (fg(cur)) {
-      auto link = [&](int by2, int bz2) {
-        const uint32_t m = (uint32_t)G::box(bxh, by2, bz2);
-        const T o = L.v[m];
-        const bool l = MODE == M_MULTI ? (o == cur) : fg(o);
-        if (l) runion(par, n, m);
-      };
-      if (by >= 2) link(by - 1, bz);
-      if (bz >= 2) {
-        link(by, bz - 1);
-        if (NB != 6) {
-          if (by >= 2) link(by - 1, bz - 1);
-          if (by <= G::TY - 1) link(by + 1, bz - 1);
+  } else {
+    // 4 voxels per thread and pass, 16 rows a pass; all loads first
+    constexpr int PASSES = (G::NROWS + 15) / 16;
+    T v[PASSES][4];
+    const int q4 = 4 * (t & 15), rr = t >> 4;
+#pragma unroll
+    for (int q = 0; q < PASSES; q++) {
+      const int r = rr + 16 * q;
+      const int bz = r / G::BY, by = r - bz * G::BY;
+#pragma unroll
+      for (int k = 0; k < 4; k++) v[q][k] = T(0);
+      if (r < G::NROWS - 1 && row_ok(by, bz)) {
+        const T* e = row_ptr(by, bz) + q4;
+        if (q4 + 4 <= xleft) {
+          load_run<T, 4>(e, v[q]);
+        } else {
+#pragma unroll
+          for (int k = 0; k < 4; k++)
+            if (q4 + k < xleft) v[q][k] = e[k];
         }
       }
     }
-  }
-  __syncthreads();
-
-  // 3. piece roots: halo nodes that are roots now
-  {
-    auto push = [&](bool is_root, uint32_t n) {
-      const uint64_t m = wave_ballot(is_root);
-      if (m == 0) return;
-      uint32_t base = 0;
-      if (lane == 0) base = atomicAdd(&L.npiece, (uint32_t)__builtin_popcountll(m));
-      base = __shfl(base, 0);
-      if (is_root) L.plist[base + mbcnt64(m)] = (uint16_t)n;
-    };
-    // halo rows: plane 0 (10 rows), by = 0 of planes 1..8, by = 9 of planes 1..7
-    for (int hr = wv; hr < 25; hr += G::NW) {
-      const int r = hr < 10 ? G::rid(hr, 0) : hr < 18 ? G::rid(0, hr - 9) : G::rid(G::TY + 1, hr - 17);
-      const T v = row_vals(r);
-      const uint64_t F = row_F(v);
-      const uint64_t S = row_S(v, F);
-      const uint32_t n = (uint32_t)(r * BX + 1 + lane);
-      push(((S >> lane) & 1ull) && pload(par, n) == n, n);
+    T hx = T(0);
+    const int hr = t >> 1, right = t & 1;
+    if (t < 2 * G::NROWS) {
+      const int bz = hr / G::BY, by = hr - bz * G::BY;
+      if (row_ok(by, bz) && (right ? xleft > 64 : x0 > 0)) hx = row_ptr(by, bz)[right ? 64 : -1];
     }
-    // x-halo voxels of the 89 staged rows (rows 0..88), a wave at a time
-    for (int i0 = wv * 64; i0 < 2 * 89; i0 += G::NT) {
-      const int i = i0 + lane;
-      const bool live = i < 2 * 89;
-      const int r = live ? i >> 1 : 0;
-      const uint32_t n = (uint32_t)(r * BX + ((i & 1) ? BX - 1 : 0));
-      push(live && fg(L.v[n]) && pload(par, n) == n, n);
-    }
-  }
-  __syncthreads();
-
-  // 4. the tile's rows: unions with the backward rows; counters
-  uint32_t my_epl = 0, my_prov = 0;
-  int my_first = 0x7FFFFFFF, my_last = -1;
-#pragma unroll 1
-  for (int by = 1; by <= G::TY; by++) {
-    const int r = G::rid(by, bzo);
-    const T cur = row_vals(r);
-    const uint64_t F = row_F(cur);
-    const T hlc = L.v[r * BX];
-    const uint64_t eqv = wave_ballot(cur == lane_shift<T>(hlc, cur, true));  // bit 0: vs the x-halo voxel
-    uint64_t S, link0;
-    if constexpr (MODE == M_MULTI) {
-      S = F & ~(eqv & ~1ull);
-      link0 = eqv & F;
-    } else {
-      S = F & ~(F << 1);
-      link0 = F & ((F << 1) | (fg(hlc) ? 1ull : 0ull));
-    }
-    const uint64_t Send = F & ~((F & ~S) >> 1);
-    my_epl += (uint32_t)__builtin_popcountll(F & ~eqv);
-    if (F) {
-      const int lr = (by - 1) + G::TY * (bzo - 1);
-      my_first = lr < my_first ? lr : my_first;
-      my_last = lr > my_last ? lr : my_last;
-    }
-    uint64_t any = link0;
-    if (link0 & 1ull) append(1ull, (uint32_t)(r * BX + 1), (uint32_t)(r * BX));  // the x-halo voxel before the row
-    // Same plane, row before (B); plane before: rows by (C), by - 1 (D) and
-    // by + 1 (E).  A link p - q of voxel p = (x, y, z) to q = (x + d, y - 1,
-    // z - 1) in D is implied when p links to (x + d, y - 1, z) in B or to
-    // (x + d, y, z - 1) in C: that voxel is adjacent to both, and its links
-    // to q (a C link of row B, a B link of row C) are always unioned by the
-    // tile that owns the later voxel.  Likewise for E through C.
-    uint64_t b0, bm, bp, c0, cm, cp, t0, tm, tp;
-    const uint32_t a = (uint32_t)(r * BX + 1) + run_start(S, lemask);
-    contact(a, cur, F, S, Send, G::rid(by - 1, bzo), DIAG, false, any, 0, 0, 0, b0, bm, bp);
-    contact(a, cur, F, S, Send, G::rid(by, bzo - 1), DIAG, false, any, 0, 0, 0, c0, cm, cp);
-    if (NB != 6) {
-      contact(a, cur, F, S, Send, G::rid(by - 1, bzo - 1), NB == 26, false, any, b0 | c0, bm | cm, bp | cp, t0, tm,
-              tp);
-      contact(a, cur, F, S, Send, G::rid(by + 1, bzo - 1), NB == 26, false, any, c0, cm, cp, t0, tm, tp);
-    }
-    my_prov += (uint32_t)__builtin_popcountll(F & ~any);
-  }
-  flush();
-  __syncthreads();
-
-  // 5. roots of the tile's run starts, 64 at a time from a per-wave queue;
-  //    mark the roots and store each run start's root as its parent.  Every
-  //    walk here and in step 7 only reads, so the only stores are these: a
-  //    run start's parent is its root from here on.
-  {
-    uint32_t fnum = 0;
-    auto fflush = [&]() {
-      for (uint32_t i = lane; i < fnum; i += 64) {
-        const uint32_t n = q[i];
-        const uint32_t root = rfind_ro(par, n);
-        if (root != n) pstore(par, n, root);
-        if (!((lload(&L.rbits[root >> 5]) >> (root & 31)) & 1u)) atomicOr(&L.rbits[root >> 5], 1u << (root & 31));
+#pragma unroll
+    for (int q = 0; q < PASSES; q++) {
+      const int r = rr + 16 * q;
+      if (r < G::NROWS) {
+        VT* d = static_cast<VT*>(__builtin_assume_aligned(L.u.v + (r * RSTR + 4 + q4), 16));
+#pragma unroll
+        for (int k = 0; k < 4; k++) d[k] = (VT)v[q][k];
       }
-      fnum = 0;
-    };
-#pragma unroll 1
-    for (int by = 1; by <= G::TY; by++) {
-      const int r = G::rid(by, bzo);
-      const T cur = row_vals(r);
-      const uint64_t S = row_S(cur, row_F(cur));
-      if (S == 0) continue;
-      if ((S >> lane) & 1ull) q[fnum + mbcnt64(S)] = (uint32_t)(r * BX + 1 + lane);
-      fnum += (uint32_t)__builtin_popcountll(S);
-      if (fnum >= 64) fflush();
     }
-    fflush();
+    if (t < 2 * G::NROWS) L.u.v[hr * RSTR + (right ? 68 : 3)] = (VT)hx;
   }
   __syncthreads();
 
-  // 6. rank the marked roots in node (= key) order
-  if (wv == 0) {
-    uint32_t c[3];
+  // 2. the segment's masks (bit k: voxel 16 seg + k of row `lane`)
+  const int ly = lane & (G::TY - 1), lz = lane / G::TY;
+  const int r0 = (ly + 1) + G::BY * (lz + 1);
+  constexpr int RB = -1, RC = -G::BY, RD = -G::BY - 1, RE = -G::BY + 1;  // box rows B, C, D, E from r0
+  const bool first = seg == 0;  // bit 0 is the tile's first column
+  uint32_t F = 0, a = 0;
+  uint32_t U[R_N];  // kept links
 #pragma unroll
-    for (int k = 0; k < 3; k++) c[k] = 3 * lane + k < RW ? (uint32_t)__popc(L.rbits[3 * lane + k]) : 0u;
-    const uint32_t tot = c[0] + c[1] + c[2];
-    uint32_t incl = tot;
+  for (int i = 0; i < R_N; i++) U[i] = 0;
+  {
+    uint32_t M[R_N];  // all links
+    uint32_t any;
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const uint32_t y = __shfl_up(incl, o);
-      if (lane >= o) incl += y;
+    for (int i = 0; i < R_N; i++) M[i] = 0;
+    uint32_t hD0 = 0;  // 6-connectivity: equal to the voxels of bm, cm (in M) and d0
+    if constexpr (MODE == M_BINARY) {
+      auto bits = [&](int r, uint32_t& m0, uint32_t& mm, uint32_t& mp) {
+        const uint16_t* b = &L.u.fb[r][seg];
+        const uint32_t c = b[1];
+        m0 = c;
+        mm = ((c << 1) | (uint32_t)(b[0] >> 15)) & 0xFFFFu;
+        mp = (c >> 1) | (((uint32_t)b[2] & 1u) << 15);
+      };
+      uint32_t mm, mp;
+      bits(r0, F, mm, mp);
+      a = F & mm;
+      auto rel = [&](int dr, int i0, int im, int ip) {
+        uint32_t m0;
+        bits(r0 + dr, m0, mm, mp);
+        M[i0] = F & m0;
+        M[im] = F & mm;
+        M[ip] = F & mp;
+      };
+      rel(RB, R_B0, R_BM, R_BP);
+      rel(RC, R_C0, R_CM, R_CP);
+      rel(RD, R_D0, R_DM, R_DP);
+      if constexpr (NB != 6) rel(RE, R_E0, R_EM, R_EP);
+      hD0 = M[R_D0];
+    } else {
+      const VT* base = static_cast<const VT*>(__builtin_assume_aligned(L.u.v + (r0 * RSTR + 4 + 16 * seg), 16));
+      VT cur[16];
+#pragma unroll
+      for (int k = 0; k < 16; k++) cur[k] = base[k];
+      const VT left = base[-1];
+      if constexpr (MODE == M_MULTI) {
+#pragma unroll
+        for (int k = 15; k >= 0; k--) {
+          push_fg(F, cur[k]);
+          push_eq(a, cur[k], k > 0 ? cur[k > 0 ? k - 1 : 0] : left);
+        }
+        a &= F;
+        my_epl = (uint32_t)__popc(F & ~a);
+        // W0/WM/WP: which of the row's three relations to form
+        auto rel = [&](int dr, int i0, int im, int ip, bool W0, bool WM, bool WP) {
+          const VT* w = base + dr * RSTR;
+          VT wv[18];  // x = -1 .. 16 of the segment
+#pragma unroll
+          for (int k = 0; k < 18; k++)
+            if ((k > 0 || WM) && (k < 17 || WP)) wv[k] = w[k - 1];
+#pragma unroll
+          for (int k = 15; k >= 0; k--) {
+            if (W0) push_eq(M[i0], cur[k], wv[k + 1]);
+            if (WM) push_eq(M[im], cur[k], wv[k]);
+            if (WP) push_eq(M[ip], cur[k], wv[k + 2]);
+          }
+          if (W0) M[i0] &= F;
+          if (WM) M[im] &= F;
+          if (WP) M[ip] &= F;
+        };
+        rel(RB, R_B0, R_BM, R_BP, true, true, NB != 6);
+        rel(RC, R_C0, R_CM, R_CP, true, true, NB != 6);
+        rel(RD, R_D0, R_DM, R_DP, true, NB == 26, NB == 26);
+        if constexpr (NB != 6) rel(RE, R_E0, R_EM, R_EP, true, NB == 26, NB == 26);
+        hD0 = M[R_D0];
+      }
     }
-    uint32_t ex = incl - tot;
+    const uint32_t ain = first ? (a & ~1u) : a;  // links a inside the tile
+    if constexpr (MODE != M_CONT) {
+      if constexpr (NB == 6) {
+        any = a | M[R_B0] | M[R_C0];
+        U[R_B0] = M[R_B0] & ~(ain & M[R_BM]);
+        U[R_C0] = M[R_C0] & ~(ain & M[R_CM]) & ~(M[R_B0] & hD0);
+        U[R_A] = a & ~ain & ~((M[R_B0] & M[R_BM]) | (M[R_C0] & M[R_CM]));
+      } else {
+        any = a;
+        uint32_t cova = 0;
 #pragma unroll
-    for (int k = 0; k < 3; k++) {
-      if (3 * lane + k < RW) L.u.rprefix[3 * lane + k] = ex;
-      ex += c[k];
+        for (int i = 0; i < R_A; i++) {
+          if (!rel_in(i, NB)) continue;
+          any |= M[i];
+          uint32_t cov = rel_adj(R_A, i, NB) ? ain : 0u;
+#pragma unroll
+          for (int j = 0; j < i; j++)
+            if (rel_in(j, NB) && rel_adj(j, i, NB)) cov |= M[j];
+          if (rel_adj(R_A, i, NB)) cova |= M[i];
+          U[i] = M[i] & ~cov;
+        }
+        U[R_A] = a & ~ain & ~cova;
+      }
     }
-    if (lane == 63) L.nroots = incl;
+    my_prov = (uint32_t)__popc(F & ~any);
+  }
+  const uint32_t S = F & (first ? ~(a & ~1u) : ~a);  // run starts inside the tile
+  const uint64_t fgrows = wave_ballot(F != 0u);
+  __syncthreads();  // the staged box is dead: par and the queues take its place
+
+  // 3. parents, and the wave's queue of kept links
+  uint32_t* par = L.u.w.par;
+  uint16_t* queue = L.u.w.queue[seg];
+  {
+    const uint32_t n0 = (uint32_t)(lane * RSTR + 16 * seg);
+    uint32_t v = n0 - 1u;  // a segment that continues a run hangs on the voxel before it
+#pragma unroll
+    for (int k = 0; k < 16; k += 4) {
+      uint32_t w[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        if (k + i == 1) v = (S & 1u) ? v : n0;
+        v = ((S >> (k + i)) & 1u) ? n0 + (uint32_t)(k + i) : v;
+        w[i] = v;
+      }
+      uint32_t* d = static_cast<uint32_t*>(__builtin_assume_aligned(par + n0 + k, 16));
+#pragma unroll
+      for (int i = 0; i < 4; i++) d[i] = w[i];
+    }
+  }
+  constexpr int NWORD = NB == 6 ? 1 : NB == 18 ? 4 : 6;
+  const uint32_t pos0 = (uint32_t)(lane * G::TX + 16 * seg);
+  uint32_t W[6];  // two relations each: 2 i in the low half, 2 i + 1 in the high half
+  uint32_t cnt = U[R_A];
+#pragma unroll
+  for (int i = 0; i < 6; i++) {
+    W[i] = i < NWORD ? (U[2 * i] | (U[2 * i + 1] << 16)) : 0u;
+    if (i < NWORD) cnt += (uint32_t)__popc(W[i]);
+  }
+  // writes this lane's links from slot q on, two words per loop
+  auto emit = [&](uint16_t* q, uint32_t ua) {
+    if (first && ua) *q++ = (uint16_t)(pos0 | ((uint32_t)R_A << 12));
+#pragma unroll
+    for (int i = 0; i < NWORD; i += 2) {
+      uint32_t m = W[i], m2 = i + 1 < NWORD ? W[i + 1] : 0u;
+      uint32_t code = pos0 + ((uint32_t)(2 * i) << 12);
+      while (m | m2) {
+        if (m == 0) {
+          m = m2;
+          m2 = 0;
+          code += 2u << 12;
+        }
+        const uint32_t k = (uint32_t)__builtin_ctz(m);
+        m &= m - 1u;
+        *q++ = (uint16_t)(code + (k & 15u) + ((k >> 4) << 12));
+      }
+    }
+  };
+  // the n queued links of the wave, one per lane
+  uint16_t* REQt = reinterpret_cast<uint16_t*>(p.REQ) + slot * p.reqcap;
+  auto drain = [&](uint32_t n) {
+    for (uint32_t i0 = 0; i0 < n; i0 += 64) {
+      const uint32_t i = i0 + (uint32_t)lane;
+      bool out = false;
+      uint32_t e = 0;
+      if (i < n) {
+        e = queue[i];
+        int dx, dy, dz;
+        rel_decode(e >> 12, dx, dy, dz);
+        const int x = (int)(e & 63u) + dx, y = (int)((e >> 6) & (G::TY - 1)) + dy, z = (int)((e >> 9) & (G::TZ - 1)) + dz;
+        out = x < 0 || x >= G::TX || y < 0 || y >= G::TY || z < 0;
+        if (!out) {
+          const uint32_t ps = e & 0xFFFu;
+          runion(par, ps + 4u * (ps >> 6), (uint32_t)(x + RSTR * (y + G::TY * z)));
+        }
+      }
+      const uint64_t m = wave_ballot(out);
+      if (m) {
+        uint32_t b = 0;
+        if (lane == 0) b = atomicAdd(&L.nreq, (uint32_t)__builtin_popcountll(m));
+        b = (uint32_t)__builtin_amdgcn_readfirstlane((int)b);
+        if (out) REQt[b + mbcnt64(m)] = (uint16_t)e;
+      }
+    }
+  };
+  const uint32_t incl = wave_incl_add(cnt);
+  const uint32_t total = wave_lane63(incl);
+  if (total <= RQCAP) emit(queue + (incl - cnt), U[R_A]);
+  __syncthreads();
+
+  // 4. unions and requests
+  if (total <= RQCAP) {
+    drain(total);
+  } else {
+    // more links than the queue holds: one relation at a time
+    uint32_t keep[6];
+#pragma unroll
+    for (int i = 0; i < 6; i++) keep[i] = W[i];
+#pragma unroll 1
+    for (int r = 0; r <= 2 * NWORD; r++) {
+      uint32_t c = 0;
+#pragma unroll
+      for (int i = 0; i < 6; i++) {
+        W[i] = (r >> 1) == i ? (keep[i] & ((r & 1) ? 0xFFFF0000u : 0xFFFFu)) : 0u;
+        c += (uint32_t)__popc(W[i]);
+      }
+      const uint32_t ua = r == 2 * NWORD ? U[R_A] : 0u;
+      c += ua;
+      const uint32_t inc = wave_incl_add(c);
+      emit(queue + (inc - c), ua);
+      wave_order();
+      drain(wave_lane63(inc));
+      wave_order();
+    }
+  }
+  // the wave's queue is dead: its place takes the segment bits by row
+  wave_order();
+  uint32_t* segbits = reinterpret_cast<uint32_t*>(queue);
+  segbits[lane] = S | (F << 16);
+  my_epl = wave_lane63(wave_incl_add(my_epl));
+  my_prov = wave_lane63(wave_incl_add(my_prov));
+  if (lane == 0) {
+    L.red_epl[seg] = my_epl;
+    L.red_prov[seg] = my_prov;
+    L.rows[seg] = fgrows;
   }
   __syncthreads();
-  static_assert(3 * 64 >= RW, "one wave scans the root bitmask");
-  const uint32_t R = L.nroots;
-  auto rank = [&](uint32_t r) -> uint32_t {
-    return L.u.rprefix[r >> 5] + (uint32_t)__popc(L.rbits[r >> 5] & ((1u << (r & 31)) - 1u));
-  };
+
+  // 5. roots.  From here thread t has segment t & 3 of row t >> 2, so its
+  //    outputs are in raster order over the workgroup.  Heads (run starts and
+  //    the first voxel of a segment) take their root as parent; all walks
+  //    only read otherwise.
+  const int hrow = t >> 2, hseg = t & 3;
+  uint32_t* qs = reinterpret_cast<uint32_t*>(L.u.w.queue[hseg]);
+  const uint32_t sf = qs[hrow];
+  const uint32_t hS = sf & 0xFFFFu, hF = sf >> 16;
+  const uint32_t H = hS | (hF & 1u);
+  const uint32_t h0 = (uint32_t)(hrow * RSTR + 16 * hseg);
+  uint32_t rb = 0;  // roots of this segment
+  for (uint32_t m = H; m; m &= m - 1u) {
+    const uint32_t k = (uint32_t)__builtin_ctz(m), n = h0 + k;
+    const uint32_t r = rfind_ro(par, n);
+    if (r == n) rb |= 1u << k;
+    else lstore(par + n, r);
+  }
+  const uint32_t nr = (uint32_t)__popc(rb);
+  const uint32_t rincl = wave_incl_add(nr);
+  if (lane == 63) L.wtot[t >> 6] = rincl;
+  __syncthreads();
+  uint32_t rbase = 0, R = 0;
+#pragma unroll
+  for (int w = 0; w < 4; w++) {
+    if (w < (t >> 6)) rbase += L.wtot[w];
+    R += L.wtot[w];
+  }
+  rbase += rincl - nr;
+  qs[64 + hrow] = rb | (rbase << 16);  // ranks of the segment's roots
+  __syncthreads();
+
+  // 6. heads: 1 + the rank of their root
+  for (uint32_t m = H; m; m &= m - 1u) {
+    const uint32_t k = (uint32_t)__builtin_ctz(m), n = h0 + k;
+    const uint32_t r = par[n];
+    const uint32_t row = (r * 61681u) >> 22;  // r / 68 for r < 64 * 68
+    const uint32_t x = r - RSTR * row;
+    const uint32_t w = reinterpret_cast<const uint32_t*>(L.u.w.queue[x >> 4])[64 + row];
+    par[n] = (w >> 16) + (uint32_t)__popc(w & ((1u << (x & 15u)) - 1u)) + 1u;
+  }
 
   // 7. outputs.  Keys in 32-bit arithmetic (below 2^32; intermediate wraps
-  //    cancel): box position (bx, by, bz) is voxel (x0 + bx - 1, ...).
-  const uint32_t kbox0 =
-    (uint32_t)(x0 - 1) + (uint32_t)sx * ((uint32_t)(y0 - 1) + (uint32_t)sy * (uint32_t)(z0 - 1)) + keybase;
+  //    cancel).  A segment's keys are consecutive, so its root marks are one
+  //    or two words.
   const uint32_t root0 = tile_root0<G>(sx, sy, sz, tx, ty, tz, keybase);
-  uint32_t* RLt = p.RL + root0;
-  if (t < RW) {
-    uint32_t bits = L.rbits[t];
-    uint32_t rk = L.u.rprefix[t];
-    while (bits) {
-      const int b = __builtin_ctz(bits);
-      bits &= bits - 1u;
-      int bx, by, bz;
-      G::halo_coords(32 * t + b, bx, by, bz);
-      const uint32_t key = kbox0 + (uint32_t)bx + (uint32_t)sx * ((uint32_t)by + (uint32_t)sy * (uint32_t)bz);
-      p.GP[root0 + rk] = root0 + rk;
-      RLt[rk++] = key;
-      atomicOr(p.bits + (key >> 5), 1u << (key & 31));
+  if (rb) {
+    const uint32_t key0 = (uint32_t)x0 + 16u * (uint32_t)hseg +
+                          (uint32_t)sx * ((uint32_t)(y0 + (hrow & (G::TY - 1))) +
+                                          (uint32_t)sy * (uint32_t)(z0 + hrow / G::TY)) + keybase;
+    uint32_t rk = root0 + rbase;
+    for (uint32_t m = rb; m; m &= m - 1u) {
+      p.GP[rk] = make_uint2(rk, key0 + (uint32_t)__builtin_ctz(m));
+      rk++;
     }
+    const uint32_t sh = key0 & 31u, lo = rb << sh, hi = sh > 16u ? rb >> (32u - sh) : 0u;
+    if (lo) atomicOr(p.bits + (key0 >> 5), lo);
+    if (hi) atomicOr(p.bits + (key0 >> 5) + 1, hi);
   }
-#pragma unroll 2
-  for (int by = 1; by <= G::TY; by++) {
-    const int r = G::rid(by, bzo);
-    const T cur = row_vals(r);
-    const uint64_t F = row_F(cur);
-    const uint64_t S = row_S(cur, F);
-    uint32_t j = 0;
-    if (fg(cur)) j = rank(pload(par, (uint32_t)(r * BX + 1) + run_start(S, lemask))) + 1u;  // its run's root
-    const int64_t e = slot * G::TV + G::jidx(lane, by - 1, bzo - 1);
-    if (R <= 255) p.J8[e] = (uint8_t)j;
-    else p.J16[e] = (uint16_t)j;
-  }
-  for (uint32_t i = t; i < L.npiece; i += G::NT) {
-    const uint32_t h = L.plist[i];
-    const uint32_t root = rfind_ro(par, h);
-    if ((L.rbits[root >> 5] >> (root & 31)) & 1u) {
-      const uint32_t k = atomicAdd(&L.nreq, 1u);
-      p.REQ[slot * G::HALO + k] = (rank(root) << 16) | h;
-    }
-  }
-  // counters
+  {
+    uint32_t j = 0, pk[8];
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const int f = __shfl_xor(my_first, o), l = __shfl_xor(my_last, o);
-    my_first = f < my_first ? f : my_first;
-    my_last = l > my_last ? l : my_last;
+    for (int k = 0; k < 16; k += 4) {
+      const uint32_t* v = static_cast<const uint32_t*>(__builtin_assume_aligned(par + h0 + k, 16));
+      uint32_t o[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        j = ((H >> (k + i)) & 1u) ? v[i] : j;
+        o[i] = ((hF >> (k + i)) & 1u) ? j : 0u;
+      }
+      pk[k / 2] = o[0] | (o[1] << 16);
+      pk[k / 2 + 1] = o[2] | (o[3] << 16);
+    }
+    if (R <= 255) {
+      uint32_t b[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) b[i] = __builtin_amdgcn_perm(pk[2 * i + 1], pk[2 * i], 0x06040200u);
+      reinterpret_cast<uint4*>(p.J8 + slot * G::TV)[t] = make_uint4(b[0], b[1], b[2], b[3]);
+    } else {
+      uint4* o = reinterpret_cast<uint4*>(p.J16 + slot * G::TV) + 2 * t;
+      o[0] = make_uint4(pk[0], pk[1], pk[2], pk[3]);
+      o[1] = make_uint4(pk[4], pk[5], pk[6], pk[7]);
+    }
   }
-  if (lane == 0) {
-    L.red_epl[wv] = my_epl;
-    L.red_prov[wv] = my_prov;
-    L.red_first[wv] = my_first;
-    L.red_last[wv] = my_last;
-  }
-  __syncthreads();
   if (t == 0) {
     uint32_t e = 0, pv = 0;
-    int fl = 0x7FFFFFFF, ll = -1;
-    for (int w = 0; w < G::NW; w++) {
+    uint64_t rows = 0;
+    for (int w = 0; w < 4; w++) {
       e += L.red_epl[w];
       pv += L.red_prov[w];
-      fl = L.red_first[w] < fl ? L.red_first[w] : fl;
-      ll = L.red_last[w] > ll ? L.red_last[w] : ll;
+      rows |= L.rows[w];
     }
     long long f = 0x7FFFFFFFFFFFFFFFll, l = -1;
-    if (ll >= 0) {
+    if (rows) {
+      const int fl = __builtin_ctzll(rows), ll = 63 - __builtin_clzll(rows);
       f = (y0 + fl % G::TY) + sy * (z0 + fl / G::TY);
       l = (y0 + ll % G::TY) + sy * (z0 + ll / G::TY);
     }
@@ -666,15 +735,16 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
 }
 
 // Waves per SIMD the row kernel is compiled for: what the LDS of one tile
-// admits (3 workgroups of 8 waves per CU up to 4-byte voxels, 2 for 8-byte).
-template <class T>
+// admits (6 workgroups of 4 waves per CU up to 4-byte voxels, 3 for 8-byte
+// ones; binary tiles stage bits and hold 6 for every type).
+template <class T, int MODE>
 __host__ __device__ constexpr int rows_waves() {
-  return sizeof(T) <= 2 ? 8 : sizeof(T) == 4 ? 6 : 4;
+  return (MODE == M_BINARY || sizeof(T) <= 4) ? 6 : 3;
 }
 
 template <class T, int MODE, int NB>
-__global__ __launch_bounds__(GeoR::NT, (rows_waves<T>())) void k_rows_local(LocalParams p) {
-  __shared__ RowLds<T> L;
+__global__ __launch_bounds__(GeoR::NT, (rows_waves<T, MODE>())) void k_rows_local(LocalParams p) {
+  __shared__ RowLds<T, MODE> L;
   const int64_t tile = xcd_tile(blockIdx.x, p.ntiles);
   rows_tile<T, MODE, NB>(p, static_cast<const T*>(p.in), p.sx, p.sy, p.sz, p.ntx, p.nty, tile, tile, 0u, L);
 }
@@ -682,10 +752,10 @@ __global__ __launch_bounds__(GeoR::NT, (rows_waves<T>())) void k_rows_local(Loca
 // Batch: tiles [gtile0, gtile0 + gtiles) of volumes of connectivity NB; each
 // workgroup reads its volume's table entry.
 template <class T, int MODE, int NB>
-__global__ __launch_bounds__(GeoR::NT, (rows_waves<T>())) void k_rows_local_batch(LocalParams p, const BatchVol* vols,
-                                                                                 const uint32_t* vix, int64_t gtile0,
-                                                                                 int64_t gtiles) {
-  __shared__ RowLds<T> L;
+__global__ __launch_bounds__(GeoR::NT, (rows_waves<T, MODE>())) void k_rows_local_batch(LocalParams p, const BatchVol* vols,
+                                                                                       const uint32_t* vix,
+                                                                                       int64_t gtile0, int64_t gtiles) {
+  __shared__ RowLds<T, MODE> L;
   const int64_t slot = gtile0 + xcd_tile(blockIdx.x, gtiles);
   const BatchVol& v = vols[vix[slot]];
   rows_tile<T, MODE, NB>(p, static_cast<const T*>(v.in), v.sx, v.sy, v.sz, v.ntx, v.nty, slot - v.tile0, slot, v.key0,

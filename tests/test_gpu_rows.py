@@ -1,0 +1,80 @@
+"""Row tiles (csrc/rows.hpp) where they can go wrong: sides around the tile
+(64 x 8 x 8) and the 16-voxel segment, every voxel width, links that fill a
+wave's queue past its capacity, and the scratch limit that sends a volume back
+to the voxel tiles.  Labels and N are whole numbers: bit for bit."""
+import numpy as np
+import pytest
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+SIDES = [(1, 9, 8), (15, 8, 9), (16, 7, 17), (17, 16, 3), (63, 9, 2), (64, 8, 8), (65, 17, 9), (130, 10, 16)]
+
+
+def _check(vol, tag, **kw):
+  import cc3d
+  print(tag, vol.shape, vol.dtype, kw, flush=True)
+  got, n = cc3d.connected_components(vol, return_N=True, **kw)
+  exp, en = oracle.connected_components(vol, return_N=True, **kw)
+  assert n == en and np.array_equal(got, exp), tag
+
+
+@pytest.mark.parametrize("connectivity", [6, 18, 26])
+@pytest.mark.parametrize("dtype", [np.uint8, np.uint16, np.uint32, np.uint64, np.float32, np.float64])
+def test_edges_of_tile_and_segment(gpu, dtype, connectivity):
+  rng = np.random.default_rng(connectivity + np.dtype(dtype).itemsize)
+  for k, shape in enumerate(SIDES):
+    vol = rng.integers(0, 3, size=shape).astype(dtype)
+    vol = np.asfortranarray(vol) if k & 1 else vol
+    _check(vol, f"multilabel {k}", connectivity=connectivity)
+    _check(vol, f"binary {k}", connectivity=connectivity, binary_image=True)
+
+
+@pytest.mark.parametrize("connectivity", [18, 26])
+@pytest.mark.parametrize("binary", [False, True])
+def test_more_links_than_a_queue_holds(gpu, connectivity, binary):
+  """A checkerboard: no face links, three kept edge links per foreground voxel."""
+  x, y, z = np.meshgrid(*[np.arange(s) for s in (130, 17, 18)], indexing="ij")
+  vol = np.asfortranarray(((x + y + z) & 1).astype(np.uint32))
+  _check(vol, "checkerboard", connectivity=connectivity, binary_image=binary)
+  vol = np.asfortranarray(1 + ((x + y + z) & 1).astype(np.uint8))  # both colours labelled
+  _check(vol, "two colours", connectivity=connectivity, binary_image=binary)
+
+
+def test_special_float_values(gpu):
+  """NaN equals nothing (not even itself), infinities and signed zeros follow ==."""
+  rng = np.random.default_rng(5)
+  pool = np.array([0.0, -0.0, np.nan, np.inf, -np.inf, 1.0, 1e-42], np.float32)
+  for dt in (np.float32, np.float64):
+    vol = pool[rng.integers(0, len(pool), size=(70, 9, 11))].astype(dt)
+    for conn in (6, 18, 26):
+      _check(vol, "special values", connectivity=conn)
+
+
+def test_scratch_limit_keeps_ragged_volumes(gpu):
+  """A volume whose row tiles exceed the fixed scratch is labelled on the voxel
+  tiles: 65 columns leave a second row tile nearly empty."""
+  import ctypes
+  import torch
+  from cc3d import _lib as L
+  lib = L.lib()
+  f = lib.cc3d_amd_connected_components3d_noalloc
+  f.restype = ctypes.c_int
+  f.argtypes = lib.cc3d_amd_connected_components3d.argtypes
+  sx, sy, sz = 65, 512, 504
+  limit = 256 << 20
+  assert lib.cc3d_amd_workspace_bytes(sx, sy, sz, 26, 0, 0) > limit
+  assert lib.cc3d_amd_workspace_bytes(sx, sy, sz, 26, 0, L.FLAG_TILES_VOXELS) <= limit
+  g = torch.Generator().manual_seed(3)
+  vol = torch.randint(0, 3, (sx * sy * sz,), generator=g, dtype=torch.int32).to(gpu)
+  exp, en = torch.empty_like(vol), ctypes.c_uint64(0)
+  got, gn = torch.empty_like(vol), ctypes.c_uint64(0)
+  d = np.zeros(1, np.uint32)
+  s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+  for fn, out, n in ((lib.cc3d_amd_connected_components3d, exp, en), (f, got, gn)):
+    rc = fn(ctypes.c_void_p(vol.data_ptr()), L.DT_U32, sx, sy, sz, vol.numel(), 26, d.ctypes.data,
+            ctypes.c_void_p(out.data_ptr()), L.DT_U32, ctypes.byref(n), 0, 0, s)
+    assert rc == L.OK
+  torch.cuda.synchronize()
+  assert en.value == gn.value and torch.equal(exp, got)
