@@ -1296,9 +1296,8 @@ static int plan(Geometry& g, int64_t sx, int64_t sy, int64_t sz, int64_t connect
   if (g.K >= 0xFFFFFFFFll || g.V >= 0xFFFFFFFFll)
     return fail(CC3D_AMD_ERR_INVALID, "volumes of 2^32-1 voxels or more are not supported");
   int TX, TY, TZ;
-  // Row tiles for 3D multilabel and binary volumes.
-  g.rows = g.is3d && g.mode != M_CONT &&
-           ((tiles & CC3D_AMD_TILES_ROWS) || !(tiles & (CC3D_AMD_TILES_VOXELS | CC3D_AMD_TILES_TALL)));
+  // Row tiles for 3D volumes.
+  g.rows = g.is3d && ((tiles & CC3D_AMD_TILES_ROWS) || !(tiles & (CC3D_AMD_TILES_VOXELS | CC3D_AMD_TILES_TALL)));
   g.tall = g.is3d && !g.rows && (tiles & CC3D_AMD_TILES_TALL) && !(tiles & CC3D_AMD_TILES_VOXELS);
   if (g.rows) {
     TX = GeoR::TX; TY = GeoR::TY; TZ = GeoR::TZ; g.TV = GeoR::TV;
@@ -1807,6 +1806,7 @@ static int job_begin(cc3d_amd_job* j, const void* in, int in_dtype, int64_t sx, 
   {
   ProfScope ps_("k_local", s);
   if (g.rows && g.mode == M_MULTI) e = launch_rows_multi(in_dtype, g.nb, lp, s);
+  else if (g.rows && g.mode == M_CONT) e = launch_rows_cont(in_dtype, g.nb, lp, s);
   else if (g.rows) e = launch_rows_binary(in_dtype, g.nb, lp, s);
   else if (g.mode == M_MULTI) e = launch_local_multi(in_dtype, g.nb, g.qk, g.tall, lp, s);
   else if (g.mode == M_BINARY) e = launch_local_binary(in_dtype, g.nb, g.qk, g.tall, lp, s);
@@ -2161,16 +2161,14 @@ static int batch_layout(const cc3d_amd_volume* vols, int n, int mode, std::vecto
       nbps[i] = v.sz > 1 ? 6 : (conn == 26 || conn == 18) ? 8 : conn == 6 ? 4 : conn;
     }
     nbs[i] = nb;
-    // the single-volume path's choice (plan): rows unless continuous, then
-    // voxels, then tall; by default rows, voxels if continuous
+    // the single-volume path's choice (plan): rows, then voxels, then tall;
+    // by default rows
     const int pref = (int)((v.connectivity >> 8) & 0xFF);
-    const bool cont = mode == CC3D_AMD_BATCH_CONTINUOUS;
-    famv[i] = qks[i] != Q_NONE                           ? cc3d_amd_batch::FAM_PLANE
-              : (!cont && (pref & CC3D_AMD_TILES_ROWS))  ? cc3d_amd_batch::FAM_ROWS
-              : (pref & CC3D_AMD_TILES_VOXELS)          ? cc3d_amd_batch::FAM_VOXELS
-              : (pref & CC3D_AMD_TILES_TALL)            ? cc3d_amd_batch::FAM_TALL
-              : !cont                                   ? cc3d_amd_batch::FAM_ROWS
-                                                        : cc3d_amd_batch::FAM_VOXELS;
+    famv[i] = qks[i] != Q_NONE                  ? cc3d_amd_batch::FAM_PLANE
+              : (pref & CC3D_AMD_TILES_ROWS)    ? cc3d_amd_batch::FAM_ROWS
+              : (pref & CC3D_AMD_TILES_VOXELS)  ? cc3d_amd_batch::FAM_VOXELS
+              : (pref & CC3D_AMD_TILES_TALL)    ? cc3d_amd_batch::FAM_TALL
+                                                : cc3d_amd_batch::FAM_ROWS;
     b.perm[i] = i;
   }
   // by tile family (voxels, tall, rows), then 26, 18, 6 within each
@@ -2483,6 +2481,8 @@ int cc3d_amd_batch_begin(cc3d_amd_batch* b) {
         e = launch_local_batch_plane_cont(b->dt, g.nb, tg.lp, tg.gp.vols, tg.gp.vix, g.tile0, g.tiles, s);
       else if (tg.rows() && b->mode == M_BINARY)
         e = launch_rows_batch_binary(b->dt, g.nb, tg.lp, tg.gp.vols, tg.gp.vix, g.tile0, g.tiles, s);
+      else if (tg.rows() && b->mode == M_CONT)
+        e = launch_rows_batch_cont(b->dt, g.nb, tg.lp, tg.gp.vols, tg.gp.vix, g.tile0, g.tiles, s);
       else if (tg.rows())
         e = launch_rows_batch_multi(b->dt, g.nb, tg.lp, tg.gp.vols, tg.gp.vix, g.tile0, g.tiles, s);
       else if (b->mode == M_BINARY)

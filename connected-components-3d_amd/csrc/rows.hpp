@@ -189,11 +189,40 @@ __device__ inline void push_fg(uint32_t& m, V a) {
   push_bit(m, a != V(0));
 }
 
-// Continuous link between two values of one volume type T, background
-// excluded (cc3d/cc3d_continuous.hpp:79-88).
-template <class T, class V>
-__device__ inline bool cont_link(V a, V b, V delta) {
-  return a != V(0) && b != V(0) && match<V>(a, b, delta);
+// Continuous link between two staged values (cc3d/cc3d_continuous.hpp:79-88).
+// Floating-point background is staged as a NaN, which links to nothing, so
+// the link is one subtraction and one compare; integers test both for zero.
+template <class V>
+__device__ inline void push_link(uint32_t& m, V a, V b, V delta) {
+  push_bit(m, a != V(0) && b != V(0) && match<V>(a, b, delta));
+}
+__device__ inline void push_link(uint32_t& m, float a, float b, float delta) {
+  asm("v_cmp_le_f32_e64 vcc, |%1|, %2\n\tv_addc_co_u32_e32 %0, vcc, %0, %0, vcc"
+      : "+v"(m) : "v"(a - b), "s"(delta) : "vcc");
+}
+__device__ inline void push_link(uint32_t& m, double a, double b, double delta) {
+  asm("v_cmp_le_f64_e64 vcc, |%1|, %2\n\tv_addc_co_u32_e32 %0, vcc, %0, %0, vcc"
+      : "+v"(m) : "v"(a - b), "s"(delta) : "vcc");
+}
+// Staged form of a value of a continuous volume: background becomes the NaN
+// of all ones, every other NaN the default one.
+__device__ inline float cont_stage(float v) {
+  const uint32_t b = v == 0.0f ? 0xFFFFFFFFu : v != v ? 0x7FC00000u : __builtin_bit_cast(uint32_t, v);
+  return __builtin_bit_cast(float, b);
+}
+__device__ inline double cont_stage(double v) {
+  const uint64_t b = v == 0.0 ? ~0ull : v != v ? 0x7FF8000000000000ull : __builtin_bit_cast(uint64_t, v);
+  return __builtin_bit_cast(double, b);
+}
+template <class V>
+__device__ inline V cont_stage(V v) {
+  return v;
+}
+__device__ inline bool cont_fg(float v) { return __builtin_bit_cast(uint32_t, v) != 0xFFFFFFFFu; }
+__device__ inline bool cont_fg(double v) { return __builtin_bit_cast(uint64_t, v) != ~0ull; }
+template <class V>
+__device__ inline bool cont_fg(V v) {
+  return v != V(0);
 }
 
 // Orders the wave's memory accesses before and after (its LDS accesses are
@@ -395,10 +424,10 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
       if (r < G::NROWS) {
         VT* d = static_cast<VT*>(__builtin_assume_aligned(L.u.v + (r * RSTR + 4 + q4), 16));
 #pragma unroll
-        for (int k = 0; k < 4; k++) d[k] = (VT)v[q][k];
+        for (int k = 0; k < 4; k++) d[k] = MODE == M_CONT ? cont_stage((VT)v[q][k]) : (VT)v[q][k];
       }
     }
-    if (t < 2 * G::NROWS) L.u.v[hr * RSTR + (right ? 68 : 3)] = (VT)hx;
+    if (t < 2 * G::NROWS) L.u.v[hr * RSTR + (right ? 68 : 3)] = MODE == M_CONT ? cont_stage((VT)hx) : (VT)hx;
   }
   __syncthreads();
 
@@ -416,7 +445,8 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
     uint32_t any;
 #pragma unroll
     for (int i = 0; i < R_N; i++) M[i] = 0;
-    uint32_t hD0 = 0;  // 6-connectivity: equal to the voxels of bm, cm (in M) and d0
+    uint32_t hD0 = 0;       // 6-connectivity: equal to the voxel of d0 (bm, cm are in M)
+    uint32_t left_cov = 0;  // continuous: bit 0, the link a of the tile's first column is covered
     if constexpr (MODE == M_BINARY) {
       auto bits = [&](int r, uint32_t& m0, uint32_t& mm, uint32_t& mp) {
         const uint16_t* b = &L.u.fb[r][seg];
@@ -477,6 +507,84 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
         if constexpr (NB != 6) rel(RE, R_E0, R_EM, R_EP, true, NB == 26, NB == 26);
         hD0 = M[R_D0];
       }
+      if constexpr (MODE == M_CONT) {
+        const VT delta = (VT)from_bits<T>(p.delta_bits);
+        uint32_t eq = 0;
+#pragma unroll
+        for (int k = 15; k >= 0; k--) {
+          const VT pv = k > 0 ? cur[k > 0 ? k - 1 : 0] : left;
+          push_bit(F, cont_fg(cur[k]));
+          push_eq(eq, cur[k], pv);
+          push_link(a, cur[k], pv, delta);
+        }
+        my_epl = (uint32_t)__popc(F & ~eq);
+        const uint32_t inner = first ? (a & ~1u) : a;
+        // One backward row: its links, and the kept ones.  Masks of 17 bits
+        // have the voxel before the segment in bit 0: the link of voxel k - 1
+        // to the voxel at x is a pair (a, q), so it covers p - q where p has
+        // the link a; xw: links along the row itself, w[k] - w[k + 1].
+        uint32_t bd = 0, ce = 0;
+        VT prow[16];  // rows B and C at 18-connectivity, for the pairs (b0, d0) and (c0, e0)
+        auto rel = [&](int dr, int i0, int im, int ip, bool diag, bool quirk, bool keep, uint32_t* pair,
+                       bool left_rule) {
+          const VT* w = base + dr * RSTR;
+          VT wv[18];
+#pragma unroll
+          for (int k = 0; k < 18; k++)
+            if (k < 17 || NB != 6) wv[k] = w[k - 1];
+          uint32_t x0m = 0, xpm = 0, xw = 0, eqm = 0;
+#pragma unroll
+          for (int k = 15; k >= -1; k--) {
+            const VT c = k >= 0 ? cur[k >= 0 ? k : 0] : left;
+            push_link(x0m, c, wv[k + 1], delta);
+            if (quirk) push_eq(eqm, c, wv[k + 1]);
+            if (diag) push_link(xpm, c, wv[k + 2], delta);
+            if (k >= 0 && diag) push_link(M[im], c, wv[k], delta);
+            if (NB == 6) {
+              if (k >= 0) push_link(xw, wv[k + 1], wv[k], delta);
+            } else if (diag) {
+              push_link(xw, wv[k + 2], wv[k + 1], delta);
+            }
+          }
+          if (pair) {
+#pragma unroll
+            for (int k = 15; k >= 0; k--) push_link(*pair, prow[k], wv[k + 1], delta);
+          }
+          if (keep) {
+#pragma unroll
+            for (int k = 0; k < 16; k++) prow[k] = wv[k + 1];
+          }
+          // equal to the voxel below: linked under 26-connectivity whatever delta says
+          // (cc3d/cc3d_continuous.hpp:147-150); a background c is masked by F below
+          if (quirk) {
+            const uint32_t f17 = (F << 1) | (cont_fg(left) ? 1u : 0u);
+            x0m |= eqm & f17;
+          }
+          M[i0] = x0m >> 1;
+          const uint32_t s0 = x0m & 0xFFFFu;  // voxel k - 1 to the voxel of im
+          if constexpr (NB == 6) {
+            const uint32_t cov = s0 & xw;
+            U[i0] = M[i0] & ~(inner & cov);
+            left_cov |= M[i0] & cov;
+          } else {
+            const uint32_t sp = xpm & 0xFFFFu;  // voxel k - 1 to the voxel of i0
+            uint32_t cov0 = rel_adj(R_A, i0, NB) ? (inner & sp) : 0u;
+            if (pair) cov0 |= M[i0 == R_D0 ? R_B0 : R_C0] & *pair;
+            U[i0] = M[i0] & ~cov0;
+            if (diag) {
+              M[ip] = xpm >> 1;
+              U[im] = M[im] & ~(inner & s0) & ~(M[i0] & xw);
+              U[ip] = M[ip] & ~(M[i0] & (xw >> 1));
+            }
+            if (left_rule) left_cov |= M[i0] & sp;
+          }
+        };
+        constexpr bool D = NB != 6, D26 = NB == 26, P18 = NB == 18;
+        rel(RB, R_B0, R_BM, R_BP, D, false, P18, nullptr, true);
+        if constexpr (NB != 6) rel(RD, R_D0, R_DM, R_DP, D26, false, false, P18 ? &bd : nullptr, false);
+        rel(RC, R_C0, R_CM, R_CP, D, NB == 26, P18, nullptr, true);
+        if constexpr (NB != 6) rel(RE, R_E0, R_EM, R_EP, D26, false, false, P18 ? &ce : nullptr, false);
+      }
     }
     const uint32_t ain = first ? (a & ~1u) : a;  // links a inside the tile
     if constexpr (MODE != M_CONT) {
@@ -501,6 +609,12 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
         }
         U[R_A] = a & ~ain & ~cova;
       }
+    } else {
+      any = a;
+#pragma unroll
+      for (int i = 0; i < R_A; i++)
+        if (rel_in(i, NB)) any |= M[i];
+      U[R_A] = a & ~ain & ~left_cov;
     }
     my_prov = (uint32_t)__popc(F & ~any);
   }
@@ -764,6 +878,9 @@ __global__ __launch_bounds__(GeoR::NT, (rows_waves<T, MODE>())) void k_rows_loca
 
 hipError_t launch_rows_multi(int dt, int nb, const LocalParams& p, hipStream_t s);
 hipError_t launch_rows_binary(int dt, int nb, const LocalParams& p, hipStream_t s);
+hipError_t launch_rows_cont(int dt, int nb, const LocalParams& p, hipStream_t s);
+hipError_t launch_rows_batch_cont(int dt, int nb, const LocalParams& p, const BatchVol* vols, const uint32_t* vix,
+                                  int64_t gtile0, int64_t gtiles, hipStream_t s);
 hipError_t launch_rows_batch_multi(int dt, int nb, const LocalParams& p, const BatchVol* vols, const uint32_t* vix,
                                    int64_t gtile0, int64_t gtiles, hipStream_t s);
 hipError_t launch_rows_batch_binary(int dt, int nb, const LocalParams& p, const BatchVol* vols, const uint32_t* vix,
