@@ -267,8 +267,8 @@ __global__ __launch_bounds__(WG) void k_requests(GlobalParams p) {
 // with its pair.  A table slot that another pair took only costs a repeated
 // union.
 constexpr int RRQ_SLOTS = 256;
+template <class G>
 __global__ __launch_bounds__(WG) void k_rrequests(GlobalParams p) {
-  using G = GeoR;
   __shared__ uint2 tab[WG / 64][RRQ_SLOTS];
   __shared__ uint32_t own[WG / 64][RRQ_SLOTS];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -299,7 +299,7 @@ __global__ __launch_bounds__(WG) void k_rrequests(GlobalParams p) {
         rel_decode(rq >> 12, dx, dy, dz);
         const int64_t gx = tx * G::TX + (ps & 63) + dx;
         const int64_t gy = ty * G::TY + ((ps >> 6) & (G::TY - 1)) + dy;
-        const int64_t gz = tz * G::TZ + (ps >> 9) + dz;
+        const int64_t gz = tz * G::TZ + ps / (64 * G::TY) + dz;
         b = lroot_index<G>(p, v, gx, gy, gz);
         a = root0 + j - 1;
       }
@@ -727,7 +727,7 @@ hipError_t scan_root_bits(const uint32_t* bits, int64_t nwords, uint32_t* bsum, 
   return hipGetLastError();
 }
 
-// Row tiles (GeoR): one workgroup per tile.  In pass i thread t takes the 4
+// Row tiles (GeoR, GeoP): one workgroup per tile.  In pass i thread t takes the 4
 // voxels at x = 4 (t & 15) of row 16 i + (t >> 4): 16 lanes read and write
 // one row, so a wave's stores cover whole 256-byte rows (uint32 labels) at
 // any row alignment.  All loads of the passes come before the label table's
@@ -735,42 +735,42 @@ hipError_t scan_root_bits(const uint32_t* bits, int64_t nwords, uint32_t* bsum, 
 // (512^3 uint32: 179 -> 166 us, with one component 148 -> 110 us); other rows
 // share lines with their neighbours and are merged in L2 instead (383 x 401 x
 // 367: 62 us, 105 us past the caches).
-template <class OUT>
+template <class OUT, class G>
 __device__ inline void rfin_tile(const GlobalParams& p, const VolGeo& v, int64_t tile, int64_t slot, uint32_t base,
                                  OUT* __restrict__ out, uint32_t* lab) {
-  constexpr int PASSES = GeoR::TV / (4 * WG);
+  constexpr int PASSES = G::TV / (4 * WG);
   const int t = threadIdx.x;
   const uint32_t R = p.TR[slot];
   uint32_t j[PASSES][2];  // two 16-bit entries per word
   if (R <= 255) {
 #pragma unroll
     for (int i = 0; i < PASSES; i++) {
-      const uint32_t w = reinterpret_cast<const uint32_t*>(p.J8 + slot * GeoR::TV)[t + WG * i];
+      const uint32_t w = reinterpret_cast<const uint32_t*>(p.J8 + slot * G::TV)[t + WG * i];
       j[i][0] = (w & 0xFFu) | ((w & 0xFF00u) << 8);
       j[i][1] = ((w >> 16) & 0xFFu) | ((w >> 8) & 0xFF0000u);
     }
   } else {
 #pragma unroll
     for (int i = 0; i < PASSES; i++) {
-      const uint2 w = reinterpret_cast<const uint2*>(p.J16 + slot * GeoR::TV)[t + WG * i];
+      const uint2 w = reinterpret_cast<const uint2*>(p.J16 + slot * G::TV)[t + WG * i];
       j[i][0] = w.x;
       j[i][1] = w.y;
     }
   }
-  const uint32_t root0 = slot_root0<GeoR>(v, slot);
+  const uint32_t root0 = slot_root0<G>(v, slot);
   if (t == 0) lab[0] = 0u;
   for (uint32_t i = t; i < R; i += WG) lab[i + 1] = root_label(p, kroot_key(p.GP, root0 + i), base);
   __syncthreads();
   const int64_t tz = tile / (v.ntx * v.nty);
   const int64_t tr = tile - tz * v.ntx * v.nty;
   const int64_t ty = tr / v.ntx, tx = tr - ty * v.ntx;
-  const int64_t gx = tx * GeoR::TX + 4 * (t & 15);
+  const int64_t gx = tx * G::TX + 4 * (t & 15);
   typedef OUT Pack __attribute__((ext_vector_type(4), aligned(sizeof(OUT))));
   const bool whole = ((uint64_t)v.sx * sizeof(OUT) % 128 | reinterpret_cast<uintptr_t>(out) % 128) == 0;
 #pragma unroll
   for (int i = 0; i < PASSES; i++) {
     const int row = 16 * i + (t >> 4);
-    const int64_t gy = ty * GeoR::TY + (row & (GeoR::TY - 1)), gz = tz * GeoR::TZ + row / GeoR::TY;
+    const int64_t gy = ty * G::TY + (row & (G::TY - 1)), gz = tz * G::TZ + row / G::TY;
     Pack k;
     k[0] = (OUT)lab[j[i][0] & 0xFFFFu];
     k[1] = (OUT)lab[j[i][0] >> 16];
@@ -789,11 +789,11 @@ __device__ inline void rfin_tile(const GlobalParams& p, const VolGeo& v, int64_t
   }
 }
 
-template <class OUT>
+template <class OUT, class G>
 __global__ __launch_bounds__(WG) void k_rfinalize(GlobalParams p, OUT* __restrict__ out) {
-  __shared__ uint32_t lab[GeoR::TV + 1];
+  __shared__ uint32_t lab[G::TV + 1];
   const int64_t tile = xcd_tile(blockIdx.x, p.ntiles);
-  rfin_tile<OUT>(p, vol_geo(p, 0), tile, tile, 0u, out, lab);
+  rfin_tile<OUT, G>(p, vol_geo(p, 0), tile, tile, 0u, out, lab);
 }
 
 __global__ __launch_bounds__(WG) void k_rfinalize_batch(GlobalParams p) {
@@ -802,9 +802,9 @@ __global__ __launch_bounds__(WG) void k_rfinalize_batch(GlobalParams p) {
   const BatchVol& bv = p.vols[p.vix[slot]];
   const VolGeo v = batch_geo(bv);
   const uint32_t base = p.prefix[bv.key0 >> 5];
-  if (bv.out_dtype == DT_U16) rfin_tile<uint16_t>(p, v, slot - bv.tile0, slot, base, static_cast<uint16_t*>(bv.out), lab);
-  else if (bv.out_dtype == DT_U64) rfin_tile<uint64_t>(p, v, slot - bv.tile0, slot, base, static_cast<uint64_t*>(bv.out), lab);
-  else rfin_tile<uint32_t>(p, v, slot - bv.tile0, slot, base, static_cast<uint32_t*>(bv.out), lab);
+  if (bv.out_dtype == DT_U16) rfin_tile<uint16_t, GeoR>(p, v, slot - bv.tile0, slot, base, static_cast<uint16_t*>(bv.out), lab);
+  else if (bv.out_dtype == DT_U64) rfin_tile<uint64_t, GeoR>(p, v, slot - bv.tile0, slot, base, static_cast<uint64_t*>(bv.out), lab);
+  else rfin_tile<uint32_t, GeoR>(p, v, slot - bv.tile0, slot, base, static_cast<uint32_t*>(bv.out), lab);
 }
 
 // Batch: the table entry of every tile (one block per volume).
@@ -1256,7 +1256,8 @@ struct Geometry {
   int64_t sx = 0, sy = 0, sz = 0, V = 0, K = 0, osx = 0;
   int nb = 0, qk = Q_NONE, mode = M_MULTI;
   bool is3d = true;
-  bool rows = false;  // row tiles (GeoR): 3D multilabel and binary
+  bool rows = false;   // row tiles (GeoR)
+  bool plane = false;  // row tiles of a single plane (GeoP)
   bool tall = false;  // tall voxel tiles (Geo3T) instead of Geo3
   int64_t ntx = 0, nty = 0, ntz = 0, ntiles = 0;
   int TV = 0;
@@ -1298,9 +1299,16 @@ static int plan(Geometry& g, int64_t sx, int64_t sy, int64_t sz, int64_t connect
   int TX, TY, TZ;
   // Row tiles for 3D volumes.
   g.rows = g.is3d && ((tiles & CC3D_AMD_TILES_ROWS) || !(tiles & (CC3D_AMD_TILES_VOXELS | CC3D_AMD_TILES_TALL)));
+  // Row tiles for single planes of at least 64 rows, which fill them, but for
+  // the continuous 2D-8 links.
+  g.plane = !g.is3d && sy >= GeoP::TY && g.qk != Q_CONT8 && !(tiles & (CC3D_AMD_TILES_VOXELS | CC3D_AMD_TILES_TALL));
   g.tall = g.is3d && !g.rows && (tiles & CC3D_AMD_TILES_TALL) && !(tiles & CC3D_AMD_TILES_VOXELS);
   if (g.rows) {
     TX = GeoR::TX; TY = GeoR::TY; TZ = GeoR::TZ; g.TV = GeoR::TV;
+    g.reqcap = row_req_cap(g.mode == M_CONT, g.nb);
+    g.req_bytes = (size_t)g.reqcap * sizeof(uint16_t);
+  } else if (g.plane) {
+    TX = GeoP::TX; TY = GeoP::TY; TZ = GeoP::TZ; g.TV = GeoP::TV;
     g.reqcap = row_req_cap(g.mode == M_CONT, g.nb);
     g.req_bytes = (size_t)g.reqcap * sizeof(uint16_t);
   } else if (g.tall) {
@@ -1455,8 +1463,9 @@ void launch_requests(const GlobalParams& p, int64_t ntiles, int mode, hipStream_
   else hipLaunchKernelGGL((k_requests<G, QK, 8>), dim3(grid_for(ntiles, WG / 8, 65536)), dim3(WG), 0, s, p);
 }
 
+template <class G>
 void launch_rrequests(const GlobalParams& p, int64_t ntiles, hipStream_t s) {
-  hipLaunchKernelGGL(k_rrequests, dim3(grid_for(ntiles, WG / 64, 65536)), dim3(WG), 0, s, p);
+  hipLaunchKernelGGL(k_rrequests<G>, dim3(grid_for(ntiles, WG / 64, 65536)), dim3(WG), 0, s, p);
 }
 
 template <class G>
@@ -1465,7 +1474,7 @@ int run_global(cc3d_amd_job* j) {
   hipStream_t s = j->stream;
   {
   ProfScope ps_("k_requests", s);
-  if constexpr (std::is_same<G, GeoR>::value) launch_rrequests(p, j->g.ntiles, s);
+  if constexpr (std::is_same<G, GeoR>::value || std::is_same<G, GeoP>::value) launch_rrequests<G>(p, j->g.ntiles, s);
   else if (j->g.qk == Q_BLOCK8) launch_requests<G, Q_BLOCK8>(p, j->g.ntiles, j->g.mode, s);
   else launch_requests<G, Q_NONE>(p, j->g.ntiles, j->g.mode, s);
   }
@@ -1784,7 +1793,7 @@ static int job_begin(cc3d_amd_job* j, const void* in, int in_dtype, int64_t sx, 
 
   LocalParams lp;
   lp.utab = nullptr;
-  if (!g.rows) {  // the row kernels need no union tables
+  if (!g.rows && !g.plane) {  // the row kernels need no union tables
     rc = utab_ready(&lp.utab, no_alloc ? s : nullptr);
     if (rc != CC3D_AMD_OK) return rc;
   }
@@ -1805,7 +1814,10 @@ static int job_begin(cc3d_amd_job* j, const void* in, int in_dtype, int64_t sx, 
   hipError_t e;
   {
   ProfScope ps_("k_local", s);
-  if (g.rows && g.mode == M_MULTI) e = launch_rows_multi(in_dtype, g.nb, lp, s);
+  if (g.plane && g.mode == M_MULTI) e = launch_rows_plane_multi(in_dtype, g.nb, g.qk, lp, s);
+  else if (g.plane && g.mode == M_CONT) e = launch_rows_plane_cont(in_dtype, g.nb, g.qk, lp, s);
+  else if (g.plane) e = launch_rows_plane_binary(in_dtype, g.nb, g.qk, lp, s);
+  else if (g.rows && g.mode == M_MULTI) e = launch_rows_multi(in_dtype, g.nb, lp, s);
   else if (g.rows && g.mode == M_CONT) e = launch_rows_cont(in_dtype, g.nb, lp, s);
   else if (g.rows) e = launch_rows_binary(in_dtype, g.nb, lp, s);
   else if (g.mode == M_MULTI) e = launch_local_multi(in_dtype, g.nb, g.qk, g.tall, lp, s);
@@ -1820,6 +1832,7 @@ static int job_begin(cc3d_amd_job* j, const void* in, int in_dtype, int64_t sx, 
   }
   if (hipGetLastError() != hipSuccess) return fail(CC3D_AMD_ERR_HIP, "k_tile_counters launch failed");
   rc = g.rows ? run_global<GeoR>(j)
+       : g.plane ? run_global<GeoP>(j)
        : g.tall ? run_global<Geo3T>(j)
        : g.is3d ? run_global<Geo3>(j)
                 : run_global<Geo2>(j);
@@ -1880,7 +1893,8 @@ int cc3d_amd_label_finish(cc3d_amd_job* j, void* out, int out_dtype) {
   ProfScope ps_("k_finalize", s);
 #define CC3D_F(OUT)                                                                                \
   do {                                                                                             \
-    if (g.rows) hipLaunchKernelGGL((k_rfinalize<OUT>), dim3((unsigned)g.ntiles), block, 0, s, j->gp, (OUT*)out); \
+    if (g.rows) hipLaunchKernelGGL((k_rfinalize<OUT, GeoR>), dim3((unsigned)g.ntiles), block, 0, s, j->gp, (OUT*)out); \
+    else if (g.plane) hipLaunchKernelGGL((k_rfinalize<OUT, GeoP>), dim3((unsigned)g.ntiles), block, 0, s, j->gp, (OUT*)out); \
     else if (g.tall) hipLaunchKernelGGL((k_finalize<OUT, Geo3T>), grid3t, block, 0, s, j->gp, (OUT*)out); \
     else if (g.is3d) hipLaunchKernelGGL((k_finalize<OUT, Geo3>), grid3, block, 0, s, j->gp, (OUT*)out); \
     else hipLaunchKernelGGL((k_finalize<OUT, Geo2>), grid2, block, 0, s, j->gp, (OUT*)out);        \
@@ -2505,7 +2519,7 @@ int cc3d_amd_batch_begin(cc3d_amd_batch* b) {
   {
     ProfScope ps_("k_requests", s);
     for (const auto& tg : b->tgroups) {
-      if (tg.rows()) launch_rrequests(tg.gp, tg.tiles, s);
+      if (tg.rows()) launch_rrequests<GeoR>(tg.gp, tg.tiles, s);
       else if (tg.fam == cc3d_amd_batch::FAM_TALL) launch_requests<Geo3T, Q_NONE>(tg.gp, tg.tiles, b->mode, s);
       else if (tg.fam == cc3d_amd_batch::FAM_PLANE) launch_requests<Geo2, Q_NONE>(tg.gp, tg.tiles, b->mode, s);
       else launch_requests<Geo3, Q_NONE>(tg.gp, tg.tiles, b->mode, s);

@@ -48,21 +48,23 @@
 
 namespace cc3d_amd {
 
-// Tile geometry of the row kernels: 64 rows of 64 voxels.  Box rows (by, bz):
-// by = y + 1, bz = z + 1, one halo row or plane on each side that backward
-// neighbours reach.
+// Tile geometry of the row kernels: 64 rows of 64 voxels, 8 x 8 of them for
+// volumes (GeoR) and 64 x 1 for single planes (GeoP).  Box rows (by, bz): by =
+// y + 1, bz = z + 1 (0 in a plane), one halo row or plane on each side that
+// backward neighbours reach.
 template <int TY_, int TZ_>
 struct RowGeo {
   static constexpr int TX = 64, TY = TY_, TZ = TZ_;
-  static constexpr bool IS3D = true;
+  static constexpr bool IS3D = TZ > 1;
   static constexpr int NT = 256;
   static constexpr int TV = TX * TY * TZ;
-  static constexpr int BY = TY + 2, BZ = TZ + 1;
+  static constexpr int BY = IS3D ? TY + 2 : TY + 1, BZ = IS3D ? TZ + 1 : 1;
   static constexpr int NROWS = BY * BZ;
   static_assert(TY * TZ == 64, "one row per lane of a wave");
   __device__ static inline int jidx(int lx, int ly, int lz) { return lx + TX * (ly + TY * lz); }
 };
 using GeoR = RowGeo<8, 8>;
+using GeoP = RowGeo<64, 1>;
 
 // Relations in covering order; index 12 is a.  Offsets as (d + 1) in 2-bit
 // fields per axis.
@@ -98,6 +100,7 @@ __host__ __device__ constexpr bool off_in(int dx, int dy, int dz, int nb) {
   const int ax = dx < 0 ? -dx : dx, ay = dy < 0 ? -dy : dy, az = dz < 0 ? -dz : dz;
   const int l1 = ax + ay + az;
   if (ax > 1 || ay > 1 || az > 1) return false;
+  if (nb == 8 || nb == 4) return az == 0 && (nb == 8 || l1 <= 1);
   return nb == 26 || (nb == 18 && l1 <= 2) || (nb == 6 && l1 <= 1);
 }
 __host__ __device__ constexpr bool rel_in(int r, int nb) {
@@ -118,9 +121,10 @@ __device__ inline void rel_decode(uint32_t r, int& dx, int& dy, int& dz) {
 // Bound on the requests of a tile.  Multilabel and binary: the largest number
 // of kept relations that leave the tile, over every set of links a voxel can
 // have, summed over the tile's voxels (4,036 at 26-connectivity, 2,537 at
-// 18, 1,088 at 6).  Continuous: all relations that leave the tile.
+// 18, 1,088 at 6).  Continuous volumes and planes: all relations that leave
+// the tile (382 in a plane).
 __host__ __device__ constexpr int row_req_cap(bool cont, int nb) {
-  return nb == 6 ? 1088 : nb == 18 ? (cont ? 5280 : 2540) : (cont ? 9316 : 4036);
+  return nb == 8 || nb == 4 ? 384 : nb == 6 ? 1088 : nb == 18 ? (cont ? 5280 : 2540) : (cont ? 9316 : 4036);
 }
 
 // Staged voxel type: 4 bytes for every type up to 4 bytes, else the type.
@@ -144,9 +148,23 @@ struct RowVal<double> {
 constexpr int RSTR = 68;     // row stride of staged values and nodes: 16-byte accesses of 64 rows spread over all banks
 constexpr int RQCAP = 1024;  // queued links per wave; one relation of a wave's segments always fits
 
-template <class T, int MODE>
+// LDS index of a tile voxel's node: raster order, or for the binary 2D
+// 8-connected numbering the order of the 2x2 block keys (pairs of rows, 4
+// nodes a block, 132 a pair).
+template <int QK>
+__device__ inline uint32_t row_node(uint32_t x, uint32_t row) {
+  if (QK == Q_BLOCK8) return 132u * (row >> 1) + 4u * (x >> 1) + 2u * (row & 1u) + (x & 1u);
+  return RSTR * row + x;
+}
+// Node of voxel k of a segment whose first voxel has node n0.
+template <int QK>
+__device__ inline uint32_t seg_node(uint32_t n0, uint32_t k) {
+  return QK == Q_BLOCK8 ? n0 + 4u * (k >> 1) + (k & 1u) : n0 + k;
+}
+
+template <class T, int MODE, class G_ = GeoR>
 struct RowLds {
-  using G = GeoR;
+  using G = G_;
   using VT = typename RowVal<T>::type;
   struct Work {
     uint32_t par[64 * RSTR];
@@ -159,6 +177,7 @@ struct RowLds {
     uint16_t fb[G::NROWS][6];
     Work w;
   } u;
+  uint16_t ne0[4];  // binary 2D-4: values of the plane's first row that differ from the one before
   uint32_t nreq;
   uint32_t wtot[4], red_epl[4], red_prov[4];
   uint64_t rows[4];
@@ -313,10 +332,11 @@ __device__ inline uint32_t nonzero_bytes(const uint32_t (&w)[4]) {
   return out[0] | (out[1] << 8);
 }
 
-template <class T, int MODE, int NB>
+template <class T, int MODE, int NB, class G, int QK>
 __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, int64_t sy, int64_t sz, int64_t ntx,
-                                 int64_t nty, int64_t tile, int64_t slot, uint32_t keybase, RowLds<T, MODE>& L) {
-  using G = GeoR;
+                                 int64_t nty, int64_t tile, int64_t slot, uint32_t keybase, RowLds<T, MODE, G>& L) {
+  constexpr bool IS3D = G::IS3D;
+  constexpr bool FACE = NB == 6 || NB == 4;  // face links only
   using VT = typename RowVal<T>::type;
   const int t = threadIdx.x, lane = t & 63;
   const int seg = __builtin_amdgcn_readfirstlane(t >> 6);  // one segment per wave
@@ -329,11 +349,12 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
 
   // 1. stage the box: rows r = by + BY * bz.  Row BY - 1 of the last plane is
   //    reached by no voxel.  Voxels outside the volume are background.
-  const T* box = in + ((x0 - 1) + sx * ((y0 - 1) + sy * (z0 - 1)));  // box position (-1, -1, -1); dereferenced inside the volume only
+  // box position (-1, -1, -1) ((-1, -1) in a plane); dereferenced inside the volume only
+  const T* box = in + ((x0 - 1) + sx * ((y0 - 1) + (IS3D ? sy * (z0 - 1) : 0)));
   const int64_t xleft = sx - x0;                                     // voxels of a row from x0 on
   auto row_ok = [&](int by, int bz) -> bool {
     const int64_t gy = y0 + by - 1, gz = z0 + bz - 1;
-    return gy >= 0 && gy < sy && gz >= 0 && gz < sz;
+    return gy >= 0 && gy < sy && (!IS3D || (gz >= 0 && gz < sz));
   };
   auto row_ptr = [&](int by, int bz) -> const T* { return box + (1 + sx * (by + sy * (int64_t)bz)); };  // its x0
   if constexpr (MODE == M_BINARY) {
@@ -349,7 +370,7 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
       uint32_t F = 0, NE = 0;  // NE: differs from the voxel before it (tile rows)
       if (row_ok(by, bz) && 16 * s < xleft) {
         const T* e = row_ptr(by, bz) + 16 * s;
-        const bool own = by >= 1 && by <= G::TY && bz >= 1;
+        const bool own = by >= 1 && by <= G::TY && (!IS3D || bz >= 1);
         T prev = T(0);
         if (own && x0 + 16 * s > 0) prev = e[-1];
         if (16 * s + 16 <= xleft) {
@@ -380,6 +401,7 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
           }
         }
         if (own) my_epl += (uint32_t)__popc(F & NE);
+        if (QK == Q_BIN4 && by == 1) L.ne0[s] = (uint16_t)NE;
       }
       L.u.fb[r][s + 1] = (uint16_t)F;
     }
@@ -401,7 +423,7 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
       const int bz = r / G::BY, by = r - bz * G::BY;
 #pragma unroll
       for (int k = 0; k < 4; k++) v[q][k] = T(0);
-      if (r < G::NROWS - 1 && row_ok(by, bz)) {
+      if (r < (IS3D ? G::NROWS - 1 : G::NROWS) && row_ok(by, bz)) {
         const T* e = row_ptr(by, bz) + q4;
         if (q4 + 4 <= xleft) {
           load_run<T, 4>(e, v[q]);
@@ -433,7 +455,7 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
 
   // 2. the segment's masks (bit k: voxel 16 seg + k of row `lane`)
   const int ly = lane & (G::TY - 1), lz = lane / G::TY;
-  const int r0 = (ly + 1) + G::BY * (lz + 1);
+  const int r0 = (ly + 1) + (IS3D ? G::BY * (lz + 1) : 0);
   constexpr int RB = -1, RC = -G::BY, RD = -G::BY - 1, RE = -G::BY + 1;  // box rows B, C, D, E from r0
   const bool first = seg == 0;  // bit 0 is the tile's first column
   uint32_t F = 0, a = 0;
@@ -466,10 +488,17 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
         M[ip] = F & mp;
       };
       rel(RB, R_B0, R_BM, R_BP);
-      rel(RC, R_C0, R_CM, R_CP);
-      rel(RD, R_D0, R_DM, R_DP);
-      if constexpr (NB != 6) rel(RE, R_E0, R_EM, R_EP);
-      hD0 = M[R_D0];
+      if constexpr (IS3D) {
+        rel(RC, R_C0, R_CM, R_CP);
+        rel(RD, R_D0, R_DM, R_DP);
+        if constexpr (!FACE) rel(RE, R_E0, R_EM, R_EP);
+        hD0 = M[R_D0];
+      }
+      if constexpr (QK == Q_BIN4) {
+        // the first row links on equal values, later rows to the left unless
+        // the two pixels above are both set (cc3d/cc3d_binary.hpp:822-935)
+        a &= y0 + ly == 0 ? ~(uint32_t)L.ne0[seg] : ~(M[R_B0] & M[R_BM]);
+      }
     } else {
       const VT* base = static_cast<const VT*>(__builtin_assume_aligned(L.u.v + (r0 * RSTR + 4 + 16 * seg), 16));
       VT cur[16];
@@ -501,11 +530,13 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
           if (WM) M[im] &= F;
           if (WP) M[ip] &= F;
         };
-        rel(RB, R_B0, R_BM, R_BP, true, true, NB != 6);
-        rel(RC, R_C0, R_CM, R_CP, true, true, NB != 6);
-        rel(RD, R_D0, R_DM, R_DP, true, NB == 26, NB == 26);
-        if constexpr (NB != 6) rel(RE, R_E0, R_EM, R_EP, true, NB == 26, NB == 26);
-        hD0 = M[R_D0];
+        rel(RB, R_B0, R_BM, R_BP, true, true, !FACE);
+        if constexpr (IS3D) {
+          rel(RC, R_C0, R_CM, R_CP, true, true, !FACE);
+          rel(RD, R_D0, R_DM, R_DP, true, NB == 26, NB == 26);
+          if constexpr (!FACE) rel(RE, R_E0, R_EM, R_EP, true, NB == 26, NB == 26);
+          hD0 = M[R_D0];
+        }
       }
       if constexpr (MODE == M_CONT) {
         const VT delta = (VT)from_bits<T>(p.delta_bits);
@@ -531,7 +562,7 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
           VT wv[18];
 #pragma unroll
           for (int k = 0; k < 18; k++)
-            if (k < 17 || NB != 6) wv[k] = w[k - 1];
+            if (k < 17 || !FACE) wv[k] = w[k - 1];
           uint32_t x0m = 0, xpm = 0, xw = 0, eqm = 0;
 #pragma unroll
           for (int k = 15; k >= -1; k--) {
@@ -540,7 +571,7 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
             if (quirk) push_eq(eqm, c, wv[k + 1]);
             if (diag) push_link(xpm, c, wv[k + 2], delta);
             if (k >= 0 && diag) push_link(M[im], c, wv[k], delta);
-            if (NB == 6) {
+            if (FACE) {
               if (k >= 0) push_link(xw, wv[k + 1], wv[k], delta);
             } else if (diag) {
               push_link(xw, wv[k + 2], wv[k + 1], delta);
@@ -562,7 +593,7 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
           }
           M[i0] = x0m >> 1;
           const uint32_t s0 = x0m & 0xFFFFu;  // voxel k - 1 to the voxel of im
-          if constexpr (NB == 6) {
+          if constexpr (FACE) {
             const uint32_t cov = s0 & xw;
             U[i0] = M[i0] & ~(inner & cov);
             left_cov |= M[i0] & cov;
@@ -579,16 +610,20 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
             if (left_rule) left_cov |= M[i0] & sp;
           }
         };
-        constexpr bool D = NB != 6, D26 = NB == 26, P18 = NB == 18;
+        constexpr bool D = !FACE, D26 = NB == 26, P18 = NB == 18;
         rel(RB, R_B0, R_BM, R_BP, D, false, P18, nullptr, true);
-        if constexpr (NB != 6) rel(RD, R_D0, R_DM, R_DP, D26, false, false, P18 ? &bd : nullptr, false);
-        rel(RC, R_C0, R_CM, R_CP, D, NB == 26, P18, nullptr, true);
-        if constexpr (NB != 6) rel(RE, R_E0, R_EM, R_EP, D26, false, false, P18 ? &ce : nullptr, false);
+        if constexpr (IS3D && !FACE) rel(RD, R_D0, R_DM, R_DP, D26, false, false, P18 ? &bd : nullptr, false);
+        if constexpr (IS3D) rel(RC, R_C0, R_CM, R_CP, D, NB == 26, P18, nullptr, true);
+        if constexpr (IS3D && !FACE) rel(RE, R_E0, R_EM, R_EP, D26, false, false, P18 ? &ce : nullptr, false);
       }
     }
     const uint32_t ain = first ? (a & ~1u) : a;  // links a inside the tile
     if constexpr (MODE != M_CONT) {
-      if constexpr (NB == 6) {
+      if constexpr (QK == Q_BIN4) {
+        any = a | M[R_B0];
+        U[R_B0] = M[R_B0];  // the reference's own links, none covered
+        U[R_A] = a & ~ain;
+      } else if constexpr (FACE) {
         any = a | M[R_B0] | M[R_C0];
         U[R_B0] = M[R_B0] & ~(ain & M[R_BM]);
         U[R_C0] = M[R_C0] & ~(ain & M[R_CM]) & ~(M[R_B0] & hD0);
@@ -616,7 +651,7 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
         if (rel_in(i, NB)) any |= M[i];
       U[R_A] = a & ~ain & ~left_cov;
     }
-    my_prov = (uint32_t)__popc(F & ~any);
+    if (QK != Q_BLOCK8) my_prov = (uint32_t)__popc(F & ~any);  // block labels are counted separately
   }
   const uint32_t S = F & (first ? ~(a & ~1u) : ~a);  // run starts inside the tile
   const uint64_t fgrows = wave_ballot(F != 0u);
@@ -626,23 +661,25 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
   uint32_t* par = L.u.w.par;
   uint16_t* queue = L.u.w.queue[seg];
   {
-    const uint32_t n0 = (uint32_t)(lane * RSTR + 16 * seg);
-    uint32_t v = n0 - 1u;  // a segment that continues a run hangs on the voxel before it
+    const uint32_t n0 = row_node<QK>(16u * (uint32_t)seg, (uint32_t)lane);
+    // a segment that continues a run hangs on the voxel before it
+    uint32_t v = QK == Q_BLOCK8 ? n0 - 3u : n0 - 1u;
+    constexpr int ST = QK == Q_BLOCK8 ? 2 : 4;  // consecutive nodes
 #pragma unroll
-    for (int k = 0; k < 16; k += 4) {
-      uint32_t w[4];
+    for (int k = 0; k < 16; k += ST) {
+      uint32_t w[ST];
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
+      for (int i = 0; i < ST; i++) {
         if (k + i == 1) v = (S & 1u) ? v : n0;
-        v = ((S >> (k + i)) & 1u) ? n0 + (uint32_t)(k + i) : v;
+        v = ((S >> (k + i)) & 1u) ? seg_node<QK>(n0, (uint32_t)(k + i)) : v;
         w[i] = v;
       }
-      uint32_t* d = static_cast<uint32_t*>(__builtin_assume_aligned(par + n0 + k, 16));
+      uint32_t* d = static_cast<uint32_t*>(__builtin_assume_aligned(par + seg_node<QK>(n0, (uint32_t)k), 4 * ST));
 #pragma unroll
-      for (int i = 0; i < 4; i++) d[i] = w[i];
+      for (int i = 0; i < ST; i++) d[i] = w[i];
     }
   }
-  constexpr int NWORD = NB == 6 ? 1 : NB == 18 ? 4 : 6;
+  constexpr int NWORD = FACE ? 1 : NB == 8 ? 2 : NB == 18 ? 4 : 6;
   const uint32_t pos0 = (uint32_t)(lane * G::TX + 16 * seg);
   uint32_t W[6];  // two relations each: 2 i in the low half, 2 i + 1 in the high half
   uint32_t cnt = U[R_A];
@@ -681,12 +718,11 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
         e = queue[i];
         int dx, dy, dz;
         rel_decode(e >> 12, dx, dy, dz);
-        const int x = (int)(e & 63u) + dx, y = (int)((e >> 6) & (G::TY - 1)) + dy, z = (int)((e >> 9) & (G::TZ - 1)) + dz;
+        const uint32_t ps = e & 0xFFFu;
+        const int x = (int)(ps & 63u) + dx, y = (int)((ps >> 6) & (G::TY - 1)) + dy, z = (int)(ps / (64u * G::TY)) + dz;
         out = x < 0 || x >= G::TX || y < 0 || y >= G::TY || z < 0;
-        if (!out) {
-          const uint32_t ps = e & 0xFFFu;
-          runion(par, ps + 4u * (ps >> 6), (uint32_t)(x + RSTR * (y + G::TY * z)));
-        }
+        if (!out)
+          runion(par, row_node<QK>(ps & 63u, ps >> 6), row_node<QK>((uint32_t)x, (uint32_t)(y + G::TY * z)));
       }
       const uint64_t m = wave_ballot(out);
       if (m) {
@@ -749,10 +785,10 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
   const uint32_t sf = qs[hrow];
   const uint32_t hS = sf & 0xFFFFu, hF = sf >> 16;
   const uint32_t H = hS | (hF & 1u);
-  const uint32_t h0 = (uint32_t)(hrow * RSTR + 16 * hseg);
+  const uint32_t h0 = row_node<QK>(16u * (uint32_t)hseg, (uint32_t)hrow);
   uint32_t rb = 0;  // roots of this segment
   for (uint32_t m = H; m; m &= m - 1u) {
-    const uint32_t k = (uint32_t)__builtin_ctz(m), n = h0 + k;
+    const uint32_t k = (uint32_t)__builtin_ctz(m), n = seg_node<QK>(h0, k);
     const uint32_t r = rfind_ro(par, n);
     if (r == n) rb |= 1u << k;
     else lstore(par + n, r);
@@ -773,10 +809,18 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
 
   // 6. heads: 1 + the rank of their root
   for (uint32_t m = H; m; m &= m - 1u) {
-    const uint32_t k = (uint32_t)__builtin_ctz(m), n = h0 + k;
+    const uint32_t k = (uint32_t)__builtin_ctz(m), n = seg_node<QK>(h0, k);
     const uint32_t r = par[n];
-    const uint32_t row = (r * 61681u) >> 22;  // r / 68 for r < 64 * 68
-    const uint32_t x = r - RSTR * row;
+    uint32_t row, x;
+    if (QK == Q_BLOCK8) {
+      const uint32_t pr = (r * 31776u) >> 22;  // r / 132 for r < 32 * 132
+      const uint32_t rem = r - 132u * pr;
+      row = 2u * pr + ((rem >> 1) & 1u);
+      x = 2u * (rem >> 2) + (rem & 1u);
+    } else {
+      row = (r * 61681u) >> 22;  // r / 68 for r < 64 * 68
+      x = r - RSTR * row;
+    }
     const uint32_t w = reinterpret_cast<const uint32_t*>(L.u.w.queue[x >> 4])[64 + row];
     par[n] = (w >> 16) + (uint32_t)__popc(w & ((1u << (x & 15u)) - 1u)) + 1u;
   }
@@ -785,7 +829,16 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
   //    cancel).  A segment's keys are consecutive, so its root marks are one
   //    or two words.
   const uint32_t root0 = tile_root0<G>(sx, sy, sz, tx, ty, tz, keybase);
-  if (rb) {
+  if (QK == Q_BLOCK8) {
+    uint32_t rk = root0 + rbase;
+    for (uint32_t m = rb; m; m &= m - 1u) {
+      const uint32_t key =
+        gkey<QK>(x0 + 16 * hseg + __builtin_ctz(m), y0 + hrow, 0, sx, sy, p.osx) + keybase;
+      p.GP[rk] = make_uint2(rk, key);
+      atomicOr(p.bits + (key >> 5), 1u << (key & 31));
+      rk++;
+    }
+  } else if (rb) {
     const uint32_t key0 = (uint32_t)x0 + 16u * (uint32_t)hseg +
                           (uint32_t)sx * ((uint32_t)(y0 + (hrow & (G::TY - 1))) +
                                           (uint32_t)sy * (uint32_t)(z0 + hrow / G::TY)) + keybase;
@@ -800,13 +853,21 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
   }
   {
     uint32_t j = 0, pk[8];
+    uint32_t v[16];
+    constexpr int ST = QK == Q_BLOCK8 ? 2 : 4;
+#pragma unroll
+    for (int k = 0; k < 16; k += ST) {
+      const uint32_t* q =
+        static_cast<const uint32_t*>(__builtin_assume_aligned(par + seg_node<QK>(h0, (uint32_t)k), 4 * ST));
+#pragma unroll
+      for (int i = 0; i < ST; i++) v[k + i] = q[i];
+    }
 #pragma unroll
     for (int k = 0; k < 16; k += 4) {
-      const uint32_t* v = static_cast<const uint32_t*>(__builtin_assume_aligned(par + h0 + k, 16));
       uint32_t o[4];
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        j = ((H >> (k + i)) & 1u) ? v[i] : j;
+        j = ((H >> (k + i)) & 1u) ? v[k + i] : j;
         o[i] = ((hF >> (k + i)) & 1u) ? j : 0u;
       }
       pk[k / 2] = o[0] | (o[1] << 16);
@@ -860,7 +921,16 @@ template <class T, int MODE, int NB>
 __global__ __launch_bounds__(GeoR::NT, (rows_waves<T, MODE>())) void k_rows_local(LocalParams p) {
   __shared__ RowLds<T, MODE> L;
   const int64_t tile = xcd_tile(blockIdx.x, p.ntiles);
-  rows_tile<T, MODE, NB>(p, static_cast<const T*>(p.in), p.sx, p.sy, p.sz, p.ntx, p.nty, tile, tile, 0u, L);
+  rows_tile<T, MODE, NB, GeoR, Q_NONE>(p, static_cast<const T*>(p.in), p.sx, p.sy, p.sz, p.ntx, p.nty, tile, tile, 0u,
+                                       L);
+}
+
+// Single planes of at least 64 rows.
+template <class T, int MODE, int NB, int QK>
+__global__ __launch_bounds__(GeoP::NT, (rows_waves<T, MODE>())) void k_rows_plane(LocalParams p) {
+  __shared__ RowLds<T, MODE, GeoP> L;
+  const int64_t tile = xcd_tile(blockIdx.x, p.ntiles);
+  rows_tile<T, MODE, NB, GeoP, QK>(p, static_cast<const T*>(p.in), p.sx, p.sy, 1, p.ntx, p.nty, tile, tile, 0u, L);
 }
 
 // Batch: tiles [gtile0, gtile0 + gtiles) of volumes of connectivity NB; each
@@ -872,12 +942,17 @@ __global__ __launch_bounds__(GeoR::NT, (rows_waves<T, MODE>())) void k_rows_loca
   __shared__ RowLds<T, MODE> L;
   const int64_t slot = gtile0 + xcd_tile(blockIdx.x, gtiles);
   const BatchVol& v = vols[vix[slot]];
-  rows_tile<T, MODE, NB>(p, static_cast<const T*>(v.in), v.sx, v.sy, v.sz, v.ntx, v.nty, slot - v.tile0, slot, v.key0,
-                         L);
+  rows_tile<T, MODE, NB, GeoR, Q_NONE>(p, static_cast<const T*>(v.in), v.sx, v.sy, v.sz, v.ntx, v.nty, slot - v.tile0,
+                                       slot, v.key0, L);
 }
 
 hipError_t launch_rows_multi(int dt, int nb, const LocalParams& p, hipStream_t s);
 hipError_t launch_rows_binary(int dt, int nb, const LocalParams& p, hipStream_t s);
+// Planes on the row tiles: every mode and numbering but continuous 2D-8
+// (Q_CONT8), whose links depend on the plane's extremes.
+hipError_t launch_rows_plane_multi(int dt, int nb, int qk, const LocalParams& p, hipStream_t s);
+hipError_t launch_rows_plane_binary(int dt, int nb, int qk, const LocalParams& p, hipStream_t s);
+hipError_t launch_rows_plane_cont(int dt, int nb, int qk, const LocalParams& p, hipStream_t s);
 hipError_t launch_rows_cont(int dt, int nb, const LocalParams& p, hipStream_t s);
 hipError_t launch_rows_batch_cont(int dt, int nb, const LocalParams& p, const BatchVol* vols, const uint32_t* vix,
                                   int64_t gtile0, int64_t gtiles, hipStream_t s);
@@ -896,6 +971,36 @@ hipError_t launch_rows_mode(int dt, int nb, const LocalParams& p, hipStream_t s)
     case 18: CC3D_R(T, 18); break;        \
     case 6: CC3D_R(T, 6); break;          \
     default: return hipErrorInvalidValue; \
+  }
+  switch (dt) {
+    case DT_U8: CC3D_RNB(uint8_t); break;
+    case DT_U16: CC3D_RNB(uint16_t); break;
+    case DT_U32: CC3D_RNB(uint32_t); break;
+    case DT_U64: CC3D_RNB(uint64_t); break;
+    case DT_F32: CC3D_RNB(float); break;
+    case DT_F64: CC3D_RNB(double); break;
+    default: return hipErrorInvalidValue;
+  }
+#undef CC3D_RNB
+#undef CC3D_R
+  return hipGetLastError();
+}
+
+template <int MODE>
+hipError_t launch_rows_plane_mode(int dt, int nb, int qk, const LocalParams& p, hipStream_t s) {
+  const dim3 grid((unsigned)p.ntiles), block(GeoP::NT);
+#define CC3D_R(T, NB, QK) hipLaunchKernelGGL((k_rows_plane<T, MODE, NB, QK>), grid, block, 0, s, p)
+#define CC3D_RNB(T)                                                                            \
+  if (nb == 8 && qk == Q_BLOCK8 && MODE == M_BINARY) {                                         \
+    CC3D_R(T, 8, (MODE == M_BINARY ? Q_BLOCK8 : Q_NONE));                                      \
+  } else if (nb == 4 && qk == Q_BIN4 && MODE == M_BINARY) {                                    \
+    CC3D_R(T, 4, (MODE == M_BINARY ? Q_BIN4 : Q_NONE));                                        \
+  } else if (nb == 8 && qk == Q_NONE) {                                                        \
+    CC3D_R(T, 8, Q_NONE);                                                                      \
+  } else if (nb == 4 && qk == Q_NONE) {                                                        \
+    CC3D_R(T, 4, Q_NONE);                                                                      \
+  } else {                                                                                     \
+    return hipErrorInvalidValue;                                                               \
   }
   switch (dt) {
     case DT_U8: CC3D_RNB(uint8_t); break;

@@ -9,4 +9,7 @@ hipError_t launch_rows_batch_cont(int dt, int nb, const LocalParams& p, const Ba
                                   int64_t gtile0, int64_t gtiles, hipStream_t s) {
   return launch_rows_batch_mode<M_CONT>(dt, nb, p, vols, vix, gtile0, gtiles, s);
 }
+hipError_t launch_rows_plane_cont(int dt, int nb, int qk, const LocalParams& p, hipStream_t s) {
+  return launch_rows_plane_mode<M_CONT>(dt, nb, qk, p, s);
+}
 }  // namespace cc3d_amd

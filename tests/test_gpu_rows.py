@@ -74,6 +74,28 @@ def test_continuous_special_values(gpu):
         _check(vol, f"special values {delta}", connectivity=conn, delta=delta)
 
 
+PLANES = [(1, 64), (15, 65), (16, 127), (17, 128), (63, 66), (64, 64), (65, 129), (130, 71)]
+
+
+@pytest.mark.parametrize("connectivity", [4, 8, 6, 26])
+@pytest.mark.parametrize("dtype", [np.uint8, np.uint32, np.uint64, np.float32])
+def test_plane_edges(gpu, dtype, connectivity):
+  """Planes on 64 x 64 tiles in every mode, with the block numbering of
+  binary 8 and the first-row rule of binary 4 (values of one image differ)."""
+  rng = np.random.default_rng(13 * connectivity + np.dtype(dtype).itemsize)
+  for k, shape in enumerate(PLANES):
+    vol = rng.integers(0, 3, size=shape).astype(dtype)
+    vol = np.asfortranarray(vol) if k & 1 else np.ascontiguousarray(vol.T)
+    _check(vol, f"multilabel {k}", connectivity=connectivity)
+    _check(vol, f"binary {k}", connectivity=connectivity, binary_image=True)
+    if connectivity in (4, 8, 6):
+      _check(vol, f"periodic {k}", connectivity=connectivity, periodic_boundary=True)
+      _check(vol, f"periodic binary {k}", connectivity=connectivity, periodic_boundary=True, binary_image=True)
+    many = (rng.integers(0, 7, size=shape) * 2).astype(dtype)
+    many = np.asfortranarray(many) if k & 1 else np.ascontiguousarray(many.T)
+    _check(many, f"continuous {k}", connectivity=connectivity, delta=2)
+
+
 def test_special_float_values(gpu):
   """NaN equals nothing (not even itself), infinities and signed zeros follow ==."""
   rng = np.random.default_rng(5)
