@@ -156,6 +156,7 @@ __global__ __launch_bounds__(WG) void k_tile_counters(const TileCnt* tc, int64_t
 struct GlobalParams {
   int64_t sx, sy, sz, osx;
   int64_t ntx, nty, ntz, ntiles;
+  Div dxy, dx;  // by ntx * nty and by ntx
   uint2* GP;
   const uint32_t* TR;
   const uint8_t* J8;
@@ -184,6 +185,7 @@ struct GlobalParams {
 struct VolGeo {
   int64_t sx, sy, sz, osx, ntx, nty, ntz, tile0;
   uint32_t key0;
+  Div dxy, dx;
 };
 
 __device__ inline VolGeo batch_geo(const BatchVol& v) {
@@ -192,6 +194,8 @@ __device__ inline VolGeo batch_geo(const BatchVol& v) {
   g.ntx = v.ntx; g.nty = v.nty; g.ntz = v.ntz;
   g.tile0 = v.tile0;
   g.key0 = v.key0;
+  g.dxy = v.dxy;
+  g.dx = v.dx;
   return g;
 }
 
@@ -202,6 +206,8 @@ __device__ inline VolGeo vol_geo(const GlobalParams& p, int64_t slot) {
   g.ntx = p.ntx; g.nty = p.nty; g.ntz = p.ntz;
   g.tile0 = p.tile0;
   g.key0 = p.key0;
+  g.dxy = p.dxy;
+  g.dx = p.dx;
   return g;
 }
 
@@ -220,10 +226,8 @@ __device__ inline uint32_t lroot_index(const GlobalParams& p, const VolGeo& v, i
 // First forest entry of tile `slot` of volume v.
 template <class G>
 __device__ inline uint32_t slot_root0(const VolGeo& v, int64_t slot) {
-  const int64_t tile = slot - v.tile0;
-  const int64_t tz = tile / (v.ntx * v.nty);
-  const int64_t tr = tile - tz * v.ntx * v.nty;
-  const int64_t ty = tr / v.ntx, tx = tr - ty * v.ntx;
+  int64_t tx, ty, tz;
+  tile_coords((uint32_t)(slot - v.tile0), v.ntx, v.nty, v.dxy, v.dx, tx, ty, tz);
   return tile_root0<G>(v.sx, v.sy, v.sz, tx, ty, tz, v.key0);
 }
 
@@ -271,7 +275,7 @@ template <class G>
 __global__ __launch_bounds__(WG) void k_rrequests(GlobalParams p) {
   __shared__ uint2 tab[WG / 64][RRQ_SLOTS];
   __shared__ uint32_t own[WG / 64][RRQ_SLOTS];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t w0 = (int64_t)blockIdx.x * (WG / 64) + wv;
   const int64_t nw = (int64_t)gridDim.x * (WG / 64);
   const uint16_t* REQ = reinterpret_cast<const uint16_t*>(p.REQ);
@@ -279,10 +283,8 @@ __global__ __launch_bounds__(WG) void k_rrequests(GlobalParams p) {
     const uint32_t nq = p.TQ[slot];
     if (nq == 0) continue;
     const VolGeo v = vol_geo(p, slot);
-    const int64_t tile = slot - v.tile0;
-    const int64_t tz = tile / (v.ntx * v.nty);
-    const int64_t tr = tile - tz * v.ntx * v.nty;
-    const int64_t ty = tr / v.ntx, tx = tr - ty * v.ntx;
+    int64_t tx, ty, tz;
+    tile_coords((uint32_t)(slot - v.tile0), v.ntx, v.nty, v.dxy, v.dx, tx, ty, tz);
     const uint32_t root0 = tile_root0<G>(v.sx, v.sy, v.sz, tx, ty, tz, v.key0);
     const bool j8 = p.TR[slot] <= 255;
 #pragma unroll
@@ -652,9 +654,8 @@ __device__ inline void fin_store(const VolGeo& v, int64_t tile, OUT* __restrict_
                                  const uint32_t (&j)[fin_ept<G>()], const uint32_t* lab) {
   constexpr int EPT = fin_ept<G>();
   const int t = threadIdx.x;
-  const int64_t tz = tile / (v.ntx * v.nty);
-  const int64_t tr = tile - tz * v.ntx * v.nty;
-  const int64_t ty = tr / v.ntx, tx = tr - ty * v.ntx;
+  int64_t tx, ty, tz;
+  tile_coords((uint32_t)tile, v.ntx, v.nty, v.dxy, v.dx, tx, ty, tz);
 #pragma unroll
   for (int k = 0; k < EPT; k++) {
     int vx, vy, vz;
@@ -761,9 +762,8 @@ __device__ inline void rfin_tile(const GlobalParams& p, const VolGeo& v, int64_t
   if (t == 0) lab[0] = 0u;
   for (uint32_t i = t; i < R; i += WG) lab[i + 1] = root_label(p, kroot_key(p.GP, root0 + i), base);
   __syncthreads();
-  const int64_t tz = tile / (v.ntx * v.nty);
-  const int64_t tr = tile - tz * v.ntx * v.nty;
-  const int64_t ty = tr / v.ntx, tx = tr - ty * v.ntx;
+  int64_t tx, ty, tz;
+  tile_coords((uint32_t)tile, v.ntx, v.nty, v.dxy, v.dx, tx, ty, tz);
   const int64_t gx = tx * G::TX + 4 * (t & 15);
   typedef OUT Pack __attribute__((ext_vector_type(4), aligned(sizeof(OUT))));
   const bool whole = ((uint64_t)v.sx * sizeof(OUT) % 128 | reinterpret_cast<uintptr_t>(out) % 128) == 0;
@@ -1643,6 +1643,8 @@ hipError_t batch_periodic(const cc3d_amd_batch* b, const cc3d_amd_batch::Periodi
   q.ntx = v.ntx;
   q.nty = v.nty;
   q.ntz = v.ntz;
+  q.dxy = v.dxy;
+  q.dx = v.dx;
   q.tile0 = v.tile0;
   q.key0 = v.key0;
   q.ctr = b->gp.ctr + 1 + pv.k;
@@ -1743,6 +1745,8 @@ static int job_begin(cc3d_amd_job* j, const void* in, int in_dtype, int64_t sx, 
   GlobalParams& gp = j->gp;
   gp.sx = g.sx; gp.sy = g.sy; gp.sz = g.sz; gp.osx = g.osx;
   gp.ntx = g.ntx; gp.nty = g.nty; gp.ntz = g.ntz; gp.ntiles = g.ntiles;
+  gp.dxy = Div(g.ntx * g.nty);
+  gp.dx = Div(g.ntx);
   gp.GP = reinterpret_cast<uint2*>(ws + g.oGP);
   gp.TR = reinterpret_cast<uint32_t*>(ws + g.oTR);
   gp.J8 = reinterpret_cast<uint8_t*>(ws + g.oJ8);
@@ -1800,6 +1804,8 @@ static int job_begin(cc3d_amd_job* j, const void* in, int in_dtype, int64_t sx, 
   lp.in = in;
   lp.sx = g.sx; lp.sy = g.sy; lp.sz = g.sz; lp.osx = g.osx;
   lp.ntx = g.ntx; lp.nty = g.nty; lp.ntz = g.ntz; lp.ntiles = g.ntiles;
+  lp.dxy = gp.dxy;
+  lp.dx = gp.dx;
   lp.delta_bits = j->delta_bits;
   lp.minmax = reinterpret_cast<const uint64_t*>(mm);
   lp.GP = gp.GP;
@@ -2217,6 +2223,8 @@ static int batch_layout(const cc3d_amd_volume* vols, int n, int mode, std::vecto
     t.nty = (v.sy + TYg - 1) / TYg;
     t.ntz = (v.sz + TZg - 1) / TZg;
     t.ntiles = t.ntx * t.nty * t.ntz;
+    t.dxy = Div(t.ntx * t.nty);
+    t.dx = Div(t.ntx);
     t.tile0 = tg.tiles;
     const uint64_t V = (uint64_t)v.sx * (uint64_t)v.sy * (uint64_t)v.sz;
     // binary 2D-8 keys are 2x2 block keys: 4 per block (plan's K)

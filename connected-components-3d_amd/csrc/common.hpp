@@ -75,6 +75,29 @@ struct TileCnt {
   long long first_row, last_row;
 };
 
+// Division of n < 2^31 by a divisor fixed on the host: with 2^s >= d and m =
+// ceil(2^(31 + s) / d), n * m >> (31 + s) is n / d.  Two scalar multiplies
+// instead of the 64-bit division routine (about 350 scalar and 50 vector
+// instructions per wave for a tile's coordinates).
+struct Div {
+  uint32_t m = 0, s = 0;
+  Div() = default;
+  __host__ explicit Div(int64_t d) {
+    while (((int64_t)1 << s) < d) s++;
+    m = (uint32_t)((((uint64_t)1 << (31 + s)) + (uint64_t)d - 1) / (uint64_t)d);
+  }
+};
+__device__ inline uint32_t div_by(uint32_t n, Div d) { return (uint32_t)(((uint64_t)n * d.m) >> (31 + d.s)); }
+
+// Coordinates of a volume's tile.
+__device__ inline void tile_coords(uint32_t tile, int64_t ntx, int64_t nty, Div dxy, Div dx, int64_t& tx, int64_t& ty,
+                                   int64_t& tz) {
+  const uint32_t z = div_by(tile, dxy), r = tile - z * (uint32_t)(ntx * nty), y = div_by(r, dx);
+  tx = r - y * (uint32_t)ntx;
+  ty = y;
+  tz = z;
+}
+
 // One volume of a batch (device-side table).
 struct BatchVol {
   const void* in;
@@ -87,6 +110,7 @@ struct BatchVol {
   int nb, out_dtype;
   int qk;                   // numbering / link variant of a single plane on the 2D tiles (Q_*)
   const uint64_t* minmax;   // continuous 2D-8: the volume's global {min, max} bit patterns
+  Div dxy, dx;              // by ntx * nty and by ntx
 };
 
 // Tile geometry.  A tile is TX x TY x TZ voxels; the local kernel's

@@ -63,6 +63,7 @@ struct LocalParams {
   const void* in;
   int64_t sx, sy, sz, osx;
   int64_t ntx, nty, ntz, ntiles;
+  Div dxy, dx;  // by ntx * nty and by ntx
   uint64_t delta_bits;
   const uint64_t* minmax;  // Q_CONT8: global {min, max} bit patterns
   uint2* GP;       // {parent, key} per local root

@@ -127,25 +127,45 @@ __host__ __device__ constexpr int row_req_cap(bool cont, int nb) {
   return nb == 8 || nb == 4 ? 384 : nb == 6 ? 1088 : nb == 18 ? (cont ? 5280 : 2540) : (cont ? 9316 : 4036);
 }
 
-// Staged voxel type: 4 bytes for every type up to 4 bytes, else the type.
-template <class T>
+// Staged voxel type: 4 bytes for every type up to 4 bytes.  Multilabel 8-byte
+// voxels are staged as 4-byte halves one after the other (their masks are
+// ANDed), which keeps 6 workgroups per CU instead of 3; continuous ones whole.
+template <class T, int MODE>
 struct RowVal {
   using type = uint32_t;
+  static constexpr bool SPLIT = sizeof(T) == 8;
 };
-template <>
-struct RowVal<float> {
+template <int MODE>
+struct RowVal<float, MODE> {
   using type = float;
+  static constexpr bool SPLIT = false;
 };
 template <>
-struct RowVal<uint64_t> {
+struct RowVal<uint64_t, M_CONT> {
   using type = uint64_t;
+  static constexpr bool SPLIT = false;
 };
 template <>
-struct RowVal<double> {
+struct RowVal<double, M_CONT> {
   using type = double;
+  static constexpr bool SPLIT = false;
 };
+// Half H of an 8-byte voxel.  Doubles compare as bits once -0 is 0 and every
+// NaN the default one, which links to nothing (NANHI, a high half that only
+// NaNs have).
+constexpr uint32_t NANHI = 0x7FF80000u;
+template <int H>
+__device__ inline uint32_t half_of(uint64_t v) {
+  return (uint32_t)(v >> (32 * H));
+}
+template <int H>
+__device__ inline uint32_t half_of(double v) {
+  const uint64_t b = v == 0.0 ? 0ull : v != v ? (uint64_t)NANHI << 32 : __builtin_bit_cast(uint64_t, v);
+  return (uint32_t)(b >> (32 * H));
+}
 
-constexpr int RSTR = 68;     // row stride of staged values and nodes: 16-byte accesses of 64 rows spread over all banks
+constexpr int RSTR = 68;   // row stride of staged values and nodes: 16-byte accesses of 64 rows spread over all banks
+constexpr int PSTR = 704;  // plane stride of staged values: 10 rows, and 24 more so that planes start on the same bank
 constexpr int RQCAP = 1024;  // queued links per wave; one relation of a wave's segments always fits
 
 // LDS index of a tile voxel's node: raster order, or for the binary 2D
@@ -165,14 +185,14 @@ __device__ inline uint32_t seg_node(uint32_t n0, uint32_t k) {
 template <class T, int MODE, class G_ = GeoR>
 struct RowLds {
   using G = G_;
-  using VT = typename RowVal<T>::type;
+  using VT = typename RowVal<T, MODE>::type;
   struct Work {
     uint32_t par[64 * RSTR];
     uint16_t queue[4][RQCAP];  // per wave; later, per wave: segment bits [row] and root bits [row]
   };
   union alignas(16) {
     // staged box: x = -1 at 3, x = 0..63 at 4..67, x = 64 at 68 (the next row's unused first element)
-    VT v[MODE == M_BINARY ? 1 : G::NROWS * RSTR + 4];
+    VT v[MODE == M_BINARY ? 4 : G::IS3D ? G::BZ * PSTR : G::NROWS * RSTR + 4];
     // staged foreground bits, 16 per half-word: x = -1 in bit 15 of 0, segments in 1..4, x = 64 in bit 0 of 5
     uint16_t fb[G::NROWS][6];
     Work w;
@@ -260,23 +280,15 @@ __device__ inline uint32_t mbcnt64(uint64_t m) {
 }
 
 // LDS union-find over 32-bit parents.  A parent is never larger than its
-// node, so walks end; a union lowers the larger root's parent with an atomic
-// minimum and goes on from the parent it displaced, so a link is never lost
-// to a racing one.  Path halving stores an ancestor of a node that is no
-// root any more.
+// node, so walks end.  A union climbs on the side of the larger parent and
+// lowers that parent to the other side's on the way (an atomic minimum that
+// returns what it replaced): either the node was a root and is linked now, or
+// the parent it gave up is the next node to join.  A join left undone is
+// always some lane's next step, so no link is lost.  Two finds to the roots
+// and then the link took 440 us on 512^3 uint32 Voronoi (26) and 1,025 us on
+// a 16384^2 mask (8), this 410 and 831 us.
 __device__ inline void lstore(uint32_t* p, uint32_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ inline uint32_t rfind(uint32_t* par, uint32_t a) {
-  uint32_t p = lload(par + a);
-  while (p != a) {
-    const uint32_t gp = lload(par + p);
-    if (gp == p) return p;
-    lstore(par + a, gp);
-    a = gp;
-    p = lload(par + a);
-  }
-  return a;
 }
 __device__ inline uint32_t rfind_ro(const uint32_t* par, uint32_t a) {
   uint32_t p = lload(par + a);
@@ -288,17 +300,13 @@ __device__ inline uint32_t rfind_ro(const uint32_t* par, uint32_t a) {
 }
 __device__ inline void runion(uint32_t* par, uint32_t a, uint32_t b) {
   while (true) {
-    a = rfind(par, a);
-    b = rfind(par, b);
-    if (a == b) return;
-    if (a < b) {
-      const uint32_t t = a;
-      a = b;
-      b = t;
-    }
-    const uint32_t old = atomicMin(par + a, b);
-    if (old == a) return;
+    const uint32_t pa = lload(par + a), pb = lload(par + b);
+    if (pa == pb) return;
+    const uint32_t c = pa > pb ? a : b, lo = pa > pb ? pb : pa;
+    const uint32_t old = atomicMin(par + c, lo);
+    if (old == c) return;  // c was a root: linked under lo
     a = old;
+    b = lo;
   }
 }
 
@@ -306,12 +314,13 @@ __device__ inline void runion(uint32_t* par, uint32_t a, uint32_t b) {
 // alignment allows.
 template <class T, int N>
 __device__ inline void load_run(const T* p, T (&v)[N]) {
-  struct __attribute__((packed, aligned(sizeof(T)))) Pack {
-    T e[N];
-  };
-  const Pack k = *reinterpret_cast<const Pack*>(p);
+  typedef T V4 __attribute__((ext_vector_type(4), aligned(sizeof(T))));
 #pragma unroll
-  for (int i = 0; i < N; i++) v[i] = k.e[i];
+  for (int i = 0; i < N; i += 4) {
+    const V4 k = *reinterpret_cast<const V4*>(p + i);
+#pragma unroll
+    for (int j = 0; j < 4; j++) v[i + j] = k[j];
+  }
 }
 
 // Bit k of the result: byte k of w is not zero, for the 16 bytes of four
@@ -334,29 +343,190 @@ __device__ inline uint32_t nonzero_bytes(const uint32_t (&w)[4]) {
 
 template <class T, int MODE, int NB, class G, int QK>
 __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, int64_t sy, int64_t sz, int64_t ntx,
-                                 int64_t nty, int64_t tile, int64_t slot, uint32_t keybase, RowLds<T, MODE, G>& L) {
+                                 int64_t nty, Div dxy, Div dx, int64_t tile, int64_t slot, uint32_t keybase,
+                                 RowLds<T, MODE, G>& L) {
   constexpr bool IS3D = G::IS3D;
   constexpr bool FACE = NB == 6 || NB == 4;  // face links only
-  using VT = typename RowVal<T>::type;
+  using VT = typename RowVal<T, MODE>::type;
+  constexpr bool SPLIT = RowVal<T, MODE>::SPLIT;
   const int t = threadIdx.x, lane = t & 63;
   const int seg = __builtin_amdgcn_readfirstlane(t >> 6);  // one segment per wave
-  const int64_t tz = tile / (ntx * nty);
-  const int64_t trem = tile - tz * ntx * nty;
-  const int64_t ty = trem / ntx, tx = trem - ty * ntx;
+  int64_t tx, ty, tz;
+  tile_coords((uint32_t)tile, ntx, nty, dxy, dx, tx, ty, tz);
   const int64_t x0 = tx * G::TX, y0 = ty * G::TY, z0 = tz * G::TZ;
   uint32_t my_epl = 0, my_prov = 0;
   if (t == 0) L.nreq = 0;
+
+  // 2. masks of the wave's segment: bit k is voxel 16 seg + k of row `lane`
+  const int ly = lane & (G::TY - 1), lz = lane / G::TY;
+  const bool first = seg == 0;  // bit 0 is the tile's first column
+  uint32_t F = 0, a = 0;
+  uint32_t U[R_N];  // kept links
+#pragma unroll
+  for (int i = 0; i < R_N; i++) U[i] = 0;
+  uint32_t M[R_N];  // all links
+#pragma unroll
+  for (int i = 0; i < R_N; i++) M[i] = 0;
+  uint32_t hD0 = 0;       // 6-connectivity: equal to the voxel of d0 (bm, cm are in M)
+  uint32_t left_cov = 0;  // continuous: bit 0, the link a of the tile's first column is covered
+  // offsets of the staged rows B, C, D, E from a row
+  constexpr int RB = -RSTR, RC = -PSTR, RD = -PSTR - RSTR, RE = -PSTR + RSTR;
+  [[maybe_unused]] auto masks = [&](auto half) {
+    [[maybe_unused]] constexpr int H = decltype(half)::value;
+    const VT* base = static_cast<const VT*>(__builtin_assume_aligned(
+      L.u.v + ((ly + 1) * RSTR + (IS3D ? (lz + 1) * PSTR : 0) + 4 + 16 * seg), 16));
+    VT cur[16];
+#pragma unroll
+    for (int k = 0; k < 16; k++) cur[k] = base[k];
+    const VT left = base[-1];
+    if constexpr (MODE == M_MULTI) {
+      // one half of a split voxel: nonzero halves ORed, equal halves ANDed
+      auto both = [&](uint32_t& m, uint32_t half_m) { m = H ? (m & half_m) : half_m; };
+      uint32_t f = 0, e = 0;
+#pragma unroll
+      for (int k = 15; k >= 0; k--) {
+        push_fg(f, cur[k]);
+        push_eq(e, cur[k], k > 0 ? cur[k > 0 ? k - 1 : 0] : left);
+      }
+      F |= f;
+      both(a, e);
+      // W0/WM/WP: which of the row's three relations to form
+      auto rel = [&](int dr, int i0, int im, int ip, bool W0, bool WM, bool WP) {
+        const VT* w = base + dr;
+        VT wv[18];  // x = -1 .. 16 of the segment
+#pragma unroll
+        for (int k = 0; k < 18; k++)
+          if ((k > 0 || WM) && (k < 17 || WP)) wv[k] = w[k - 1];
+        uint32_t m0 = 0, mm = 0, mp = 0;
+#pragma unroll
+        for (int k = 15; k >= 0; k--) {
+          if (W0) push_eq(m0, cur[k], wv[k + 1]);
+          if (WM) push_eq(mm, cur[k], wv[k]);
+          if (WP) push_eq(mp, cur[k], wv[k + 2]);
+        }
+        if (W0) both(M[i0], m0);
+        if (WM) both(M[im], mm);
+        if (WP) both(M[ip], mp);
+      };
+      rel(RB, R_B0, R_BM, R_BP, true, true, !FACE);
+      if constexpr (IS3D) {
+        rel(RC, R_C0, R_CM, R_CP, true, true, !FACE);
+        rel(RD, R_D0, R_DM, R_DP, true, NB == 26, NB == 26);
+        if constexpr (!FACE) rel(RE, R_E0, R_EM, R_EP, true, NB == 26, NB == 26);
+      }
+      if (H == 1 || !SPLIT) {
+        uint32_t lk = F;
+        if constexpr (std::is_same<T, double>::value) {
+          uint32_t nan = 0;
+#pragma unroll
+          for (int k = 15; k >= 0; k--) push_eq(nan, cur[k], NANHI);
+          lk &= ~nan;
+        }
+        a &= lk;
+#pragma unroll
+        for (int i = 0; i < R_A; i++) M[i] &= lk;
+        hD0 = M[R_D0];
+        my_epl = (uint32_t)__popc(F & ~a);
+      }
+    }
+    if constexpr (MODE == M_CONT) {
+      const VT delta = (VT)from_bits<T>(p.delta_bits);
+      uint32_t eq = 0;
+#pragma unroll
+      for (int k = 15; k >= 0; k--) {
+        const VT pv = k > 0 ? cur[k > 0 ? k - 1 : 0] : left;
+        push_bit(F, cont_fg(cur[k]));
+        push_eq(eq, cur[k], pv);
+        push_link(a, cur[k], pv, delta);
+      }
+      my_epl = (uint32_t)__popc(F & ~eq);
+      const uint32_t inner = first ? (a & ~1u) : a;
+      // One backward row: its links, and the kept ones.  Masks of 17 bits
+      // have the voxel before the segment in bit 0: the link of voxel k - 1
+      // to the voxel at x is a pair (a, q), so it covers p - q where p has
+      // the link a; xw: links along the row itself, w[k] - w[k + 1].
+      uint32_t bd = 0, ce = 0;
+      VT prow[16];  // rows B and C at 18-connectivity, for the pairs (b0, d0) and (c0, e0)
+      auto rel = [&](int dr, int i0, int im, int ip, bool diag, bool quirk, bool keep, uint32_t* pair,
+                     bool left_rule) {
+        const VT* w = base + dr;
+        VT wv[18];
+#pragma unroll
+        for (int k = 0; k < 18; k++)
+          if (k < 17 || !FACE) wv[k] = w[k - 1];
+        uint32_t x0m = 0, xpm = 0, xw = 0, eqm = 0;
+#pragma unroll
+        for (int k = 15; k >= -1; k--) {
+          const VT c = k >= 0 ? cur[k >= 0 ? k : 0] : left;
+          push_link(x0m, c, wv[k + 1], delta);
+          if (quirk) push_eq(eqm, c, wv[k + 1]);
+          if (diag) push_link(xpm, c, wv[k + 2], delta);
+          if (k >= 0 && diag) push_link(M[im], c, wv[k], delta);
+          if (FACE) {
+            if (k >= 0) push_link(xw, wv[k + 1], wv[k], delta);
+          } else if (diag) {
+            push_link(xw, wv[k + 2], wv[k + 1], delta);
+          }
+        }
+        if (pair) {
+#pragma unroll
+          for (int k = 15; k >= 0; k--) push_link(*pair, prow[k], wv[k + 1], delta);
+        }
+        if (keep) {
+#pragma unroll
+          for (int k = 0; k < 16; k++) prow[k] = wv[k + 1];
+        }
+        // equal to the voxel below: linked under 26-connectivity whatever delta says
+        // (cc3d/cc3d_continuous.hpp:147-150); a background c is masked by F below
+        if (quirk) {
+          const uint32_t f17 = (F << 1) | (cont_fg(left) ? 1u : 0u);
+          x0m |= eqm & f17;
+        }
+        M[i0] = x0m >> 1;
+        const uint32_t s0 = x0m & 0xFFFFu;  // voxel k - 1 to the voxel of im
+        if constexpr (FACE) {
+          const uint32_t cov = s0 & xw;
+          U[i0] = M[i0] & ~(inner & cov);
+          left_cov |= M[i0] & cov;
+        } else {
+          const uint32_t sp = xpm & 0xFFFFu;  // voxel k - 1 to the voxel of i0
+          uint32_t cov0 = rel_adj(R_A, i0, NB) ? (inner & sp) : 0u;
+          if (pair) cov0 |= M[i0 == R_D0 ? R_B0 : R_C0] & *pair;
+          U[i0] = M[i0] & ~cov0;
+          if (diag) {
+            M[ip] = xpm >> 1;
+            U[im] = M[im] & ~(inner & s0) & ~(M[i0] & xw);
+            U[ip] = M[ip] & ~(M[i0] & (xw >> 1));
+          }
+          if (left_rule) left_cov |= M[i0] & sp;
+        }
+      };
+      constexpr bool D = !FACE, D26 = NB == 26, P18 = NB == 18;
+      rel(RB, R_B0, R_BM, R_BP, D, false, P18, nullptr, true);
+      if constexpr (IS3D && !FACE) rel(RD, R_D0, R_DM, R_DP, D26, false, false, P18 ? &bd : nullptr, false);
+      if constexpr (IS3D) rel(RC, R_C0, R_CM, R_CP, D, NB == 26, P18, nullptr, true);
+      if constexpr (IS3D && !FACE) rel(RE, R_E0, R_EM, R_EP, D26, false, false, P18 ? &ce : nullptr, false);
+    }
+  };
 
   // 1. stage the box: rows r = by + BY * bz.  Row BY - 1 of the last plane is
   //    reached by no voxel.  Voxels outside the volume are background.
   // box position (-1, -1, -1) ((-1, -1) in a plane); dereferenced inside the volume only
   const T* box = in + ((x0 - 1) + sx * ((y0 - 1) + (IS3D ? sy * (z0 - 1) : 0)));
-  const int64_t xleft = sx - x0;                                     // voxels of a row from x0 on
-  auto row_ok = [&](int by, int bz) -> bool {
-    const int64_t gy = y0 + by - 1, gz = z0 + bz - 1;
-    return gy >= 0 && gy < sy && (!IS3D || (gz >= 0 && gz < sz));
+  const int xleft = (int)(sx - x0 < 128 ? sx - x0 : 128);  // voxels of a row from x0 on
+  // box rows and planes inside the volume: [ylo, yhi) and [zlo, zhi)
+  const int ylo = y0 == 0 ? 1 : 0, yhi = (int)(sy - y0 + 1 < G::BY ? sy - y0 + 1 : G::BY);
+  const int zlo = IS3D && z0 == 0 ? 1 : 0, zhi = IS3D && sz - z0 + 1 < G::BZ ? (int)(sz - z0 + 1) : G::BZ;
+  auto row_ok = [&](int by, int bz) -> bool { return by >= ylo && by < yhi && bz >= zlo && bz < zhi; };
+  const int64_t pitch = sx * sy;
+  auto row_ptr = [&](int by, int bz) -> const T* {  // its x0
+    return box + (1 + (int64_t)by * sx + (IS3D ? (int64_t)bz * pitch : 0));
   };
-  auto row_ptr = [&](int by, int bz) -> const T* { return box + (1 + sx * (by + sy * (int64_t)bz)); };  // its x0
+  auto row_of = [&](int r, int& by, int& bz) {  // box row r < 128
+    bz = IS3D ? (r * 205) >> 11 : 0;  // r / 10
+    static_assert(!IS3D || G::BY == 10, "division by 10");
+    by = r - bz * G::BY;
+  };
   if constexpr (MODE == M_BINARY) {
     // 16 voxels (one segment) per thread and pass
     constexpr int ITEMS = 4 * G::NROWS;
@@ -366,7 +536,8 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
       const int i = t + G::NT * q;
       if (i >= ITEMS) break;
       const int r = i >> 2, s = i & 3;
-      const int bz = r / G::BY, by = r - bz * G::BY;
+      int by, bz;
+      row_of(r, by, bz);
       uint32_t F = 0, NE = 0;  // NE: differs from the voxel before it (tile rows)
       if (row_ok(by, bz) && 16 * s < xleft) {
         const T* e = row_ptr(by, bz) + 16 * s;
@@ -375,16 +546,18 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
         if (own && x0 + 16 * s > 0) prev = e[-1];
         if (16 * s + 16 <= xleft) {
           T v[16];
-          load_run<T, 16>(e, v);
           if constexpr (sizeof(T) == 1) {
-            uint32_t w[4], d[4];
-            __builtin_memcpy(w, v, 16);
+            typedef uint32_t Words __attribute__((ext_vector_type(4), aligned(1)));
+            const Words q4 = *reinterpret_cast<const Words*>(e);
+            const uint32_t w[4] = {q4[0], q4[1], q4[2], q4[3]};
+            uint32_t d[4];
             F = nonzero_bytes(w);
             d[0] = w[0] ^ ((w[0] << 8) | (uint32_t)(uint8_t)prev);
 #pragma unroll
             for (int k = 1; k < 4; k++) d[k] = w[k] ^ __builtin_amdgcn_alignbyte(w[k], w[k - 1], 3);
             NE = nonzero_bytes(d);
           } else {
+            load_run<T, 16>(e, v);
 #pragma unroll
             for (int k = 15; k >= 0; k--) {
               push_bit(F, v[k] != T(0));
@@ -407,24 +580,50 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
     }
     if (t < 2 * G::NROWS) {
       const int r = t >> 1, right = t & 1;
-      const int bz = r / G::BY, by = r - bz * G::BY;
+      int by, bz;
+      row_of(r, by, bz);
       const bool ok = row_ok(by, bz) && (right ? xleft > 64 : x0 > 0);
       const bool f = ok && row_ptr(by, bz)[right ? 64 : -1] != T(0);
       L.u.fb[r][right ? 5 : 0] = (uint16_t)(f ? (right ? 1u : 0x8000u) : 0u);
     }
   } else {
-    // 4 voxels per thread and pass, 16 rows a pass; all loads first
-    constexpr int PASSES = (G::NROWS + 15) / 16;
+    // 4 voxels per lane and load, 4 rows a wave; all loads first.  The rows of
+    // load l = seg + 4 q: in a volume rows 0-3 or 4-7 of plane l / 2 for l <
+    // 18, then rows 8 and 9 of planes 2 (l - 18) and the next; in a plane
+    // rows 4 l to 4 l + 3.  Bases are wave-uniform, a lane's offset is one of
+    // two constants.
+    constexpr int PASSES = IS3D ? 6 : (G::NROWS + 15) / 16;
+    const int q4 = 4 * (lane & 15), sub = lane >> 4;
     T v[PASSES][4];
-    const int q4 = 4 * (t & 15), rr = t >> 4;
+    const bool inner = x0 + G::TX <= sx && ylo == 0 && yhi == G::BY && zlo == 0 && zhi == G::BZ;
+    auto base_row = [&](int q, int& by, int& bz) -> bool {  // false: the two-plane form
+      const int l = seg + 4 * q;
+      if (!IS3D) {
+        by = 4 * l;
+        bz = 0;
+        return true;
+      }
+      if (l < 18) {
+        by = (l & 1) * 4;
+        bz = l >> 1;
+        return true;
+      }
+      by = 8;
+      bz = 2 * (l - 18);
+      return false;
+    };
+    const int64_t offa = (int64_t)sub * sx + q4, offb = (int64_t)(sub & 1) * sx + (int64_t)(sub >> 1) * pitch + q4;
+    const int sub_y = sub & 1, sub_z = sub >> 1;
 #pragma unroll
     for (int q = 0; q < PASSES; q++) {
-      const int r = rr + 16 * q;
-      const int bz = r / G::BY, by = r - bz * G::BY;
+      int by, bz;
+      const bool quad = base_row(q, by, bz);
 #pragma unroll
       for (int k = 0; k < 4; k++) v[q][k] = T(0);
-      if (r < (IS3D ? G::NROWS - 1 : G::NROWS) && row_ok(by, bz)) {
-        const T* e = row_ptr(by, bz) + q4;
+      const T* e = row_ptr(by, bz) + (quad ? offa : offb);
+      if (inner && quad && by + 3 < G::BY && bz < G::BZ) {
+        load_run<T, 4>(e, v[q]);
+      } else if (quad ? row_ok(by + sub, bz) : row_ok(by + sub_y, bz + sub_z)) {
         if (q4 + 4 <= xleft) {
           load_run<T, 4>(e, v[q]);
         } else {
@@ -436,187 +635,77 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
     }
     T hx = T(0);
     const int hr = t >> 1, right = t & 1;
-    if (t < 2 * G::NROWS) {
-      const int bz = hr / G::BY, by = hr - bz * G::BY;
-      if (row_ok(by, bz) && (right ? xleft > 64 : x0 > 0)) hx = row_ptr(by, bz)[right ? 64 : -1];
-    }
+    int hby, hbz;
+    row_of(hr, hby, hbz);
+    if (t < 2 * G::NROWS && row_ok(hby, hbz) && (right ? xleft > 64 : x0 > 0))
+      hx = row_ptr(hby, hbz)[right ? 64 : -1];
+    // half: which half of a split voxel
+    auto put = [&](auto half) {
+      auto staged = [&](T c) -> VT {
+        if constexpr (SPLIT) return half_of<decltype(half)::value>(c);
+        else if constexpr (MODE == M_CONT) return cont_stage((VT)c);
+        else return (VT)c;
+      };
 #pragma unroll
-    for (int q = 0; q < PASSES; q++) {
-      const int r = rr + 16 * q;
-      if (r < G::NROWS) {
-        VT* d = static_cast<VT*>(__builtin_assume_aligned(L.u.v + (r * RSTR + 4 + q4), 16));
+      for (int q = 0; q < PASSES; q++) {
+        int by, bz;
+        const bool quad = base_row(q, by, bz);
+        const int dy = quad ? sub : sub_y, dz = quad ? 0 : sub_z;
+        if (by + dy < G::BY && bz + dz < G::BZ) {
+          VT* d = static_cast<VT*>(
+            __builtin_assume_aligned(L.u.v + (by * RSTR + bz * PSTR + (dy * RSTR + dz * PSTR + 4 + q4)), 16));
 #pragma unroll
-        for (int k = 0; k < 4; k++) d[k] = MODE == M_CONT ? cont_stage((VT)v[q][k]) : (VT)v[q][k];
+          for (int k = 0; k < 4; k++) d[k] = staged(v[q][k]);
+        }
       }
+      if (t < 2 * G::NROWS) L.u.v[hby * RSTR + hbz * PSTR + (right ? 68 : 3)] = staged(hx);
+    };
+    put(std::integral_constant<int, 0>());
+    __syncthreads();
+    masks(std::integral_constant<int, 0>());
+    if constexpr (SPLIT) {
+      __syncthreads();
+      put(std::integral_constant<int, 1>());
+      __syncthreads();
+      masks(std::integral_constant<int, 1>());
     }
-    if (t < 2 * G::NROWS) L.u.v[hr * RSTR + (right ? 68 : 3)] = MODE == M_CONT ? cont_stage((VT)hx) : (VT)hx;
   }
-  __syncthreads();
-
-  // 2. the segment's masks (bit k: voxel 16 seg + k of row `lane`)
-  const int ly = lane & (G::TY - 1), lz = lane / G::TY;
-  const int r0 = (ly + 1) + (IS3D ? G::BY * (lz + 1) : 0);
-  constexpr int RB = -1, RC = -G::BY, RD = -G::BY - 1, RE = -G::BY + 1;  // box rows B, C, D, E from r0
-  const bool first = seg == 0;  // bit 0 is the tile's first column
-  uint32_t F = 0, a = 0;
-  uint32_t U[R_N];  // kept links
-#pragma unroll
-  for (int i = 0; i < R_N; i++) U[i] = 0;
-  {
-    uint32_t M[R_N];  // all links
-    uint32_t any;
-#pragma unroll
-    for (int i = 0; i < R_N; i++) M[i] = 0;
-    uint32_t hD0 = 0;       // 6-connectivity: equal to the voxel of d0 (bm, cm are in M)
-    uint32_t left_cov = 0;  // continuous: bit 0, the link a of the tile's first column is covered
-    if constexpr (MODE == M_BINARY) {
-      auto bits = [&](int r, uint32_t& m0, uint32_t& mm, uint32_t& mp) {
-        const uint16_t* b = &L.u.fb[r][seg];
-        const uint32_t c = b[1];
-        m0 = c;
-        mm = ((c << 1) | (uint32_t)(b[0] >> 15)) & 0xFFFFu;
-        mp = (c >> 1) | (((uint32_t)b[2] & 1u) << 15);
-      };
-      uint32_t mm, mp;
-      bits(r0, F, mm, mp);
-      a = F & mm;
-      auto rel = [&](int dr, int i0, int im, int ip) {
-        uint32_t m0;
-        bits(r0 + dr, m0, mm, mp);
-        M[i0] = F & m0;
-        M[im] = F & mm;
-        M[ip] = F & mp;
-      };
-      rel(RB, R_B0, R_BM, R_BP);
-      if constexpr (IS3D) {
-        rel(RC, R_C0, R_CM, R_CP);
-        rel(RD, R_D0, R_DM, R_DP);
-        if constexpr (!FACE) rel(RE, R_E0, R_EM, R_EP);
-        hD0 = M[R_D0];
-      }
-      if constexpr (QK == Q_BIN4) {
-        // the first row links on equal values, later rows to the left unless
-        // the two pixels above are both set (cc3d/cc3d_binary.hpp:822-935)
-        a &= y0 + ly == 0 ? ~(uint32_t)L.ne0[seg] : ~(M[R_B0] & M[R_BM]);
-      }
-    } else {
-      const VT* base = static_cast<const VT*>(__builtin_assume_aligned(L.u.v + (r0 * RSTR + 4 + 16 * seg), 16));
-      VT cur[16];
-#pragma unroll
-      for (int k = 0; k < 16; k++) cur[k] = base[k];
-      const VT left = base[-1];
-      if constexpr (MODE == M_MULTI) {
-#pragma unroll
-        for (int k = 15; k >= 0; k--) {
-          push_fg(F, cur[k]);
-          push_eq(a, cur[k], k > 0 ? cur[k > 0 ? k - 1 : 0] : left);
-        }
-        a &= F;
-        my_epl = (uint32_t)__popc(F & ~a);
-        // W0/WM/WP: which of the row's three relations to form
-        auto rel = [&](int dr, int i0, int im, int ip, bool W0, bool WM, bool WP) {
-          const VT* w = base + dr * RSTR;
-          VT wv[18];  // x = -1 .. 16 of the segment
-#pragma unroll
-          for (int k = 0; k < 18; k++)
-            if ((k > 0 || WM) && (k < 17 || WP)) wv[k] = w[k - 1];
-#pragma unroll
-          for (int k = 15; k >= 0; k--) {
-            if (W0) push_eq(M[i0], cur[k], wv[k + 1]);
-            if (WM) push_eq(M[im], cur[k], wv[k]);
-            if (WP) push_eq(M[ip], cur[k], wv[k + 2]);
-          }
-          if (W0) M[i0] &= F;
-          if (WM) M[im] &= F;
-          if (WP) M[ip] &= F;
-        };
-        rel(RB, R_B0, R_BM, R_BP, true, true, !FACE);
-        if constexpr (IS3D) {
-          rel(RC, R_C0, R_CM, R_CP, true, true, !FACE);
-          rel(RD, R_D0, R_DM, R_DP, true, NB == 26, NB == 26);
-          if constexpr (!FACE) rel(RE, R_E0, R_EM, R_EP, true, NB == 26, NB == 26);
-          hD0 = M[R_D0];
-        }
-      }
-      if constexpr (MODE == M_CONT) {
-        const VT delta = (VT)from_bits<T>(p.delta_bits);
-        uint32_t eq = 0;
-#pragma unroll
-        for (int k = 15; k >= 0; k--) {
-          const VT pv = k > 0 ? cur[k > 0 ? k - 1 : 0] : left;
-          push_bit(F, cont_fg(cur[k]));
-          push_eq(eq, cur[k], pv);
-          push_link(a, cur[k], pv, delta);
-        }
-        my_epl = (uint32_t)__popc(F & ~eq);
-        const uint32_t inner = first ? (a & ~1u) : a;
-        // One backward row: its links, and the kept ones.  Masks of 17 bits
-        // have the voxel before the segment in bit 0: the link of voxel k - 1
-        // to the voxel at x is a pair (a, q), so it covers p - q where p has
-        // the link a; xw: links along the row itself, w[k] - w[k + 1].
-        uint32_t bd = 0, ce = 0;
-        VT prow[16];  // rows B and C at 18-connectivity, for the pairs (b0, d0) and (c0, e0)
-        auto rel = [&](int dr, int i0, int im, int ip, bool diag, bool quirk, bool keep, uint32_t* pair,
-                       bool left_rule) {
-          const VT* w = base + dr * RSTR;
-          VT wv[18];
-#pragma unroll
-          for (int k = 0; k < 18; k++)
-            if (k < 17 || !FACE) wv[k] = w[k - 1];
-          uint32_t x0m = 0, xpm = 0, xw = 0, eqm = 0;
-#pragma unroll
-          for (int k = 15; k >= -1; k--) {
-            const VT c = k >= 0 ? cur[k >= 0 ? k : 0] : left;
-            push_link(x0m, c, wv[k + 1], delta);
-            if (quirk) push_eq(eqm, c, wv[k + 1]);
-            if (diag) push_link(xpm, c, wv[k + 2], delta);
-            if (k >= 0 && diag) push_link(M[im], c, wv[k], delta);
-            if (FACE) {
-              if (k >= 0) push_link(xw, wv[k + 1], wv[k], delta);
-            } else if (diag) {
-              push_link(xw, wv[k + 2], wv[k + 1], delta);
-            }
-          }
-          if (pair) {
-#pragma unroll
-            for (int k = 15; k >= 0; k--) push_link(*pair, prow[k], wv[k + 1], delta);
-          }
-          if (keep) {
-#pragma unroll
-            for (int k = 0; k < 16; k++) prow[k] = wv[k + 1];
-          }
-          // equal to the voxel below: linked under 26-connectivity whatever delta says
-          // (cc3d/cc3d_continuous.hpp:147-150); a background c is masked by F below
-          if (quirk) {
-            const uint32_t f17 = (F << 1) | (cont_fg(left) ? 1u : 0u);
-            x0m |= eqm & f17;
-          }
-          M[i0] = x0m >> 1;
-          const uint32_t s0 = x0m & 0xFFFFu;  // voxel k - 1 to the voxel of im
-          if constexpr (FACE) {
-            const uint32_t cov = s0 & xw;
-            U[i0] = M[i0] & ~(inner & cov);
-            left_cov |= M[i0] & cov;
-          } else {
-            const uint32_t sp = xpm & 0xFFFFu;  // voxel k - 1 to the voxel of i0
-            uint32_t cov0 = rel_adj(R_A, i0, NB) ? (inner & sp) : 0u;
-            if (pair) cov0 |= M[i0 == R_D0 ? R_B0 : R_C0] & *pair;
-            U[i0] = M[i0] & ~cov0;
-            if (diag) {
-              M[ip] = xpm >> 1;
-              U[im] = M[im] & ~(inner & s0) & ~(M[i0] & xw);
-              U[ip] = M[ip] & ~(M[i0] & (xw >> 1));
-            }
-            if (left_rule) left_cov |= M[i0] & sp;
-          }
-        };
-        constexpr bool D = !FACE, D26 = NB == 26, P18 = NB == 18;
-        rel(RB, R_B0, R_BM, R_BP, D, false, P18, nullptr, true);
-        if constexpr (IS3D && !FACE) rel(RD, R_D0, R_DM, R_DP, D26, false, false, P18 ? &bd : nullptr, false);
-        if constexpr (IS3D) rel(RC, R_C0, R_CM, R_CP, D, NB == 26, P18, nullptr, true);
-        if constexpr (IS3D && !FACE) rel(RE, R_E0, R_EM, R_EP, D26, false, false, P18 ? &ce : nullptr, false);
-      }
+  if constexpr (MODE == M_BINARY) {
+    __syncthreads();
+    const int r0 = (ly + 1) + (IS3D ? G::BY * (lz + 1) : 0);
+    constexpr int B = -1, C = -G::BY, D = -G::BY - 1, E = -G::BY + 1;  // box rows from r0
+    auto bits = [&](int r, uint32_t& m0, uint32_t& mm, uint32_t& mp) {
+      const uint16_t* b = &L.u.fb[r][seg];
+      const uint32_t c = b[1];
+      m0 = c;
+      mm = ((c << 1) | (uint32_t)(b[0] >> 15)) & 0xFFFFu;
+      mp = (c >> 1) | (((uint32_t)b[2] & 1u) << 15);
+    };
+    uint32_t mm, mp;
+    bits(r0, F, mm, mp);
+    a = F & mm;
+    auto rel = [&](int dr, int i0, int im, int ip) {
+      uint32_t m0;
+      bits(r0 + dr, m0, mm, mp);
+      M[i0] = F & m0;
+      M[im] = F & mm;
+      M[ip] = F & mp;
+    };
+    rel(B, R_B0, R_BM, R_BP);
+    if constexpr (IS3D) {
+      rel(C, R_C0, R_CM, R_CP);
+      rel(D, R_D0, R_DM, R_DP);
+      if constexpr (!FACE) rel(E, R_E0, R_EM, R_EP);
+      hD0 = M[R_D0];
     }
+    if constexpr (QK == Q_BIN4) {
+      // the first row links on equal values, later rows to the left unless
+      // the two pixels above are both set (cc3d/cc3d_binary.hpp:822-935)
+      a &= y0 + ly == 0 ? ~(uint32_t)L.ne0[seg] : ~(M[R_B0] & M[R_BM]);
+    }
+  }
+  {
+    uint32_t any;
     const uint32_t ain = first ? (a & ~1u) : a;  // links a inside the tile
     if constexpr (MODE != M_CONT) {
       if constexpr (QK == Q_BIN4) {
@@ -910,18 +999,20 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
 }
 
 // Waves per SIMD the row kernel is compiled for: what the LDS of one tile
-// admits (6 workgroups of 4 waves per CU up to 4-byte voxels, 3 for 8-byte
-// ones; binary tiles stage bits and hold 6 for every type).
+// admits (6 workgroups of 4 waves per CU; 3 for continuous 8-byte voxels),
+// less one for 8-byte voxels staged by halves, which hold a tile's share in
+// registers meanwhile.
 template <class T, int MODE>
 __host__ __device__ constexpr int rows_waves() {
-  return (MODE == M_BINARY || sizeof(T) <= 4) ? 6 : 3;
+  return sizeof(T) < 8 || MODE == M_BINARY ? 6 : MODE == M_CONT ? 3 : 5;
 }
 
 template <class T, int MODE, int NB>
 __global__ __launch_bounds__(GeoR::NT, (rows_waves<T, MODE>())) void k_rows_local(LocalParams p) {
   __shared__ RowLds<T, MODE> L;
   const int64_t tile = xcd_tile(blockIdx.x, p.ntiles);
-  rows_tile<T, MODE, NB, GeoR, Q_NONE>(p, static_cast<const T*>(p.in), p.sx, p.sy, p.sz, p.ntx, p.nty, tile, tile, 0u,
+  rows_tile<T, MODE, NB, GeoR, Q_NONE>(p, static_cast<const T*>(p.in), p.sx, p.sy, p.sz, p.ntx, p.nty, p.dxy,
+                                       p.dx, tile, tile, 0u,
                                        L);
 }
 
@@ -930,7 +1021,8 @@ template <class T, int MODE, int NB, int QK>
 __global__ __launch_bounds__(GeoP::NT, (rows_waves<T, MODE>())) void k_rows_plane(LocalParams p) {
   __shared__ RowLds<T, MODE, GeoP> L;
   const int64_t tile = xcd_tile(blockIdx.x, p.ntiles);
-  rows_tile<T, MODE, NB, GeoP, QK>(p, static_cast<const T*>(p.in), p.sx, p.sy, 1, p.ntx, p.nty, tile, tile, 0u, L);
+  rows_tile<T, MODE, NB, GeoP, QK>(p, static_cast<const T*>(p.in), p.sx, p.sy, 1, p.ntx, p.nty, p.dxy, p.dx, tile,
+                                     tile, 0u, L);
 }
 
 // Batch: tiles [gtile0, gtile0 + gtiles) of volumes of connectivity NB; each
@@ -942,8 +1034,8 @@ __global__ __launch_bounds__(GeoR::NT, (rows_waves<T, MODE>())) void k_rows_loca
   __shared__ RowLds<T, MODE> L;
   const int64_t slot = gtile0 + xcd_tile(blockIdx.x, gtiles);
   const BatchVol& v = vols[vix[slot]];
-  rows_tile<T, MODE, NB, GeoR, Q_NONE>(p, static_cast<const T*>(v.in), v.sx, v.sy, v.sz, v.ntx, v.nty, slot - v.tile0,
-                                       slot, v.key0, L);
+  rows_tile<T, MODE, NB, GeoR, Q_NONE>(p, static_cast<const T*>(v.in), v.sx, v.sy, v.sz, v.ntx, v.nty, v.dxy, v.dx,
+                                       slot - v.tile0, slot, v.key0, L);
 }
 
 hipError_t launch_rows_multi(int dt, int nb, const LocalParams& p, hipStream_t s);
