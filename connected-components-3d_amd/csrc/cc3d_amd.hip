@@ -218,7 +218,7 @@ __device__ inline uint32_t lroot_index(const GlobalParams& p, const VolGeo& v, i
   const int64_t slot = v.tile0 + tx + v.ntx * (ty + v.nty * tz);
   const int ji = G::jidx((int)(gx - tx * G::TX), (int)(gy - ty * G::TY), (int)(gz - tz * G::TZ));
   const uint32_t R = p.TR[slot];
-  const uint32_t j = R <= 255 ? p.J8[slot * G::TV + ji] : p.J16[slot * G::TV + ji];
+  const uint32_t j = R <= 255 ? p.J8[slot * (2 * G::TV) + ji] : p.J16[slot * G::TV + ji];
   if (j == 0) return 0xFFFFFFFFu;
   return tile_root0<G>(v.sx, v.sy, v.sz, tx, ty, tz, v.key0) + j - 1;
 }
@@ -262,14 +262,194 @@ __global__ __launch_bounds__(WG) void k_requests(GlobalParams p) {
   }
 }
 
-// The same for row tiles, whose requests are (voxel position in the tile |
-// relation << 12): the forest entries of the two voxels, both foreground.
-// One wave per tile.  The links of a border join the same few pairs of local
-// roots again and again, so a wave drops the pairs that one of its lanes has
-// taken before: a table of the tile's pairs in LDS, and within the 64
-// requests of a round the lane that wrote a slot last stands for the others
-// with its pair.  A table slot that another pair took only costs a repeated
-// union.
+// Row tiles: requests are (voxel position in the tile | relation << 12).
+
+// Forest side of request e of a tile at (tx, ty, tz) (number `slot`): the
+// local roots jp of its voxel p and jq of the neighbour q, 1-based in their
+// tiles, and the offset (ox, oy, oz) of q's tile.  8-bit root indices are loaded
+// beside the counts that say whether they are valid.
+template <class G>
+__device__ inline void request_ends(const GlobalParams& p, int64_t ntx, int64_t nty, int64_t slot, bool j8, uint32_t e,
+                                    int& ox, int& oy, int& oz, uint32_t& jp, uint32_t& jq) {
+  const int ps = (int)(e & 0xFFFu);
+  int dx, dy, dz;
+  rel_decode(e >> 12, dx, dy, dz);
+  const int x = (ps & 63) + dx, y = ((ps >> 6) & (G::TY - 1)) + dy, z = ps / (64 * G::TY) + dz;
+  ox = x < 0 ? -1 : x >= G::TX ? 1 : 0;
+  oy = y < 0 ? -1 : y >= G::TY ? 1 : 0;
+  oz = z < 0 ? -1 : 0;
+  const int64_t qs = slot + ox + ntx * (oy + nty * oz);
+  const int qp = G::jidx(x - ox * G::TX, y - oy * G::TY, z - oz * G::TZ);
+  const uint32_t Rq = p.TR[qs];
+  jp = p.J8[slot * (2 * G::TV) + ps];
+  jq = p.J8[qs * (2 * G::TV) + qp];
+  if (!j8) jp = p.J16[slot * G::TV + ps];
+  if (Rq > 255) jq = p.J16[qs * G::TV + qp];
+}
+
+// Unions inside groups of 16 tiles, in LDS: 1 x 4 x 4 tiles of a volume (most
+// of a 64 x 8 x 8 tile's border is its y and z faces), 4 x 4 of a plane.  Of
+// the global unions' time nearly all is their device-scope compare-and-swaps
+// (512^3 uint32 Voronoi 26: 183 us, 39 us without them), and a group settles
+// about 70 % of them among its own tiles.  Every entry leaves with its group
+// root as parent, the group root with its component's smallest key; the bits
+// of the other keys are cleared, and the requests that leave the group are
+// moved to the front of their tile's list.  A group with more local roots than the LDS
+// table holds leaves its requests to the global kernel.
+constexpr int GRP = 16, GRP_NT = 512, GRP_CAP = 4096;  // two tiles per wave: 4 workgroups per CU
+template <class G>
+struct GroupGeo {
+  static constexpr int X = G::IS3D ? 1 : 4, Y = 4, Z = G::IS3D ? 4 : 1;
+  static_assert(X * Y * Z == GRP, "16 tiles a group");
+};
+struct GroupGrid {
+  uint32_t nx, ny, n;  // groups along x, along y, in all
+  Div dxy, dx;         // by nx * ny and by nx
+};
+template <class G>
+__global__ __launch_bounds__(GRP_NT) void k_group(GlobalParams p, GroupGrid gg) {
+  using GG = GroupGeo<G>;
+  __shared__ uint32_t par[GRP_CAP], key[GRP_CAP];
+  __shared__ uint32_t base[GRP + 1], root0s[GRP];
+  const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
+  int64_t gx, gy, gz;
+  tile_coords((uint32_t)xcd_tile(blockIdx.x, gg.n), gg.nx, gg.ny, gg.dxy, gg.dx, gx, gy, gz);
+  // tile l of the group: its coordinates and number; false outside the volume
+  auto tile_of = [&](int l, int64_t& tx, int64_t& ty, int64_t& tz, int64_t& slot) -> bool {
+    tx = gx * GG::X + (l % GG::X);
+    ty = gy * GG::Y + (l / GG::X) % GG::Y;
+    tz = gz * GG::Z + l / (GG::X * GG::Y);
+    slot = tx + p.ntx * (ty + p.nty * tz);
+    return tx < p.ntx && ty < p.nty && tz < p.ntz;
+  };
+  // the wave's tiles: their counts and first requests, and their ends
+  constexpr int TPW = GRP / (GRP_NT / 64);
+  auto number = [&](int h) { return TPW * wv + h; };
+  uint16_t* list[TPW];
+  uint32_t R[TPW], nq[TPW], r0[TPW], rq[TPW][2], jp[TPW][2], jq[TPW][2];
+  int64_t slot[TPW];
+  int ql[TPW][2];  // q's tile in the group, -1 outside
+  bool valid[TPW];
+#pragma unroll
+  for (int h = 0; h < TPW; h++) {
+    int64_t tx, ty, tz;
+    valid[h] = tile_of(number(h), tx, ty, tz, slot[h]);
+    list[h] = nullptr;
+    R[h] = nq[h] = r0[h] = rq[h][0] = rq[h][1] = 0;
+    if (valid[h]) {
+      list[h] = reinterpret_cast<uint16_t*>(const_cast<uint32_t*>(p.REQ)) + slot[h] * p.reqcap;
+      rq[h][0] = list[h][lane];  // the storage holds more than 128 whatever nq is
+      rq[h][1] = list[h][lane + 64];
+      R[h] = p.TR[slot[h]];
+      nq[h] = p.TQ[slot[h]];
+      r0[h] = tile_root0<G>(p.sx, p.sy, p.sz, tx, ty, tz, p.key0);
+    }
+  }
+  auto ends = [&](int h, uint32_t e, uint32_t& p1, uint32_t& q1) -> int {
+    const int l = number(h), lx = l % GG::X, ly = (l / GG::X) % GG::Y, lz = l / (GG::X * GG::Y);
+    int ox, oy, oz;
+    request_ends<G>(p, p.ntx, p.nty, slot[h], R[h] <= 255, e, ox, oy, oz, p1, q1);
+    const int qx = lx + ox, qy = ly + oy, qz = lz + oz;
+    return qx < 0 || qx >= GG::X || qy < 0 || qy >= GG::Y || qz < 0 ? -1 : qx + GG::X * (qy + GG::Y * qz);
+  };
+#pragma unroll
+  for (int h = 0; h < TPW; h++) {
+    if (lane == 0) {
+      base[number(h) + 1] = R[h];
+      root0s[number(h)] = r0[h];
+    }
+  }
+  __syncthreads();
+  if (wv == 0) {
+    const uint32_t c = lane < GRP ? base[lane + 1] : 0u;
+    const uint32_t incl = wave_incl_add(c);
+    if (lane < GRP) base[lane + 1] = incl;
+    if (lane == GRP) base[0] = 0;
+  }
+#pragma unroll
+  for (int h = 0; h < TPW; h++) {
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      ql[h][k] = -1;
+      if (64u * k + (uint32_t)lane < nq[h]) ql[h][k] = ends(h, rq[h][k], jp[h][k], jq[h][k]);
+    }
+  }
+  __syncthreads();
+  const uint32_t total = base[GRP];
+  if (total > GRP_CAP) return;
+#pragma unroll
+  for (int h = 0; h < TPW; h++) {
+    const uint32_t b = base[number(h)];
+    for (uint32_t i = lane; i < R[h]; i += 64) {
+      par[b + i] = b + i;
+      key[b + i] = p.GP[r0[h] + i].y;
+    }
+  }
+  __syncthreads();
+  // unions inside the group; the others move to the front of the list, never
+  // past an entry that is still to be read
+#pragma unroll
+  for (int h = 0; h < TPW; h++) {
+    const uint32_t b = base[number(h)];
+    uint32_t kept = 0;
+    auto settle = [&](uint32_t i, uint32_t e, int l, uint32_t p1, uint32_t q1) {
+      const bool out = i < nq[h] && l < 0;
+      if (l >= 0) runion(par, b + p1 - 1u, base[l] + q1 - 1u);
+      const uint64_t m = wave_ballot(out);
+      if (out) list[h][kept + mbcnt64(m)] = (uint16_t)e;
+      kept += (uint32_t)__builtin_popcountll(m);
+    };
+#pragma unroll
+    for (int k = 0; k < 2; k++) settle(64u * k + (uint32_t)lane, rq[h][k], ql[h][k], jp[h][k], jq[h][k]);
+    for (uint32_t i0 = 128; i0 < nq[h]; i0 += 64) {
+      const uint32_t i = i0 + (uint32_t)lane;
+      uint32_t e = 0, p1 = 0, q1 = 0;
+      int l = -1;
+      if (i < nq[h]) {
+        e = list[h][i];
+        l = ends(h, e, p1, q1);
+      }
+      settle(i, e, l, p1, q1);
+      wave_order();
+    }
+    if (valid[h] && lane == 0) const_cast<uint32_t*>(p.TQ)[slot[h]] = kept;
+  }
+  __syncthreads();
+  for (uint32_t i = t; i < total; i += GRP_NT) {
+    const uint32_t r = rfind_ro(par, i);
+    if (r != i) {
+      lstore(par + i, r);
+      atomicMin(key + r, key[i]);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int h = 0; h < TPW; h++) {
+    const uint32_t b = base[number(h)];
+    for (uint32_t i = lane; i < R[h]; i += 64) {
+      const uint32_t n = b + i, r = par[n], k = key[r];
+      const uint32_t own = r == n ? p.GP[r0[h] + i].y : key[n];
+      if (own != k) atomicAnd(p.bits + (own >> 5), ~(1u << (own & 31)));
+      if (r != n) {
+        int lr = 0;  // r's tile
+#pragma unroll
+        for (int s = GRP / 2; s > 0; s >>= 1) lr += base[lr + s] <= r ? s : 0;
+        p.GP[r0[h] + i].x = root0s[lr] + (r - base[lr]);
+      } else if (own != k) {
+        p.GP[r0[h] + i].y = k;
+      }
+    }
+  }
+}
+
+// Cross-tile unions of row tiles on the global forest, one wave per tile.  The
+// links of a border join the same few pairs of local roots again and again,
+// so a wave drops the pairs that one of its lanes has taken before: a table of
+// the tile's pairs in LDS, and within the requests of a round the lane that
+// wrote a slot last stands for the others with its pair.  A table slot that
+// another pair took only costs a repeated union.  (8 lanes per tile without
+// the table: 192 us on the 512^3 uint32 Voronoi volume, 285 us on a p = 0.3
+// mask; with it 182 and 243 us.)
 constexpr int RRQ_SLOTS = 256;
 template <class G>
 __global__ __launch_bounds__(WG) void k_rrequests(GlobalParams p) {
@@ -280,45 +460,56 @@ __global__ __launch_bounds__(WG) void k_rrequests(GlobalParams p) {
   const int64_t nw = (int64_t)gridDim.x * (WG / 64);
   const uint16_t* REQ = reinterpret_cast<const uint16_t*>(p.REQ);
   for (int64_t slot = w0; slot < p.ntiles; slot += nw) {
+    // the first requests are loaded beside their number: the list's storage
+    // holds more than 128 whatever the number is
+    const uint16_t* list = REQ + slot * p.reqcap;
+    const uint32_t rq[2] = {list[lane], list[lane + 64]};
     const uint32_t nq = p.TQ[slot];
+    const bool j8 = p.TR[slot] <= 255;
     if (nq == 0) continue;
     const VolGeo v = vol_geo(p, slot);
     int64_t tx, ty, tz;
     tile_coords((uint32_t)(slot - v.tile0), v.ntx, v.nty, v.dxy, v.dx, tx, ty, tz);
     const uint32_t root0 = tile_root0<G>(v.sx, v.sy, v.sz, tx, ty, tz, v.key0);
-    const bool j8 = p.TR[slot] <= 255;
 #pragma unroll
     for (int k = 0; k < RRQ_SLOTS / 64; k++) tab[wv][lane + 64 * k] = make_uint2(0xFFFFFFFFu, 0xFFFFFFFFu);
     wave_order();
-    for (uint32_t i0 = 0; i0 < nq; i0 += 64) {
-      const uint32_t i = i0 + (uint32_t)lane;
-      uint32_t a = 0xFFFFFFFFu, b = 0xFFFFFFFFu;
-      if (i < nq) {
-        const uint32_t rq = REQ[slot * p.reqcap + i];
-        const int ps = (int)(rq & 0xFFFu);
-        const uint32_t j = j8 ? p.J8[slot * G::TV + ps] : p.J16[slot * G::TV + ps];
-        int dx, dy, dz;
-        rel_decode(rq >> 12, dx, dy, dz);
-        const int64_t gx = tx * G::TX + (ps & 63) + dx;
-        const int64_t gy = ty * G::TY + ((ps >> 6) & (G::TY - 1)) + dy;
-        const int64_t gz = tz * G::TZ + ps / (64 * G::TY) + dz;
-        b = lroot_index<G>(p, v, gx, gy, gz);
-        a = root0 + j - 1;
+    // two requests per lane and round, so that their loads overlap
+    for (uint32_t i0 = 0; i0 < nq; i0 += 128) {
+      uint32_t a[2], b[2];
+#pragma unroll
+      for (int k = 0; k < 2; k++) {
+        const uint32_t i = i0 + 64u * k + (uint32_t)lane;
+        a[k] = b[k] = 0xFFFFFFFFu;
+        if (i < nq) {
+          const uint32_t e = i0 == 0 ? rq[k] : list[i];
+          int ox, oy, oz;
+          uint32_t jp, jq;
+          request_ends<G>(p, v.ntx, v.nty, slot, j8, e, ox, oy, oz, jp, jq);
+          a[k] = root0 + jp - 1u;
+          b[k] = tile_root0<G>(v.sx, v.sy, v.sz, tx + ox, ty + oy, tz + oz, v.key0) + jq - 1u;
+        }
       }
-      bool live = b != 0xFFFFFFFFu;
-      const uint32_t h = (((a * 0x9E3779B1u) ^ (b * 0x85EBCA77u)) >> 24) & (RRQ_SLOTS - 1);
-      if (live) {
-        const uint2 q = tab[wv][h];
-        live = q.x != a || q.y != b;
+      bool live[2];
+#pragma unroll
+      for (int k = 0; k < 2; k++) {
+        live[k] = b[k] != 0xFFFFFFFFu;
+        const uint32_t h = (((a[k] * 0x9E3779B1u) ^ (b[k] * 0x85EBCA77u)) >> 24) & (RRQ_SLOTS - 1);
+        if (live[k]) {
+          const uint2 q = tab[wv][h];
+          live[k] = q.x != a[k] || q.y != b[k];
+        }
+        if (live[k]) own[wv][h] = (uint32_t)lane;
+        wave_order();
+        const int o = live[k] ? (int)own[wv][h] : lane;
+        const uint32_t oa = __shfl(a[k], o), ob = __shfl(b[k], o);
+        if (live[k] && o != lane && oa == a[k] && ob == b[k]) live[k] = false;
+        if (live[k]) tab[wv][h] = make_uint2(a[k], b[k]);
+        wave_order();
       }
-      if (live) own[wv][h] = (uint32_t)lane;
-      wave_order();
-      const int o = live ? (int)own[wv][h] : lane;
-      const uint32_t oa = __shfl(a, o), ob = __shfl(b, o);
-      if (live && o != lane && oa == a && ob == b) live = false;
-      if (live) tab[wv][h] = make_uint2(a, b);
-      wave_order();
-      if (live) kunion(p.GP, p.bits, a, b);
+#pragma unroll
+      for (int k = 0; k < 2; k++)
+        if (live[k]) kunion(p.GP, p.bits, a[k], b[k]);
     }
     wave_order();
   }
@@ -630,7 +821,7 @@ __device__ inline void fin_load(const GlobalParams& p, int64_t slot, uint32_t ro
   if (R <= 255) {
 #pragma unroll
     for (int h = 0; h < EPT / 8; h++) {
-      const uint2 w = reinterpret_cast<const uint2*>(p.J8 + slot * G::TV)[t + WG * h];
+      const uint2 w = reinterpret_cast<const uint2*>(p.J8 + slot * (2 * G::TV))[t + WG * h];
 #pragma unroll
       for (int k = 0; k < 8; k++) j[8 * h + k] = ((k < 4 ? w.x : w.y) >> (8 * (k & 3))) & 0xFFu;
     }
@@ -746,7 +937,7 @@ __device__ inline void rfin_tile(const GlobalParams& p, const VolGeo& v, int64_t
   if (R <= 255) {
 #pragma unroll
     for (int i = 0; i < PASSES; i++) {
-      const uint32_t w = reinterpret_cast<const uint32_t*>(p.J8 + slot * G::TV)[t + WG * i];
+      const uint32_t w = reinterpret_cast<const uint32_t*>(p.J8 + slot * (2 * G::TV))[t + WG * i];
       j[i][0] = (w & 0xFFu) | ((w & 0xFF00u) << 8);
       j[i][1] = ((w >> 16) & 0xFFu) | ((w >> 8) & 0xFF0000u);
     }
@@ -1258,6 +1449,7 @@ struct Geometry {
   bool is3d = true;
   bool rows = false;   // row tiles (GeoR)
   bool plane = false;  // row tiles of a single plane (GeoP)
+  bool grouped = false;  // row tiles: unions inside groups of tiles first (k_group)
   bool tall = false;  // tall voxel tiles (Geo3T) instead of Geo3
   int64_t ntx = 0, nty = 0, ntz = 0, ntiles = 0;
   int TV = 0;
@@ -1325,6 +1517,15 @@ static int plan(Geometry& g, int64_t sx, int64_t sy, int64_t sz, int64_t connect
   g.nty = (sy + TY - 1) / TY;
   g.ntz = (sz + TZ - 1) / TZ;
   g.ntiles = g.ntx * g.nty * g.ntz;
+  // Unions inside groups of tiles first, where that saves more global unions
+  // than it costs (k_group + k_requests against k_requests alone, us):
+  // continuous volumes from 4,096 tiles (256^3 tones 26 59 and 95, 512^3 155
+  // and 277; 192^3 44 and 40), multilabel ones at 26 and 18 from 8,000 (320^3
+  // 45 and 52, 512^3 159 and 182; 256^3 41 and 33; at 6 512^3 uint64 142 and
+  // 123), binary 8-connected planes from 32,768 (16384^2 213 and 272; 8192^2
+  // 105 and 99).  Binary volumes gain nothing (512^3 p = 0.3 221 and 227).
+  g.grouped = g.rows ? (g.mode == M_CONT && g.ntiles >= 4096) || (g.mode == M_MULTI && g.nb != 6 && g.ntiles >= 8000)
+                     : g.plane && g.mode == M_BINARY && g.nb == 8 && g.ntiles >= 32768;
   g.nwords = (g.K + 31) / 32;
   g.nblk = (g.nwords + SCAN_WPB - 1) / SCAN_WPB;
   if (g.qk == Q_BLOCK8) {
@@ -1343,8 +1544,7 @@ static int plan(Geometry& g, int64_t sx, int64_t sy, int64_t sz, int64_t connect
   g.oTR = take((size_t)g.ntiles * 4);
   g.oTQ = take((size_t)g.ntiles * 4);
   g.oTC = take((size_t)g.ntiles * sizeof(TileCnt));
-  g.oJ8 = take(slots);
-  g.oJ16 = take(slots * 2);
+  g.oJ8 = g.oJ16 = take(slots * 2);  // a tile has one of the two, in the same place
   g.oREQ = take((size_t)g.ntiles * g.req_bytes);
   g.oBITS = take((size_t)g.nwords * 4);
   g.oPRE = take((size_t)g.nwords * 4);
@@ -1464,6 +1664,18 @@ void launch_requests(const GlobalParams& p, int64_t ntiles, int mode, hipStream_
 }
 
 template <class G>
+void launch_group(const GlobalParams& p, hipStream_t s) {
+  using GG = GroupGeo<G>;
+  GroupGrid gg;
+  gg.nx = (uint32_t)((p.ntx + GG::X - 1) / GG::X);
+  gg.ny = (uint32_t)((p.nty + GG::Y - 1) / GG::Y);
+  gg.n = gg.nx * gg.ny * (uint32_t)((p.ntz + GG::Z - 1) / GG::Z);
+  gg.dxy = Div((int64_t)gg.nx * gg.ny);
+  gg.dx = Div(gg.nx);
+  hipLaunchKernelGGL(k_group<G>, dim3(gg.n), dim3(GRP_NT), 0, s, p, gg);
+}
+
+template <class G>
 void launch_rrequests(const GlobalParams& p, int64_t ntiles, hipStream_t s) {
   hipLaunchKernelGGL(k_rrequests<G>, dim3(grid_for(ntiles, WG / 64, 65536)), dim3(WG), 0, s, p);
 }
@@ -1472,6 +1684,12 @@ template <class G>
 int run_global(cc3d_amd_job* j) {
   const GlobalParams& p = j->gp;
   hipStream_t s = j->stream;
+  if constexpr (std::is_same<G, GeoR>::value || std::is_same<G, GeoP>::value) {
+    if (j->g.grouped) {
+      ProfScope ps_("k_group", s);
+      launch_group<G>(p, s);
+    }
+  }
   {
   ProfScope ps_("k_requests", s);
   if constexpr (std::is_same<G, GeoR>::value || std::is_same<G, GeoP>::value) launch_rrequests<G>(p, j->g.ntiles, s);
@@ -2296,8 +2514,7 @@ static int batch_layout(const cc3d_amd_volume* vols, int n, int mode, std::vecto
     tg.oTR = take((size_t)tg.tiles * 4);
     tg.oTQ = take((size_t)tg.tiles * 4);
     tg.oTC = take((size_t)tg.tiles * sizeof(TileCnt));
-    tg.oJ8 = take(slots);
-    tg.oJ16 = take(slots * 2);
+    tg.oJ8 = tg.oJ16 = take(slots * 2);
     tg.oREQ = take((size_t)tg.tiles * req_bytes);
   }
   for (auto& m : b.minmax) m.oMM = take(64);  // {min, max} and the last NaN index

@@ -428,13 +428,19 @@ __device__ inline uint32_t lunion(uint16_t* par, uint32_t a, uint32_t b) {
 struct KWord {
   uint32_t parent, key;
 };
+template <bool COHERENT>
 __device__ inline KWord kload(const uint2* GP, uint32_t a) {
+  if constexpr (!COHERENT) {
+    const uint2 q = GP[a];
+    return {q.x, q.y};
+  }
   const unsigned long long w = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(GP + a),
                                                  __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   return {(uint32_t)w, (uint32_t)(w >> 32)};
 }
 __device__ inline uint32_t* kparent(uint2* GP, uint32_t a) { return &GP[a].x; }
 // Root of entry a, whose word is w; on return w is the root's word.
+template <bool COHERENT>
 __device__ inline uint32_t kfind(uint2* GP, uint32_t a, KWord& w) {
   uint32_t n0 = a, n1 = a, n2 = a;  // path nodes 0..2 (only those below the root are stored)
   int depth = 0;
@@ -444,7 +450,7 @@ __device__ inline uint32_t kfind(uint2* GP, uint32_t a, KWord& w) {
     r = w.parent;
     if (depth == 1) n1 = r;
     else if (depth == 2) n2 = r;
-    w = kload(GP, r);
+    w = kload<COHERENT>(GP, r);
   }
   // node i (i < depth) has parent node i + 1; store where that is not r
   if (depth >= 2) __hip_atomic_store(kparent(GP, n0), r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -460,12 +466,18 @@ __device__ inline uint32_t kfind(uint2* GP, uint32_t a, KWord& w) {
 // and cleared it; a root with the minimum key is only ever linked under an
 // entry with that same key (entries sharing a key are one component), which
 // clears nothing.
+//
+// The first walks read through the caches, which may be behind other XCDs'
+// links: what they hold as a parent is an ancestor all the same, what they
+// hold as a root may have been linked since.  The compare-and-swap finds that
+// out for the entry it links (the other one need not be a root: it has the
+// smaller key, so it is no descendant), and the walks after a failed one are
+// coherent.
 __device__ inline void kunion(uint2* GP, uint32_t* bits, uint32_t a, uint32_t b) {
-  while (true) {
-    KWord wa = kload(GP, a), wb = kload(GP, b);
-    a = kfind(GP, a, wa);
-    b = kfind(GP, b, wb);
-    if (a == b) return;
+  KWord wa = kload<false>(GP, a), wb = kload<false>(GP, b);
+  a = kfind<false>(GP, a, wa);
+  b = kfind<false>(GP, b, wb);
+  while (a != b) {
     uint64_t ka = ((uint64_t)wa.key << 32) | a, kb = ((uint64_t)wb.key << 32) | b;
     if (ka < kb) {
       const uint32_t t = a;
@@ -475,11 +487,17 @@ __device__ inline void kunion(uint2* GP, uint32_t* bits, uint32_t a, uint32_t b)
       ka = kb;
       kb = tk;
     }
-    if (atomicCAS(kparent(GP, a), a, b) == a) {  // a was still a root: linked under b
+    const uint32_t old = atomicCAS(kparent(GP, a), a, b);
+    if (old == a) {  // a was still a root: linked under b
       const uint32_t key = (uint32_t)(ka >> 32);
       if (key != (uint32_t)(kb >> 32)) atomicAnd(bits + (key >> 5), ~(1u << (key & 31)));
       return;
     }
+    a = old;
+    wa = kload<true>(GP, a);
+    wb = kload<true>(GP, b);
+    a = kfind<true>(GP, a, wa);
+    b = kfind<true>(GP, b, wb);
   }
 }
 // Key of the global root of entry a, once every union is made (plain loads:

@@ -1123,8 +1123,8 @@ __device__ inline void local_tile(const LocalParams& p, int64_t tile, int64_t sl
 #pragma unroll
     for (int i = 0; i < PT / 4; i++) w8[i] = (jw[2 * i] & 0xFFu) | ((jw[2 * i] >> 8) & 0xFF00u) |
                                              ((jw[2 * i + 1] & 0xFFu) << 16) | ((jw[2 * i + 1] >> 16) << 24);
-    if constexpr (PT == 8) reinterpret_cast<uint2*>(p.J8 + slot * G::TV)[t] = make_uint2(w8[0], w8[PT / 4 - 1]);
-    else reinterpret_cast<uint32_t*>(p.J8 + slot * G::TV)[t] = w8[0];
+    if constexpr (PT == 8) reinterpret_cast<uint2*>(p.J8 + slot * (2 * G::TV))[t] = make_uint2(w8[0], w8[PT / 4 - 1]);
+    else reinterpret_cast<uint32_t*>(p.J8 + slot * (2 * G::TV))[t] = w8[0];
   } else {
     if constexpr (PT == 8)
       reinterpret_cast<uint4*>(p.J16 + slot * G::TV)[t] = make_uint4(jw[0], jw[1], jw[PT / 2 - 2], jw[PT / 2 - 1]);

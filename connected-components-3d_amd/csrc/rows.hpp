@@ -966,7 +966,7 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
       uint32_t b[4];
 #pragma unroll
       for (int i = 0; i < 4; i++) b[i] = __builtin_amdgcn_perm(pk[2 * i + 1], pk[2 * i], 0x06040200u);
-      reinterpret_cast<uint4*>(p.J8 + slot * G::TV)[t] = make_uint4(b[0], b[1], b[2], b[3]);
+      reinterpret_cast<uint4*>(p.J8 + slot * (2 * G::TV))[t] = make_uint4(b[0], b[1], b[2], b[3]);
     } else {
       uint4* o = reinterpret_cast<uint4*>(p.J16 + slot * G::TV) + 2 * t;
       o[0] = make_uint4(pk[0], pk[1], pk[2], pk[3]);

@@ -96,6 +96,20 @@ def test_plane_edges(gpu, dtype, connectivity):
     _check(many, f"continuous {k}", connectivity=connectivity, delta=2)
 
 
+@pytest.mark.parametrize("connectivity", [18, 26])
+def test_groups_of_tiles(gpu, connectivity):
+  """Volumes large enough for unions inside groups of tiles: ragged sides (the
+  last groups are partly outside), and a region of distinct voxels whose groups
+  hold more local roots than the group's table."""
+  import synth
+  vol = synth.voronoi((1250, 157, 163), 4000, seed=21)
+  vol[600:760, 40:110, 30:80] = np.arange(1, 160 * 70 * 50 + 1, dtype=np.uint32).reshape(160, 70, 50)
+  _check(vol, "multilabel groups", connectivity=connectivity, out_dtype=np.uint32)
+  tones = synth.tones((700, 160, 170), 700, seed=22)
+  tones[300:400, 60:120, 40:90] = np.arange(100 * 60 * 50, dtype=np.float32).reshape(100, 60, 50) * 50 + 1000
+  _check(tones, "continuous groups", connectivity=connectivity, delta=20, out_dtype=np.uint32)
+
+
 def test_special_float_values(gpu):
   """NaN equals nothing (not even itself), infinities and signed zeros follow ==."""
   rng = np.random.default_rng(5)
