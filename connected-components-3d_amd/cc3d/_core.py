@@ -344,6 +344,17 @@ def _decide(pl, st):
   return odt, N
 
 
+def _known_out_dtype(pl):
+  """The output dtype when it does not depend on the labels, else None: given
+  by the caller, chosen from the voxel count alone (binary_image=True), or
+  uint16 because no estimate can exceed the voxel count."""
+  if pl.out_dtype is not None:
+    return pl.out_dtype
+  if pl.binary_flag_given:
+    return _choose_out_dtype(pl, _binary_bound(pl, pl.voxels))
+  return np.dtype(np.uint16) if pl.voxels < np.iinfo(np.uint16).max else None
+
+
 def connected_components(
   data,
   max_labels: int = -1,
@@ -392,11 +403,20 @@ def _label_one(pl):
     ctypes.c_void_p(ws.data_ptr()), ws_bytes, stream))
   try:
     st = L.Stats()
+    # A known output dtype: the labels are written right behind stage 1 instead
+    # of after the host has read the counters (a gap of about 35 us in which
+    # the GPU idles).  Where the counters then raise, or the volume turns out to
+    # be a single row, the written labels are dropped.
+    known = _known_out_dtype(pl)
+    if known is not None:
+      out_dev = torch.empty(pl.voxels, dtype=_torch_out_dtype(known), device=buf.device)
+      L.check(L.lib().cc3d_amd_label_finish(job, ctypes.c_void_p(out_dev.data_ptr()), _OUT_CODE[known]))
     L.check(L.lib().cc3d_amd_job_stats(job, ctypes.byref(st)))
     odt, N = _decide(pl, st)
-    out_dev = torch.empty(pl.voxels, dtype=_torch_out_dtype(odt), device=buf.device)
-    if pl.special_row is None:
-      L.check(L.lib().cc3d_amd_label_finish(job, ctypes.c_void_p(out_dev.data_ptr()), _OUT_CODE[odt]))
+    if known is None:
+      out_dev = torch.empty(pl.voxels, dtype=_torch_out_dtype(odt), device=buf.device)
+      if pl.special_row is None:
+        L.check(L.lib().cc3d_amd_label_finish(job, ctypes.c_void_p(out_dev.data_ptr()), _OUT_CODE[odt]))
   finally:
     L.lib().cc3d_amd_job_free(job)
   if pl.special_row is not None:

@@ -1414,30 +1414,52 @@ struct ProfScope {
 
 static inline size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
-// Pinned host buffers for the jobs' counter read-back, reused across calls
-// (pinned allocation and release cost far more than a small labelling call).
-static std::mutex g_pin_mu;
-static std::vector<Counters*> g_pin_pool;
-
-static Counters* pinned_counters() {
-  {
-    std::lock_guard<std::mutex> g(g_pin_mu);
-    if (!g_pin_pool.empty()) {
-      Counters* c = g_pin_pool.back();
-      g_pin_pool.pop_back();
-      return c;
-    }
-  }
+// Pinned host buffers for the jobs' counter read-back, each with an event that
+// marks its arrival, reused across calls of one device (pinned allocation and
+// release cost far more than a small labelling call).
+struct PinnedCounters {
   Counters* c = nullptr;
-  if (hipHostMalloc(reinterpret_cast<void**>(&c), sizeof(Counters), hipHostMallocDefault) != hipSuccess) return nullptr;
-  return c;
+  hipEvent_t ready = nullptr;
+  int dev = -1;
+};
+static std::mutex g_pin_mu;
+static std::vector<PinnedCounters> g_pin_pool;
+
+static void free_pinned_counters(const PinnedCounters& p) {
+  if (p.ready) (void)hipEventDestroy(p.ready);
+  if (p.c) (void)hipHostFree(p.c);
 }
 
-static void release_pinned_counters(Counters* c) {
-  if (!c) return;
-  std::lock_guard<std::mutex> g(g_pin_mu);
-  if (g_pin_pool.size() < 64) g_pin_pool.push_back(c);
-  else (void)hipHostFree(c);
+static PinnedCounters pinned_counters() {
+  PinnedCounters p;
+  if (hipGetDevice(&p.dev) != hipSuccess) return PinnedCounters();
+  {
+    std::lock_guard<std::mutex> g(g_pin_mu);
+    for (size_t i = g_pin_pool.size(); i-- > 0;) {
+      if (g_pin_pool[i].dev != p.dev) continue;
+      p = g_pin_pool[i];
+      g_pin_pool.erase(g_pin_pool.begin() + (std::ptrdiff_t)i);
+      return p;
+    }
+  }
+  if (hipHostMalloc(reinterpret_cast<void**>(&p.c), sizeof(Counters), hipHostMallocDefault) != hipSuccess ||
+      hipEventCreateWithFlags(&p.ready, hipEventDisableTiming) != hipSuccess) {
+    free_pinned_counters(p);
+    return PinnedCounters();
+  }
+  return p;
+}
+
+static void release_pinned_counters(const PinnedCounters& p) {
+  if (!p.c) return;
+  {
+    std::lock_guard<std::mutex> g(g_pin_mu);
+    if (g_pin_pool.size() < 64) {
+      g_pin_pool.push_back(p);
+      return;
+    }
+  }
+  free_pinned_counters(p);
 }
 static inline unsigned grid_for(int64_t items, int64_t per_block, int64_t cap) {
   return (unsigned)std::max<int64_t>(1, std::min<int64_t>((items + per_block - 1) / per_block, cap));
@@ -1578,6 +1600,8 @@ struct cc3d_amd_job {
   uint32_t* qprefix = nullptr;
   uint32_t* qbsum = nullptr;
   Counters* h_ctr = nullptr;
+  PinnedCounters pin;
+  bool copied = false;     // the counters' copy to h_ctr is under way (pin.ready marks its end)
   Counters h_ctr_local{};  // host copy of the counters when nothing may be allocated
   bool ctr_local = false;
   bool have_stats = false;
@@ -1956,7 +1980,8 @@ static int job_begin(cc3d_amd_job* j, const void* in, int in_dtype, int64_t sx, 
     j->h_ctr = &j->h_ctr_local;
     j->ctr_local = true;
   } else {
-    j->h_ctr = pinned_counters();
+    j->pin = pinned_counters();
+    j->h_ctr = j->pin.c;
     if (!j->h_ctr) return fail(CC3D_AMD_ERR_NOMEM, "could not allocate pinned counters");
   }
   char* ws = j->ws;
@@ -2094,8 +2119,12 @@ int cc3d_amd_label_begin(cc3d_amd_job** out_job, const void* in, int in_dtype, i
 int cc3d_amd_job_stats(cc3d_amd_job* j, cc3d_amd_stats* st) {
   if (!j || !st) return fail(CC3D_AMD_ERR_INVALID, "NULL job or stats");
   if (!j->have_stats) {
-    HIPCHECK(hipMemcpyAsync(j->h_ctr, j->gp.ctr, sizeof(Counters), hipMemcpyDeviceToHost, j->stream));
-    HIPCHECK(hipStreamSynchronize(j->stream));
+    if (j->copied) {
+      HIPCHECK(hipEventSynchronize(j->pin.ready));
+    } else {
+      HIPCHECK(hipMemcpyAsync(j->h_ctr, j->gp.ctr, sizeof(Counters), hipMemcpyDeviceToHost, j->stream));
+      HIPCHECK(hipStreamSynchronize(j->stream));
+    }
     j->have_stats = true;
   }
   st->N = j->h_ctr->N;
@@ -2108,8 +2137,17 @@ int cc3d_amd_job_stats(cc3d_amd_job* j, cc3d_amd_stats* st) {
 
 int cc3d_amd_label_finish(cc3d_amd_job* j, void* out, int out_dtype) {
   if (!j || !out) return fail(CC3D_AMD_ERR_INVALID, "NULL job or output");
+  if (out_dtype != DT_U16 && out_dtype != DT_U32 && out_dtype != DT_U64)
+    return fail(CC3D_AMD_ERR_INVALID, "output dtype must be uint16, uint32 or uint64");
   const Geometry& g = j->g;
   hipStream_t s = j->stream;
+  // Called before the counters were asked for: their copy goes first, so that
+  // cc3d_amd_job_stats waits for stage 1 only while stage 2 already runs.
+  if (!j->have_stats && !j->copied && !j->ctr_local) {
+    HIPCHECK(hipMemcpyAsync(j->h_ctr, j->gp.ctr, sizeof(Counters), hipMemcpyDeviceToHost, s));
+    HIPCHECK(hipEventRecord(j->pin.ready, s));
+    j->copied = true;
+  }
   const dim3 grid3((unsigned)((g.ntiles + fin_tiles<Geo3>() - 1) / fin_tiles<Geo3>()));
   const dim3 grid3t((unsigned)((g.ntiles + fin_tiles<Geo3T>() - 1) / fin_tiles<Geo3T>()));
   const dim3 grid2((unsigned)((g.ntiles + fin_tiles<Geo2>() - 1) / fin_tiles<Geo2>())), block(WG);
@@ -2148,7 +2186,8 @@ int cc3d_amd_label_finish(cc3d_amd_job* j, void* out, int out_dtype) {
 void cc3d_amd_job_free(cc3d_amd_job* j) {
   if (!j) return;
   if (j->own_ws && j->ws) (void)hipFreeAsync(j->ws, j->stream);
-  if (!j->ctr_local) release_pinned_counters(j->h_ctr);
+  if (j->copied && !j->have_stats) (void)hipEventSynchronize(j->pin.ready);  // the copy still writes the buffer
+  release_pinned_counters(j->pin);
   delete j;
 }
 

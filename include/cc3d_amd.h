@@ -132,7 +132,8 @@ int cc3d_amd_label_begin(cc3d_amd_job** job, const void* in, int in_dtype, int64
                          void* workspace, size_t workspace_bytes, void* stream);
 /* Waits for stage 1 and returns its counters. */
 int cc3d_amd_job_stats(cc3d_amd_job* job, cc3d_amd_stats* stats);
-/* Stage 2: writes every voxel of `out` (out_dtype 1/2/3). */
+/* Stage 2: writes every voxel of `out` (out_dtype 1/2/3).  May be called before
+ * cc3d_amd_job_stats, which then waits for stage 1 only, while stage 2 runs. */
 int cc3d_amd_label_finish(cc3d_amd_job* job, void* out, int out_dtype);
 /* Releases the job (and its workspace when the library allocated it). */
 void cc3d_amd_job_free(cc3d_amd_job* job);
