@@ -161,6 +161,19 @@ def _stream():
   return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
+def _to_numpy(t, dtype) -> np.ndarray:
+  """A contiguous device tensor's bytes as a new 1D numpy array of `dtype`.
+
+  The copy lands in memory numpy allocated (large blocks on huge pages): a
+  pageable copy into a new torch CPU tensor runs at 4 GB/s, page faults and
+  all, this at 10 GB/s."""
+  torch = _torch()
+  out = np.empty(t.numel() * t.element_size() // np.dtype(dtype).itemsize, dtype=dtype)
+  if out.size:
+    torch.from_numpy(out.view(np.uint8)).copy_(t.view(torch.uint8))
+  return out
+
+
 def _require_gpu():
   torch = _torch()
   if not torch.cuda.is_available():
@@ -493,7 +506,7 @@ def _deliver(out_dev, vol, sx, sy, sz, dims, order, out_dtype, out_file, N, retu
         strides.append(strides[-1] * s)
       out = out_dev.as_strided(shp, tuple(strides))
     return (out, N) if return_N else out
-  host = out_dev.cpu().numpy()
+  host = _to_numpy(out_dev, out_dtype)
   if out_file is not None:
     if isinstance(out_file, str):
       with open(out_file, "wb") as f:

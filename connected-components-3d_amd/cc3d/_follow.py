@@ -8,7 +8,7 @@ from typing import Union
 import numpy as np
 
 from . import _lib as L
-from ._core import _NP_TO_CODE, _Vol, _is_torch, _require_gpu, _stream, _torch, connected_components
+from ._core import _NP_TO_CODE, _Vol, _is_torch, _require_gpu, _stream, _to_numpy, _torch, connected_components
 
 
 def _bind():
@@ -28,6 +28,8 @@ def _bind():
                                        ci, ci, vp, vp, vp]
     lib.cc3d_amd_keep_labels.restype = ci
     lib.cc3d_amd_keep_labels.argtypes = [vp, ci, i64, vp, i64, u64, vp, vp, ci, vp]
+    lib.cc3d_amd_narrow_boxes.restype = ci
+    lib.cc3d_amd_narrow_boxes.argtypes = [vp, i64, vp, vp]
     lib.cc3d_amd_follow_last_error.restype = ctypes.c_char_p
     lib._follow_bound = True
   return lib
@@ -117,12 +119,16 @@ def statistics(out_labels, no_slice_conversion: bool = False) -> dict:
   voxels = sx * sy * sz
   counts, bbox, cen = _device_stats(buf, code, sx, sy, sz, ndim, f_order, N)
   nd = 2 if ndim == 2 else 3
-  counts = counts.cpu().numpy().view(np.uint32)
-  bb = bbox.cpu().numpy().view(np.uint32)
+  counts = _to_numpy(counts, np.uint32)
   big = max(sx, sy, sz) > np.iinfo(np.uint16).max
-  bdt = np.uint32 if big else np.uint16
-  bb = np.minimum(bb, np.iinfo(bdt).max).astype(bdt).reshape((N + 1, 2 * nd))
-  cen = cen.cpu().numpy().reshape((N + 1, nd))
+  if not big:  # 16-bit boxes: narrowed on the device, half the bytes to copy
+    torch = _torch()
+    narrow = torch.empty(bbox.numel(), dtype=torch.int16, device=bbox.device)
+    _fcheck(_bind().cc3d_amd_narrow_boxes(ctypes.c_void_p(bbox.data_ptr()), bbox.numel(),
+                                          ctypes.c_void_p(narrow.data_ptr()), _stream()))
+    bbox = narrow
+  bb = _to_numpy(bbox, np.uint32 if big else np.uint16).reshape((N + 1, 2 * nd))
+  cen = _to_numpy(cen, np.float64).reshape((N + 1, nd))
   output = {"voxel_counts": counts, "bounding_boxes": bb, "centroids": cen}
   if no_slice_conversion:
     return output
@@ -211,12 +217,13 @@ def dust(img, threshold: Union[int, float, tuple, list], connectivity: int = 26,
       img = np.zeros(img.shape, dtype=img.dtype, order="F")
     return (img, dust_N) if return_N else img
 
-  host = img_dev.cpu().numpy().view(img.dtype if img.dtype != np.bool_ else np.uint8)
-  if img.dtype == np.bool_:
-    host = host.view(np.bool_)
-  # write through the caller's array (a strided view included), as the
-  # reference's img[mask] = 0 does
-  img[...] = host.reshape(img.shape, order=order)
+  # write through the caller's array, as the reference's img[mask] = 0 does:
+  # straight into its memory where it is packed, through numpy's assignment
+  # into a strided view, a subclass or (an error there) a read-only array
+  if type(img) is np.ndarray and img.flags.writeable and (img.flags.c_contiguous or img.flags.f_contiguous):
+    torch.from_numpy(np.ravel(img, order="K").view(np.uint8)).copy_(img_dev.view(torch.uint8))
+  else:
+    img[...] = _to_numpy(img_dev, img.dtype).reshape(img.shape, order=order)
   img = img.view(orig_dtype)
   return (img, dust_N) if return_N else img
 
@@ -267,7 +274,10 @@ def largest_k(img, k: int, connectivity: int = 26, delta: Union[int, float] = 0,
     cc_t, N = connected_components(tview, connectivity=connectivity, return_N=True, delta=delta,
                                    binary_image=bool(binary_image))
     if N <= k:
-      cc_labels = cc_t.cpu().numpy()  # the input's shape and memory order
+      # the input's shape and memory order
+      flat = _to_numpy(cc_t.as_strided((cc_t.numel(),), (1,)),
+                       {torch.uint16: np.uint16, torch.uint32: np.uint32, torch.uint64: np.uint64}[cc_t.dtype])
+      cc_labels = flat.reshape(tuple(cc_t.shape), order=io)
       return (cc_labels, N) if return_N else cc_labels
     cc_shape, cc_c = img.shape, img.flags.c_contiguous
     cc_dtype = np.dtype({torch.uint16: np.uint16, torch.uint32: np.uint32, torch.uint64: np.uint64}[cc_t.dtype])
@@ -282,7 +292,7 @@ def largest_k(img, k: int, connectivity: int = 26, delta: Union[int, float] = 0,
 
   buf, code, sx, sy, sz, ndim, f_order, NL = lv
   counts, _, _ = _device_stats(buf, code, sx, sy, sz, ndim, f_order, NL, bbox=False, centroids=False)
-  cts = counts.cpu().numpy().view(np.uint32)
+  cts = _to_numpy(counts, np.uint32)
   if k == 1:
     keep = [int(np.argmax(cts[1:])) + 1]
     out_np = np.dtype(np.bool_)
@@ -298,10 +308,7 @@ def largest_k(img, k: int, connectivity: int = 26, delta: Union[int, float] = 0,
   _fcheck(_bind().cc3d_amd_keep_labels(
     ctypes.c_void_p(buf.data_ptr()), code, voxels, ctypes.c_void_p(keep_t.data_ptr()), len(keep), NL,
     ctypes.c_void_p(lut.data_ptr()), ctypes.c_void_p(out_t.data_ptr()), _NP_TO_CODE[out_np], _stream()))
-  host = out_t.cpu().numpy()
-  cc_out = np.zeros(cc_shape, dtype=out_np, order="C" if cc_c else "F")
-  flat = np.ravel(cc_out, order="K")
-  flat[:] = host.view(flat.dtype)
+  cc_out = _to_numpy(out_t, out_np).reshape(cc_shape, order="C" if cc_c else "F")
   if return_N:
     return cc_out, (1 if k == 1 else len(keep))
   return cc_out

@@ -7,7 +7,7 @@ import ctypes
 import numpy as np
 
 from . import _lib as L
-from ._core import DimensionError, _require_gpu, _stream, _torch
+from ._core import DimensionError, _require_gpu, _stream, _to_numpy, _torch
 
 _UNSIGNED = {8: np.uint64, 4: np.uint32, 2: np.uint16, 1: np.uint8}
 _CODE = {1: L.DT_U8, 2: L.DT_U16, 4: L.DT_U32, 8: L.DT_U64}
@@ -61,7 +61,7 @@ def voxel_connectivity_graph(data: np.ndarray, connectivity: int = 26) -> np.nda
   if rc != L.OK:
     msg = lib.cc3d_amd_graphs_last_error().decode(errors="replace")
     raise (RuntimeError if rc == L.ERR_RUNTIME else ValueError)(msg)
-  graph = out.cpu().numpy().view(out_dtype)
+  graph = _to_numpy(out, out_dtype)
   if dims == 3:
     return graph.reshape((sx, sy, sz), order="F")
   elif dims == 2:
@@ -105,7 +105,7 @@ def color_connectivity_graph(vcg, connectivity=26, return_N=False):
   if rc != L.OK:
     msg = lib.cc3d_amd_color_last_error().decode(errors="replace")
     raise (RuntimeError if rc == L.ERR_RUNTIME else MemoryError if rc == L.ERR_NOMEM else ValueError)(msg)
-  labels = out.cpu().numpy().view(np.uint32).reshape((sx, sy, sz), order="F")
+  labels = _to_numpy(out, np.uint32).reshape((sx, sy, sz), order="F")
   while labels.ndim > dims:
     labels = labels[..., 0]
   if return_N:

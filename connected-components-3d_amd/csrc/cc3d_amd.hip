@@ -1461,6 +1461,47 @@ static void release_pinned_counters(const PinnedCounters& p) {
   }
   free_pinned_counters(p);
 }
+// Pinned blocks for the batches' tables, kept for the next batch of the same
+// device (at most 16 blocks of at most 1 MiB each). A block comes back when the
+// batch's stream has drained, so no copy reads it any more.
+struct PinnedBlock {
+  char* p = nullptr;
+  size_t bytes = 0;
+  int dev = -1;
+};
+static std::vector<PinnedBlock> g_block_pool;  // under g_pin_mu
+constexpr size_t BLOCK_KEEP = 1 << 20;
+
+static PinnedBlock pinned_block(size_t bytes) {
+  PinnedBlock b;
+  if (hipGetDevice(&b.dev) != hipSuccess) return PinnedBlock();
+  {
+    std::lock_guard<std::mutex> g(g_pin_mu);
+    for (size_t i = g_block_pool.size(); i-- > 0;) {
+      if (g_block_pool[i].dev != b.dev || g_block_pool[i].bytes < bytes) continue;
+      b = g_block_pool[i];
+      g_block_pool.erase(g_block_pool.begin() + (std::ptrdiff_t)i);
+      return b;
+    }
+  }
+  b.bytes = 1 << 14;
+  while (b.bytes < bytes) b.bytes <<= 1;
+  if (hipHostMalloc(reinterpret_cast<void**>(&b.p), b.bytes, hipHostMallocDefault) != hipSuccess) return PinnedBlock();
+  return b;
+}
+
+static void release_block(const PinnedBlock& b) {
+  if (!b.p) return;
+  {
+    std::lock_guard<std::mutex> g(g_pin_mu);
+    if (g_block_pool.size() < 16 && b.bytes <= BLOCK_KEEP) {
+      g_block_pool.push_back(b);
+      return;
+    }
+  }
+  (void)hipHostFree(b.p);
+}
+
 static inline unsigned grid_for(int64_t items, int64_t per_block, int64_t cap) {
   return (unsigned)std::max<int64_t>(1, std::min<int64_t>((items + per_block - 1) / per_block, cap));
 }
@@ -1616,6 +1657,7 @@ struct cc3d_amd_batch {
   size_t total = 0;
   int64_t ntiles = 0, nkeys = 0, nwords = 0, nblk = 0;
   size_t oVOL = 0, oGP = 0, oBITS = 0, oPRE = 0, oBSUM = 0, oCTR = 0;
+  PinnedBlock pin;            // holds the three tables below
   BatchVol* h_tab = nullptr;  // pinned host copy of the volume table
   int64_t* h_t0 = nullptr;    // pinned: first tile of each volume, per tile group (n + tile groups)
   Counters* h_ctr = nullptr;  // pinned: entry 0 whole batch, 1 + k table entry k
@@ -2609,14 +2651,15 @@ int cc3d_amd_batch_create(cc3d_amd_batch** out_batch, const cc3d_amd_volume* vol
     b->ws = static_cast<char*>(p);
     b->own_ws = true;
   }
-  if (hipHostMalloc(reinterpret_cast<void**>(&b->h_tab), n * sizeof(BatchVol), hipHostMallocDefault) != hipSuccess ||
-      hipHostMalloc(reinterpret_cast<void**>(&b->h_t0), t0.size() * sizeof(int64_t), hipHostMallocDefault) !=
-        hipSuccess ||
-      hipHostMalloc(reinterpret_cast<void**>(&b->h_ctr), (n + 1) * sizeof(Counters), hipHostMallocDefault) !=
-        hipSuccess) {
+  const size_t tab_bytes = align256(n * sizeof(BatchVol)), t0_bytes = align256(t0.size() * sizeof(int64_t));
+  b->pin = pinned_block(tab_bytes + t0_bytes + (n + 1) * sizeof(Counters));
+  if (!b->pin.p) {
     cc3d_amd_batch_free(b);
     return fail(CC3D_AMD_ERR_NOMEM, "could not allocate pinned batch tables");
   }
+  b->h_tab = reinterpret_cast<BatchVol*>(b->pin.p);
+  b->h_t0 = reinterpret_cast<int64_t*>(b->pin.p + tab_bytes);
+  b->h_ctr = reinterpret_cast<Counters*>(b->pin.p + tab_bytes + t0_bytes);
   for (const auto& m : b->minmax) tab[m.k].minmax = reinterpret_cast<const uint64_t*>(b->ws + m.oMM);
   std::memcpy(b->h_tab, tab.data(), n * sizeof(BatchVol));
   std::memcpy(b->h_t0, t0.data(), t0.size() * sizeof(int64_t));
@@ -2909,11 +2952,9 @@ void cc3d_amd_batch_free(cc3d_amd_batch* b) {
   if (!b) return;
   if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
   if (b->graph) (void)hipGraphDestroy(b->graph);
-  if (b->h_tab || b->h_t0 || b->h_ctr) (void)hipStreamSynchronize(b->stream);
+  if (b->pin.p) (void)hipStreamSynchronize(b->stream);
   if (b->own_ws && b->ws) (void)hipFreeAsync(b->ws, b->stream);
-  if (b->h_tab) (void)hipHostFree(b->h_tab);
-  if (b->h_t0) (void)hipHostFree(b->h_t0);
-  if (b->h_ctr) (void)hipHostFree(b->h_ctr);
+  release_block(b->pin);
   delete b;
 }
 

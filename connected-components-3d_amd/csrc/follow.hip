@@ -325,6 +325,14 @@ __global__ void k_centroids(const uint32_t* counts, const unsigned long long* su
   }
 }
 
+// Boxes as uint16, clamped (absent labels have 0xFFFFFFFF as minimum).
+__global__ __launch_bounds__(WG) void k_narrow_boxes(const uint32_t* bbox, int64_t n, uint16_t* out) {
+  for (int64_t i = (int64_t)blockIdx.x * WG + threadIdx.x; i < n; i += (int64_t)gridDim.x * WG) {
+    const uint32_t v = bbox[i];
+    out[i] = (uint16_t)(v < 65535u ? v : 65535u);
+  }
+}
+
 // dust: erase[l] = 1 when voxels of label l are to be zeroed.
 __global__ void k_dust_table(const uint32_t* counts, int64_t N, double lo, double hi, int ranged, int invert,
                              uint8_t* erase, unsigned long long* nmask) {
@@ -522,6 +530,16 @@ int cc3d_amd_statistics(const void* labels, int dtype, int64_t s0, int64_t s1, i
   if (centroids)
     hipLaunchKernelGGL(k_centroids, dim3(fgrid(n1, WG, 8192)), dim3(WG), 0, s, counts, sums, centroids, n1, nd);
   if (hipGetLastError() != hipSuccess) return ffail(CC3D_AMD_ERR_HIP, "statistics launch failed");
+  return CC3D_AMD_OK;
+}
+
+// Box coordinates bbox[n] clamped to 16 bits (sides up to 65,535).
+int cc3d_amd_narrow_boxes(const uint32_t* bbox, int64_t n, uint16_t* out, void* stream) {
+  if (!bbox || !out || n < 0) return ffail(CC3D_AMD_ERR_INVALID, "narrow_boxes: bad argument");
+  if (n == 0) return CC3D_AMD_OK;
+  hipLaunchKernelGGL(k_narrow_boxes, dim3(fgrid(n, 4 * WG, 8192)), dim3(WG), 0, static_cast<hipStream_t>(stream), bbox,
+                     n, out);
+  if (hipGetLastError() != hipSuccess) return ffail(CC3D_AMD_ERR_HIP, "narrow_boxes launch failed");
   return CC3D_AMD_OK;
 }
 

@@ -215,6 +215,10 @@ int cc3d_amd_statistics(const void* labels, int dtype, int64_t s0, int64_t s1, i
                         int ndim, int f_order, uint64_t N, uint32_t* counts, uint32_t* bbox,
                         double* centroids, unsigned long long* sums_scratch, void* stream);
 
+/* Box coordinates bbox[n] of cc3d_amd_statistics clamped to 16 bits, for
+ * volumes whose sides are at most 65,535: half the bytes to copy to the host. */
+int cc3d_amd_narrow_boxes(const uint32_t* bbox, int64_t n, uint16_t* out, void* stream);
+
 /* The masking step of cc3d.dust (cc3d/__init__.py:121-150): zero img where
  * the voxel's component fails `size < lo` (ranged == 0) or
  * `!(lo <= size < hi)` (ranged != 0), inverted when invert != 0.
