@@ -1,7 +1,7 @@
 // Global phases of the labelling pipeline and the C ABI (include/cc3d_amd.h).
 //
 // Pipeline for one volume (stream-ordered, no host round trip until stats):
-//   k_init       reset counters, clear the root bitmask
+//   [k_init]     clear the root bitmask, where the local kernel does not store all of it
 //   [k_minmax]   continuous 2D-8 only: global min/max (cc3d/cc3d_continuous.hpp:298-303)
 //   k_local      per tile: LDS union-find, local roots, J tables, requests; every
 //                local root sets the bit of its key in the root bitmask
@@ -10,7 +10,8 @@
 //                its smallest key; a link clears the bit of the root it buries,
 //                so the bits left mark the global roots (kunion)
 //   [k_periodic] wrap-around unions (cc3d/cc3d.hpp:1048-1073, :1265-1277, :1377-1418)
-//   k_scan_*     exclusive popcount prefix over the bitmask -> N
+//   k_scan_*     exclusive popcount prefix over the bitmask -> N; the tiles'
+//                counters summed; both written to the job's pinned host copy
 //   --- stage 2 ---
 //   k_finalize   per local root: its global root's key (a find on the settled
 //                forest), final label = 1 + rank of that key;
@@ -39,6 +40,10 @@
 
 namespace cc3d_amd {
 
+static inline unsigned grid_for(int64_t items, int64_t per_block, int64_t cap) {
+  return (unsigned)std::max<int64_t>(1, std::min<int64_t>((items + per_block - 1) / per_block, cap));
+}
+
 // ---------------------------------------------------------------------------
 // small kernels
 // ---------------------------------------------------------------------------
@@ -62,6 +67,14 @@ __global__ void k_init(Counters* c, uint32_t* bits, int64_t nwords) {
     for (int64_t w = i; w < nwords; w += stride) bits[w] = 0;
   }
 }
+
+// Sums and extremes of the local kernel's counters.
+struct TileSum {
+  unsigned long long epl, prov;
+  long long first, last;
+};
+constexpr TileSum NO_TILES = {0, 0, 0x7FFFFFFFFFFFFFFFll, -1};
+constexpr unsigned FOLD_MAX = WG;  // TileSums of one scan, at most
 
 // Union tables (UTab in common.hpp), one copy per device, built once by
 // k_build_utab: each thread grows one (border class, link mask) entry.
@@ -108,49 +121,44 @@ __global__ void k_batch_init(Counters* c, int nc, uint32_t* bits, int64_t nwords
   for (int64_t w = i; w < nwords; w += (int64_t)gridDim.x * blockDim.x) bits[w] = 0;
 }
 
-// Folds the local kernel's per-tile counters into Counters.
-__global__ __launch_bounds__(WG) void k_tile_counters(const TileCnt* tc, int64_t ntiles, Counters* c) {
-  __shared__ unsigned long long se[WG / 64], sp[WG / 64];
-  __shared__ long long sf[WG / 64], sl[WG / 64];
-  unsigned long long e = 0, pv = 0;
-  long long f = 0x7FFFFFFFFFFFFFFFll, l = -1;
-  for (int64_t i = (int64_t)blockIdx.x * WG + threadIdx.x; i < ntiles; i += (int64_t)gridDim.x * WG) {
-    const TileCnt v = tc[i];
-    e += v.epl;
-    pv += v.prov;
-    f = v.first_row < f ? v.first_row : f;
-    l = v.last_row > l ? v.last_row : l;
-  }
+// The total of a block's TileSums, in thread 0.
+template <int NT>
+__device__ inline TileSum block_sum(TileSum t) {
+  __shared__ TileSum ws[NT / 64];
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
-    e += __shfl_xor(e, o);
-    pv += __shfl_xor(pv, o);
-    const long long f2 = __shfl_xor(f, o), l2 = __shfl_xor(l, o);
-    f = f2 < f ? f2 : f;
-    l = l2 > l ? l2 : l;
+    t.epl += __shfl_xor(t.epl, o);
+    t.prov += __shfl_xor(t.prov, o);
+    const long long f2 = __shfl_xor(t.first, o), l2 = __shfl_xor(t.last, o);
+    t.first = f2 < t.first ? f2 : t.first;
+    t.last = l2 > t.last ? l2 : t.last;
   }
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  if (lane == 0) {
-    se[wv] = e;
-    sp[wv] = pv;
-    sf[wv] = f;
-    sl[wv] = l;
-  }
+  if (lane == 0) ws[wv] = t;
   __syncthreads();
   if (threadIdx.x == 0) {
-    for (int w = 1; w < WG / 64; w++) {
-      e += se[w];
-      pv += sp[w];
-      f = sf[w] < f ? sf[w] : f;
-      l = sl[w] > l ? sl[w] : l;
-    }
-    if (e) atomicAdd(&c->epl, e);
-    if (pv) atomicAdd(&c->prov, pv);
-    if (l >= 0) {
-      atomicMin(&c->first_row, f);
-      atomicMax(&c->last_row, l);
+    for (int w = 1; w < NT / 64; w++) {
+      t.epl += ws[w].epl;
+      t.prov += ws[w].prov;
+      t.first = ws[w].first < t.first ? ws[w].first : t.first;
+      t.last = ws[w].last > t.last ? ws[w].last : t.last;
     }
   }
+  return t;
+}
+
+// The same over tiles i0, i0 + stride, ... below n.
+template <int NT>
+__device__ inline TileSum tile_sum(const TileCnt* tc, int64_t i0, int64_t n, int64_t stride) {
+  TileSum t = NO_TILES;
+  for (int64_t i = i0; i < n; i += stride) {
+    const TileCnt c = tc[i];
+    t.epl += c.epl;
+    t.prov += c.prov;
+    t.first = c.first_row < t.first ? c.first_row : t.first;
+    t.last = c.last_row > t.last ? c.last_row : t.last;
+  }
+  return block_sum<NT>(t);
 }
 
 struct GlobalParams {
@@ -626,6 +634,7 @@ __global__ __launch_bounds__(WG) void k_periodic(GlobalParams p, const T* in, in
 constexpr int SCAN_WPT = 16;
 constexpr int SCAN_WPB = SCAN_WPT * WG;
 
+template <int NT = WG>
 __device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t* tmp, uint32_t& total) {
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   uint32_t x = v;
@@ -637,7 +646,7 @@ __device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t* tmp, uint3
   if (lane == 63) tmp[wv] = x;
   __syncthreads();
   uint32_t base = 0, tot = 0;
-  for (int w = 0; w < WG / 64; w++) {
+  for (int w = 0; w < NT / 64; w++) {
     if (w < wv) base += tmp[w];
     tot += tmp[w];
   }
@@ -664,7 +673,43 @@ __device__ inline void load_words(const uint32_t* bits, int64_t base, int64_t nw
   }
 }
 
-__global__ __launch_bounds__(WG) void k_scan_a(const uint32_t* bits, int64_t nwords, uint32_t* bsum) {
+// Where a job's counters go: the workspace and, where the host reads them
+// without a copy, its pinned buffer.
+struct CounterSink {
+  const TileCnt* tc;  // null: only N is known
+  int64_t ntiles;
+  TileSum* sums;      // one per folding block of k_scan_a
+  unsigned folds;
+  Counters *ctr, *host;
+};
+
+__device__ inline void publish(const CounterSink& k, const TileSum& t, bool tiles, uint64_t N) {
+  for (int i = 0; i < 2; i++) {
+    Counters* c = i ? k.host : k.ctr;
+    if (!c) continue;
+    c->N = N;
+    if (!tiles) continue;
+    c->epl = t.epl;
+    c->prov = t.prov;
+    c->first_row = t.first;
+    c->last_row = t.last;
+  }
+}
+// By one block, after k_scan_a.
+__device__ inline void publish_folded(const CounterSink& k, uint64_t N) {
+  const TileSum t = block_sum<WG>(threadIdx.x < k.folds ? k.sums[threadIdx.x] : NO_TILES);
+  if (threadIdx.x == 0) publish(k, t, k.tc != nullptr, N);
+}
+
+// Blocks from nblk on fold the tiles' counters.
+__global__ __launch_bounds__(WG) void k_scan_a(const uint32_t* bits, int64_t nwords, uint32_t* bsum, int64_t nblk,
+                                               CounterSink k) {
+  if ((int64_t)blockIdx.x >= nblk) {
+    const int64_t b = (int64_t)blockIdx.x - nblk;
+    const TileSum t = tile_sum<WG>(k.tc, b * WG + threadIdx.x, k.ntiles, (int64_t)k.folds * WG);
+    if (threadIdx.x == 0) k.sums[b] = t;
+    return;
+  }
   __shared__ uint32_t tmp[WG / 64];
   const int64_t base = (int64_t)blockIdx.x * SCAN_WPB + (int64_t)threadIdx.x * SCAN_WPT;
   uint32_t w[SCAN_WPT];
@@ -677,7 +722,7 @@ __global__ __launch_bounds__(WG) void k_scan_a(const uint32_t* bits, int64_t nwo
   if (threadIdx.x == 0) bsum[blockIdx.x] = total;
 }
 
-__global__ __launch_bounds__(WG) void k_scan_b(uint32_t* bsum, int64_t nblk, Counters* ctr) {
+__global__ __launch_bounds__(WG) void k_scan_b(uint32_t* bsum, int64_t nblk, CounterSink k) {
   __shared__ uint32_t tmp[WG / 64];
   uint32_t carry = 0;
   for (int64_t off = 0; off < nblk; off += WG) {
@@ -688,7 +733,7 @@ __global__ __launch_bounds__(WG) void k_scan_b(uint32_t* bsum, int64_t nblk, Cou
     if (i < nblk) bsum[i] = carry + ex;
     carry += total;
   }
-  if (threadIdx.x == 0 && ctr) ctr->N = carry;
+  publish_folded(k, carry);
 }
 
 __global__ __launch_bounds__(WG) void k_scan_c(const uint32_t* bits, int64_t nwords, const uint32_t* bsum,
@@ -728,14 +773,14 @@ __global__ __launch_bounds__(WG) void k_scan_c(const uint32_t* bits, int64_t nwo
 // the total.
 constexpr int64_t SCAN_FUSE_MAX = 4096;
 __global__ __launch_bounds__(WG) void k_scan_bc(const uint32_t* bits, int64_t nwords, const uint32_t* bsum,
-                                                int64_t nblk, uint32_t* prefix, Counters* ctr) {
+                                                int64_t nblk, uint32_t* prefix, CounterSink k) {
   __shared__ uint32_t tmp[WG / 64];
   const int64_t lim = blockIdx.x == 0 ? nblk : (int64_t)blockIdx.x;
   uint32_t part = 0;
   for (int64_t i = threadIdx.x; i < lim; i += WG) part += bsum[i];
   uint32_t sum;
   block_exclusive_scan(part, tmp, sum);
-  if (blockIdx.x == 0 && threadIdx.x == 0 && ctr) ctr->N = sum;
+  if (blockIdx.x == 0) publish_folded(k, sum);
   const uint32_t carry = blockIdx.x == 0 ? 0u : sum;
   const int64_t base = (int64_t)blockIdx.x * SCAN_WPB + (int64_t)threadIdx.x * SCAN_WPT;
   uint32_t w[SCAN_WPT];
@@ -765,18 +810,82 @@ __global__ __launch_bounds__(WG) void k_scan_bc(const uint32_t* bits, int64_t nw
   }
 }
 
-// Exclusive popcount prefix of nwords bitmask words (nblk = blocks of
-// SCAN_WPB words); the total goes to ctr->N when ctr is given.
+// One launch for small bitmasks: each block counts the words before its own
+// 4096 itself (four rounds of eight 16-byte loads per thread at the limit, from
+// L2), and block nblk folds the counters, 16 tiles per thread at the limit. On
+// 96^3 voxels (7 blocks) k_tile_counters, k_scan_a and k_scan_bc of their own
+// took 3.8 + 3.8 + 2.8 us and a copy of the counters 2.2 more; this takes 4.6.
+constexpr int SCAN1_NT = 1024;
+constexpr int64_t SCAN1_MAX = 32, SCAN1_TILES = 16 * SCAN1_NT;
+__global__ __launch_bounds__(SCAN1_NT) void k_scan_small(const uint32_t* bits, int64_t nwords, int nblk,
+                                                         uint32_t* prefix, CounterSink k) {
+  static_assert(SCAN_WPB == 4 * SCAN1_NT, "four words per thread");
+  if ((int)blockIdx.x == nblk) {
+    const TileSum t = tile_sum<SCAN1_NT>(k.tc, threadIdx.x, k.ntiles, SCAN1_NT);
+    if (threadIdx.x != 0) return;
+    for (int i = 0; i < 2; i++) {
+      Counters* c = i ? k.host : k.ctr;
+      if (!c) continue;
+      c->epl = t.epl;
+      c->prov = t.prov;
+      c->first_row = t.first;
+      c->last_row = t.last;
+    }
+    return;
+  }
+  __shared__ uint32_t tmp[SCAN1_NT / 64];
+  const int b = (int)blockIdx.x;
+  const uint4* before = reinterpret_cast<const uint4*>(bits) + threadIdx.x;
+  uint32_t part = 0, carry, total;
+#pragma unroll 8
+  for (int i = 0; i < b; i++) {
+    const uint4 q = before[(int64_t)i * SCAN1_NT];
+    part += __popc(q.x) + __popc(q.y) + __popc(q.z) + __popc(q.w);
+  }
+  block_exclusive_scan<SCAN1_NT>(part, tmp, carry);
+  const int64_t base = (int64_t)b * SCAN_WPB + 4 * (int64_t)threadIdx.x;
+  uint32_t w[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) w[i] = base + i < nwords ? __popc(bits[base + i]) : 0u;
+  uint32_t run = carry + block_exclusive_scan<SCAN1_NT>(w[0] + w[1] + w[2] + w[3], tmp, total);
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    if (base + i < nwords) prefix[base + i] = run;
+    run += w[i];
+  }
+  if (b == nblk - 1 && threadIdx.x == 0) {
+    if (k.ctr) k.ctr->N = carry + total;
+    if (k.host) k.host->N = carry + total;
+  }
+}
+
+// Exclusive popcount prefix of nwords bitmask words (nblk = blocks of SCAN_WPB
+// words); the total goes to k.ctr->N when that is given, the counters of k's
+// tiles with it, and all of them to k.host when that is given too.
 static void launch_scan(const uint32_t* bits, int64_t nwords, uint32_t* bsum, int64_t nblk, uint32_t* prefix,
-                        Counters* ctr, hipStream_t s) {
-  hipLaunchKernelGGL(k_scan_a, dim3((unsigned)nblk), dim3(WG), 0, s, bits, nwords, bsum);
+                        CounterSink k, hipStream_t s) {
+  if (nblk <= SCAN1_MAX && k.ntiles <= SCAN1_TILES) {
+    hipLaunchKernelGGL(k_scan_small, dim3((unsigned)nblk + (k.tc ? 1u : 0u)), dim3(SCAN1_NT), 0, s, bits, nwords,
+                       (int)nblk, prefix, k);
+    return;
+  }
+  k.folds = k.tc ? grid_for(k.ntiles, WG * 2, FOLD_MAX) : 0u;
+  hipLaunchKernelGGL(k_scan_a, dim3((unsigned)nblk + k.folds), dim3(WG), 0, s, bits, nwords, bsum, nblk, k);
   if (nblk <= SCAN_FUSE_MAX) {
-    hipLaunchKernelGGL(k_scan_bc, dim3((unsigned)nblk), dim3(WG), 0, s, bits, nwords, bsum, nblk, prefix, ctr);
+    hipLaunchKernelGGL(k_scan_bc, dim3((unsigned)nblk), dim3(WG), 0, s, bits, nwords, bsum, nblk, prefix, k);
   } else {
-    hipLaunchKernelGGL(k_scan_b, dim3(1), dim3(WG), 0, s, bsum, nblk, ctr);
+    hipLaunchKernelGGL(k_scan_b, dim3(1), dim3(WG), 0, s, bsum, nblk, k);
     hipLaunchKernelGGL(k_scan_c, dim3((unsigned)nblk), dim3(WG), 0, s, bits, nwords, bsum, prefix);
   }
 }
+// The tiles' counters alone, before the scan.
+static void launch_fold(CounterSink k, hipStream_t s) {
+  k.folds = grid_for(k.ntiles, WG * 2, FOLD_MAX);
+  k.host = nullptr;
+  hipLaunchKernelGGL(k_scan_a, dim3(k.folds), dim3(WG), 0, s, nullptr, (int64_t)0, nullptr, (int64_t)0, k);
+  hipLaunchKernelGGL(k_scan_b, dim3(1), dim3(WG), 0, s, nullptr, (int64_t)0, k);
+}
+static CounterSink only_N(Counters* ctr) { return {nullptr, 0, nullptr, 0u, ctr, nullptr}; }
 
 // Stage 2: every voxel of the tile gets its local root's label.  Thread t
 // owns the column the local kernel gave it: its 8 root indices are one 8- or
@@ -915,7 +1024,7 @@ __global__ __launch_bounds__(WG) void k_finalize_batch(GlobalParams p) {
 hipError_t scan_root_bits(const uint32_t* bits, int64_t nwords, uint32_t* bsum, uint32_t* prefix, Counters* ctr,
                           hipStream_t s) {
   const int64_t nblk = (nwords + SCAN_WPB - 1) / SCAN_WPB;
-  launch_scan(bits, nwords, bsum, nblk, prefix, ctr, s);
+  launch_scan(bits, nwords, bsum, nblk, prefix, only_N(ctr), s);
   return hipGetLastError();
 }
 
@@ -1006,46 +1115,14 @@ __global__ __launch_bounds__(WG) void k_fill_vix(const int64_t* vtile0, uint32_t
 
 // Batch: per-volume counters from the per-tile records (one block per volume).
 __global__ __launch_bounds__(WG) void k_tile_counters_batch(const TileCnt* tc, const int64_t* vtile0, Counters* ctrs) {
-  __shared__ unsigned long long se[WG / 64], sp[WG / 64];
-  __shared__ long long sf[WG / 64], sl[WG / 64];
   const int v = blockIdx.x;
-  unsigned long long e = 0, pv = 0;
-  long long f = 0x7FFFFFFFFFFFFFFFll, l = -1;
-  for (int64_t i = vtile0[v] + threadIdx.x; i < vtile0[v + 1]; i += WG) {
-    const TileCnt c = tc[i];
-    e += c.epl;
-    pv += c.prov;
-    f = c.first_row < f ? c.first_row : f;
-    l = c.last_row > l ? c.last_row : l;
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    e += __shfl_xor(e, o);
-    pv += __shfl_xor(pv, o);
-    const long long f2 = __shfl_xor(f, o), l2 = __shfl_xor(l, o);
-    f = f2 < f ? f2 : f;
-    l = l2 > l ? l2 : l;
-  }
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  if (lane == 0) {
-    se[wv] = e;
-    sp[wv] = pv;
-    sf[wv] = f;
-    sl[wv] = l;
-  }
-  __syncthreads();
+  const TileSum t = tile_sum<WG>(tc, vtile0[v] + threadIdx.x, vtile0[v + 1], WG);
   if (threadIdx.x == 0) {
-    for (int w = 1; w < WG / 64; w++) {
-      e += se[w];
-      pv += sp[w];
-      f = sf[w] < f ? sf[w] : f;
-      l = sl[w] > l ? sl[w] : l;
-    }
     Counters& c = ctrs[v];
-    c.epl = e;
-    c.prov = pv;
-    c.first_row = f;
-    c.last_row = l;
+    c.epl = t.epl;
+    c.prov = t.prov;
+    c.first_row = t.first;
+    c.last_row = t.last;
   }
 }
 
@@ -1417,8 +1494,18 @@ static inline size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 // Pinned host buffers for the jobs' counter read-back, each with an event that
 // marks its arrival, reused across calls of one device (pinned allocation and
 // release cost far more than a small labelling call).
+static bool stream_capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return st != hipStreamCaptureStatusNone;
+}
+
 struct PinnedCounters {
   Counters* c = nullptr;
+  Counters* dev_c = nullptr;  // the same memory as the GPU addresses it
   hipEvent_t ready = nullptr;
   int dev = -1;
 };
@@ -1442,7 +1529,8 @@ static PinnedCounters pinned_counters() {
       return p;
     }
   }
-  if (hipHostMalloc(reinterpret_cast<void**>(&p.c), sizeof(Counters), hipHostMallocDefault) != hipSuccess ||
+  if (hipHostMalloc(reinterpret_cast<void**>(&p.c), sizeof(Counters), hipHostMallocCoherent) != hipSuccess ||
+      hipHostGetDevicePointer(reinterpret_cast<void**>(&p.dev_c), p.c, 0) != hipSuccess ||
       hipEventCreateWithFlags(&p.ready, hipEventDisableTiming) != hipSuccess) {
     free_pinned_counters(p);
     return PinnedCounters();
@@ -1502,9 +1590,6 @@ static void release_block(const PinnedBlock& b) {
   (void)hipHostFree(b.p);
 }
 
-static inline unsigned grid_for(int64_t items, int64_t per_block, int64_t cap) {
-  return (unsigned)std::max<int64_t>(1, std::min<int64_t>((items + per_block - 1) / per_block, cap));
-}
 
 struct Geometry {
   int64_t sx = 0, sy = 0, sz = 0, V = 0, K = 0, osx = 0;
@@ -1520,7 +1605,7 @@ struct Geometry {
   int64_t reqcap = 0;    // row tiles: requests in it
   int64_t nwords = 0, nblk = 0;
   int64_t qblocks = 0, qwords = 0, qnblk = 0;  // binary 2D-8 block bitmask
-  size_t oGP, oTR, oTQ, oTC, oJ8, oJ16, oREQ, oBITS, oPRE, oBSUM, oCTR, oMM, oQB, oQP, oQS, total;
+  size_t oGP, oTR, oTQ, oTC, oJ8, oJ16, oREQ, oBITS, oPRE, oBSUM, oTS, oCTR, oMM, oQB, oQP, oQS, total;
 };
 
 // tiles: CC3D_AMD_TILES_ROWS / _VOXELS / _TALL bits (else the default family)
@@ -1612,6 +1697,7 @@ static int plan(Geometry& g, int64_t sx, int64_t sy, int64_t sz, int64_t connect
   g.oBITS = take((size_t)g.nwords * 4);
   g.oPRE = take((size_t)g.nwords * 4);
   g.oBSUM = take((size_t)(g.nblk + 1) * 4);
+  g.oTS = take(FOLD_MAX * sizeof(TileSum));
   g.oCTR = take(sizeof(Counters));
   g.oMM = take(64);
   g.oQB = take((size_t)g.qwords * 4);
@@ -1642,6 +1728,10 @@ struct cc3d_amd_job {
   uint32_t* qbsum = nullptr;
   Counters* h_ctr = nullptr;
   PinnedCounters pin;
+  bool capturing = false;  // begun while the stream is being captured
+  bool direct = false;     // the scan writes h_ctr itself
+  const TileCnt* tcnt = nullptr;
+  TileSum* tsum = nullptr;
   bool copied = false;     // the counters' copy to h_ctr is under way (pin.ready marks its end)
   Counters h_ctr_local{};  // host copy of the counters when nothing may be allocated
   bool ctr_local = false;
@@ -1763,7 +1853,9 @@ int run_global(cc3d_amd_job* j) {
   else launch_requests<G, Q_NONE>(p, j->g.ntiles, j->g.mode, s);
   }
   HIPCHECK(hipGetLastError());
+  const CounterSink sink = {j->tcnt, j->g.ntiles, j->tsum, 0u, p.ctr, j->direct ? j->pin.dev_c : nullptr};
   if (j->periodic && j->g.mode != M_CONT) {
+    if (j->special_row_rule) launch_fold(sink, s);  // k_periodic asks whether one row holds all foreground
     // a 6-connected single plane wraps like the 4-neighbourhood (its z wrap pairs a voxel with itself)
     const int nbp = j->g.is3d ? 6 : j->g.nb;
     const int64_t npairs = nbp == 6 ? (j->g.sy * j->g.sz + j->g.sx * j->g.sz + j->g.sx * j->g.sy)
@@ -1797,7 +1889,7 @@ int run_global(cc3d_amd_job* j) {
   }
   {
   ProfScope ps_("k_scan", s);
-  launch_scan(p.bits, p.nwords, p.bsum, (int64_t)j->g.nblk, p.prefix, p.ctr, s);
+  launch_scan(p.bits, p.nwords, p.bsum, (int64_t)j->g.nblk, p.prefix, sink, s);
   }
   HIPCHECK(hipGetLastError());
   return CC3D_AMD_OK;
@@ -1828,7 +1920,7 @@ int launch_q1(cc3d_amd_job* j) {
                      static_cast<const T*>(j->in), g.sx, g.sy, j->qbits, j->gp.ctr);
   HIPCHECK(hipGetLastError());
   if (j->stale) {
-    launch_scan(j->qbits, g.qwords, j->qbsum, g.qnblk, j->qprefix, nullptr, s);
+    launch_scan(j->qbits, g.qwords, j->qbsum, g.qnblk, j->qprefix, only_N(nullptr), s);
     HIPCHECK(hipGetLastError());
   }
   return CC3D_AMD_OK;
@@ -1884,7 +1976,7 @@ hipError_t batch_q1(const cc3d_amd_batch* b, hipStream_t s) {
     hipLaunchKernelGGL(k_zero_words, dim3(grid_for(st.qwords, WG, 8192)), dim3(WG), 0, s, qb, st.qwords);
     hipLaunchKernelGGL((k_q1_newblocks<T>), dim3(grid_for(st.qblocks, WG, 65536)), dim3(WG), 0, s,
                        static_cast<const T*>(v.in), v.sx, v.sy, qb, b->gp.ctr + 1 + st.k);
-    launch_scan(qb, st.qwords, qs, st.qnblk, qp, nullptr, s);
+    launch_scan(qb, st.qwords, qs, st.qnblk, qp, only_N(nullptr), s);
   }
   return hipGetLastError();
 }
@@ -2025,6 +2117,10 @@ static int job_begin(cc3d_amd_job* j, const void* in, int in_dtype, int64_t sx, 
     j->pin = pinned_counters();
     j->h_ctr = j->pin.c;
     if (!j->h_ctr) return fail(CC3D_AMD_ERR_NOMEM, "could not allocate pinned counters");
+    // a captured launch would write the pooled buffer again at every replay,
+    // and the 2D-8 rules count after the scan: those jobs copy the counters
+    j->capturing = stream_capturing(j->stream);
+    j->direct = !j->capturing && !j->count_prov && !j->stale;
   }
   char* ws = j->ws;
   GlobalParams& gp = j->gp;
@@ -2050,7 +2146,8 @@ static int job_begin(cc3d_amd_job* j, const void* in, int in_dtype, int64_t sx, 
   unsigned long long* mm = reinterpret_cast<unsigned long long*>(ws + g.oMM);
   hipStream_t s = j->stream;
 
-  {
+  // not where the row kernel stores every word of the bitmask; the counters are stored by the scan
+  if (!(g.rows || g.plane) || g.qk == Q_BLOCK8 || (g.sx & 15)) {
     ProfScope ps_("k_init", s);
     hipLaunchKernelGGL(k_init, dim3(grid_for((g.nwords + 3) / 4, WG, 8192)), dim3(WG), 0, s, gp.ctr, gp.bits, g.nwords);
   }
@@ -2116,12 +2213,8 @@ static int job_begin(cc3d_amd_job* j, const void* in, int in_dtype, int64_t sx, 
   else e = launch_local_cont(in_dtype, g.nb, g.qk, g.tall, lp, s);
   }
   if (e != hipSuccess) return fail(CC3D_AMD_ERR_HIP, std::string("k_local: ") + hipGetErrorString(e));
-  {
-    ProfScope ps_("k_tile_counters", s);
-    hipLaunchKernelGGL(k_tile_counters, dim3(grid_for(g.ntiles, WG * 2, 256)), dim3(WG), 0, s, lp.tcnt, g.ntiles,
-                       gp.ctr);
-  }
-  if (hipGetLastError() != hipSuccess) return fail(CC3D_AMD_ERR_HIP, "k_tile_counters launch failed");
+  j->tcnt = lp.tcnt;
+  j->tsum = reinterpret_cast<TileSum*>(ws + g.oTS);
   rc = g.rows ? run_global<GeoR>(j)
        : g.plane ? run_global<GeoP>(j)
        : g.tall ? run_global<Geo3T>(j)
@@ -2164,7 +2257,8 @@ int cc3d_amd_job_stats(cc3d_amd_job* j, cc3d_amd_stats* st) {
     if (j->copied) {
       HIPCHECK(hipEventSynchronize(j->pin.ready));
     } else {
-      HIPCHECK(hipMemcpyAsync(j->h_ctr, j->gp.ctr, sizeof(Counters), hipMemcpyDeviceToHost, j->stream));
+      if (!j->direct)
+        HIPCHECK(hipMemcpyAsync(j->h_ctr, j->gp.ctr, sizeof(Counters), hipMemcpyDeviceToHost, j->stream));
       HIPCHECK(hipStreamSynchronize(j->stream));
     }
     j->have_stats = true;
@@ -2183,10 +2277,11 @@ int cc3d_amd_label_finish(cc3d_amd_job* j, void* out, int out_dtype) {
     return fail(CC3D_AMD_ERR_INVALID, "output dtype must be uint16, uint32 or uint64");
   const Geometry& g = j->g;
   hipStream_t s = j->stream;
-  // Called before the counters were asked for: their copy goes first, so that
-  // cc3d_amd_job_stats waits for stage 1 only while stage 2 already runs.
-  if (!j->have_stats && !j->copied && !j->ctr_local) {
-    HIPCHECK(hipMemcpyAsync(j->h_ctr, j->gp.ctr, sizeof(Counters), hipMemcpyDeviceToHost, s));
+  // Called before the counters were asked for: an event (behind their copy,
+  // unless the scan wrote them) marks their place, so that cc3d_amd_job_stats
+  // waits for stage 1 only while stage 2 already runs.
+  if (!j->have_stats && !j->copied && !j->ctr_local && !j->capturing) {
+    if (!j->direct) HIPCHECK(hipMemcpyAsync(j->h_ctr, j->gp.ctr, sizeof(Counters), hipMemcpyDeviceToHost, s));
     HIPCHECK(hipEventRecord(j->pin.ready, s));
     j->copied = true;
   }
@@ -2228,7 +2323,10 @@ int cc3d_amd_label_finish(cc3d_amd_job* j, void* out, int out_dtype) {
 void cc3d_amd_job_free(cc3d_amd_job* j) {
   if (!j) return;
   if (j->own_ws && j->ws) (void)hipFreeAsync(j->ws, j->stream);
-  if (j->copied && !j->have_stats) (void)hipEventSynchronize(j->pin.ready);  // the copy still writes the buffer
+  if (!j->have_stats) {  // the pinned counters may still be written
+    if (j->copied) (void)hipEventSynchronize(j->pin.ready);
+    else if (j->direct && j->ws) (void)hipStreamSynchronize(j->stream);
+  }
   release_pinned_counters(j->pin);
   delete j;
 }
@@ -2846,7 +2944,7 @@ int cc3d_amd_batch_begin(cc3d_amd_batch* b) {
   }
   {
     ProfScope ps_("k_scan", s);
-    launch_scan(p.bits, p.nwords, p.bsum, (int64_t)b->nblk, p.prefix, p.ctr, s);
+    launch_scan(p.bits, p.nwords, p.bsum, (int64_t)b->nblk, p.prefix, only_N(p.ctr), s);
   }
   {
     hipLaunchKernelGGL(k_batch_N, dim3((b->n + 63) / 64), dim3(64), 0, s, p.vols, b->n, p.prefix, p.nwords, p.ctr,

@@ -927,18 +927,28 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
       atomicOr(p.bits + (key >> 5), 1u << (key & 31));
       rk++;
     }
-  } else if (rb) {
-    const uint32_t key0 = (uint32_t)x0 + 16u * (uint32_t)hseg +
-                          (uint32_t)sx * ((uint32_t)(y0 + (hrow & (G::TY - 1))) +
-                                          (uint32_t)sy * (uint32_t)(z0 + hrow / G::TY)) + keybase;
+  } else {
+    const int hx = x0 + 16 * hseg, hy = y0 + (hrow & (G::TY - 1)), hz = z0 + hrow / G::TY;
+    const uint32_t key0 = (uint32_t)hx + (uint32_t)sx * ((uint32_t)hy + (uint32_t)sy * (uint32_t)hz) + keybase;
     uint32_t rk = root0 + rbase;
     for (uint32_t m = rb; m; m &= m - 1u) {
       p.GP[rk] = make_uint2(rk, key0 + (uint32_t)__builtin_ctz(m));
       rk++;
     }
-    const uint32_t sh = key0 & 31u, lo = rb << sh, hi = sh > 16u ? rb >> (32u - sh) : 0u;
-    if (lo) atomicOr(p.bits + (key0 >> 5), lo);
-    if (hi) atomicOr(p.bits + (key0 >> 5) + 1, hi);
+    if ((sx & 15) == 0) {
+      // every segment is a half-word of the bitmask that no other tile holds:
+      // stored whether or not it has roots, so nothing clears the bitmask
+      // before; the volume's last half-word clears the rest of its word
+      if (hx < sx && hy < sy && hz < sz) {
+        uint16_t* half = reinterpret_cast<uint16_t*>(p.bits) + (key0 >> 4);
+        half[0] = (uint16_t)rb;
+        if (!((key0 >> 4) & 1u) && hx + 16 == sx && hy + 1 == sy && hz + 1 == sz) half[1] = 0;
+      }
+    } else if (rb) {
+      const uint32_t sh = key0 & 31u, lo = rb << sh, hi = sh > 16u ? rb >> (32u - sh) : 0u;
+      if (lo) atomicOr(p.bits + (key0 >> 5), lo);
+      if (hi) atomicOr(p.bits + (key0 >> 5) + 1, hi);
+    }
   }
   {
     uint32_t j = 0, pk[8];

@@ -146,3 +146,31 @@ def test_scratch_limit_keeps_ragged_volumes(gpu):
     assert rc == L.OK
   torch.cuda.synchronize()
   assert en.value == gn.value and torch.equal(exp, got)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (64, 64, 1023), (64, 64, 1024), (64, 64, 1025), (1, 1, 131072),
+                                   (1, 1, 131073), (64, 2048, 1), (64, 2049, 1)])
+def test_one_launch_scan_limits(gpu, shape):
+  """Bitmasks of up to 32 blocks of 131,072 voxels and up to 16,384 tiles are
+  ranked, and their counters folded, in one launch."""
+  vol = np.asfortranarray(np.random.default_rng(len(str(shape))).integers(0, 3, size=shape).astype(np.uint16))
+  _check(vol, "scan", connectivity=6)
+  _check(vol, "scan", connectivity=26, binary_image=True)
+
+
+@pytest.mark.parametrize("shape", [(16, 1, 1), (48, 3, 1), (16, 9, 17), (80, 65, 1), (112, 8, 9), (144, 5, 8),
+                                   (96, 96, 96)])
+def test_stored_root_bits(gpu, shape):
+  """Rows of whole segments: the root bitmask is stored, not cleared first, an
+  odd last half-word included. The scratch is filled with ones before."""
+  import torch
+  rng = np.random.default_rng(sum(shape))
+  vol = np.asfortranarray(rng.integers(0, 3, size=shape).astype(np.uint32))
+  for kw in ({"connectivity": 6}, {"connectivity": 26}, {"connectivity": 18, "binary_image": True}):
+    junk = torch.full((1 << 24,), -1, dtype=torch.int32, device="cuda")
+    del junk
+    _check(vol, "bits", **kw)
+  if shape[2] == 1:
+    for conn in (4, 8):
+      _check(vol[:, :, 0], "bits 2D", connectivity=conn)
+      _check(vol[:, :, 0], "bits 2D binary", connectivity=conn, binary_image=True)
