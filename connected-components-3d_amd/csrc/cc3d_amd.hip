@@ -295,28 +295,27 @@ __device__ inline void request_ends(const GlobalParams& p, int64_t ntx, int64_t 
   if (Rq > 255) jq = p.J16[qs * G::TV + qp];
 }
 
-// Unions inside groups of 16 tiles, in LDS: 1 x 4 x 4 tiles of a volume (most
-// of a 64 x 8 x 8 tile's border is its y and z faces), 4 x 4 of a plane.  Of
-// the global unions' time nearly all is their device-scope compare-and-swaps
-// (512^3 uint32 Voronoi 26: 183 us, 39 us without them), and a group settles
-// about 70 % of them among its own tiles.  Every entry leaves with its group
+// Unions inside groups of 16 tiles of a continuous volume, in LDS: 1 x 4 x 4
+// tiles (most of a 64 x 8 x 8 tile's border is its y and z faces). Components
+// within a tolerance are few and span most tiles, so their global unions all
+// meet at a few roots, and a group settles about 70 % of them among its own
+// tiles (512^3 float32 grey levels 215 us without, 50 + 95 with). Every entry leaves with its group
 // root as parent, the group root with its component's smallest key; the bits
 // of the other keys are cleared, and the requests that leave the group are
 // moved to the front of their tile's list.  A group with more local roots than the LDS
 // table holds leaves its requests to the global kernel.
 constexpr int GRP = 16, GRP_NT = 512, GRP_CAP = 4096;  // two tiles per wave: 4 workgroups per CU
-template <class G>
 struct GroupGeo {
-  static constexpr int X = G::IS3D ? 1 : 4, Y = 4, Z = G::IS3D ? 4 : 1;
+  static constexpr int X = 1, Y = 4, Z = 4;
   static_assert(X * Y * Z == GRP, "16 tiles a group");
 };
 struct GroupGrid {
   uint32_t nx, ny, n;  // groups along x, along y, in all
   Div dxy, dx;         // by nx * ny and by nx
 };
-template <class G>
 __global__ __launch_bounds__(GRP_NT) void k_group(GlobalParams p, GroupGrid gg) {
-  using GG = GroupGeo<G>;
+  using GG = GroupGeo;
+  using G = GeoR;
   __shared__ uint32_t par[GRP_CAP], key[GRP_CAP];
   __shared__ uint32_t base[GRP + 1], root0s[GRP];
   const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -450,6 +449,73 @@ __global__ __launch_bounds__(GRP_NT) void k_group(GlobalParams p, GroupGrid gg) 
   }
 }
 
+constexpr int RRQ_SLOTS = 256;
+
+// kunion by the lanes of a wave that are live, their links sorted out in LDS
+// before any goes to memory: of the lanes that would link the same root, the
+// one with the lowest target links it, and each of the others takes that
+// target's part instead (its own root joins it: both ends are in the same
+// component in the end). own: 64 words, low: 64 double words of the wave.
+__device__ inline void kunion_wave(uint2* GP, uint32_t* bits, uint32_t a, uint32_t b, bool live, uint32_t* own,
+                                   unsigned long long* low) {
+  const uint32_t lane = threadIdx.x & 63;
+  KWord wa = {0, 0}, wb = {0, 0};
+  if (live) {
+    wa = kload<false>(GP, a);
+    wb = kload<false>(GP, b);
+    a = kfind<false>(GP, a, wa);
+    b = kfind<false>(GP, b, wb);
+    live = a != b;
+  }
+  while (wave_ballot(live)) {
+    uint64_t ka = ((uint64_t)wa.key << 32) | a, kb = ((uint64_t)wb.key << 32) | b;
+    bool moved;
+    do {
+      if (ka < kb) {
+        const uint64_t t = ka;
+        ka = kb;
+        kb = t;
+      }
+      const uint32_t h = ((uint32_t)ka * 0x9E3779B1u) >> 26;
+      if (live) {
+        own[h] = (uint32_t)ka;
+        low[h] = ~0ull;
+      }
+      wave_order();
+      const bool group = live && own[h] == (uint32_t)ka;
+      if (group) atomicMin(low + h, (unsigned long long)kb);
+      wave_order();
+      const uint64_t m = group ? low[h] : kb;
+      wave_order();
+      if (group && m == kb) own[h] = lane;
+      wave_order();
+      if (group && m == kb && own[h] != lane) live = false;  // another lane's link
+      wave_order();
+      moved = live && m != kb;
+      if (moved) {
+        ka = m;
+      }
+    } while (wave_ballot(moved));
+    if (live) {
+      a = (uint32_t)ka;
+      b = (uint32_t)kb;
+      const uint32_t old = atomicCAS(kparent(GP, a), a, b);
+      if (old == a) {  // a was still a root: linked under b
+        const uint32_t key = (uint32_t)(ka >> 32);
+        if (key != (uint32_t)(kb >> 32)) atomicAnd(bits + (key >> 5), ~(1u << (key & 31)));
+        live = false;
+      } else {
+        a = old;
+        wa = kload<true>(GP, a);
+        wb = kload<true>(GP, b);
+        a = kfind<true>(GP, a, wa);
+        b = kfind<true>(GP, b, wb);
+        live = a != b;
+      }
+    }
+  }
+}
+
 // Cross-tile unions of row tiles on the global forest, one wave per tile.  The
 // links of a border join the same few pairs of local roots again and again,
 // so a wave drops the pairs that one of its lanes has taken before: a table of
@@ -458,13 +524,26 @@ __global__ __launch_bounds__(GRP_NT) void k_group(GlobalParams p, GroupGrid gg) 
 // another pair took only costs a repeated union.  (8 lanes per tile without
 // the table: 192 us on the 512^3 uint32 Voronoi volume, 285 us on a p = 0.3
 // mask; with it 182 and 243 us.)
-constexpr int RRQ_SLOTS = 256;
+//
+// What is left is the unions' own time: without them the kernel takes 47 us on
+// the p = 0.3 mask and 25 on the 512^3 uint64 Voronoi volume at 6. Sorting the
+// links out in the wave first (kunion_wave) took these from 232 to 157 us and
+// from 122 to 118, and 383 x 401 x 367 p = 0.5 at 6 from 154 to 74. Two links a
+// lane in one pass, for fewer serial steps, is slower (183, 120 and 80): the
+// second link mostly finds its ends joined when the first is made before it.
+//
+// by_xcd: consecutive tiles on one XCD, whose L2 then holds both sides of most
+// borders. That is faster where components are small (512^3 uint32 Voronoi 26
+// 160 -> 131 us, uint64 at 6 118 -> 98) and slower where one root gathers most
+// tiles, which in raster order find it settled (p = 0.3 157 -> 212 us, p = 0.5
+// at 6 77 -> 160, 512^3 grey levels after k_group 92 -> 129): multilabel only.
 template <class G>
-__global__ __launch_bounds__(WG) void k_rrequests(GlobalParams p) {
+__global__ __launch_bounds__(WG) void k_rrequests(GlobalParams p, int by_xcd) {
   __shared__ uint2 tab[WG / 64][RRQ_SLOTS];
   __shared__ uint32_t own[WG / 64][RRQ_SLOTS];
+  __shared__ unsigned long long low[WG / 64][64];
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t w0 = (int64_t)blockIdx.x * (WG / 64) + wv;
+  const int64_t w0 = (by_xcd ? xcd_tile(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x) * (WG / 64) + wv;
   const int64_t nw = (int64_t)gridDim.x * (WG / 64);
   const uint16_t* REQ = reinterpret_cast<const uint16_t*>(p.REQ);
   for (int64_t slot = w0; slot < p.ntiles; slot += nw) {
@@ -516,8 +595,7 @@ __global__ __launch_bounds__(WG) void k_rrequests(GlobalParams p) {
         wave_order();
       }
 #pragma unroll
-      for (int k = 0; k < 2; k++)
-        if (live[k]) kunion(p.GP, p.bits, a[k], b[k]);
+      for (int k = 0; k < 2; k++) kunion_wave(p.GP, p.bits, a[k], b[k], live[k], own[wv], low[wv]);
     }
     wave_order();
   }
@@ -813,7 +891,7 @@ __global__ __launch_bounds__(WG) void k_scan_bc(const uint32_t* bits, int64_t nw
 // One launch for small bitmasks: each block counts the words before its own
 // 4096 itself (four rounds of eight 16-byte loads per thread at the limit, from
 // L2), and block nblk folds the counters, 16 tiles per thread at the limit. On
-// 96^3 voxels (7 blocks) k_tile_counters, k_scan_a and k_scan_bc of their own
+// 64^3 voxels (2 blocks) k_tile_counters, k_scan_a and k_scan_bc of their own
 // took 3.8 + 3.8 + 2.8 us and a copy of the counters 2.2 more; this takes 4.6.
 constexpr int SCAN1_NT = 1024;
 constexpr int64_t SCAN1_MAX = 32, SCAN1_TILES = 16 * SCAN1_NT;
@@ -1666,14 +1744,13 @@ static int plan(Geometry& g, int64_t sx, int64_t sy, int64_t sz, int64_t connect
   g.ntz = (sz + TZ - 1) / TZ;
   g.ntiles = g.ntx * g.nty * g.ntz;
   // Unions inside groups of tiles first, where that saves more global unions
-  // than it costs (k_group + k_requests against k_requests alone, us):
-  // continuous volumes from 4,096 tiles (256^3 tones 26 59 and 95, 512^3 155
-  // and 277; 192^3 44 and 40), multilabel ones at 26 and 18 from 8,000 (320^3
-  // 45 and 52, 512^3 159 and 182; 256^3 41 and 33; at 6 512^3 uint64 142 and
-  // 123), binary 8-connected planes from 32,768 (16384^2 213 and 272; 8192^2
-  // 105 and 99).  Binary volumes gain nothing (512^3 p = 0.3 221 and 227).
-  g.grouped = g.rows ? (g.mode == M_CONT && g.ntiles >= 4096) || (g.mode == M_MULTI && g.nb != 6 && g.ntiles >= 8000)
-                     : g.plane && g.mode == M_BINARY && g.nb == 8 && g.ntiles >= 32768;
+  // than it costs: continuous volumes from 4,096 tiles (k_group + k_rrequests
+  // against k_rrequests alone, float32 grey levels: 192^3 16 + 25 and 34 us,
+  // 256^3 15 + 38 and 71, 384^3 26 + 108 and 154, 512^3 50 + 95 and 215).
+  // Multilabel and binary volumes gain nothing (512^3 uint32 Voronoi 26
+  // 80 + 52 and 131 us, uint64 at 6 73 + 44 and 98; p = 0.3 67 + 105 and 157;
+  // 16384^2 plane at 8 90 + 119 and 200).
+  g.grouped = g.rows && g.mode == M_CONT && g.ntiles >= 4096;
   g.nwords = (g.K + 31) / 32;
   g.nblk = (g.nwords + SCAN_WPB - 1) / SCAN_WPB;
   if (g.qk == Q_BLOCK8) {
@@ -1819,36 +1896,34 @@ void launch_requests(const GlobalParams& p, int64_t ntiles, int mode, hipStream_
   else hipLaunchKernelGGL((k_requests<G, QK, 8>), dim3(grid_for(ntiles, WG / 8, 65536)), dim3(WG), 0, s, p);
 }
 
-template <class G>
 void launch_group(const GlobalParams& p, hipStream_t s) {
-  using GG = GroupGeo<G>;
+  using GG = GroupGeo;
   GroupGrid gg;
   gg.nx = (uint32_t)((p.ntx + GG::X - 1) / GG::X);
   gg.ny = (uint32_t)((p.nty + GG::Y - 1) / GG::Y);
   gg.n = gg.nx * gg.ny * (uint32_t)((p.ntz + GG::Z - 1) / GG::Z);
   gg.dxy = Div((int64_t)gg.nx * gg.ny);
   gg.dx = Div(gg.nx);
-  hipLaunchKernelGGL(k_group<G>, dim3(gg.n), dim3(GRP_NT), 0, s, p, gg);
+  hipLaunchKernelGGL(k_group, dim3(gg.n), dim3(GRP_NT), 0, s, p, gg);
 }
 
 template <class G>
-void launch_rrequests(const GlobalParams& p, int64_t ntiles, hipStream_t s) {
-  hipLaunchKernelGGL(k_rrequests<G>, dim3(grid_for(ntiles, WG / 64, 65536)), dim3(WG), 0, s, p);
+void launch_rrequests(const GlobalParams& p, int64_t ntiles, int mode, hipStream_t s) {
+  hipLaunchKernelGGL(k_rrequests<G>, dim3(grid_for(ntiles, WG / 64, 65536)), dim3(WG), 0, s, p,
+                     (int)(mode == M_MULTI));
 }
 
 template <class G>
 int run_global(cc3d_amd_job* j) {
   const GlobalParams& p = j->gp;
   hipStream_t s = j->stream;
-  if constexpr (std::is_same<G, GeoR>::value || std::is_same<G, GeoP>::value) {
-    if (j->g.grouped) {
-      ProfScope ps_("k_group", s);
-      launch_group<G>(p, s);
-    }
+  if (j->g.grouped) {
+    ProfScope ps_("k_group", s);
+    launch_group(p, s);
   }
   {
   ProfScope ps_("k_requests", s);
-  if constexpr (std::is_same<G, GeoR>::value || std::is_same<G, GeoP>::value) launch_rrequests<G>(p, j->g.ntiles, s);
+  if constexpr (std::is_same<G, GeoR>::value || std::is_same<G, GeoP>::value) launch_rrequests<G>(p, j->g.ntiles, j->g.mode, s);
   else if (j->g.qk == Q_BLOCK8) launch_requests<G, Q_BLOCK8>(p, j->g.ntiles, j->g.mode, s);
   else launch_requests<G, Q_NONE>(p, j->g.ntiles, j->g.mode, s);
   }
@@ -2924,7 +2999,7 @@ int cc3d_amd_batch_begin(cc3d_amd_batch* b) {
   {
     ProfScope ps_("k_requests", s);
     for (const auto& tg : b->tgroups) {
-      if (tg.rows()) launch_rrequests<GeoR>(tg.gp, tg.tiles, s);
+      if (tg.rows()) launch_rrequests<GeoR>(tg.gp, tg.tiles, b->mode, s);
       else if (tg.fam == cc3d_amd_batch::FAM_TALL) launch_requests<Geo3T, Q_NONE>(tg.gp, tg.tiles, b->mode, s);
       else if (tg.fam == cc3d_amd_batch::FAM_PLANE) launch_requests<Geo2, Q_NONE>(tg.gp, tg.tiles, b->mode, s);
       else launch_requests<Geo3, Q_NONE>(tg.gp, tg.tiles, b->mode, s);

@@ -174,3 +174,27 @@ def test_stored_root_bits(gpu, shape):
     for conn in (4, 8):
       _check(vol[:, :, 0], "bits 2D", connectivity=conn)
       _check(vol[:, :, 0], "bits 2D binary", connectivity=conn, binary_image=True)
+
+
+@pytest.mark.parametrize("pattern", ["comb", "chain", "sponge", "cells"])
+def test_unions_that_meet_at_one_root(gpu, pattern):
+  """Links of a wave that would hang the same root: one component over every
+  tile joined at one end, along a path, and at random; and many small ones."""
+  rng = np.random.default_rng(len(pattern))
+  vol = np.zeros((200, 70, 68), dtype=np.uint32, order="F")
+  if pattern == "comb":
+    vol[::2, :, ::2] = 1
+    vol[:, -1, ::2] = 1
+    vol[0, 0, :] = 1
+  elif pattern == "chain":
+    vol[:, ::2, ::2] = 1
+    vol[-1, 1::4, ::2] = vol[0, 3::4, ::2] = 1
+    vol[-1, 69, 1::4] = vol[-1, 0, 3::4] = 1
+    vol[-1, 68:, ::2] = 1
+  elif pattern == "sponge":
+    vol[:] = rng.random(vol.shape) < 0.35
+  else:
+    vol[:] = np.repeat(np.repeat(np.repeat(rng.integers(1, 5, (40, 14, 17)), 5, 0), 5, 1), 4, 2)
+  for connectivity in (6, 18, 26):
+    _check(vol, pattern, connectivity=connectivity, out_dtype=np.uint32)
+    _check(vol, pattern, connectivity=connectivity, out_dtype=np.uint32, binary_image=True)
