@@ -188,7 +188,7 @@ struct RowLds {
   using VT = typename RowVal<T, MODE>::type;
   struct Work {
     uint32_t par[64 * RSTR];
-    uint16_t queue[4][RQCAP];  // per wave; later, per wave: segment bits [row] and root bits [row]
+    uint16_t queue[4][RQCAP];  // per wave; later, per wave: segment bits [row]
   };
   union alignas(16) {
     // staged box: x = -1 at 3, x = 0..63 at 4..67, x = 64 at 68 (the next row's unused first element)
@@ -893,48 +893,26 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
     R += L.wtot[w];
   }
   rbase += rincl - nr;
-  qs[64 + hrow] = rb | (rbase << 16);  // ranks of the segment's roots
-  __syncthreads();
 
-  // 6. heads: 1 + the rank of their root
-  for (uint32_t m = H; m; m &= m - 1u) {
-    const uint32_t k = (uint32_t)__builtin_ctz(m), n = seg_node<QK>(h0, k);
-    const uint32_t r = par[n];
-    uint32_t row, x;
-    if (QK == Q_BLOCK8) {
-      const uint32_t pr = (r * 31776u) >> 22;  // r / 132 for r < 32 * 132
-      const uint32_t rem = r - 132u * pr;
-      row = 2u * pr + ((rem >> 1) & 1u);
-      x = 2u * (rem >> 2) + (rem & 1u);
-    } else {
-      row = (r * 61681u) >> 22;  // r / 68 for r < 64 * 68
-      x = r - RSTR * row;
-    }
-    const uint32_t w = reinterpret_cast<const uint32_t*>(L.u.w.queue[x >> 4])[64 + row];
-    par[n] = (w >> 16) + (uint32_t)__popc(w & ((1u << (x & 15u)) - 1u)) + 1u;
-  }
-
-  // 7. outputs.  Keys in 32-bit arithmetic (below 2^32; intermediate wraps
-  //    cancel).  A segment's keys are consecutive, so its root marks are one
-  //    or two words.
+  // 6. roots take 1 + their rank as parent and go to the global forest.  Keys
+  //    in 32-bit arithmetic (below 2^32; intermediate wraps cancel).  A
+  //    segment's keys are consecutive, so its root marks are one or two words.
   const uint32_t root0 = tile_root0<G>(sx, sy, sz, tx, ty, tz, keybase);
-  if (QK == Q_BLOCK8) {
-    uint32_t rk = root0 + rbase;
-    for (uint32_t m = rb; m; m &= m - 1u) {
-      const uint32_t key =
-        gkey<QK>(x0 + 16 * hseg + __builtin_ctz(m), y0 + hrow, 0, sx, sy, p.osx) + keybase;
-      p.GP[rk] = make_uint2(rk, key);
+  const int hx = x0 + 16 * hseg, hy = y0 + (hrow & (G::TY - 1)), hz = z0 + hrow / G::TY;
+  const uint32_t key0 =
+    QK == Q_BLOCK8 ? 0u : (uint32_t)hx + (uint32_t)sx * ((uint32_t)hy + (uint32_t)sy * (uint32_t)hz) + keybase;
+  uint32_t rk = rbase;
+  for (uint32_t m = rb; m; m &= m - 1u) {
+    const uint32_t k = (uint32_t)__builtin_ctz(m);
+    uint32_t key = key0 + k;
+    if (QK == Q_BLOCK8) {
+      key = gkey<QK>(hx + (int)k, hy, 0, sx, sy, p.osx) + keybase;
       atomicOr(p.bits + (key >> 5), 1u << (key & 31));
-      rk++;
     }
-  } else {
-    const int hx = x0 + 16 * hseg, hy = y0 + (hrow & (G::TY - 1)), hz = z0 + hrow / G::TY;
-    const uint32_t key0 = (uint32_t)hx + (uint32_t)sx * ((uint32_t)hy + (uint32_t)sy * (uint32_t)hz) + keybase;
-    uint32_t rk = root0 + rbase;
-    for (uint32_t m = rb; m; m &= m - 1u) {
-      p.GP[rk] = make_uint2(rk, key0 + (uint32_t)__builtin_ctz(m));
-      rk++;
-    }
+    p.GP[root0 + rk] = make_uint2(root0 + rk, key);
+    par[seg_node<QK>(h0, k)] = ++rk;
+  }
+  if (QK != Q_BLOCK8) {
     if ((sx & 15) == 0) {
       // every segment is a half-word of the bitmask that no other tile holds:
       // stored whether or not it has roots, so nothing clears the bitmask
@@ -949,6 +927,13 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
       if (lo) atomicOr(p.bits + (key0 >> 5), lo);
       if (hi) atomicOr(p.bits + (key0 >> 5) + 1, hi);
     }
+  }
+  __syncthreads();
+
+  // 7. the other heads take their root's, and the outputs
+  for (uint32_t m = H & ~rb; m; m &= m - 1u) {
+    const uint32_t n = seg_node<QK>(h0, (uint32_t)__builtin_ctz(m));
+    par[n] = par[par[n]];
   }
   {
     uint32_t j = 0, pk[8];
