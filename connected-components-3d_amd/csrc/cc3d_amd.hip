@@ -1805,11 +1805,10 @@ struct cc3d_amd_job {
   uint32_t* qbsum = nullptr;
   Counters* h_ctr = nullptr;
   PinnedCounters pin;
-  bool capturing = false;  // begun while the stream is being captured
   bool direct = false;     // the scan writes h_ctr itself
   const TileCnt* tcnt = nullptr;
   TileSum* tsum = nullptr;
-  bool copied = false;     // the counters' copy to h_ctr is under way (pin.ready marks its end)
+  bool copied = false;     // the counters are on their way to h_ctr (pin.ready marks the end)
   Counters h_ctr_local{};  // host copy of the counters when nothing may be allocated
   bool ctr_local = false;
   bool have_stats = false;
@@ -2194,8 +2193,7 @@ static int job_begin(cc3d_amd_job* j, const void* in, int in_dtype, int64_t sx, 
     if (!j->h_ctr) return fail(CC3D_AMD_ERR_NOMEM, "could not allocate pinned counters");
     // a captured launch would write the pooled buffer again at every replay,
     // and the 2D-8 rules count after the scan: those jobs copy the counters
-    j->capturing = stream_capturing(j->stream);
-    j->direct = !j->capturing && !j->count_prov && !j->stale;
+    j->direct = !j->count_prov && !j->stale && !stream_capturing(j->stream);
   }
   char* ws = j->ws;
   GlobalParams& gp = j->gp;
@@ -2305,6 +2303,10 @@ static int job_begin(cc3d_amd_job* j, const void* in, int in_dtype, int64_t sx, 
       default: rc = launch_q1<double>(j); break;
     }
   }
+  if (rc == CC3D_AMD_OK && j->direct) {  // marks the end of the scan's writes to h_ctr
+    HIPCHECK(hipEventRecord(j->pin.ready, s));
+    j->copied = true;
+  }
   return rc;
 }
 
@@ -2332,8 +2334,7 @@ int cc3d_amd_job_stats(cc3d_amd_job* j, cc3d_amd_stats* st) {
     if (j->copied) {
       HIPCHECK(hipEventSynchronize(j->pin.ready));
     } else {
-      if (!j->direct)
-        HIPCHECK(hipMemcpyAsync(j->h_ctr, j->gp.ctr, sizeof(Counters), hipMemcpyDeviceToHost, j->stream));
+      HIPCHECK(hipMemcpyAsync(j->h_ctr, j->gp.ctr, sizeof(Counters), hipMemcpyDeviceToHost, j->stream));
       HIPCHECK(hipStreamSynchronize(j->stream));
     }
     j->have_stats = true;
@@ -2352,11 +2353,11 @@ int cc3d_amd_label_finish(cc3d_amd_job* j, void* out, int out_dtype) {
     return fail(CC3D_AMD_ERR_INVALID, "output dtype must be uint16, uint32 or uint64");
   const Geometry& g = j->g;
   hipStream_t s = j->stream;
-  // Called before the counters were asked for: an event (behind their copy,
-  // unless the scan wrote them) marks their place, so that cc3d_amd_job_stats
-  // waits for stage 1 only while stage 2 already runs.
-  if (!j->have_stats && !j->copied && !j->ctr_local && !j->capturing) {
-    if (!j->direct) HIPCHECK(hipMemcpyAsync(j->h_ctr, j->gp.ctr, sizeof(Counters), hipMemcpyDeviceToHost, s));
+  // Called before the counters were asked for: where the scan does not write
+  // them to the host their copy goes first, so that cc3d_amd_job_stats waits
+  // for stage 1 only while stage 2 already runs.
+  if (!j->have_stats && !j->copied && !j->ctr_local && !stream_capturing(s)) {
+    HIPCHECK(hipMemcpyAsync(j->h_ctr, j->gp.ctr, sizeof(Counters), hipMemcpyDeviceToHost, s));
     HIPCHECK(hipEventRecord(j->pin.ready, s));
     j->copied = true;
   }

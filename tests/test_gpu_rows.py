@@ -198,3 +198,45 @@ def test_unions_that_meet_at_one_root(gpu, pattern):
   for connectivity in (6, 18, 26):
     _check(vol, pattern, connectivity=connectivity, out_dtype=np.uint32)
     _check(vol, pattern, connectivity=connectivity, out_dtype=np.uint32, binary_image=True)
+
+
+@pytest.mark.parametrize("connectivity,binary,shape", [(26, 0, (96, 70, 50)), (8, 1, (200, 131, 1)), (6, 1, (64, 64, 64))])
+def test_captured_job(gpu, connectivity, binary, shape):
+  """Both stages recorded in a graph: every replay equals the eager labels,
+  whatever the scratch held, with other calls between the replays."""
+  import ctypes
+  import cc3d
+  import torch
+  from cc3d import _lib as L
+  lib = L.lib()
+  sx, sy, sz = shape
+  rng = np.random.default_rng(connectivity)
+  vol = torch.from_numpy(rng.integers(0, 3, size=(sz, sy, sx)).astype(np.uint8)).cuda()
+  out = torch.zeros(sx * sy * sz, dtype=torch.int32, device="cuda")
+  ws = torch.empty(64 << 20, dtype=torch.uint8, device="cuda")
+  delta = ctypes.c_uint64(0)
+  stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+
+  def both_stages():
+    job = ctypes.c_void_p(0)
+    L.check(lib.cc3d_amd_label_begin(ctypes.byref(job), ctypes.c_void_p(vol.data_ptr()), L.DT_U8, sx, sy, sz,
+                                     connectivity, ctypes.byref(delta), 0, 0, binary,
+                                     ctypes.c_void_p(ws.data_ptr()), ws.numel(), ctypes.c_void_p(stream.cuda_stream)))
+    L.check(lib.cc3d_amd_label_finish(job, ctypes.c_void_p(out.data_ptr()), L.DT_U32))
+    return job
+
+  torch.cuda.synchronize()
+  lib.cc3d_amd_job_free(both_stages())
+  torch.cuda.synchronize()
+  eager = out.clone()
+  with torch.cuda.graph(graph, stream=stream):
+    job = both_stages()
+  lib.cc3d_amd_job_free(job)
+  for rep in range(4):
+    out.zero_()
+    ws.fill_(255)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(out, eager), rep
+    _, n = cc3d.connected_components(vol[0].cpu().numpy(), connectivity=8, return_N=True)
+    assert n == oracle.connected_components(vol[0].cpu().numpy(), connectivity=8, return_N=True)[1]
