@@ -54,8 +54,6 @@ __global__ void k_init(Counters* c, uint32_t* bits, int64_t nwords) {
     c->prov = 0;
     c->first_row = 0x7FFFFFFFFFFFFFFFll;
     c->last_row = -1;
-    c->req_count = 0;
-    c->req_overflow = 0;
     c->N = 0;
   }
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -114,8 +112,6 @@ __global__ void k_batch_init(Counters* c, int nc, uint32_t* bits, int64_t nwords
     c[i].prov = 0;
     c[i].first_row = 0x7FFFFFFFFFFFFFFFll;
     c[i].last_row = -1;
-    c[i].req_count = 0;
-    c[i].req_overflow = 0;
     c[i].N = 0;
   }
   for (int64_t w = i; w < nwords; w += (int64_t)gridDim.x * blockDim.x) bits[w] = 0;
@@ -532,17 +528,29 @@ __device__ inline void kunion_wave(uint2* GP, uint32_t* bits, uint32_t a, uint32
 // lane in one pass, for fewer serial steps, is slower (183, 120 and 80): the
 // second link mostly finds its ends joined when the first is made before it.
 //
-// by_xcd: consecutive tiles on one XCD, whose L2 then holds both sides of most
-// borders. That is faster where components are small (512^3 uint32 Voronoi 26
-// 160 -> 131 us, uint64 at 6 118 -> 98) and slower where one root gathers most
-// tiles, which in raster order find it settled (p = 0.3 157 -> 212 us, p = 0.5
-// at 6 77 -> 160, 512^3 grey levels after k_group 92 -> 129): multilabel only.
+// order: consecutive tiles on one XCD, whose L2 then holds both sides of most
+// borders, or raster order. The first is faster where components are small
+// (512^3 uint32 Voronoi 26 161 -> 131 us, uint64 at 6 118 -> 98), the second
+// where one root gathers most tiles, which it finds settled (p = 0.3 at 26 157
+// us, by XCD 212; p = 0.5 at 6 152 and 213; 383 x 401 x 367 p = 0.3 81 and 175,
+// p = 0.5 77 and 160; 512^3 grey levels after k_group 92 and 129), and a 0/1
+// mask is that volume whether or not the caller says so. Orders between the
+// two (chunks of 16 to 1,024 tiles to an XCD in turn) lose at both. Binary and
+// continuous volumes take raster order; a multilabel one goes by XCD, but above
+// ORDER_TILES only if its labels are spread (label_spread): below, all tiles
+// are in flight at once and content makes no difference (256^3 p = 0.3 by
+// raster 37 us, by XCD 38; 293^3 45 and 68). Multilabel batches go by XCD: a
+// volume's unions stay on one (16 masks of 256^3, p = 0.3: 315 us, raster 510;
+// volumes of 64 to 256 and mixed connectivities 187, raster 155).
+constexpr int64_t ORDER_TILES = 4096;
+enum : int { BY_RASTER, BY_XCD, BY_SPREAD };
 template <class G>
-__global__ __launch_bounds__(WG) void k_rrequests(GlobalParams p, int by_xcd) {
+__global__ __launch_bounds__(WG) void k_rrequests(GlobalParams p, int order) {
   __shared__ uint2 tab[WG / 64][RRQ_SLOTS];
   __shared__ uint32_t own[WG / 64][RRQ_SLOTS];
   __shared__ unsigned long long low[WG / 64][64];
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool by_xcd = order == BY_XCD || (order == BY_SPREAD && p.ctr->spread);
   const int64_t w0 = (by_xcd ? xcd_tile(blockIdx.x, gridDim.x) : (int64_t)blockIdx.x) * (WG / 64) + wv;
   const int64_t nw = (int64_t)gridDim.x * (WG / 64);
   const uint16_t* REQ = reinterpret_cast<const uint16_t*>(p.REQ);
@@ -1907,9 +1915,12 @@ void launch_group(const GlobalParams& p, hipStream_t s) {
 }
 
 template <class G>
-void launch_rrequests(const GlobalParams& p, int64_t ntiles, int mode, hipStream_t s) {
-  hipLaunchKernelGGL(k_rrequests<G>, dim3(grid_for(ntiles, WG / 64, 65536)), dim3(WG), 0, s, p,
-                     (int)(mode == M_MULTI));
+void launch_rrequests(const GlobalParams& p, int64_t ntiles, int order, hipStream_t s) {
+  hipLaunchKernelGGL(k_rrequests<G>, dim3(grid_for(ntiles, WG / 64, 65536)), dim3(WG), 0, s, p, order);
+}
+// A single volume's order; BY_SPREAD has its row kernel look at the labels.
+int union_order(const Geometry& g) {
+  return g.mode != M_MULTI ? BY_RASTER : g.ntiles > ORDER_TILES ? BY_SPREAD : BY_XCD;
 }
 
 template <class G>
@@ -1922,7 +1933,7 @@ int run_global(cc3d_amd_job* j) {
   }
   {
   ProfScope ps_("k_requests", s);
-  if constexpr (std::is_same<G, GeoR>::value || std::is_same<G, GeoP>::value) launch_rrequests<G>(p, j->g.ntiles, j->g.mode, s);
+  if constexpr (std::is_same<G, GeoR>::value || std::is_same<G, GeoP>::value) launch_rrequests<G>(p, j->g.ntiles, union_order(j->g), s);
   else if (j->g.qk == Q_BLOCK8) launch_requests<G, Q_BLOCK8>(p, j->g.ntiles, j->g.mode, s);
   else launch_requests<G, Q_NONE>(p, j->g.ntiles, j->g.mode, s);
   }
@@ -2226,17 +2237,7 @@ static int job_begin(cc3d_amd_job* j, const void* in, int in_dtype, int64_t sx, 
   }
   if (hipGetLastError() != hipSuccess) return fail(CC3D_AMD_ERR_HIP, "k_init launch failed");
 
-#define CC3D_DT_SWITCH(FN)                      \
-  switch (in_dtype) {                           \
-    case DT_U8: rc = FN<uint8_t>; break;        \
-    case DT_U16: rc = FN<uint16_t>; break;      \
-    case DT_U32: rc = FN<uint32_t>; break;      \
-    case DT_U64: rc = FN<uint64_t>; break;      \
-    case DT_F32: rc = FN<float>; break;         \
-    default: rc = FN<double>; break;            \
-  }
   if (g.qk == Q_CONT8) {
-#define CC3D_MM launch_minmax
     switch (in_dtype) {
       case DT_U8: rc = launch_minmax<uint8_t>(j, mm); break;
       case DT_U16: rc = launch_minmax<uint16_t>(j, mm); break;
@@ -2245,10 +2246,8 @@ static int job_begin(cc3d_amd_job* j, const void* in, int in_dtype, int64_t sx, 
       case DT_F32: rc = launch_minmax<float>(j, mm); break;
       default: rc = launch_minmax<double>(j, mm); break;
     }
-#undef CC3D_MM
     if (rc != CC3D_AMD_OK) return rc;
   }
-#undef CC3D_DT_SWITCH
 
   LocalParams lp;
   lp.utab = nullptr;
@@ -2272,6 +2271,7 @@ static int job_begin(cc3d_amd_job* j, const void* in, int in_dtype, int64_t sx, 
   lp.reqcap = g.reqcap;
   lp.TQ = reinterpret_cast<uint32_t*>(ws + g.oTQ);
   lp.tcnt = reinterpret_cast<TileCnt*>(ws + g.oTC);
+  lp.spread = union_order(g) == BY_SPREAD ? &gp.ctr->spread : nullptr;  // row kernels
   hipError_t e;
   {
   ProfScope ps_("k_local", s);
@@ -3000,7 +3000,7 @@ int cc3d_amd_batch_begin(cc3d_amd_batch* b) {
   {
     ProfScope ps_("k_requests", s);
     for (const auto& tg : b->tgroups) {
-      if (tg.rows()) launch_rrequests<GeoR>(tg.gp, tg.tiles, b->mode, s);
+      if (tg.rows()) launch_rrequests<GeoR>(tg.gp, tg.tiles, b->mode == M_MULTI ? BY_XCD : BY_RASTER, s);
       else if (tg.fam == cc3d_amd_batch::FAM_TALL) launch_requests<Geo3T, Q_NONE>(tg.gp, tg.tiles, b->mode, s);
       else if (tg.fam == cc3d_amd_batch::FAM_PLANE) launch_requests<Geo2, Q_NONE>(tg.gp, tg.tiles, b->mode, s);
       else launch_requests<Geo3, Q_NONE>(tg.gp, tg.tiles, b->mode, s);

@@ -62,8 +62,8 @@ struct Counters {
   unsigned long long prov;       // voxels (or blocks) taking a new provisional label
   long long first_row;           // first row holding foreground (INT64_MAX if none)
   long long last_row;            // last row holding foreground (-1 if none)
-  unsigned int req_count;        // cross-tile union requests emitted
-  unsigned int req_overflow;     // 1 when the request buffer overflowed
+  unsigned int spread;           // large multilabel volumes: 1 when no label gathers much of the volume
+  unsigned int unused;
   unsigned long long N;          // number of components
   unsigned long long pad[2];
 };

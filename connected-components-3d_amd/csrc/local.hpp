@@ -75,6 +75,7 @@ struct LocalParams {
   int64_t reqcap;        // row tiles: requests per tile (16-bit entries)
   uint32_t* TQ;
   TileCnt* tcnt;
+  uint32_t* spread;      // row tiles: Counters::spread, or null where nothing asks for it
   const uint16_t* utab;  // union tables (UTab), UTAB_TOTAL entries
 };
 
