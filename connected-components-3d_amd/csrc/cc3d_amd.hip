@@ -183,6 +183,7 @@ struct GlobalParams {
   // a batch addressed on its own (its periodic unions)
   int64_t tile0;
   uint32_t key0;
+  int jl;  // row tiles: 2^jl J entries per row (row_pitch)
 };
 
 // Geometry of the volume owning batch tile `slot`.
@@ -220,9 +221,17 @@ template <class G>
 __device__ inline uint32_t lroot_index(const GlobalParams& p, const VolGeo& v, int64_t gx, int64_t gy, int64_t gz) {
   const int64_t tx = gx / G::TX, ty = gy / G::TY, tz = G::IS3D ? gz / G::TZ : 0;
   const int64_t slot = v.tile0 + tx + v.ntx * (ty + v.nty * tz);
-  const int ji = G::jidx((int)(gx - tx * G::TX), (int)(gy - ty * G::TY), (int)(gz - tz * G::TZ));
+  const int lx = (int)(gx - tx * G::TX), ly = (int)(gy - ty * G::TY), lz = (int)(gz - tz * G::TZ);
+  int ji, entries;  // J entries of a tile
+  if constexpr (is_row_geo<G>) {
+    ji = G::jidx(lx, ly, lz, p.jl);
+    entries = 64 << G::jlog(p.jl);
+  } else {
+    ji = G::jidx(lx, ly, lz);
+    entries = G::TV;
+  }
   const uint32_t R = p.TR[slot];
-  const uint32_t j = R <= 255 ? p.J8[slot * (2 * G::TV) + ji] : p.J16[slot * G::TV + ji];
+  const uint32_t j = R <= 255 ? p.J8[slot * (2 * entries) + ji] : p.J16[slot * entries + ji];
   if (j == 0) return 0xFFFFFFFFu;
   return tile_root0<G>(v.sx, v.sy, v.sz, tx, ty, tz, v.key0) + j - 1;
 }
@@ -283,12 +292,14 @@ __device__ inline void request_ends(const GlobalParams& p, int64_t ntx, int64_t 
   oy = y < 0 ? -1 : y >= G::TY ? 1 : 0;
   oz = z < 0 ? -1 : 0;
   const int64_t qs = slot + ox + ntx * (oy + nty * oz);
-  const int qp = G::jidx(x - ox * G::TX, y - oy * G::TY, z - oz * G::TZ);
+  const int jl = G::jlog(p.jl);
+  const int pp = (ps & 63) + ((ps >> 6) << jl);
+  const int qp = G::jidx(x - ox * G::TX, y - oy * G::TY, z - oz * G::TZ, jl);
   const uint32_t Rq = p.TR[qs];
-  jp = p.J8[slot * (2 * G::TV) + ps];
-  jq = p.J8[qs * (2 * G::TV) + qp];
-  if (!j8) jp = p.J16[slot * G::TV + ps];
-  if (Rq > 255) jq = p.J16[qs * G::TV + qp];
+  jp = p.J8[(slot << (7 + jl)) + pp];
+  jq = p.J8[(qs << (7 + jl)) + qp];
+  if (!j8) jp = p.J16[(slot << (6 + jl)) + pp];
+  if (Rq > 255) jq = p.J16[(qs << (6 + jl)) + qp];
 }
 
 // Unions inside groups of 16 tiles of a continuous volume, in LDS: 1 x 4 x 4
@@ -309,9 +320,9 @@ struct GroupGrid {
   uint32_t nx, ny, n;  // groups along x, along y, in all
   Div dxy, dx;         // by nx * ny and by nx
 };
+template <class G>
 __global__ __launch_bounds__(GRP_NT) void k_group(GlobalParams p, GroupGrid gg) {
   using GG = GroupGeo;
-  using G = GeoR;
   __shared__ uint32_t par[GRP_CAP], key[GRP_CAP];
   __shared__ uint32_t base[GRP + 1], root0s[GRP];
   const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -1129,17 +1140,22 @@ __device__ inline void rfin_tile(const GlobalParams& p, const VolGeo& v, int64_t
   const int t = threadIdx.x;
   const uint32_t R = p.TR[slot];
   uint32_t j[PASSES][2];  // two 16-bit entries per word
+  const int jl = G::jlog(p.jl);
+  // in a narrow tile, columns past the row are past the volume: their lanes read others
+  const uint32_t j0 = G::NARROW ? ((uint32_t)(t >> 4) << jl) + ((4u * (t & 15)) & ((1u << jl) - 1u)) : 4u * (uint32_t)t;
   if (R <= 255) {
+    const uint8_t* q = p.J8 + (slot << (7 + jl));
 #pragma unroll
     for (int i = 0; i < PASSES; i++) {
-      const uint32_t w = reinterpret_cast<const uint32_t*>(p.J8 + slot * (2 * G::TV))[t + WG * i];
+      const uint32_t w = *reinterpret_cast<const uint32_t*>(q + (j0 + (16u * i << jl)));
       j[i][0] = (w & 0xFFu) | ((w & 0xFF00u) << 8);
       j[i][1] = ((w >> 16) & 0xFFu) | ((w >> 8) & 0xFF0000u);
     }
   } else {
+    const uint16_t* q = p.J16 + (slot << (6 + jl));
 #pragma unroll
     for (int i = 0; i < PASSES; i++) {
-      const uint2 w = reinterpret_cast<const uint2*>(p.J16 + slot * G::TV)[t + WG * i];
+      const uint2 w = *reinterpret_cast<const uint2*>(q + (j0 + (16u * i << jl)));
       j[i][0] = w.x;
       j[i][1] = w.y;
     }
@@ -1182,15 +1198,16 @@ __global__ __launch_bounds__(WG) void k_rfinalize(GlobalParams p, OUT* __restric
   rfin_tile<OUT, G>(p, vol_geo(p, 0), tile, tile, 0u, out, lab);
 }
 
+template <class G>
 __global__ __launch_bounds__(WG) void k_rfinalize_batch(GlobalParams p) {
-  __shared__ uint32_t lab[GeoR::TV + 1];
+  __shared__ uint32_t lab[G::TV + 1];
   const int64_t slot = xcd_tile(blockIdx.x, p.ntiles);
   const BatchVol& bv = p.vols[p.vix[slot]];
   const VolGeo v = batch_geo(bv);
   const uint32_t base = p.prefix[bv.key0 >> 5];
-  if (bv.out_dtype == DT_U16) rfin_tile<uint16_t, GeoR>(p, v, slot - bv.tile0, slot, base, static_cast<uint16_t*>(bv.out), lab);
-  else if (bv.out_dtype == DT_U64) rfin_tile<uint64_t, GeoR>(p, v, slot - bv.tile0, slot, base, static_cast<uint64_t*>(bv.out), lab);
-  else rfin_tile<uint32_t, GeoR>(p, v, slot - bv.tile0, slot, base, static_cast<uint32_t*>(bv.out), lab);
+  if (bv.out_dtype == DT_U16) rfin_tile<uint16_t, G>(p, v, slot - bv.tile0, slot, base, static_cast<uint16_t*>(bv.out), lab);
+  else if (bv.out_dtype == DT_U64) rfin_tile<uint64_t, G>(p, v, slot - bv.tile0, slot, base, static_cast<uint64_t*>(bv.out), lab);
+  else rfin_tile<uint32_t, G>(p, v, slot - bv.tile0, slot, base, static_cast<uint32_t*>(bv.out), lab);
 }
 
 // Batch: the table entry of every tile (one block per volume).
@@ -1686,9 +1703,10 @@ struct Geometry {
   bool grouped = false;  // row tiles: unions inside groups of tiles first (k_group)
   bool tall = false;  // tall voxel tiles (Geo3T) instead of Geo3
   int64_t ntx = 0, nty = 0, ntz = 0, ntiles = 0;
-  int TV = 0;
+  int TV = 0;  // J entries of one tile
   size_t req_bytes = 0;  // request storage of one tile
   int64_t reqcap = 0;    // row tiles: requests in it
+  int jl = 0;            // row tiles: 2^jl J entries per row
   int64_t nwords = 0, nblk = 0;
   int64_t qblocks = 0, qwords = 0, qnblk = 0;  // binary 2D-8 block bitmask
   size_t oGP, oTR, oTQ, oTC, oJ8, oJ16, oREQ, oBITS, oPRE, oBSUM, oTS, oCTR, oMM, oQB, oQP, oQS, total;
@@ -1730,12 +1748,16 @@ static int plan(Geometry& g, int64_t sx, int64_t sy, int64_t sz, int64_t connect
   g.plane = !g.is3d && sy >= GeoP::TY && g.qk != Q_CONT8 && !(tiles & (CC3D_AMD_TILES_VOXELS | CC3D_AMD_TILES_TALL));
   g.tall = g.is3d && !g.rows && (tiles & CC3D_AMD_TILES_TALL) && !(tiles & CC3D_AMD_TILES_VOXELS);
   if (g.rows) {
-    TX = GeoR::TX; TY = GeoR::TY; TZ = GeoR::TZ; g.TV = GeoR::TV;
-    g.reqcap = row_req_cap(g.mode == M_CONT, g.nb);
+    TX = GeoR::TX; TY = GeoR::TY; TZ = GeoR::TZ;
+    g.jl = row_pitch(sx);
+    g.TV = 64 << g.jl;
+    g.reqcap = row_req_cap(g.mode == M_CONT, g.nb, g.jl);
     g.req_bytes = (size_t)g.reqcap * sizeof(uint16_t);
   } else if (g.plane) {
-    TX = GeoP::TX; TY = GeoP::TY; TZ = GeoP::TZ; g.TV = GeoP::TV;
-    g.reqcap = row_req_cap(g.mode == M_CONT, g.nb);
+    TX = GeoP::TX; TY = GeoP::TY; TZ = GeoP::TZ;
+    g.jl = row_pitch(sx);
+    g.TV = 64 << g.jl;
+    g.reqcap = row_req_cap(g.mode == M_CONT, g.nb, g.jl);
     g.req_bytes = (size_t)g.reqcap * sizeof(uint16_t);
   } else if (g.tall) {
     TX = Geo3T::TX; TY = Geo3T::TY; TZ = Geo3T::TZ; g.TV = Geo3T::TV;
@@ -1853,6 +1875,7 @@ struct cc3d_amd_batch {
     int v0 = 0, v1 = 0;  // table entries
     int64_t tiles = 0;
     int64_t reqcap = 0;  // row tiles: requests per tile, for the group's largest neighbourhood
+    int jl = 0;          // row tiles: 2^jl J entries per row, for its widest volume
     size_t oT0 = 0, oVIX = 0, oTR = 0, oTQ = 0, oTC = 0, oJ8 = 0, oJ16 = 0, oREQ = 0;
     GlobalParams gp{};
     LocalParams lp{};
@@ -1903,6 +1926,7 @@ void launch_requests(const GlobalParams& p, int64_t ntiles, int mode, hipStream_
   else hipLaunchKernelGGL((k_requests<G, QK, 8>), dim3(grid_for(ntiles, WG / 8, 65536)), dim3(WG), 0, s, p);
 }
 
+template <class G>
 void launch_group(const GlobalParams& p, hipStream_t s) {
   using GG = GroupGeo;
   GroupGrid gg;
@@ -1911,12 +1935,18 @@ void launch_group(const GlobalParams& p, hipStream_t s) {
   gg.n = gg.nx * gg.ny * (uint32_t)((p.ntz + GG::Z - 1) / GG::Z);
   gg.dxy = Div((int64_t)gg.nx * gg.ny);
   gg.dx = Div(gg.nx);
-  hipLaunchKernelGGL(k_group, dim3(gg.n), dim3(GRP_NT), 0, s, p, gg);
+  hipLaunchKernelGGL(k_group<G>, dim3(gg.n), dim3(GRP_NT), 0, s, p, gg);
 }
 
 template <class G>
 void launch_rrequests(const GlobalParams& p, int64_t ntiles, int order, hipStream_t s) {
   hipLaunchKernelGGL(k_rrequests<G>, dim3(grid_for(ntiles, WG / 64, 65536)), dim3(WG), 0, s, p, order);
+}
+template <class OUT, class G, class GN>
+void launch_rfinalize(const GlobalParams& p, int64_t ntiles, OUT* out, hipStream_t s) {
+  const dim3 grid((unsigned)ntiles);
+  if (p.jl < 6) hipLaunchKernelGGL((k_rfinalize<OUT, GN>), grid, dim3(WG), 0, s, p, out);
+  else hipLaunchKernelGGL((k_rfinalize<OUT, G>), grid, dim3(WG), 0, s, p, out);
 }
 // A single volume's order; BY_SPREAD has its row kernel look at the labels.
 int union_order(const Geometry& g) {
@@ -1927,13 +1957,15 @@ template <class G>
 int run_global(cc3d_amd_job* j) {
   const GlobalParams& p = j->gp;
   hipStream_t s = j->stream;
-  if (j->g.grouped) {
-    ProfScope ps_("k_group", s);
-    launch_group(p, s);
+  if constexpr (is_row_geo<G> && G::IS3D) {
+    if (j->g.grouped) {
+      ProfScope ps_("k_group", s);
+      launch_group<G>(p, s);
+    }
   }
   {
   ProfScope ps_("k_requests", s);
-  if constexpr (std::is_same<G, GeoR>::value || std::is_same<G, GeoP>::value) launch_rrequests<G>(p, j->g.ntiles, union_order(j->g), s);
+  if constexpr (is_row_geo<G>) launch_rrequests<G>(p, j->g.ntiles, union_order(j->g), s);
   else if (j->g.qk == Q_BLOCK8) launch_requests<G, Q_BLOCK8>(p, j->g.ntiles, j->g.mode, s);
   else launch_requests<G, Q_NONE>(p, j->g.ntiles, j->g.mode, s);
   }
@@ -2218,6 +2250,7 @@ static int job_begin(cc3d_amd_job* j, const void* in, int in_dtype, int64_t sx, 
   gp.J16 = reinterpret_cast<uint16_t*>(ws + g.oJ16);
   gp.REQ = reinterpret_cast<uint32_t*>(ws + g.oREQ);
   gp.reqcap = g.reqcap;
+  gp.jl = g.jl;
   gp.TQ = reinterpret_cast<uint32_t*>(ws + g.oTQ);
   gp.bits = reinterpret_cast<uint32_t*>(ws + g.oBITS);
   gp.prefix = reinterpret_cast<uint32_t*>(ws + g.oPRE);
@@ -2269,6 +2302,7 @@ static int job_begin(cc3d_amd_job* j, const void* in, int in_dtype, int64_t sx, 
   lp.J16 = reinterpret_cast<uint16_t*>(ws + g.oJ16);
   lp.REQ = reinterpret_cast<uint32_t*>(ws + g.oREQ);
   lp.reqcap = g.reqcap;
+  lp.jl = g.jl;
   lp.TQ = reinterpret_cast<uint32_t*>(ws + g.oTQ);
   lp.tcnt = reinterpret_cast<TileCnt*>(ws + g.oTC);
   lp.spread = union_order(g) == BY_SPREAD ? &gp.ctr->spread : nullptr;  // row kernels
@@ -2288,8 +2322,9 @@ static int job_begin(cc3d_amd_job* j, const void* in, int in_dtype, int64_t sx, 
   if (e != hipSuccess) return fail(CC3D_AMD_ERR_HIP, std::string("k_local: ") + hipGetErrorString(e));
   j->tcnt = lp.tcnt;
   j->tsum = reinterpret_cast<TileSum*>(ws + g.oTS);
-  rc = g.rows ? run_global<GeoR>(j)
-       : g.plane ? run_global<GeoP>(j)
+  const bool narrow = g.jl < 6;
+  rc = g.rows ? (narrow ? run_global<GeoRN>(j) : run_global<GeoR>(j))
+       : g.plane ? (narrow ? run_global<GeoPN>(j) : run_global<GeoP>(j))
        : g.tall ? run_global<Geo3T>(j)
        : g.is3d ? run_global<Geo3>(j)
                 : run_global<Geo2>(j);
@@ -2368,8 +2403,8 @@ int cc3d_amd_label_finish(cc3d_amd_job* j, void* out, int out_dtype) {
   ProfScope ps_("k_finalize", s);
 #define CC3D_F(OUT)                                                                                \
   do {                                                                                             \
-    if (g.rows) hipLaunchKernelGGL((k_rfinalize<OUT, GeoR>), dim3((unsigned)g.ntiles), block, 0, s, j->gp, (OUT*)out); \
-    else if (g.plane) hipLaunchKernelGGL((k_rfinalize<OUT, GeoP>), dim3((unsigned)g.ntiles), block, 0, s, j->gp, (OUT*)out); \
+    if (g.rows) launch_rfinalize<OUT, GeoR, GeoRN>(j->gp, g.ntiles, (OUT*)out, s);                 \
+    else if (g.plane) launch_rfinalize<OUT, GeoP, GeoPN>(j->gp, g.ntiles, (OUT*)out, s);           \
     else if (g.tall) hipLaunchKernelGGL((k_finalize<OUT, Geo3T>), grid3t, block, 0, s, j->gp, (OUT*)out); \
     else if (g.is3d) hipLaunchKernelGGL((k_finalize<OUT, Geo3>), grid3, block, 0, s, j->gp, (OUT*)out); \
     else hipLaunchKernelGGL((k_finalize<OUT, Geo2>), grid2, block, 0, s, j->gp, (OUT*)out);        \
@@ -2755,10 +2790,12 @@ static int batch_layout(const cc3d_amd_volume* vols, int n, int mode, std::vecto
   for (auto& tg : b.tgroups) {
     int TXg, TYg, TZg;
     batch_tile_dims(tg.fam, TXg, TYg, TZg);
-    const size_t TVg = (size_t)TXg * TYg * TZg;
-    tg.reqcap = 0;
+    // row tiles: the widest volume's J rows, the largest request list
+    tg.reqcap = tg.jl = 0;
+    for (int k = tg.v0; tg.rows() && k < tg.v1; k++) tg.jl = std::max(tg.jl, row_pitch(tab[k].sx));
     for (int k = tg.v0; tg.rows() && k < tg.v1; k++)
-      tg.reqcap = std::max<int64_t>(tg.reqcap, row_req_cap(mode == CC3D_AMD_BATCH_CONTINUOUS, tab[k].nb));
+      tg.reqcap = std::max<int64_t>(tg.reqcap, row_req_cap(mode == CC3D_AMD_BATCH_CONTINUOUS, tab[k].nb, tg.jl));
+    const size_t TVg = tg.rows() ? (size_t)64 << tg.jl : (size_t)TXg * TYg * TZg;  // J entries of a tile
     const size_t req_bytes = tg.rows() ? (size_t)tg.reqcap * sizeof(uint16_t)
                              : tg.fam == cc3d_amd_batch::FAM_TALL  ? (size_t)Geo3T::HALO * 4
                              : tg.fam == cc3d_amd_batch::FAM_PLANE ? (size_t)Geo2::HALO * 4
@@ -2869,6 +2906,7 @@ int cc3d_amd_batch_create(cc3d_amd_batch** out_batch, const cc3d_amd_volume* vol
     q.J16 = reinterpret_cast<uint16_t*>(ws + tg.oJ16);
     q.REQ = reinterpret_cast<uint32_t*>(ws + tg.oREQ);
     q.reqcap = tg.reqcap;
+    q.jl = tg.jl;
     q.TQ = reinterpret_cast<uint32_t*>(ws + tg.oTQ);
     q.vols = gp.vols + tg.v0;
     q.vtile0 = reinterpret_cast<const int64_t*>(ws + tg.oT0);
@@ -2892,6 +2930,7 @@ int cc3d_amd_batch_create(cc3d_amd_batch** out_batch, const cc3d_amd_volume* vol
     lp.J16 = reinterpret_cast<uint16_t*>(ws + tg.oJ16);
     lp.REQ = reinterpret_cast<uint32_t*>(ws + tg.oREQ);
     lp.reqcap = tg.reqcap;
+    lp.jl = tg.jl;
     lp.TQ = reinterpret_cast<uint32_t*>(ws + tg.oTQ);
     lp.tcnt = reinterpret_cast<TileCnt*>(ws + tg.oTC);
     need_utab = need_utab || !tg.rows();
@@ -3000,7 +3039,9 @@ int cc3d_amd_batch_begin(cc3d_amd_batch* b) {
   {
     ProfScope ps_("k_requests", s);
     for (const auto& tg : b->tgroups) {
-      if (tg.rows()) launch_rrequests<GeoR>(tg.gp, tg.tiles, b->mode == M_MULTI ? BY_XCD : BY_RASTER, s);
+      const int order = b->mode == M_MULTI ? BY_XCD : BY_RASTER;
+      if (tg.rows() && tg.jl < 6) launch_rrequests<GeoRN>(tg.gp, tg.tiles, order, s);
+      else if (tg.rows()) launch_rrequests<GeoR>(tg.gp, tg.tiles, order, s);
       else if (tg.fam == cc3d_amd_batch::FAM_TALL) launch_requests<Geo3T, Q_NONE>(tg.gp, tg.tiles, b->mode, s);
       else if (tg.fam == cc3d_amd_batch::FAM_PLANE) launch_requests<Geo2, Q_NONE>(tg.gp, tg.tiles, b->mode, s);
       else launch_requests<Geo3, Q_NONE>(tg.gp, tg.tiles, b->mode, s);
@@ -3011,7 +3052,8 @@ int cc3d_amd_batch_begin(cc3d_amd_batch* b) {
     ProfScope ps_("k_periodic", s);
     for (const auto& pv : b->periodic) {
       const int fam = b->tgroups[pv.tg].fam;
-      e = fam == cc3d_amd_batch::FAM_ROWS    ? batch_periodic<GeoR>(b, pv, s)
+      const bool narrow = b->tgroups[pv.tg].jl < 6;
+      e = fam == cc3d_amd_batch::FAM_ROWS    ? (narrow ? batch_periodic<GeoRN>(b, pv, s) : batch_periodic<GeoR>(b, pv, s))
           : fam == cc3d_amd_batch::FAM_TALL  ? batch_periodic<Geo3T>(b, pv, s)
           : fam == cc3d_amd_batch::FAM_PLANE ? batch_periodic<Geo2>(b, pv, s)
                                              : batch_periodic<Geo3>(b, pv, s);
@@ -3057,7 +3099,8 @@ int cc3d_amd_batch_finish(cc3d_amd_batch* b) {
   ProfScope ps_("k_finalize", b->stream);
   for (const auto& tg : b->tgroups) {
     if (tg.rows())
-      hipLaunchKernelGGL(k_rfinalize_batch, dim3((unsigned)tg.tiles), dim3(WG), 0, b->stream, tg.gp);
+      hipLaunchKernelGGL(tg.jl < 6 ? k_rfinalize_batch<GeoRN> : k_rfinalize_batch<GeoR>, dim3((unsigned)tg.tiles), dim3(WG),
+                         0, b->stream, tg.gp);
     else if (tg.fam == cc3d_amd_batch::FAM_TALL)
       hipLaunchKernelGGL((k_finalize_batch<Geo3T>), dim3((unsigned)((tg.tiles + fin_tiles<Geo3T>() - 1) / fin_tiles<Geo3T>())),
                          dim3(WG), 0, b->stream, tg.gp);

@@ -77,6 +77,7 @@ struct LocalParams {
   TileCnt* tcnt;
   uint32_t* spread;      // row tiles: Counters::spread, or null where nothing asks for it
   const uint16_t* utab;  // union tables (UTab), UTAB_TOTAL entries
+  int jl;                // row tiles: 2^jl J entries per row (row_pitch)
 };
 
 // Offsets of backward position i in the staged box and in the tile's node

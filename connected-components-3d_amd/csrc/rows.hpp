@@ -40,7 +40,7 @@
 // inside the tile as LDS unions, links out of it as cross-tile requests
 // (voxel position | relation << 12) for the global kernels.  Outputs (GP, TR,
 // J8/J16, REQ/TQ, tcnt) are those of the voxel kernel in local.hpp except
-// for the request format; J is row-major: entry x + 64 * (y + 8 * z).
+// for the request format; J is row-major: entry x + 2^jl * (y + 8 * z).
 //
 // What bounds it: VALU issue, 1,500 instructions per 1,024-voxel wave and 80 %
 // of the issue slots, of which about a third form the masks and a sixth make
@@ -59,11 +59,13 @@
 namespace cc3d_amd {
 
 // Tile geometry of the row kernels: 64 rows of 64 voxels, 8 x 8 of them for
-// volumes (GeoR) and 64 x 1 for single planes (GeoP).  Box rows (by, bz): by =
+// volumes (GeoR) and 64 x 1 for single planes (GeoP); GeoRN and GeoPN are the
+// same tiles with shorter J rows, for narrow volumes (row_pitch).  Box rows (by, bz): by =
 // y + 1, bz = z + 1 (0 in a plane), one halo row or plane on each side that
 // backward neighbours reach.
-template <int TY_, int TZ_>
+template <int TY_, int TZ_, bool NARROW_ = false>
 struct RowGeo {
+  static constexpr bool NARROW = NARROW_;
   static constexpr int TX = 64, TY = TY_, TZ = TZ_;
   static constexpr bool IS3D = TZ > 1;
   static constexpr int NT = 256;
@@ -71,10 +73,17 @@ struct RowGeo {
   static constexpr int BY = IS3D ? TY + 2 : TY + 1, BZ = IS3D ? TZ + 1 : 1;
   static constexpr int NROWS = BY * BZ;
   static_assert(TY * TZ == 64, "one row per lane of a wave");
-  __device__ static inline int jidx(int lx, int ly, int lz) { return lx + TX * (ly + TY * lz); }
+  // J: 2^jl entries a row
+  __device__ static inline int jlog(int jl) { return NARROW ? jl : 6; }
+  __device__ static inline int jidx(int lx, int ly, int lz, int jl) { return lx + ((ly + TY * lz) << jlog(jl)); }
 };
 using GeoR = RowGeo<8, 8>;
 using GeoP = RowGeo<64, 1>;
+using GeoRN = RowGeo<8, 8, true>;
+using GeoPN = RowGeo<64, 1, true>;
+template <class G>
+constexpr bool is_row_geo = std::is_same<G, GeoR>::value || std::is_same<G, GeoP>::value ||
+                            std::is_same<G, GeoRN>::value || std::is_same<G, GeoPN>::value;
 
 // Relations in covering order; index 12 is a.  Offsets as (d + 1) in 2-bit
 // fields per axis.
@@ -128,12 +137,26 @@ __device__ inline void rel_decode(uint32_t r, int& dx, int& dy, int& dz) {
   dz = (int)((PZ >> (2 * r)) & 3u) - 1;
 }
 
+// J entries per row of a tile, as a power of two: 16, 32 or 64 columns.  A
+// narrow volume has one tile in x, of whose 64 columns the rest would be scratch
+// that nothing uses (at 16 x N x N and 26-connectivity 24 bytes of scratch a
+// voxel, 34 for continuous links; voxel tiles of 32 x 8 x 8 take 18).  Kernels of
+// their own, because the general address costs the others up to 1.5 % (16384^2
+// mask at 8: 801 and 813 us).
+__host__ constexpr int row_pitch(int64_t sx) { return sx <= 16 ? 4 : sx <= 32 ? 5 : 6; }
+
 // Bound on the requests of a tile.  Multilabel and binary: the largest number
 // of kept relations that leave the tile, over every set of links a voxel can
 // have, summed over the tile's voxels (4,036 at 26-connectivity, 2,537 at
 // 18, 1,088 at 6).  Continuous volumes and planes: all relations that leave
-// the tile (382 in a plane).
-__host__ __device__ constexpr int row_req_cap(bool cont, int nb) {
+// the tile (382 in a plane).  Narrow tiles have no neighbour in x: what is left
+// is the sum over a column of 64 rows (60, 38, 16; continuous 138, 78, 16; 3
+// in a plane).  Never below the 128 that the union kernels load unasked.
+__host__ __device__ constexpr int row_req_cap(bool cont, int nb, int jl) {
+  if (jl < 6) {
+    const int n = (nb == 8 || nb == 4 ? 3 : nb == 6 ? 16 : nb == 18 ? (cont ? 78 : 38) : (cont ? 138 : 60)) << jl;
+    return n < 128 ? 128 : n;
+  }
   return nb == 8 || nb == 4 ? 384 : nb == 6 ? 1088 : nb == 18 ? (cont ? 5280 : 2540) : (cont ? 9316 : 4036);
 }
 
@@ -967,15 +990,23 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
       pk[k / 2] = o[0] | (o[1] << 16);
       pk[k / 2 + 1] = o[2] | (o[3] << 16);
     }
+    uint4* o8 = reinterpret_cast<uint4*>(p.J8 + slot * (2 * G::TV)) + t;
+    uint4* o16 = reinterpret_cast<uint4*>(p.J16 + slot * G::TV) + 2 * t;
+    bool stored = true;
+    if constexpr (G::NARROW) {
+      const uint32_t at = ((uint32_t)hrow << p.jl) + 16u * (uint32_t)hseg;
+      o8 = reinterpret_cast<uint4*>(p.J8 + (slot << (7 + p.jl)) + at);
+      o16 = reinterpret_cast<uint4*>(p.J16 + (slot << (6 + p.jl)) + at);
+      stored = 16 * hseg < 1 << p.jl;  // else columns that the volume does not have
+    }
     if (R <= 255) {
       uint32_t b[4];
 #pragma unroll
       for (int i = 0; i < 4; i++) b[i] = __builtin_amdgcn_perm(pk[2 * i + 1], pk[2 * i], 0x06040200u);
-      reinterpret_cast<uint4*>(p.J8 + slot * (2 * G::TV))[t] = make_uint4(b[0], b[1], b[2], b[3]);
-    } else {
-      uint4* o = reinterpret_cast<uint4*>(p.J16 + slot * G::TV) + 2 * t;
-      o[0] = make_uint4(pk[0], pk[1], pk[2], pk[3]);
-      o[1] = make_uint4(pk[4], pk[5], pk[6], pk[7]);
+      if (stored) *o8 = make_uint4(b[0], b[1], b[2], b[3]);
+    } else if (stored) {
+      o16[0] = make_uint4(pk[0], pk[1], pk[2], pk[3]);
+      o16[1] = make_uint4(pk[4], pk[5], pk[6], pk[7]);
     }
   }
   if (t == 0) {
@@ -1034,38 +1065,39 @@ __host__ __device__ constexpr int rows_waves() {
   return sizeof(T) < 8 || MODE == M_BINARY ? 6 : MODE == M_CONT ? 3 : 5;
 }
 
-template <class T, int MODE, int NB>
-__global__ __launch_bounds__(GeoR::NT, (rows_waves<T, MODE>())) void k_rows_local(LocalParams p) {
-  __shared__ RowLds<T, MODE> L;
+template <class T, int MODE, int NB, class G>
+__global__ __launch_bounds__(G::NT, (rows_waves<T, MODE>())) void k_rows_local(LocalParams p) {
+  __shared__ RowLds<T, MODE, G> L;
   const int64_t tile = xcd_tile(blockIdx.x, p.ntiles);
-  rows_tile<T, MODE, NB, GeoR, Q_NONE>(p, static_cast<const T*>(p.in), p.sx, p.sy, p.sz, p.ntx, p.nty, p.dxy,
-                                       p.dx, tile, tile, 0u, L);
+  rows_tile<T, MODE, NB, G, Q_NONE>(p, static_cast<const T*>(p.in), p.sx, p.sy, p.sz, p.ntx, p.nty, p.dxy, p.dx, tile,
+                                    tile, 0u, L);
   if (MODE == M_MULTI && p.spread && blockIdx.x == 0 && threadIdx.x < 64)
     label_spread(static_cast<const T*>(p.in), (uint64_t)(p.sx * p.sy * p.sz), p.spread);
 }
 
 // Single planes of at least 64 rows.
-template <class T, int MODE, int NB, int QK>
-__global__ __launch_bounds__(GeoP::NT, (rows_waves<T, MODE>())) void k_rows_plane(LocalParams p) {
-  __shared__ RowLds<T, MODE, GeoP> L;
+template <class T, int MODE, int NB, int QK, class G>
+__global__ __launch_bounds__(G::NT, (rows_waves<T, MODE>())) void k_rows_plane(LocalParams p) {
+  __shared__ RowLds<T, MODE, G> L;
   const int64_t tile = xcd_tile(blockIdx.x, p.ntiles);
-  rows_tile<T, MODE, NB, GeoP, QK>(p, static_cast<const T*>(p.in), p.sx, p.sy, 1, p.ntx, p.nty, p.dxy, p.dx, tile,
-                                     tile, 0u, L);
+  rows_tile<T, MODE, NB, G, QK>(p, static_cast<const T*>(p.in), p.sx, p.sy, 1, p.ntx, p.nty, p.dxy, p.dx, tile, tile,
+                                0u, L);
   if (MODE == M_MULTI && p.spread && blockIdx.x == 0 && threadIdx.x < 64)
     label_spread(static_cast<const T*>(p.in), (uint64_t)(p.sx * p.sy), p.spread);
 }
 
 // Batch: tiles [gtile0, gtile0 + gtiles) of volumes of connectivity NB; each
 // workgroup reads its volume's table entry.
-template <class T, int MODE, int NB>
-__global__ __launch_bounds__(GeoR::NT, (rows_waves<T, MODE>())) void k_rows_local_batch(LocalParams p, const BatchVol* vols,
-                                                                                       const uint32_t* vix,
-                                                                                       int64_t gtile0, int64_t gtiles) {
-  __shared__ RowLds<T, MODE> L;
+template <class T, int MODE, int NB, class G>
+__global__ __launch_bounds__(G::NT, (rows_waves<T, MODE>())) void k_rows_local_batch(LocalParams p,
+                                                                                    const BatchVol* vols,
+                                                                                    const uint32_t* vix,
+                                                                                    int64_t gtile0, int64_t gtiles) {
+  __shared__ RowLds<T, MODE, G> L;
   const int64_t slot = gtile0 + xcd_tile(blockIdx.x, gtiles);
   const BatchVol& v = vols[vix[slot]];
-  rows_tile<T, MODE, NB, GeoR, Q_NONE>(p, static_cast<const T*>(v.in), v.sx, v.sy, v.sz, v.ntx, v.nty, v.dxy, v.dx,
-                                       slot - v.tile0, slot, v.key0, L);
+  rows_tile<T, MODE, NB, G, Q_NONE>(p, static_cast<const T*>(v.in), v.sx, v.sy, v.sz, v.ntx, v.nty, v.dxy, v.dx,
+                                    slot - v.tile0, slot, v.key0, L);
 }
 
 hipError_t launch_rows_multi(int dt, int nb, const LocalParams& p, hipStream_t s);
@@ -1086,7 +1118,9 @@ hipError_t launch_rows_batch_binary(int dt, int nb, const LocalParams& p, const 
 template <int MODE>
 hipError_t launch_rows_mode(int dt, int nb, const LocalParams& p, hipStream_t s) {
   const dim3 grid((unsigned)p.ntiles), block(GeoR::NT);
-#define CC3D_R(T, NB) hipLaunchKernelGGL((k_rows_local<T, MODE, NB>), grid, block, 0, s, p)
+#define CC3D_R(T, NB)                                                                            \
+  if (p.jl < 6) hipLaunchKernelGGL((k_rows_local<T, MODE, NB, GeoRN>), grid, block, 0, s, p);    \
+  else hipLaunchKernelGGL((k_rows_local<T, MODE, NB, GeoR>), grid, block, 0, s, p)
 #define CC3D_RNB(T)                       \
   switch (nb) {                           \
     case 26: CC3D_R(T, 26); break;        \
@@ -1111,7 +1145,9 @@ hipError_t launch_rows_mode(int dt, int nb, const LocalParams& p, hipStream_t s)
 template <int MODE>
 hipError_t launch_rows_plane_mode(int dt, int nb, int qk, const LocalParams& p, hipStream_t s) {
   const dim3 grid((unsigned)p.ntiles), block(GeoP::NT);
-#define CC3D_R(T, NB, QK) hipLaunchKernelGGL((k_rows_plane<T, MODE, NB, QK>), grid, block, 0, s, p)
+#define CC3D_R(T, NB, QK)                                                                        \
+  if (p.jl < 6) hipLaunchKernelGGL((k_rows_plane<T, MODE, NB, QK, GeoPN>), grid, block, 0, s, p); \
+  else hipLaunchKernelGGL((k_rows_plane<T, MODE, NB, QK, GeoP>), grid, block, 0, s, p)
 #define CC3D_RNB(T)                                                                            \
   if (nb == 8 && qk == Q_BLOCK8 && MODE == M_BINARY) {                                         \
     CC3D_R(T, 8, (MODE == M_BINARY ? Q_BLOCK8 : Q_NONE));                                      \
@@ -1142,8 +1178,10 @@ template <int MODE>
 hipError_t launch_rows_batch_mode(int dt, int nb, const LocalParams& p, const BatchVol* vols, const uint32_t* vix,
                                   int64_t gtile0, int64_t gtiles, hipStream_t s) {
   const dim3 grid((unsigned)gtiles), block(GeoR::NT);
-#define CC3D_R(T, NB) \
-  hipLaunchKernelGGL((k_rows_local_batch<T, MODE, NB>), grid, block, 0, s, p, vols, vix, gtile0, gtiles)
+#define CC3D_R(T, NB)                                                                                              \
+  if (p.jl < 6)                                                                                                    \
+    hipLaunchKernelGGL((k_rows_local_batch<T, MODE, NB, GeoRN>), grid, block, 0, s, p, vols, vix, gtile0, gtiles); \
+  else hipLaunchKernelGGL((k_rows_local_batch<T, MODE, NB, GeoR>), grid, block, 0, s, p, vols, vix, gtile0, gtiles)
 #define CC3D_RNB(T)                       \
   switch (nb) {                           \
     case 26: CC3D_R(T, 26); break;        \
