@@ -302,6 +302,11 @@ __device__ inline void request_ends(const GlobalParams& p, int64_t ntx, int64_t 
   if (Rq > 255) jq = p.J16[(qs << (6 + jl)) + qp];
 }
 
+// Voxel of entry i of the link masks of the segment that is the lowest bit of d.
+__device__ inline uint32_t mask_voxel(uint32_t i, uint32_t d) {
+  return 64u * (i >> 4) + 16u * (uint32_t)__builtin_ctz(d) + (i & 15u);
+}
+
 // Unions inside groups of 16 tiles of a continuous volume, in LDS: 1 x 4 x 4
 // tiles (most of a 64 x 8 x 8 tile's border is its y and z faces). Components
 // within a tolerance are few and span most tiles, so their global unions all
@@ -310,7 +315,8 @@ __device__ inline void request_ends(const GlobalParams& p, int64_t ntx, int64_t 
 // root as parent, the group root with its component's smallest key; the bits
 // of the other keys are cleared, and the requests that leave the group are
 // moved to the front of their tile's list.  A group with more local roots than the LDS
-// table holds leaves its requests to the global kernel.
+// table holds leaves its requests to the global kernel, and so does every tile
+// with the links that it stored as masks.
 constexpr int GRP = 16, GRP_NT = 512, GRP_CAP = 4096;  // two tiles per wave: 4 workgroups per CU
 struct GroupGeo {
   static constexpr int X = 1, Y = 4, Z = 4;
@@ -555,7 +561,9 @@ __device__ inline void kunion_wave(uint2* GP, uint32_t* bits, uint32_t a, uint32
 // volumes of 64 to 256 and mixed connectivities 187, raster 155).
 constexpr int64_t ORDER_TILES = 4096;
 enum : int { BY_RASTER, BY_XCD, BY_SPREAD };
-template <class G>
+//
+// MASKS: links may be stored as masks too (continuous volumes), one voxel a lane.
+template <class G, bool MASKS>
 __global__ __launch_bounds__(WG) void k_rrequests(GlobalParams p, int order) {
   __shared__ uint2 tab[WG / 64][RRQ_SLOTS];
   __shared__ uint32_t own[WG / 64][RRQ_SLOTS];
@@ -570,9 +578,9 @@ __global__ __launch_bounds__(WG) void k_rrequests(GlobalParams p, int order) {
     // holds more than 128 whatever the number is
     const uint16_t* list = REQ + slot * p.reqcap;
     const uint32_t rq[2] = {list[lane], list[lane + 64]};
-    const uint32_t nq = p.TQ[slot];
+    const uint32_t nq = p.TQ[slot], masked = MASKS ? list[64u << G::jlog(p.jl)] : 0u;
     const bool j8 = p.TR[slot] <= 255;
-    if (nq == 0) continue;
+    if ((nq | masked) == 0) continue;
     const VolGeo v = vol_geo(p, slot);
     int64_t tx, ty, tz;
     tile_coords((uint32_t)(slot - v.tile0), v.ntx, v.nty, v.dxy, v.dx, tx, ty, tz);
@@ -580,6 +588,22 @@ __global__ __launch_bounds__(WG) void k_rrequests(GlobalParams p, int order) {
 #pragma unroll
     for (int k = 0; k < RRQ_SLOTS / 64; k++) tab[wv][lane + 64 * k] = make_uint2(0xFFFFFFFFu, 0xFFFFFFFFu);
     wave_order();
+    // is a lane's pair one that no lane has taken before
+    auto fresh = [&](uint32_t a, uint32_t b, bool live) -> bool {
+      const uint32_t h = (((a * 0x9E3779B1u) ^ (b * 0x85EBCA77u)) >> 24) & (RRQ_SLOTS - 1);
+      if (live) {
+        const uint2 q = tab[wv][h];
+        live = q.x != a || q.y != b;
+      }
+      if (live) own[wv][h] = (uint32_t)lane;
+      wave_order();
+      const int o = live ? (int)own[wv][h] : lane;
+      const uint32_t oa = __shfl(a, o), ob = __shfl(b, o);
+      if (live && o != lane && oa == a && ob == b) live = false;
+      if (live) tab[wv][h] = make_uint2(a, b);
+      wave_order();
+      return live;
+    };
     // two requests per lane and round, so that their loads overlap
     for (uint32_t i0 = 0; i0 < nq; i0 += 128) {
       uint32_t a[2], b[2];
@@ -598,23 +622,33 @@ __global__ __launch_bounds__(WG) void k_rrequests(GlobalParams p, int order) {
       }
       bool live[2];
 #pragma unroll
-      for (int k = 0; k < 2; k++) {
-        live[k] = b[k] != 0xFFFFFFFFu;
-        const uint32_t h = (((a[k] * 0x9E3779B1u) ^ (b[k] * 0x85EBCA77u)) >> 24) & (RRQ_SLOTS - 1);
-        if (live[k]) {
-          const uint2 q = tab[wv][h];
-          live[k] = q.x != a[k] || q.y != b[k];
-        }
-        if (live[k]) own[wv][h] = (uint32_t)lane;
-        wave_order();
-        const int o = live[k] ? (int)own[wv][h] : lane;
-        const uint32_t oa = __shfl(a[k], o), ob = __shfl(b[k], o);
-        if (live[k] && o != lane && oa == a[k] && ob == b[k]) live[k] = false;
-        if (live[k]) tab[wv][h] = make_uint2(a[k], b[k]);
-        wave_order();
-      }
+      for (int k = 0; k < 2; k++) live[k] = fresh(a[k], b[k], b[k] != 0xFFFFFFFFu);
 #pragma unroll
       for (int k = 0; k < 2; k++) kunion_wave(p.GP, p.bits, a[k], b[k], live[k], own[wv], low[wv]);
+    }
+    if constexpr (MASKS) {
+      uint32_t at = 64u << G::jlog(p.jl);
+      for (uint32_t d = (uint32_t)__builtin_amdgcn_readfirstlane((int)masked); d; d &= d - 1u) {
+        at -= 1024u;
+        for (uint32_t i = lane; i < 1024u; i += 64) {
+          const uint32_t e0 = mask_voxel(i, d);
+          uint32_t m = list[at + i];
+          while (wave_ballot(m != 0u)) {
+            uint32_t a = 0, b = 0;
+            const bool live = m != 0u;
+            if (live) {
+              const uint32_t e = e0 | ((uint32_t)__builtin_ctz(m) << 12);
+              int ox, oy, oz;
+              uint32_t jp, jq;
+              request_ends<G>(p, v.ntx, v.nty, slot, j8, e, ox, oy, oz, jp, jq);
+              a = root0 + jp - 1u;
+              b = tile_root0<G>(v.sx, v.sy, v.sz, tx + ox, ty + oy, tz + oz, v.key0) + jq - 1u;
+              m &= m - 1u;
+            }
+            kunion_wave(p.GP, p.bits, a, b, fresh(a, b, live), own[wv], low[wv]);
+          }
+        }
+      }
     }
     wave_order();
   }
@@ -1876,6 +1910,7 @@ struct cc3d_amd_batch {
     int64_t tiles = 0;
     int64_t reqcap = 0;  // row tiles: requests per tile, for the group's largest neighbourhood
     int jl = 0;          // row tiles: 2^jl J entries per row, for its widest volume
+    bool masks = false;  // row tiles: some may hold link masks
     size_t oT0 = 0, oVIX = 0, oTR = 0, oTQ = 0, oTC = 0, oJ8 = 0, oJ16 = 0, oREQ = 0;
     GlobalParams gp{};
     LocalParams lp{};
@@ -1939,8 +1974,10 @@ void launch_group(const GlobalParams& p, hipStream_t s) {
 }
 
 template <class G>
-void launch_rrequests(const GlobalParams& p, int64_t ntiles, int order, hipStream_t s) {
-  hipLaunchKernelGGL(k_rrequests<G>, dim3(grid_for(ntiles, WG / 64, 65536)), dim3(WG), 0, s, p, order);
+void launch_rrequests(const GlobalParams& p, int64_t ntiles, bool masks, int order, hipStream_t s) {
+  const dim3 grid(grid_for(ntiles, WG / 64, 65536));
+  if (G::IS3D && masks) hipLaunchKernelGGL((k_rrequests<G, G::IS3D>), grid, dim3(WG), 0, s, p, order);
+  else hipLaunchKernelGGL((k_rrequests<G, false>), grid, dim3(WG), 0, s, p, order);
 }
 template <class OUT, class G, class GN>
 void launch_rfinalize(const GlobalParams& p, int64_t ntiles, OUT* out, hipStream_t s) {
@@ -1965,7 +2002,7 @@ int run_global(cc3d_amd_job* j) {
   }
   {
   ProfScope ps_("k_requests", s);
-  if constexpr (is_row_geo<G>) launch_rrequests<G>(p, j->g.ntiles, union_order(j->g), s);
+  if constexpr (is_row_geo<G>) launch_rrequests<G>(p, j->g.ntiles, row_masks(j->g.mode == M_CONT, j->g.nb), union_order(j->g), s);
   else if (j->g.qk == Q_BLOCK8) launch_requests<G, Q_BLOCK8>(p, j->g.ntiles, j->g.mode, s);
   else launch_requests<G, Q_NONE>(p, j->g.ntiles, j->g.mode, s);
   }
@@ -2792,9 +2829,13 @@ static int batch_layout(const cc3d_amd_volume* vols, int n, int mode, std::vecto
     batch_tile_dims(tg.fam, TXg, TYg, TZg);
     // row tiles: the widest volume's J rows, the largest request list
     tg.reqcap = tg.jl = 0;
+    tg.masks = false;
     for (int k = tg.v0; tg.rows() && k < tg.v1; k++) tg.jl = std::max(tg.jl, row_pitch(tab[k].sx));
-    for (int k = tg.v0; tg.rows() && k < tg.v1; k++)
-      tg.reqcap = std::max<int64_t>(tg.reqcap, row_req_cap(mode == CC3D_AMD_BATCH_CONTINUOUS, tab[k].nb, tg.jl));
+    for (int k = tg.v0; tg.rows() && k < tg.v1; k++) {
+      const bool cont = mode == CC3D_AMD_BATCH_CONTINUOUS;
+      tg.reqcap = std::max<int64_t>(tg.reqcap, row_req_cap(cont, tab[k].nb, tg.jl));
+      tg.masks = tg.masks || row_masks(cont, tab[k].nb);
+    }
     const size_t TVg = tg.rows() ? (size_t)64 << tg.jl : (size_t)TXg * TYg * TZg;  // J entries of a tile
     const size_t req_bytes = tg.rows() ? (size_t)tg.reqcap * sizeof(uint16_t)
                              : tg.fam == cc3d_amd_batch::FAM_TALL  ? (size_t)Geo3T::HALO * 4
@@ -3040,8 +3081,8 @@ int cc3d_amd_batch_begin(cc3d_amd_batch* b) {
     ProfScope ps_("k_requests", s);
     for (const auto& tg : b->tgroups) {
       const int order = b->mode == M_MULTI ? BY_XCD : BY_RASTER;
-      if (tg.rows() && tg.jl < 6) launch_rrequests<GeoRN>(tg.gp, tg.tiles, order, s);
-      else if (tg.rows()) launch_rrequests<GeoR>(tg.gp, tg.tiles, order, s);
+      if (tg.rows() && tg.jl < 6) launch_rrequests<GeoRN>(tg.gp, tg.tiles, tg.masks, order, s);
+      else if (tg.rows()) launch_rrequests<GeoR>(tg.gp, tg.tiles, tg.masks, order, s);
       else if (tg.fam == cc3d_amd_batch::FAM_TALL) launch_requests<Geo3T, Q_NONE>(tg.gp, tg.tiles, b->mode, s);
       else if (tg.fam == cc3d_amd_batch::FAM_PLANE) launch_requests<Geo2, Q_NONE>(tg.gp, tg.tiles, b->mode, s);
       else launch_requests<Geo3, Q_NONE>(tg.gp, tg.tiles, b->mode, s);

@@ -145,19 +145,26 @@ __device__ inline void rel_decode(uint32_t r, int& dx, int& dy, int& dz) {
 // mask at 8: 801 and 813 us).
 __host__ constexpr int row_pitch(int64_t sx) { return sx <= 16 ? 4 : sx <= 32 ? 5 : 6; }
 
+// Whether a tile's requests may be link masks (see there).
+__host__ __device__ constexpr bool row_masks(bool cont, int nb) { return cont && (nb == 26 || nb == 18); }
+
 // Bound on the requests of a tile.  Multilabel and binary: the largest number
 // of kept relations that leave the tile, over every set of links a voxel can
 // have, summed over the tile's voxels (4,036 at 26-connectivity, 2,537 at
-// 18, 1,088 at 6).  Continuous volumes and planes: all relations that leave
-// the tile (382 in a plane).  Narrow tiles have no neighbour in x: what is left
-// is the sum over a column of 64 rows (60, 38, 16; continuous 138, 78, 16; 3
-// in a plane).  Never below the 128 that the union kernels load unasked.
+// 18, 1,088 at 6).  Narrow tiles have no neighbour in x: what is left is the
+// sum over a column of 64 rows (60, 38, 16).  Planes and 6-connected continuous
+// volumes: all relations that leave the tile (382 in a plane).  Continuous
+// links at 26 and 18 could leave 9,316 and 5,280, but only in a lattice made for
+// it (noise at its worst tolerance leaves 2,520): there a tile has 1,024 entries
+// per segment, and one that says which segments hold link masks instead (in
+// 16 bytes).  Never below the 128 that the union kernels load unasked.
 __host__ __device__ constexpr int row_req_cap(bool cont, int nb, int jl) {
+  if (row_masks(cont, nb)) return (64 << jl) + 8;
   if (jl < 6) {
-    const int n = (nb == 8 || nb == 4 ? 3 : nb == 6 ? 16 : nb == 18 ? (cont ? 78 : 38) : (cont ? 138 : 60)) << jl;
+    const int n = (nb == 8 || nb == 4 ? 3 : nb == 6 ? 16 : nb == 18 ? 38 : 60) << jl;
     return n < 128 ? 128 : n;
   }
-  return nb == 8 || nb == 4 ? 384 : nb == 6 ? 1088 : nb == 18 ? (cont ? 5280 : 2540) : (cont ? 9316 : 4036);
+  return nb == 8 || nb == 4 ? 384 : nb == 6 ? 1088 : nb == 18 ? 2540 : 4036;
 }
 
 // Staged voxel type: 4 bytes for every type up to 4 bytes.  Multilabel 8-byte
@@ -199,6 +206,7 @@ __device__ inline uint32_t half_of(double v) {
 
 constexpr int RSTR = 68;   // row stride of staged values and nodes: 16-byte accesses of 64 rows spread over all banks
 constexpr int PSTR = 704;  // plane stride of staged values: 10 rows, and 24 more so that planes start on the same bank
+constexpr uint32_t SLOW = 0x8000u;
 constexpr int RQCAP = 1024;  // queued links per wave; one relation of a wave's segments always fits
 
 // LDS index of a tile voxel's node: raster order, or for the binary 2D
@@ -230,7 +238,10 @@ struct RowLds {
     uint16_t fb[G::NROWS][6];
     Work w;
   } u;
-  uint16_t ne0[4];  // binary 2D-4: values of the plane's first row that differ from the one before
+  // binary 2D-4: values of the plane's first row that differ from the one
+  // before; continuous volumes: bound on the wave's requests (SLOW: more links
+  // than its queue holds)
+  uint16_t ne0[4];
   uint32_t nreq;
   uint32_t wtot[4], red_epl[4], red_prov[4];
   uint64_t rows[4];
@@ -829,9 +840,11 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
       }
     }
   };
-  // the n queued links of the wave, one per lane
+  // the n queued links of the wave, one per lane; those that leave the tile are
+  // appended to its list if that is asked for
   uint16_t* REQt = reinterpret_cast<uint16_t*>(p.REQ) + slot * p.reqcap;
-  auto drain = [&](uint32_t n) {
+  constexpr bool MASKS = row_masks(MODE == M_CONT, NB);
+  auto drain = [&](uint32_t n, bool append) {
     for (uint32_t i0 = 0; i0 < n; i0 += 64) {
       const uint32_t i = i0 + (uint32_t)lane;
       bool out = false;
@@ -846,7 +859,7 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
         if (!out)
           runion(par, row_node<QK>(ps & 63u, ps >> 6), row_node<QK>((uint32_t)x, (uint32_t)(y + G::TY * z)));
       }
-      const uint64_t m = wave_ballot(out);
+      const uint64_t m = wave_ballot(out && append);
       if (m) {
         uint32_t b = 0;
         if (lane == 0) b = atomicAdd(&L.nreq, (uint32_t)__builtin_popcountll(m));
@@ -858,16 +871,59 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
   const uint32_t incl = wave_incl_add(cnt);
   const uint32_t total = wave_lane63(incl);
   if (total <= RQCAP) emit(queue + (incl - cnt), U[R_A]);
+  if constexpr (MASKS) {
+    uint32_t bound = total;
+    if (total > RQCAP) {  // the links that leave the tile
+      bound = U[R_A];
+#pragma unroll
+      for (int i = 0; i < 2 * NWORD; i++) {
+        constexpr uint32_t ALL = 0xFFFFu;
+        const Off o = rel_off(i);
+        const uint32_t face = (o.dz < 0 && lz == 0) || (o.dy < 0 && ly == 0) || (o.dy > 0 && ly == G::TY - 1) ? ALL : 0u;
+        const uint32_t side = (o.dx < 0 && first ? 1u : 0u) | (o.dx > 0 && seg == 3 ? 0x8000u : 0u);
+        bound += (uint32_t)__popc((W[i >> 1] >> (16 * (i & 1))) & (face | side));
+      }
+      bound = SLOW | wave_lane63(wave_incl_add(bound));
+    }
+    if (lane == 0) L.ne0[seg] = (uint16_t)bound;
+  }
   __syncthreads();
 
   // 4. unions and requests
+  // segments whose links are stored as masks: none unless the list may be too short
+  auto masked_segments = [&]() -> uint32_t {
+    uint32_t sum = 0, m = 0;
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+      const uint32_t b = L.ne0[w];
+      sum += b & (SLOW - 1u);
+      m |= b & SLOW ? 1u << w : 0u;
+    }
+    return sum <= 64u << G::jlog(p.jl) ? 0u : m;
+  };
   if (total <= RQCAP) {
-    drain(total);
+    drain(total, true);
   } else {
     // more links than the queue holds: one relation at a time
     uint32_t keep[6];
 #pragma unroll
     for (int i = 0; i < 6; i++) keep[i] = W[i];
+    const uint32_t masked = MASKS ? masked_segments() : 0u;
+    if (MASKS && masked) {
+      // link masks: 13 bits per voxel of the segment, relation r in bit r, row by
+      // row; the first such segment at the end of the tile's entries, the next
+      // before it.  The list needs no more than the other segments' places.
+      const uint32_t at = (64u << G::jlog(p.jl)) - 1024u * (uint32_t)__popc(masked & ((2u << seg) - 1u));
+      uint16_t* d = REQt + at + 16 * lane;
+#pragma unroll 1
+      for (int k = 0; k < 16; k++) {
+        uint32_t m = ((U[R_A] >> k) & 1u) << R_A;
+#pragma unroll
+        for (int i = 0; i < NWORD; i++)
+          m |= (((keep[i] >> k) & 1u) << (2 * i)) | (((keep[i] >> (16 + k)) & 1u) << (2 * i + 1));
+        d[k] = (uint16_t)m;
+      }
+    }
 #pragma unroll 1
     for (int r = 0; r <= 2 * NWORD; r++) {
       uint32_t c = 0;
@@ -881,7 +937,7 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
       const uint32_t inc = wave_incl_add(c);
       emit(queue + (inc - c), ua);
       wave_order();
-      drain(wave_lane63(inc));
+      drain(wave_lane63(inc), masked == 0);
       wave_order();
     }
   }
@@ -1025,6 +1081,11 @@ __device__ inline void rows_tile(const LocalParams& p, const T* in, int64_t sx, 
     }
     p.TR[slot] = R;
     p.TQ[slot] = L.nreq;
+    if constexpr (MODE == M_CONT && IS3D) {
+      // 6-connected volumes of a batch with others say it too
+      const int n = 64 << G::jlog(p.jl);
+      if (MASKS || p.reqcap > n) REQt[n] = (uint16_t)(MASKS ? masked_segments() : 0u);
+    }
     TileCnt c;
     c.epl = e;
     c.prov = pv;

@@ -51,3 +51,11 @@ def test_narrow_batches():
     assert 0 < got <= 8.25 * voxels + tiles * VOXEL_TILE + (1 << 20)
   table[n - 1].sx = 33
   assert lib.cc3d_amd_batch_workspace_bytes(table, n, L.BATCH_MULTILABEL) > got + tiles * 8192
+
+
+@pytest.mark.parametrize("connectivity", [6, 18, 26])
+def test_continuous_volumes(connectivity):
+  from cc3d import _lib as L
+  for sx in WIDTHS:
+    for sy, sz in ((2, 2), (7, 100), (64, 64), (100, 3), (333, 2000), (1, 5000), (5000, 5)):
+      _check(sx, sy, sz, connectivity, 0, L.FLAG_CONTINUOUS)
