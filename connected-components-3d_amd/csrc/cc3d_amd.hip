@@ -1654,9 +1654,17 @@ static void free_pinned_counters(const PinnedCounters& p) {
   if (p.c) (void)hipHostFree(p.c);
 }
 
-static PinnedCounters pinned_counters() {
+// For jobs on stream s: an event is recorded on streams of its own device only,
+// which need not be the calling thread's.
+static PinnedCounters pinned_counters(hipStream_t s) {
   PinnedCounters p;
-  if (hipGetDevice(&p.dev) != hipSuccess) return PinnedCounters();
+  int current = -1;
+  if (hipGetDevice(&current) != hipSuccess) return PinnedCounters();
+  p.dev = current;
+  if (s && hipStreamGetDevice(s, &p.dev) != hipSuccess) {
+    (void)hipGetLastError();
+    p.dev = current;
+  }
   {
     std::lock_guard<std::mutex> g(g_pin_mu);
     for (size_t i = g_pin_pool.size(); i-- > 0;) {
@@ -1666,9 +1674,13 @@ static PinnedCounters pinned_counters() {
       return p;
     }
   }
-  if (hipHostMalloc(reinterpret_cast<void**>(&p.c), sizeof(Counters), hipHostMallocCoherent) != hipSuccess ||
-      hipHostGetDevicePointer(reinterpret_cast<void**>(&p.dev_c), p.c, 0) != hipSuccess ||
-      hipEventCreateWithFlags(&p.ready, hipEventDisableTiming) != hipSuccess) {
+  if (p.dev != current && hipSetDevice(p.dev) != hipSuccess) return PinnedCounters();
+  const bool made =
+    hipHostMalloc(reinterpret_cast<void**>(&p.c), sizeof(Counters), hipHostMallocCoherent) == hipSuccess &&
+    hipHostGetDevicePointer(reinterpret_cast<void**>(&p.dev_c), p.c, 0) == hipSuccess &&
+    hipEventCreateWithFlags(&p.ready, hipEventDisableTiming) == hipSuccess;
+  if (p.dev != current) (void)hipSetDevice(current);
+  if (!made) {
     free_pinned_counters(p);
     return PinnedCounters();
   }
@@ -2268,7 +2280,7 @@ static int job_begin(cc3d_amd_job* j, const void* in, int in_dtype, int64_t sx, 
     j->h_ctr = &j->h_ctr_local;
     j->ctr_local = true;
   } else {
-    j->pin = pinned_counters();
+    j->pin = pinned_counters(j->stream);
     j->h_ctr = j->pin.c;
     if (!j->h_ctr) return fail(CC3D_AMD_ERR_NOMEM, "could not allocate pinned counters");
     // a captured launch would write the pooled buffer again at every replay,
