@@ -105,6 +105,12 @@ def _label_volume(out_labels):
   return buf, code, sx, sy, sz, ndim, int(order == "F"), N
 
 
+# 16-bit boxes of more coordinates than this are narrowed on the device, half the
+# bytes to copy; below, the launch costs more (10 labels 23 us on the device and
+# 15 on the host, 8,000 33 and 34, 40,000 49 and 121).
+_NARROW_ON_DEVICE = 48000
+
+
 def statistics(out_labels, no_slice_conversion: bool = False) -> dict:
   """Voxel counts, bounding boxes and centroids per label (cc3d/fastcc3d.pyx:681-938).
 
@@ -121,13 +127,16 @@ def statistics(out_labels, no_slice_conversion: bool = False) -> dict:
   nd = 2 if ndim == 2 else 3
   counts = _to_numpy(counts, np.uint32)
   big = max(sx, sy, sz) > np.iinfo(np.uint16).max
-  if not big:  # 16-bit boxes: narrowed on the device, half the bytes to copy
+  if not big and bbox.numel() > _NARROW_ON_DEVICE:
     torch = _torch()
     narrow = torch.empty(bbox.numel(), dtype=torch.int16, device=bbox.device)
     _fcheck(_bind().cc3d_amd_narrow_boxes(ctypes.c_void_p(bbox.data_ptr()), bbox.numel(),
                                           ctypes.c_void_p(narrow.data_ptr()), _stream()))
-    bbox = narrow
-  bb = _to_numpy(bbox, np.uint32 if big else np.uint16).reshape((N + 1, 2 * nd))
+    bb = _to_numpy(narrow, np.uint16)
+  else:
+    bb = _to_numpy(bbox, np.uint32)
+    bb = bb if big else np.minimum(bb, np.iinfo(np.uint16).max).astype(np.uint16)
+  bb = bb.reshape((N + 1, 2 * nd))
   cen = _to_numpy(cen, np.float64).reshape((N + 1, nd))
   output = {"voxel_counts": counts, "bounding_boxes": bb, "centroids": cen}
   if no_slice_conversion:
