@@ -360,7 +360,10 @@ def _decide(pl, st):
 def _known_out_dtype(pl):
   """The output dtype when it does not depend on the labels, else None: given
   by the caller, chosen from the voxel count alone (binary_image=True), or
-  uint16 because no estimate can exceed the voxel count."""
+  uint16 because no estimate can exceed the voxel count.  Nor where the volume
+  is a single row, whose labels come from its runs (_special_row)."""
+  if pl.sy * pl.sz == 1 and pl.delta == 0 and not pl.binary_flag_given:
+    return None
   if pl.out_dtype is not None:
     return pl.out_dtype
   if pl.binary_flag_given:
