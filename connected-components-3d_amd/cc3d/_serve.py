@@ -20,7 +20,8 @@ Scheduling:
   * every result is identical to labelling the request alone.
 
 Footprint of a request: at admission, the labelling workspace + uint32 labels
-+ the dusted copy.  Once the labelling has returned N, the workspace is given
++ the dusted copy; a batch whose shared workspace takes more than its members'
+own reserves the difference too.  Once the labelling has returned N, the workspace is given
 back and the per-label outputs (voxel counts and bounding boxes, 28 bytes for
 each of N + 1 labels) are reserved in its place; when they need more than the
 workspace gave back, the worker waits for the difference, unless no other
@@ -59,6 +60,7 @@ class Request:
     self.error: Optional[BaseException] = None
     self.done = threading.Event()
     self.footprint = 0
+    self.workspace = 0  # the part of the footprint that labelling takes
     self.batched_with = 1
     self.ready = None
     self.keep = True
@@ -76,6 +78,12 @@ def request_footprint(volume, connectivity: int) -> int:
 def _workspace(volume, connectivity: int) -> int:
   sx, sy, sz = _dims(volume)
   return int(L.lib().cc3d_amd_workspace_bytes(sx, sy, sz, connectivity, 0, 0))
+
+
+def _batch_workspace(requests) -> int:
+  table = (L.Volume * len(requests))(*[L.Volume(r.volume.data_ptr(), *_dims(r.volume), r.connectivity)
+                                       for r in requests])
+  return int(L.lib().cc3d_amd_batch_workspace_bytes(table, len(requests), L.BATCH_MULTILABEL))
 
 
 def _outputs(volume) -> int:
@@ -147,6 +155,7 @@ class LabelServer:
     r.ready = _torch().cuda.Event()
     r.ready.record()  # the volume's producers on the caller's stream come first
     r.keep = bool(keep)
+    r.workspace = _workspace(volume, connectivity)
     r.footprint = request_footprint(volume, connectivity)
     if r.footprint > self.budget:
       r.error = MemoryError(f"request needs {r.footprint} bytes of HBM; the budget is {self.budget}")
@@ -189,7 +198,13 @@ class LabelServer:
         keep = collections.deque()
         while self.waiting and len(group) < self.max_batch:
           r = self.waiting.popleft()
-          if self._small(r) and r.footprint <= self.free and r.volume.dtype == head.volume.dtype:
+          joins = self._small(r) and r.volume.dtype == head.volume.dtype
+          # the volumes of a batch share tiles and request lists of one size: what
+          # the batch takes beyond its members' own workspaces is the last one's
+          extra = max(0, _batch_workspace(group + [r]) - sum(q.workspace for q in group) - r.workspace) if joins else 0
+          if joins and r.footprint + extra <= self.free:
+            r.workspace += extra
+            r.footprint += extra
             self.free -= r.footprint
             self._note()
             group.append(r)
@@ -210,10 +225,10 @@ class LabelServer:
       self.stats_waiters += len(group)
       self.cv.notify_all()
       for r, n in zip(group, ns):
-        ws = _workspace(r.volume, r.connectivity)
         stats = _STAT_BYTES_PER_LABEL * (n + 1)
-        self.free += ws
-        r.footprint -= ws
+        self.free += r.workspace
+        r.footprint -= r.workspace
+        r.workspace = 0
         while stats > self.free and self.active > self.stats_waiters:
           self.cv.wait()
         self.free -= stats
