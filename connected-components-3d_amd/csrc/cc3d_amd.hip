@@ -179,12 +179,12 @@ struct GlobalParams {
   const int64_t* vtile0;
   const uint32_t* vix;
   int nvol;
+  int in_order;  // stage 2 takes the tiles in raster order
   // single volume (nvol == 0) placed at a tile and key offset: one volume of
   // a batch addressed on its own (its periodic unions)
   int64_t tile0;
   uint32_t key0;
   int jl;  // row tiles: 2^jl J entries per row (row_pitch)
-  int in_order;  // stage 2 takes the tiles in raster order
 };
 
 // Geometry of the volume owning batch tile `slot`.
@@ -582,10 +582,10 @@ __device__ inline void kunion_wave(uint2* GP, uint32_t* bits, uint32_t a, uint32
 // raster 37 us, by XCD 38; 293^3 45 and 68). Multilabel batches go by XCD: a
 // volume's unions stay on one (16 masks of 256^3, p = 0.3: 315 us, raster 510;
 // volumes of 64 to 256 and mixed connectivities 187, raster 155).
-constexpr int64_t ORDER_TILES = 4096;
-enum : int { BY_RASTER, BY_XCD, BY_SPREAD };
 //
 // MASKS: links may be stored as masks too (continuous volumes), one voxel a lane.
+constexpr int64_t ORDER_TILES = 4096;
+enum : int { BY_RASTER, BY_XCD, BY_SPREAD };
 template <class G, bool MASKS>
 __global__ __launch_bounds__(WG) void k_rrequests(GlobalParams p, int order) {
   __shared__ uint2 tab[WG / 64][RRQ_SLOTS];
@@ -967,7 +967,7 @@ __global__ __launch_bounds__(WG) void k_scan_bc(const uint32_t* bits, int64_t nw
 // One launch for small bitmasks: each block counts the words before its own
 // 4096 itself (four rounds of eight 16-byte loads per thread at the limit, from
 // L2), and block nblk folds the counters, 16 tiles per thread at the limit. On
-// 64^3 voxels (2 blocks) k_tile_counters, k_scan_a and k_scan_bc of their own
+// 64^3 voxels (2 blocks) a counter kernel, k_scan_a and k_scan_bc of their own
 // took 3.8 + 3.8 + 2.8 us and a copy of the counters 2.2 more; this takes 4.6.
 constexpr int SCAN1_NT = 1024;
 constexpr int64_t SCAN1_MAX = 32, SCAN1_TILES = 16 * SCAN1_NT;
@@ -1932,11 +1932,10 @@ struct cc3d_amd_batch {
   BatchVol* h_tab = nullptr;  // pinned host copy of the volume table
   int64_t* h_t0 = nullptr;    // pinned: first tile of each volume, per tile group (n + tile groups)
   Counters* h_ctr = nullptr;  // pinned: entry 0 whole batch, 1 + k table entry k
-  // The table holds the volumes grouped by connectivity (one local launch
-  // per group, 26 and 18 first); perm[k] is the caller's index of table
-  // entry k.  The volumes of a tile group share one tile geometry and their
-  // per-tile arrays: 26- and 18-connected volumes the voxel tiles (Geo3),
-  // 6-connected ones the row tiles (GeoR).  Tiles are numbered from 0 within
+  // The table holds the volumes grouped by tile family (row tiles by default)
+  // and connectivity (one local launch per group, 26 and 18 first); perm[k] is
+  // the caller's index of table entry k.  The volumes of a tile group share one
+  // tile geometry and their per-tile arrays.  Tiles are numbered from 0 within
   // their tile group; the key space, bitmask and counters are shared.
   struct Group {
     int nb, tg;
@@ -2716,9 +2715,9 @@ int cc3d_amd_profile_collect(char* names, int name_len, double* total_ms, int* c
 // Volumes of a batch run the single-volume path's kernels on their own tiles.
 // A single plane is labelled on the 3D tiles: its 26/18-neighbourhood within
 // the plane is the 8-neighbourhood and its 6-neighbourhood the
-// 4-neighbourhood, so 8 and 4 map to 26 and 6.  Not covered: binary 2D-8 and
-// 2D-4 (their block and first-row numberings) and continuous 2D-8 (its global
-// min/max rule).
+// 4-neighbourhood, so 8 and 4 map to 26 and 6.  Binary 2D-8 and 2D-4 (their block
+// and first-row numberings) and continuous 2D-8 (its global min/max rule) take
+// the 2D tiles (FAM_PLANE).
 static void batch_tile_dims(int fam, int& TX, int& TY, int& TZ) {
   if (fam == cc3d_amd_batch::FAM_PLANE) {
     TX = Geo2::TX; TY = Geo2::TY; TZ = 1;

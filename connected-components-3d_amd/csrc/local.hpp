@@ -51,7 +51,7 @@
 //                    component
 //   tcnt[tile]       epl transitions, provisional-label count, first/last
 //                    foreground row (cc3d/cc3d.hpp:287-315), folded by
-//                    k_tile_counters (one store per tile: thousands of
+//                    the scan's extra blocks (one store per tile: thousands of
 //                    workgroups atomically updating one address serialise)
 #pragma once
 
@@ -77,7 +77,10 @@ struct LocalParams {
   TileCnt* tcnt;
   uint32_t* spread;      // row tiles: Counters::spread, or null where nothing asks for it
   const uint16_t* utab;  // union tables (UTab), UTAB_TOTAL entries
-  int jl;                // row tiles: 2^jl J entries per row (row_pitch)
+  // row tiles: 2^jl J entries per row (row_pitch); behind the fields that all row
+  // kernels read, since a hole among them splits their loads (16384^2 mask at 8:
+  // 801 and 813 us)
+  int jl;
 };
 
 // Offsets of backward position i in the staged box and in the tile's node

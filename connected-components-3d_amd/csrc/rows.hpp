@@ -42,9 +42,11 @@
 // J8/J16, REQ/TQ, tcnt) are those of the voxel kernel in local.hpp except
 // for the request format; J is row-major: entry x + 2^jl * (y + 8 * z).
 //
-// What bounds it: VALU issue, 1,500 instructions per 1,024-voxel wave and 80 %
-// of the issue slots, of which about a third form the masks and a sixth make
-// the unions; LDS is busy half of the time. Against the kernels it replaced,
+// What bounds it: VALU issue, 1,430 to 1,500 instructions per 1,024-voxel wave and
+// 75 to 85 % of the issue slots for voxels of up to 4 bytes (grey levels 1,975 and
+// 94 %), of which about a third form the masks and a sixth make the unions; LDS is
+// busy 40 to 50 % of the time (8-byte voxels, whose masks are formed by halves:
+// VALU 62 %, LDS 59 %). Against the kernels it replaced,
 // per launch: 512^3 uint32 Voronoi 26 988 -> 390 us, uint64 at 6 1,646 -> 466,
 // float32 grey levels 3,068 -> 440, p = 0.3 mask 26 1,057 -> 357, 16384^2 p =
 // 0.5 mask 8 1,571 -> 809. That is 64 rows of 64 because a wave then reads
@@ -1132,7 +1134,7 @@ __global__ __launch_bounds__(G::NT, (rows_waves<T, MODE>())) void k_rows_local(L
   const int64_t tile = xcd_tile(blockIdx.x, p.ntiles);
   rows_tile<T, MODE, NB, G, Q_NONE>(p, static_cast<const T*>(p.in), p.sx, p.sy, p.sz, p.ntx, p.nty, p.dxy, p.dx, tile,
                                     tile, 0u, L);
-  if (MODE == M_MULTI && p.spread && blockIdx.x == 0 && threadIdx.x < 64)
+  if (MODE == M_MULTI && blockIdx.x == 0 && threadIdx.x < 64 && p.spread)
     label_spread(static_cast<const T*>(p.in), (uint64_t)(p.sx * p.sy * p.sz), p.spread);
 }
 
@@ -1143,7 +1145,7 @@ __global__ __launch_bounds__(G::NT, (rows_waves<T, MODE>())) void k_rows_plane(L
   const int64_t tile = xcd_tile(blockIdx.x, p.ntiles);
   rows_tile<T, MODE, NB, G, QK>(p, static_cast<const T*>(p.in), p.sx, p.sy, 1, p.ntx, p.nty, p.dxy, p.dx, tile, tile,
                                 0u, L);
-  if (MODE == M_MULTI && p.spread && blockIdx.x == 0 && threadIdx.x < 64)
+  if (MODE == M_MULTI && blockIdx.x == 0 && threadIdx.x < 64 && p.spread)
     label_spread(static_cast<const T*>(p.in), (uint64_t)(p.sx * p.sy), p.spread);
 }
 

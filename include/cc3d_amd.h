@@ -109,9 +109,9 @@ typedef struct {
 #define CC3D_AMD_NO_SINGLE_ROW_RULE 4  /* do not mimic the binding's single-row shortcut */
 /* Tile family of the local labelling kernel for 3D volumes (no reference
  * counterpart: a performance choice, results are identical): row tiles
- * (64x8x8, x-runs as union-find nodes), voxel tiles (32x8x8, one node per
- * voxel) or tall voxel tiles (32x16x8, one node per voxel, 512 threads).
- * None: row tiles for 6-connectivity, voxel tiles otherwise. */
+ * (64x8x8, link bit masks of 16-voxel row segments), voxel tiles (32x8x8, one
+ * union-find node per voxel) or tall voxel tiles (32x16x8, one node per voxel,
+ * 512 threads).  None: row tiles. */
 #define CC3D_AMD_TILES_ROWS 8
 #define CC3D_AMD_TILES_VOXELS 16
 #define CC3D_AMD_TILES_TALL 32
